@@ -35,8 +35,10 @@ int fail(int status, const char* fmt, ...) {
 
 bool valid_block(int b) { return b >= 64 && b <= fl::kMaxBlock && (b % 64) == 0; }
 
-int resolve_tuning(const fl_tuning* t, fl_tuning* out) {
+int resolve_tuning(const fl_tuning* t, fl_tuning* out, int32_t* shape) {
   fl_tuning n;
+  if (t && (t->x_block || t->x_rows)) shape[0] = kShapeTuning;
+  if (t && (t->y_block || t->y_rows)) shape[1] = kShapeTuning;
   n.x_block = t && t->x_block ? t->x_block : 256;
   n.x_rows = t && t->x_rows ? t->x_rows : 32;
   n.y_block = t && t->y_block ? t->y_block : 256;
@@ -138,6 +140,8 @@ fl::SweepArgs<T> make_args(const fl_context* ctx, const fl_field* in, const fl_f
   strides(in, a.es, a.cs);
   a.nx = in->n[0];
   a.ny = in->ndim > 1 ? in->n[1] : 1;
+  a.rowb = a.nx * a.es * (int64_t)sizeof(T);
+  a.csb = a.cs * (int64_t)sizeof(T);
   a.mat = make_material<T>(s);
   a.mat64 = make_material<double>(s);
   a.limiter = s->limiter;
@@ -152,7 +156,7 @@ fl::SweepArgs<T> make_args(const fl_context* ctx, const fl_field* in, const fl_f
   return a;
 }
 
-// Rows per workgroup, halved (down to 4) while the launch would have fewer
+// Rows per workgroup of a caller's tuning, halved (down to 4) while the launch would have fewer
 // than kMinWaves waves (1.5 per SIMD of the 1024 on the device): small grids
 // keep the machine filled whatever the tuning says.
 constexpr int64_t kMinWaves = 1536;
@@ -170,10 +174,65 @@ inline bool is_vlc(int limiter, int form) {
   return FL_VLC_KERNELS && limiter == fl::kLimVanLeer && form == fl::kFormCons;
 }
 
+// The launch of one 2D sweep.
+struct SweepShape {
+  bool cell;  // the cell-parallel kernel (block and rows unused)
+  int block;  // lanes per workgroup of the march
+  int rows;   // rows per workgroup of the march
+};
+
+// Cells (of all grids of the launch) up to which the cell-parallel sweeps are
+// the faster ones.
+template <typename T> constexpr int64_t kCellMax = 5 << 17;
+template <> constexpr int64_t kCellMax<float> = 3 << 19;
+
+// Launch shape of the sweep of dimension dim over ngrids grids of nx x ny
+// cells.  By rule: small grids go cell-parallel (a 64^2 FP64 sweep takes 7 us
+// against 16 (x) and 21 us (y) marching; 512^2 17 against 19 and 22; 1024^2
+// 46 and 51 against 41 and 45).  Larger ones march, x in 128-lane workgroups of
+// about 10500 waves and y in 64-lane ones of about 4096 in all: fewer, taller
+// tiles end unevenly, shorter ones pay more warm-up rows (FP64 x at 2048^2: 8
+// rows 133 us, 32 rows 186 us; y at 4096^2: 64 rows 441 us, 22 rows 455 us).
+template <typename T>
+SweepShape pick_shape(const fl_context* ctx, int dim, int64_t nx, int64_t ny, int ngrids) {
+  const fl_tuning& tu = ctx->tuning;
+  if (ctx->shape[dim] == kShapeTuning) {
+    const int B = dim ? tu.y_block : tu.x_block;
+    const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
+    return {false, B, fit_rows(dim ? tu.y_rows : tu.x_rows, ngrids * bands, ny, B)};
+  }
+  if (ctx->shape[dim] == kShapeCell || nx * ny * ngrids <= kCellMax<T>) return {true, 0, 0};
+  const int B = dim ? 64 : 128;
+  const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
+  const int64_t waves = ngrids * bands * (B / 64) * ny;  // of one-row tiles
+  const int64_t fit = dim ? (waves + 4095) / 4096 : (waves + 10499) / 10500;
+  int64_t rows = std::max<int64_t>(dim ? 8 : 6, std::min<int64_t>(dim ? 64 : 32, fit));
+  rows = std::max(rows, (ny + 65534) / 65535);  // tile rows are the launch's y extent
+  return {false, B, (int)rows};
+}
+
+// Workgroups of a sweep: the marching tiles over (x, y), or the cell-parallel
+// ones in one dimension; z (march) or y (cell-parallel) counts the grids.
+dim3 shape_grid(const SweepShape& sh, int dim, int64_t nx, int64_t ny, int ngrids) {
+  if (sh.cell) {
+    const int cols = dim ? fl::kCellYCols : fl::kCellXCols;
+    const int rows = dim ? fl::kCellYRows : fl::kCellXRows;
+    return dim3((unsigned)(((nx + cols - 1) / cols) * ((ny + rows - 1) / rows)), ngrids, 1);
+  }
+  const int B = sh.block;
+  return dim3((unsigned)(dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2)),
+              (unsigned)((ny + sh.rows - 1) / sh.rows), ngrids);
+}
+
 template <typename T, int FLUX, bool FAST, bool VLC>
-void launch_flux_v(int ndim, int dim, dim3 grid, int B, const fl::SweepArgs<T>& a,
+void launch_flux_v(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a,
                    hipStream_t stream) {
-  if (ndim == 1)
+  const int B = sh.block;
+  if (sh.cell) {
+    auto k = dim == 0 ? fl::cell_x_kernel<T, FLUX, FAST, VLC> : fl::cell_y_kernel<T, FLUX, FAST, VLC>;
+    hipLaunchKernelGGL(k, grid, dim3(64 * fl::kCellWaves), fl::cell_tile_lds_bytes(sizeof(T)),
+                       stream, a, a);
+  } else if (ndim == 1)
     hipLaunchKernelGGL((fl::sweep_x_kernel<T, 1, FLUX, FAST, VLC>), grid, dim3(B),
                        fl::x_tile_lds_bytes(B, 3, sizeof(T)), stream, a);
   else if (dim == 0)
@@ -186,15 +245,15 @@ void launch_flux_v(int ndim, int dim, dim3 grid, int B, const fl::SweepArgs<T>& 
 
 // One sweep kernel of flux FLUX: the 1D sweep, or the x or y sweep of a 2D grid.
 template <typename T, int FLUX, bool FAST>
-void launch_flux(int ndim, int dim, dim3 grid, int B, const fl::SweepArgs<T>& a,
+void launch_flux(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a,
                  hipStream_t stream) {
   if constexpr (has_vlc<FLUX>()) {
     if (is_vlc(a.limiter, a.form)) {
-      launch_flux_v<T, FLUX, FAST, true>(ndim, dim, grid, B, a, stream);
+      launch_flux_v<T, FLUX, FAST, true>(ndim, dim, grid, sh, a, stream);
       return;
     }
   }
-  launch_flux_v<T, FLUX, FAST, false>(ndim, dim, grid, B, a, stream);
+  launch_flux_v<T, FLUX, FAST, false>(ndim, dim, grid, sh, a, stream);
 }
 
 // The fast FP64 numerics were requested (FP32 sweeps use them always).
@@ -257,15 +316,15 @@ std::vector<int> row_candidates(const int* base, int nbase, int64_t bands, int64
 }
 
 template <typename T, bool FAST>
-void launch_flux_t(int flux, int ndim, int dim, dim3 grid, int B, const fl::SweepArgs<T>& a,
-                   hipStream_t stream) {
+void launch_flux_t(int flux, int ndim, int dim, dim3 grid, const SweepShape& sh,
+                   const fl::SweepArgs<T>& a, hipStream_t stream) {
   switch (flux) {
-    case FL_FLUX_HLLC: launch_flux<T, fl::kFluxHllc, FAST>(ndim, dim, grid, B, a, stream); break;
-    case FL_FLUX_FORCE: launch_flux<T, fl::kFluxForce, FAST>(ndim, dim, grid, B, a, stream); break;
+    case FL_FLUX_HLLC: launch_flux<T, fl::kFluxHllc, FAST>(ndim, dim, grid, sh, a, stream); break;
+    case FL_FLUX_FORCE: launch_flux<T, fl::kFluxForce, FAST>(ndim, dim, grid, sh, a, stream); break;
     case FL_FLUX_LAX_FRIEDRICHS:
-      launch_flux<T, fl::kFluxLaxFriedrichs, FAST>(ndim, dim, grid, B, a, stream);
+      launch_flux<T, fl::kFluxLaxFriedrichs, FAST>(ndim, dim, grid, sh, a, stream);
       break;
-    default: launch_flux<T, fl::kFluxRichtmyer, FAST>(ndim, dim, grid, B, a, stream); break;
+    default: launch_flux<T, fl::kFluxRichtmyer, FAST>(ndim, dim, grid, sh, a, stream); break;
   }
 }
 
@@ -273,33 +332,19 @@ template <typename T>
 int launch_sweep_t(const fl_context* ctx, const fl_field* in, const fl_field* out, int dim,
                    const fl_scheme* s, double dtdh, const fl::StepCtl* ctl,
                    unsigned long long* ws_out, hipStream_t stream) {
-  fl_tuning tu = ctx->tuning;
-  if (in->ndim == 2) {
-    const int64_t nx = in->n[0], ny = in->n[1];
-    tu.x_rows = fit_rows(tu.x_rows, (nx + tu.x_block - 3) / (tu.x_block - 2), ny, tu.x_block);
-    tu.y_rows = fit_rows(tu.y_rows, (nx + tu.y_block - 1) / tu.y_block, ny, tu.y_block);
-  }
   dim3 grid;
-  int B;
-  fl::SweepArgs<T> a;
+  SweepShape sh{false, ctx->tuning.x_block, 1};
   if (in->ndim == 1) {
-    B = tu.x_block;
-    a = make_args<T>(ctx, in, out, s, dtdh, ctl, ws_out, 1);
-    grid = dim3((unsigned)((a.nx + (B - 3)) / (B - 2)), 1, 1);
-  } else if (dim == 0) {
-    B = tu.x_block;
-    a = make_args<T>(ctx, in, out, s, dtdh, ctl, ws_out, tu.x_rows);
-    grid = dim3((unsigned)((a.nx + (B - 3)) / (B - 2)),
-                (unsigned)((a.ny + tu.x_rows - 1) / tu.x_rows), 1);
+    grid = dim3((unsigned)((in->n[0] + (sh.block - 3)) / (sh.block - 2)), 1, 1);
   } else {
-    B = tu.y_block;
-    a = make_args<T>(ctx, in, out, s, dtdh, ctl, ws_out, tu.y_rows);
-    grid = dim3((unsigned)((a.nx + B - 1) / B), (unsigned)((a.ny + tu.y_rows - 1) / tu.y_rows), 1);
+    sh = pick_shape<T>(ctx, dim, in->n[0], in->n[1], 1);
+    grid = shape_grid(sh, dim, in->n[0], in->n[1], 1);
   }
+  const fl::SweepArgs<T> a = make_args<T>(ctx, in, out, s, dtdh, ctl, ws_out, sh.rows);
   if (std::is_same<T, double>::value && fast_numerics(s))
-    launch_flux_t<T, true>(s->flux, in->ndim, dim, grid, B, a, stream);
+    launch_flux_t<T, true>(s->flux, in->ndim, dim, grid, sh, a, stream);
   else
-    launch_flux_t<T, false>(s->flux, in->ndim, dim, grid, B, a, stream);
+    launch_flux_t<T, false>(s->flux, in->ndim, dim, grid, sh, a, stream);
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
@@ -317,9 +362,14 @@ int launch_sweep(const fl_context* ctx, const fl_field* in, const fl_field* out,
 // methods must be equal (the launch instantiates one), else each grid is
 // swept on its own.
 template <typename T, int FLUX, bool FAST, bool VLC>
-void launch_flux2_v(int ndim, int dim, dim3 grid, int B, const fl::SweepArgs<T>& a0,
+void launch_flux2_v(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a0,
                     const fl::SweepArgs<T>& a1, hipStream_t stream) {
-  if (ndim == 1)
+  const int B = sh.block;
+  if (sh.cell) {
+    auto k = dim == 0 ? fl::cell_x_kernel<T, FLUX, FAST, VLC> : fl::cell_y_kernel<T, FLUX, FAST, VLC>;
+    hipLaunchKernelGGL(k, grid, dim3(64 * fl::kCellWaves), fl::cell_tile_lds_bytes(sizeof(T)),
+                       stream, a0, a1);
+  } else if (ndim == 1)
     hipLaunchKernelGGL((fl::sweep_x2_kernel<T, 1, FLUX, FAST, VLC>), grid, dim3(B),
                        fl::x_tile_lds_bytes(B, 3, sizeof(T)), stream, a0, a1);
   else if (dim == 0)
@@ -332,62 +382,50 @@ void launch_flux2_v(int ndim, int dim, dim3 grid, int B, const fl::SweepArgs<T>&
 
 // fast: the fast FP64 numerics (FP64 only; the FP32 kernels have their own)
 template <typename T, int FLUX>
-void launch_flux2(int ndim, int dim, dim3 grid, int B, const fl::SweepArgs<T>& a0,
+void launch_flux2(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a0,
                   const fl::SweepArgs<T>& a1, bool fast, hipStream_t stream) {
   const bool vlc = has_vlc<FLUX>() && is_vlc(a0.limiter, a0.form) && is_vlc(a1.limiter, a1.form);
   if constexpr (std::is_same<T, double>::value) {
     if (fast) {
       if constexpr (has_vlc<FLUX>())
-        if (vlc) return launch_flux2_v<T, FLUX, true, true>(ndim, dim, grid, B, a0, a1, stream);
-      return launch_flux2_v<T, FLUX, true, false>(ndim, dim, grid, B, a0, a1, stream);
+        if (vlc) return launch_flux2_v<T, FLUX, true, true>(ndim, dim, grid, sh, a0, a1, stream);
+      return launch_flux2_v<T, FLUX, true, false>(ndim, dim, grid, sh, a0, a1, stream);
     }
   }
   if constexpr (has_vlc<FLUX>())
-    if (vlc) return launch_flux2_v<T, FLUX, false, true>(ndim, dim, grid, B, a0, a1, stream);
-  launch_flux2_v<T, FLUX, false, false>(ndim, dim, grid, B, a0, a1, stream);
+    if (vlc) return launch_flux2_v<T, FLUX, false, true>(ndim, dim, grid, sh, a0, a1, stream);
+  launch_flux2_v<T, FLUX, false, false>(ndim, dim, grid, sh, a0, a1, stream);
 }
 
 template <typename T>
 int launch_sweep2_t(const fl_context* ctx, const fl_field* const in[2],
                     const fl_field* const out[2], int dim, const fl_scheme* const s[2],
                     double dtdh, hipStream_t stream, const fl::StepCtl* ctl) {
-  fl_tuning tu = ctx->tuning;
   const fl_field* f = in[0];
-  int rows = 0, B;
   dim3 grid;
+  SweepShape sh{false, ctx->tuning.x_block, 1};
   if (f->ndim == 1) {
-    B = tu.x_block;
-    grid = dim3((unsigned)((f->n[0] + (B - 3)) / (B - 2)), 1, 2);
+    grid = dim3((unsigned)((f->n[0] + (sh.block - 3)) / (sh.block - 2)), 1, 2);
   } else {
-    const int64_t nx = f->n[0], ny = f->n[1];
-    // the waves of both grids count towards filling the machine
-    if (dim == 0) {
-      B = tu.x_block;
-      rows = fit_rows(tu.x_rows, 2 * ((nx + B - 3) / (B - 2)), ny, B);
-      grid = dim3((unsigned)((nx + B - 3) / (B - 2)), (unsigned)((ny + rows - 1) / rows), 2);
-    } else {
-      B = tu.y_block;
-      rows = fit_rows(tu.y_rows, 2 * ((nx + B - 1) / B), ny, B);
-      grid = dim3((unsigned)((nx + B - 1) / B), (unsigned)((ny + rows - 1) / rows), 2);
-    }
+    // the cells of both grids count towards filling the machine
+    sh = pick_shape<T>(ctx, dim, f->n[0], f->n[1], 2);
+    grid = shape_grid(sh, dim, f->n[0], f->n[1], 2);
   }
-  const fl::SweepArgs<T> a0 = make_args<T>(ctx, in[0], out[0], s[0], dtdh, ctl, nullptr,
-                                           f->ndim == 1 ? 1 : rows);
-  const fl::SweepArgs<T> a1 = make_args<T>(ctx, in[1], out[1], s[1], dtdh, ctl, nullptr,
-                                           f->ndim == 1 ? 1 : rows);
+  const fl::SweepArgs<T> a0 = make_args<T>(ctx, in[0], out[0], s[0], dtdh, ctl, nullptr, sh.rows);
+  const fl::SweepArgs<T> a1 = make_args<T>(ctx, in[1], out[1], s[1], dtdh, ctl, nullptr, sh.rows);
   const bool fast = fast_numerics(s[0]);
   switch (s[0]->flux) {
     case FL_FLUX_HLLC:
-      launch_flux2<T, fl::kFluxHllc>(f->ndim, dim, grid, B, a0, a1, fast, stream);
+      launch_flux2<T, fl::kFluxHllc>(f->ndim, dim, grid, sh, a0, a1, fast, stream);
       break;
     case FL_FLUX_FORCE:
-      launch_flux2<T, fl::kFluxForce>(f->ndim, dim, grid, B, a0, a1, fast, stream);
+      launch_flux2<T, fl::kFluxForce>(f->ndim, dim, grid, sh, a0, a1, fast, stream);
       break;
     case FL_FLUX_LAX_FRIEDRICHS:
-      launch_flux2<T, fl::kFluxLaxFriedrichs>(f->ndim, dim, grid, B, a0, a1, fast, stream);
+      launch_flux2<T, fl::kFluxLaxFriedrichs>(f->ndim, dim, grid, sh, a0, a1, fast, stream);
       break;
     default:
-      launch_flux2<T, fl::kFluxRichtmyer>(f->ndim, dim, grid, B, a0, a1, fast, stream);
+      launch_flux2<T, fl::kFluxRichtmyer>(f->ndim, dim, grid, sh, a0, a1, fast, stream);
       break;
   }
   FL_HIP(hipGetLastError());
@@ -628,7 +666,7 @@ int fl_ctx_create(int device, fl_context** out) {
   fl_context* c = new fl_context();
   memset(c, 0, sizeof(*c));
   c->device = device;
-  (void)resolve_tuning(nullptr, &c->tuning);
+  (void)resolve_tuning(nullptr, &c->tuning, c->shape);
   hipError_t e = hipMalloc((void**)&c->ctl, sizeof(fl::StepCtl));
   if (e == hipSuccess) e = hipMalloc((void**)&c->ws_tmp, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMalloc((void**)&c->partial, sizeof(double) * kSumBlocks * 4);
@@ -678,9 +716,12 @@ int fl_ctx_set_tuning(fl_context* c, const fl_tuning* t) {
   if (t->x_rows) n.x_rows = t->x_rows;
   if (t->y_block) n.y_block = t->y_block;
   if (t->y_rows) n.y_rows = t->y_rows;
-  int rc = resolve_tuning(&n, &n);
+  int32_t unused[2];
+  int rc = resolve_tuning(&n, &n, unused);
   if (rc) return rc;
   c->tuning = n;
+  if (t->x_block || t->x_rows) c->shape[0] = kShapeTuning;
+  if (t->y_block || t->y_rows) c->shape[1] = kShapeTuning;
   return FL_OK;
 }
 
@@ -708,9 +749,26 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
   FL_HIP(hipEventCreate(&e0));
   FL_HIP(hipEventCreate(&e1));
   const fl_tuning saved = c->tuning;
+  const int32_t saved_shape[2] = {c->shape[0], c->shape[1]};
   fl_tuning best = c->tuning;
+  // the sweep with the context's current shape: milliseconds over reps launches
+  auto timed = [&](int dim, float* total) -> int {
+    int err = FL_OK;
+    *total = 0.0f;
+    for (int r = 0; r <= reps && !err; ++r) {  // r = 0 warms up
+      if (hipEventRecord(e0, st) != hipSuccess) err = fail(FL_ERR_HIP, "hipEventRecord");
+      if (!err) err = launch_sweep(c, in, work, dim, s, 1e-3, nullptr, nullptr, st);
+      if (!err && hipEventRecord(e1, st) != hipSuccess) err = fail(FL_ERR_HIP, "hipEventRecord");
+      if (!err && hipEventSynchronize(e1) != hipSuccess) err = fail(FL_ERR_HIP, "hipEventSynchronize");
+      float ms = 0.0f;
+      if (!err) (void)hipEventElapsedTime(&ms, e0, e1);
+      if (r > 0) *total += ms;
+    }
+    return err;
+  };
   for (int dim = 0; dim < in->ndim && !rc; ++dim) {
     float best_ms = 1e30f;
+    if (in->ndim == 2) c->shape[dim] = kShapeTuning;
     for (int w : widths) {
       std::vector<int> rows(1, 0);  // 1D: the height is unused
       if (in->ndim == 2) {
@@ -731,26 +789,26 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
         }
         c->tuning = t;
         float total = 0.0f;
-        for (int r = 0; r <= reps && !rc; ++r) {  // r = 0 warms up
-          if (hipEventRecord(e0, st) != hipSuccess) rc = fail(FL_ERR_HIP, "hipEventRecord");
-          if (!rc) rc = launch_sweep(c, in, work, dim, s, 1e-3, nullptr, nullptr, st);
-          if (!rc && hipEventRecord(e1, st) != hipSuccess) rc = fail(FL_ERR_HIP, "hipEventRecord");
-          if (!rc && hipEventSynchronize(e1) != hipSuccess)
-            rc = fail(FL_ERR_HIP, "hipEventSynchronize");
-          float ms = 0.0f;
-          if (!rc) (void)hipEventElapsedTime(&ms, e0, e1);
-          if (r > 0) total += ms;
-        }
+        rc = timed(dim, &total);
         if (!rc && total < best_ms) {
           best_ms = total;
           best = t;
         }
       }
     }
+    // the cell-parallel kernel, on grids where it can be the faster one
+    if (in->ndim == 2 && !rc && in->n[0] * in->n[1] <= 4 * kCellMax<float>) {
+      float total = 0.0f;
+      c->shape[dim] = kShapeCell;
+      rc = timed(dim, &total);
+      if (!rc && total >= best_ms) c->shape[dim] = kShapeTuning;
+    }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   c->tuning = rc ? saved : best;
+  if (rc)
+    for (int d = 0; d < 2; ++d) c->shape[d] = saved_shape[d];
   if (!rc && chosen) *chosen = best;
   return rc;
 }
@@ -978,6 +1036,7 @@ int fl_simulate(fl_context* c, fl_field* state, fl_field* work, const fl_scheme*
     key.sim_time = p->sim_time;
     key.max_iters = p->max_iters;
     key.tuning = c->tuning;
+    for (int d = 0; d < 2; ++d) key.shape[d] = c->shape[d];
     if (!c->sim_exec || !c->sim_exec_run || memcmp(&key, &c->sim_key, sizeof(key)) != 0) {
       if (c->sim_exec) (void)hipGraphExecDestroy(c->sim_exec);
       if (c->sim_graph) (void)hipGraphDestroy(c->sim_graph);

@@ -28,7 +28,13 @@ struct SimGraphKey {
   double cfl, dh, sim_time;
   int64_t max_iters;
   fl_tuning tuning;
+  int32_t shape[2];
 };
+
+// Where the launch shape of a 2D sweep (x, y) comes from: the built-in rule
+// on the grid, the march heights and widths in `tuning`, or the cell-parallel
+// kernel (the autotuner's choice).
+enum : int { kShapeRule = 0, kShapeTuning = 1, kShapeCell = 2 };
 
 struct fl_context {
   int device;
@@ -40,6 +46,7 @@ struct fl_context {
   fl::ls::EikCtl* eik;         // device control words of the eikonal loop, 2 jobs
   fl::ls::EikCtl* host_eik;    // pinned host mirror of eik
   fl_tuning tuning;
+  int32_t shape[2];            // kShape* of the x and the y sweep
   hipEvent_t step_ev;          // fl_mm_simulate: the step's control block is on the host
   int64_t eik_sweeps;          // sweeps the last eikonal solve took (first batch size)
   int use_graphs;              // fl_simulate replays a captured pair of steps
@@ -98,8 +105,9 @@ inline fl::Material<T> make_material(const fl_scheme* s) {
 
 double bits_to_double(unsigned long long b);
 // `t` (nullable: all defaults) with zeros replaced by the built-in launch
-// shapes, validated, into *out.
-int resolve_tuning(const fl_tuning* t, fl_tuning* out);
+// shapes, validated, into *out; shape[d] becomes kShapeTuning where t names a
+// width or height of that sweep.
+int resolve_tuning(const fl_tuning* t, fl_tuning* out, int32_t* shape);
 int check_pair(const fl_field* in, const fl_field* out);
 int check_field(const fl_field* f, const char* name);
 int check_scheme(const fl_scheme* s, int ndim);

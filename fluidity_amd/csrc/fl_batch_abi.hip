@@ -116,6 +116,8 @@ std::vector<bt::Prob<T>> make_probs(const fl_batch* b, const fl_tuning& t) {
     strides(&q.state, a.es, a.cs);
     a.nx = q.state.n[0];
     a.ny = q.state.ndim > 1 ? q.state.n[1] : 1;
+    a.rowb = a.nx * a.es * (int64_t)sizeof(T);
+    a.csb = a.cs * (int64_t)sizeof(T);
     a.mat = make_material<T>(&q.scheme);
     a.mat64 = make_material<double>(&q.scheme);
     a.limiter = q.scheme.limiter;

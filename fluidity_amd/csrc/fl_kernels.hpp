@@ -44,6 +44,8 @@ struct SweepArgs {
   T* out;
   int64_t es;          // element stride (in T units): S for AoS, 1 for SoA
   int64_t cs;          // component stride: 1 for AoS, nx*ny for SoA
+  int64_t rowb;        // bytes from one row to the next
+  int64_t csb;         // component stride in bytes
   int64_t nx, ny;      // interior cells
   Material<T> mat;     // material in the sweep precision
   Material<double> mat64;  // FP64 material for the fused wavespeed
@@ -58,6 +60,7 @@ struct SweepArgs {
 
 // Maximum workgroup width of the sweep kernels (LDS arrays are sized for it).
 constexpr int kMaxBlock = 256;
+constexpr int kMaxWaves = 8;  // waves of the widest workgroup (the cell-parallel sweeps')
 constexpr int kHalo = 3;  // extra cells each side staged in LDS for chi
 
 // Dynamic LDS of an x-sweep tile of B lanes over states of S components of
@@ -73,6 +76,25 @@ __host__ __device__ constexpr size_t y_tile_lds_bytes(int B, int tsize) {
   return (size_t)(3 * (B + 2 * kHalo) + kYRing * 4 * B) * (size_t)tsize;
 }
 
+// Cell-parallel 2D sweeps: kCellWaves waves per workgroup, one row of 64
+// columns each.  LDS of FP size tsize: pressures and y velocities of
+// kCellWaves + 6 rows, x velocities of kCellWaves rows (columns with their
+// halo where the x direction reads it), one state per thread.
+constexpr int kCellWaves = 8;
+constexpr int kCellCols = 64 + 2 * kHalo;  // columns of a staged row with its halo
+__host__ __device__ constexpr size_t cell_tile_lds_bytes(int tsize) {
+  return (size_t)((kCellWaves + 6) * (kCellCols + 64) + kCellWaves * (kCellCols + 4 * 64)) *
+         (size_t)tsize;
+}
+// Cells of one tile: 62 columns x kCellWaves rows (x sweep), 64 columns x
+// kCellWaves - 2 rows (y sweep).
+constexpr int kCellXCols = 62, kCellXRows = kCellWaves;
+constexpr int kCellYCols = 64, kCellYRows = kCellWaves - 2;
+
+// Blocks of a cell-parallel launch up to which each issues its atomicMax
+// unseen (two rounds of the blocks the device holds).
+constexpr unsigned kCellFewBlocks = 1024;
+
 // Standalone wavespeed max: at most kMaxWsBlocks workgroups of kMaxBlock
 // threads, each thread loading kMaxWsUnroll cells per iteration.
 constexpr int kMaxWsBlocks = 512;
@@ -84,6 +106,10 @@ constexpr int kMaxWsUnroll = 4;
 namespace fl {
 template <typename T, int ND, int FLUX, bool FAST, bool VLC> __global__ void sweep_x_kernel(SweepArgs<T> a);
 template <typename T, int FLUX, bool FAST, bool VLC> __global__ void sweep_y_kernel(SweepArgs<T> a);
+template <typename T, int FLUX, bool FAST, bool VLC>
+__global__ void cell_x_kernel(SweepArgs<T> a0, SweepArgs<T> a1);
+template <typename T, int FLUX, bool FAST, bool VLC>
+__global__ void cell_y_kernel(SweepArgs<T> a0, SweepArgs<T> a1);
 template <typename T, int ND, int FLUX, bool FAST, bool VLC>
 __global__ void sweep_x2_kernel(SweepArgs<T> a0, SweepArgs<T> a1);
 template <typename T, int FLUX, bool FAST, bool VLC>

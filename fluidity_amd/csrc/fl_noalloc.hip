@@ -68,7 +68,7 @@ int fl_simulate_noalloc(const fl_tuning* tuning, fl_field* state, fl_field* work
   fl_context c;
   memset(&c, 0, sizeof(c));
   FL_HIP(hipGetDevice(&c.device));
-  if ((rc = resolve_tuning(tuning, &c.tuning))) return rc;
+  if ((rc = resolve_tuning(tuning, &c.tuning, c.shape))) return rc;
   fl::StepCtl* ctl = nullptr;
   if ((rc = scratch_of(c.device, &ctl))) return rc;
   hipStream_t st = (hipStream_t)stream;

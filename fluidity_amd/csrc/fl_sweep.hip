@@ -46,6 +46,23 @@ sweep_y_kernel(SweepArgs<T> a) {
   sweep_y_tile<T, FLUX, FAST, VLC>(a, bx, by);
 }
 
+// Cell-parallel sweeps of small grids (cell_x_tile, cell_y_tile), of one grid
+// or of two of one shape (blockIdx.y selects the grid), one tile per
+// workgroup, tiles numbered along x first.
+template <typename T, int FLUX, bool FAST, bool VLC>
+__global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(4)))
+cell_x_kernel(SweepArgs<T> a0, SweepArgs<T> a1) {
+  const unsigned nbx = (unsigned)((a0.nx + kCellXCols - 1) / kCellXCols);
+  cell_x_tile<T, FLUX, FAST, VLC>(blockIdx.y ? a1 : a0, blockIdx.x % nbx, blockIdx.x / nbx);
+}
+
+template <typename T, int FLUX, bool FAST, bool VLC>
+__global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(4)))
+cell_y_kernel(SweepArgs<T> a0, SweepArgs<T> a1) {
+  const unsigned nbx = (unsigned)((a0.nx + kCellYCols - 1) / kCellYCols);
+  cell_y_tile<T, FLUX, FAST, VLC>(blockIdx.y ? a1 : a0, blockIdx.x % nbx, blockIdx.x / nbx);
+}
+
 // The same sweeps over two grids of one shape in one launch (the two
 // materials of a two-material step): blockIdx.z selects the grid.
 template <typename T, int ND, int FLUX, bool FAST, bool VLC>
@@ -449,7 +466,9 @@ FL_INST_PERSIST(float)
 #define FL_SWEEPS_V(T, FLUX, FAST, VLC)                                          \
   template __global__ void sweep_x_kernel<T, 1, FLUX, FAST, VLC>(SweepArgs<T>);  \
   template __global__ void sweep_x_kernel<T, 2, FLUX, FAST, VLC>(SweepArgs<T>);  \
-  template __global__ void sweep_y_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>);
+  template __global__ void sweep_y_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>);     \
+  template __global__ void cell_x_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>, SweepArgs<T>); \
+  template __global__ void cell_y_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>, SweepArgs<T>);
 #define FL_SWEEPS(T, FLUX, FAST) FL_SWEEPS_V(T, FLUX, FAST, false)
 
 #define FL_INST_SWEEPS(T)                                                      \

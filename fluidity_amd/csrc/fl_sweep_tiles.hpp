@@ -251,9 +251,14 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 }
 
 // Block-wide max of v; thread 0 issues one atomicMax.  Must be reached by every
-// thread of the block.
-__device__ __forceinline__ void block_atomic_max(unsigned long long v, unsigned long long* dst) {
-  __shared__ unsigned long long red[kMaxBlock / 64];
+// thread of the block.  The atomics of a launch serialise at about 10 ns
+// each, so a launch of many short blocks reads the maximum so far first and
+// leaves out those that cannot raise it (FP32 at 1024^2, 2900 cell-parallel
+// blocks: 61 -> 48 us a step); with few blocks that read is one more device
+// round trip in each.
+__device__ __forceinline__ void block_atomic_max(unsigned long long v, unsigned long long* dst,
+                                                 bool many = false) {
+  __shared__ unsigned long long red[kMaxWaves];
   v = wave_max_u64(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) red[wave] = v;
@@ -261,7 +266,8 @@ __device__ __forceinline__ void block_atomic_max(unsigned long long v, unsigned 
   if (threadIdx.x == 0) {
     const int nw = (blockDim.x + 63) >> 6;
     for (int i = 1; i < nw; ++i) v = red[i] > v ? red[i] : v;
-    atomicMax(dst, v);
+    if (!many || v > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(dst, v);
   }
 }
 
@@ -762,6 +768,258 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, int64_t bx, 
   }
   }
   if (a.ws_out) block_atomic_max(wsmax, a.ws_out);
+}
+
+// ---------------------------------------------------------------------------
+// cell-parallel 2D sweeps
+// ---------------------------------------------------------------------------
+
+// The march above hides a row's latency behind the rows before it; on a small
+// grid its six or eight warm-up rows are the whole run time (each row is one
+// dependent FP64 chain of 1 to 2 us).  Here a workgroup of kCellWaves waves
+// takes a tile at once, one row of 64 columns per wave: the primitives that
+// the flattening factors read are staged in LDS for the tile and the rows and
+// columns around it, so the chain is one load, one cell's arithmetic and two
+// or three barriers whatever the tile.  The rows around a tile cost 14 rows of
+// primitives per 8 (x) or 6 (y) and the y sweep evolves two rows more than it
+// writes, so large grids march.
+
+// First byte of grid row y through the ghost map; flip: bit 1 set for a
+// reflective ghost row (y momentum flips).
+template <typename T>
+__device__ __forceinline__ const char* row_ptr(const SweepArgs<T>& a, int64_t y, int& flip) {
+  bool fy = false;
+  const int yi = map_row((int)y, (int)a.ny, a.bcy, fy);
+  flip = fy ? 2 : 0;
+  return (const char*)a.in + (int64_t)yi * a.rowb;
+}
+
+// Issues the loads of a lane's cell of the row at `row` (row_ptr), each a
+// scalar base plus a 32-bit lane offset as in issue_row.
+template <typename T, int S>
+__device__ __forceinline__ void issue_at(const SweepArgs<T>& a, const char* row, int flip,
+                                         const LaneCol& lc, Pending<T, S>& q) {
+  uint32_t off = lc.off;
+  asm volatile("" : "+v"(off));
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    const char* base = row;
+    asm volatile("" : "+s"(base));
+    q.u[k] = *(const __attribute__((address_space(1))) T*)(
+        (const __attribute__((address_space(1))) char*)base + off);
+    row += a.csb;
+  }
+  q.flip = lc.flip | flip;
+}
+
+// issue_at of row y.
+template <typename T, int S>
+__device__ __forceinline__ void issue_near(const SweepArgs<T>& a, int64_t y, const LaneCol& lc,
+                                           Pending<T, S>& q) {
+  int flip;
+  const char* row = row_ptr(a, y, flip);
+  issue_at<T, S>(a, row, flip, lc, q);
+}
+
+// Stages the primitives that the flattening factors of rows yb .. yb +
+// kCellWaves - 1 of the 64 columns from xc read: pressures and y velocities
+// of those rows and three above and below, pressures and x velocities of the
+// kHalo columns on either side of the rows.  Wave w stages its own row yb + w
+// (its first byte `row`), whose states it keeps in u0, and one of the six
+// rows above and below (w < 6) or the halo cells (w = 6).
+template <typename T, bool F>
+__device__ __forceinline__ void cell_stage(const SweepArgs<T>& a, int64_t xc, int64_t yb, int w,
+                                           int t, const char* row, int flip, const LaneCol& lc,
+                                           T* sP, T* sVX, T* sVY, T* u0) {
+  constexpr int S = 4, ND = 2, NW = kCellWaves, PW = kCellCols;
+  static_assert(NW >= 7 && 6 * NW <= 64, "one wave stages the halo cells");
+  Pending<T, S> Q, H;
+  issue_at<T, S>(a, row, flip, lc, Q);
+  const int j = t / 6, h = t - 6 * j;       // halo cell of this lane (w = 6)
+  const int hcol = h < kHalo ? h : 64 + h;  // its column in the staged row
+  const bool halo = w == 6 && j < NW;
+  const int q2 = w < 3 ? w : NW + w;        // second staged row of this wave (w < 6)
+  if (w < 6) issue_near<T, S>(a, yb - 3 + q2, lc, H);
+  else if (halo) issue_load<T, ND>(a, xc - kHalo + hcol, yb + j, H);
+  take<T, ND>(Q, u0);
+  {
+    const Prim<T, ND> p = prim_sel<F, T, ND>(u0, a.mat);
+    sP[(w + 3) * PW + kHalo + t] = p.p;
+    sVX[w * PW + kHalo + t] = p.vel[0];
+    sVY[(w + 3) * 64 + t] = p.vel[1];
+  }
+  if (w < 6 || halo) {
+    T uh[S];
+    take<T, ND>(H, uh);
+    const Prim<T, ND> p = prim_sel<F, T, ND>(uh, a.mat);
+    if (w < 6) {
+      sP[q2 * PW + kHalo + t] = p.p;
+      sVY[q2 * 64 + t] = p.vel[1];
+    } else {
+      sP[(j + 3) * PW + hcol] = p.p;
+      sVX[j * PW + hcol] = p.vel[0];
+    }
+  }
+}
+
+// chi of lane t in row w of the staged tile (muscl_reconstructor.hpp:106-114):
+// the factors about the cell and about its neighbour on the higher-pressure
+// side, the latter evaluated where they are needed instead of exchanged.
+template <typename T, bool F>
+__device__ __forceinline__ T cell_chi(const SweepArgs<T>& a, int w, int t, const T* sP,
+                                      const T* sVX, const T* sVY) {
+  constexpr int PW = kCellCols;
+  const T* p = sP + (w + 3) * PW + kHalo + t;
+  const T* vx = sVX + w * PW + kHalo + t;
+  const T* vy = sVY + (w + 3) * 64 + t;
+  const T pl = p[-1], pr = p[1], pd = p[-PW], pu = p[PW];
+  const int sx = signum(pr - pl), sy = signum(pu - pd);
+  const T* pn = p + sx;
+  const T* vn = vx + sx;
+  const T* pm = p + sy * PW;
+  const T* vm = vy + sy * 64;
+  const T kx = chi_sel<F>(p[-2], pl, pr, p[2], vx[-1], vx[1], a.mat);
+  const T kxn = chi_sel<F>(pn[-2], pn[-1], pn[1], pn[2], vn[-1], vn[1], a.mat);
+  const T ky = chi_sel<F>(p[-2 * PW], pd, pu, p[2 * PW], vy[-64], vy[64], a.mat);
+  const T kyn = chi_sel<F>(pm[-2 * PW], pm[-PW], pm[PW], pm[2 * PW], vm[-64], vm[64], a.mat);
+  const T chi = min_sel<F>(Limits<T>::max(), min_sel<F>(kx, kxn));
+  return min_sel<F>(chi, min_sel<F>(ky, kyn));
+}
+
+// Orders a wave's LDS accesses: what its other lanes wrote before is read
+// after (the LDS serves one wave's accesses in order).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// x sweep of columns [62 bx, 62 bx + 62) of rows [kCellWaves by, kCellWaves
+// (by + 1)).  Lanes 0 and 63 hold the columns beside them, whose face states
+// the tile's outer faces need.  Called by every thread of a workgroup of
+// kCellWaves waves.
+template <typename T, int FLUX, bool FAST, bool VLC>
+__device__ __forceinline__ void cell_x_tile(const SweepArgs<T>& a, int64_t bx, int64_t by) {
+  constexpr int ND = 2, S = 4, NW = kCellWaves;
+  constexpr bool F = UseFast<T, FAST>::value;
+  const int limiter = VLC ? int(kLimVanLeer) : a.limiter;
+  const int form = VLC ? int(kFormCons) : a.form;
+  T dtdh;
+  if (!sweep_dtdh(a, dtdh)) return;
+  const T half_dtdh = T(0.5) * dtdh;
+  const T dhdt = T(1) / dtdh;
+  const int t = (int)(threadIdx.x & 63);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  extern __shared__ __align__(16) unsigned char fl_c_lds[];
+  T* const sP = reinterpret_cast<T*>(fl_c_lds);  // [NW + 6][kCellCols]
+  T* const sVX = sP + (NW + 6) * kCellCols;      // [NW][kCellCols]
+  T* const sVY = sVX + NW * kCellCols;           // [NW + 6][64]
+  T* const sX = sVY + (NW + 6) * 64 + w * (S * 64);  // this wave's [S][64]
+  const int64_t xc = bx * kCellXCols - 1;
+  const int64_t c = xc + t;
+  const int64_t yb = by * NW, r = yb + w;
+  const LaneCol lc = lane_col(a, c), ll = lane_col(a, c - 1), lr = lane_col(a, c + 1);
+  int fy;
+  const char* row = row_ptr(a, r, fy);
+  Pending<T, S> Ql, Qr;
+  T u0[S];
+  issue_at<T, S>(a, row, fy, ll, Ql);
+  issue_at<T, S>(a, row, fy, lr, Qr);
+  cell_stage<T, F>(a, xc, yb, w, t, row, fy, lc, sP, sVX, sVY, u0);
+  __syncthreads();
+  unsigned long long wsmax = 0ull;
+  if (r < a.ny) {  // uniform over the wave
+    const T chi = cell_chi<T, F>(a, w, t, sP, sVX, sVY);
+    T um[S], up[S], R[S], L[S];
+    take<T, ND>(Ql, um);
+    take<T, ND>(Qr, up);
+    evolve_sel<F, T, ND, 0>(um, u0, up, chi, half_dtdh, limiter, form, a.mat, R, L);
+#pragma unroll
+    for (int k = 0; k < S; ++k) sX[k * 64 + t] = L[k];
+    wave_sync();
+    T Lr[S], G[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) Lr[k] = sX[k * 64 + ((t + 1) & 63)];
+    wave_sync();
+    flux_sel<F, T, ND, 0, FLUX>(R, Lr, dtdh, dhdt, a.mat, G);
+#pragma unroll
+    for (int k = 0; k < S; ++k) sX[k * 64 + t] = G[k];
+    wave_sync();
+    if (t >= 1 && t <= 62 && c < a.nx) {
+      T o[S];
+#pragma unroll
+      for (int k = 0; k < S; ++k) o[k] = u0[k] + (sX[k * 64 + t - 1] - G[k]) * dtdh;
+      store_row<T, S>(a, r, col_off(a, c), o);
+      if (a.ws_out) ws_fold<F, T, ND>(o, a, wsmax);
+    }
+  }
+  if (a.ws_out) block_atomic_max(wsmax, a.ws_out, gridDim.x > kCellFewBlocks);
+}
+
+// y sweep of columns [64 bx, 64 bx + 64) of rows [(kCellWaves - 2) by,
+// (kCellWaves - 2) (by + 1)).  Waves 0 and kCellWaves - 1 hold the rows beside
+// them.  Called as cell_x_tile.
+template <typename T, int FLUX, bool FAST, bool VLC>
+__device__ __forceinline__ void cell_y_tile(const SweepArgs<T>& a, int64_t bx, int64_t by) {
+  constexpr int ND = 2, S = 4, NW = kCellWaves;
+  constexpr bool F = UseFast<T, FAST>::value;
+  const int limiter = VLC ? int(kLimVanLeer) : a.limiter;
+  const int form = VLC ? int(kFormCons) : a.form;
+  T dtdh;
+  if (!sweep_dtdh(a, dtdh)) return;
+  const T half_dtdh = T(0.5) * dtdh;
+  const T dhdt = T(1) / dtdh;
+  const int t = (int)(threadIdx.x & 63);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  extern __shared__ __align__(16) unsigned char fl_c_lds[];
+  T* const sP = reinterpret_cast<T*>(fl_c_lds);  // as in cell_x_tile
+  T* const sVX = sP + (NW + 6) * kCellCols;
+  T* const sVY = sVX + NW * kCellCols;
+  T* const sX = sVY + (NW + 6) * 64;             // [NW][S][64]
+  const int64_t xc = bx * kCellYCols;
+  const int64_t c = xc + t;
+  const int64_t yb = by * kCellYRows - 1, r = yb + w;
+  const LaneCol lc = lane_col(a, c);
+  int fy;
+  const char* row = row_ptr(a, r, fy);
+  Pending<T, S> Ql, Qr;
+  T u0[S];
+  cell_stage<T, F>(a, xc, yb, w, t, row, fy, lc, sP, sVX, sVY, u0);
+  issue_near<T, S>(a, r - 1, lc, Ql);
+  issue_near<T, S>(a, r + 1, lc, Qr);
+  __syncthreads();
+  T R[S], L[S], G[S];
+  const bool live = r <= a.ny;  // uniform over the wave; row ny is the ghost above the grid
+  if (live) {
+    const T chi = cell_chi<T, F>(a, w, t, sP, sVX, sVY);
+    T um[S], up[S];
+    take<T, ND>(Ql, um);
+    take<T, ND>(Qr, up);
+    evolve_sel<F, T, ND, 1>(um, u0, up, chi, half_dtdh, limiter, form, a.mat, R, L);
+#pragma unroll
+    for (int k = 0; k < S; ++k) sX[(w * S + k) * 64 + t] = R[k];
+  }
+  __syncthreads();
+  if (live && w > 0) {
+    // the face between rows r - 1 and r; slot w - 1, which this wave alone
+    // reads, takes its flux for the wave below
+    T Rp[S];
+    T* const x = sX + (w - 1) * S * 64 + t;
+#pragma unroll
+    for (int k = 0; k < S; ++k) Rp[k] = x[k * 64];
+    flux_sel<F, T, ND, 1, FLUX>(Rp, L, dtdh, dhdt, a.mat, G);
+#pragma unroll
+    for (int k = 0; k < S; ++k) x[k * 64] = G[k];
+  }
+  __syncthreads();
+  unsigned long long wsmax = 0ull;
+  if (r < a.ny && w > 0 && w < NW - 1 && c < a.nx) {
+    T o[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) o[k] = u0[k] + (G[k] - sX[(w * S + k) * 64 + t]) * dtdh;
+    store_row<T, S>(a, r, col_off(a, c), o);
+    if (a.ws_out) ws_fold<F, T, ND>(o, a, wsmax);
+  }
+  if (a.ws_out) block_atomic_max(wsmax, a.ws_out, gridDim.x > kCellFewBlocks);
 }
 
 }  // namespace fl

@@ -1,0 +1,77 @@
+"""The built-in launch rule of the 2D sweeps: cell-parallel tiles on small
+grids and marching tiles on larger ones, against the oracle and against each
+other, at the edges of the tiles (62 or 64 columns, 8 or 6 rows) and of the rule.
+"""
+import numpy as np
+import pytest
+import torch
+
+from tests.fields import cons_field
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def E():
+    from fluidity_amd import euler
+    return euler
+
+
+def _dev(U, layout, dtype=torch.float64):
+    a = np.moveaxis(U, -1, 0) if layout == 1 else U
+    return torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dtype=dtype)
+
+
+def _host(a, layout):
+    a = a.cpu().numpy()
+    return np.ascontiguousarray(np.moveaxis(a, 0, -1)) if layout == 1 else a
+
+
+def _bits(a):
+    return a.view(np.uint64 if a.dtype == np.float64 else np.uint32)
+
+
+CASES = [
+    # (ny, nx), limiter, form, flux, bc per dimension, layout
+    ((4, 4), 0, 0, 0, (0, 0), 0),
+    ((6, 62), 0, 0, 0, (0, 1), 1),
+    ((7, 63), 1, 0, 0, (1, 0), 0),
+    ((8, 64), 0, 1, 1, (2, 2), 1),
+    ((9, 65), 0, 0, 0, (2, 0), 0),
+    ((12, 124), 1, 1, 0, (1, 1), 1),
+    ((13, 125), 0, 0, 2, (0, 2), 0),
+    ((5, 190), 0, 1, 3, (1, 2), 1),
+    ((131, 5), 0, 0, 0, (2, 1), 0),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[0])))
+@pytest.mark.parametrize("dim", [0, 1])
+def test_rule_sweeps_bitwise(E, oracle, case, dim):
+    shape, lim, form, flux, bc, layout = case
+    U = cons_field("rough", shape, seed=3 + shape[0] * shape[1])
+    os_ = oracle.scheme(limiter=lim, form=form, flux=flux, bc=bc + (0,))
+    dtdh = 0.4 / oracle.max_wavespeed_grid(U, os_)
+    ref = oracle.sweep(U, os_, dtdh, dim)
+    solver = E.SplitSolver(E.Scheme(limiter=lim, form=form, flux=flux, bc=bc + (0,)), layout=layout)
+    a = _dev(U, layout)
+    b = torch.empty_like(a)
+    solver.sweep(a, b, dim, dtdh)
+    assert np.array_equal(_bits(_host(b, layout)), _bits(ref))
+
+
+@pytest.mark.parametrize("shape", [(640, 1024), (641, 1024)])  # the rule's line for FP64
+def test_rule_line_matches_marching_loop(E, shape):
+    """The step loop (fused CFL maximum included) on either side of the rule's
+    line equals the loop with a caller's marching shapes bit for bit."""
+    U = cons_field("riemann", shape, seed=1001)  # a run the oracle completes
+    out = []
+    for tuning in (None, dict(x_block=128, x_rows=16, y_block=64, y_rows=32)):
+        solver = E.SplitSolver(E.Scheme(), layout=1)
+        if tuning:
+            solver.set_tuning(**tuning)
+        a = _dev(U, 1)
+        r = solver.simulate(a, torch.empty_like(a), 0.9, 1.0 / shape[1], max_iters=5)
+        out.append((_bits(_host(a, 1)), r.run_time, r.max_wavespeed))
+    assert np.array_equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:]
