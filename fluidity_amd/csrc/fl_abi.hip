@@ -328,10 +328,20 @@ void launch_flux_t(int flux, int ndim, int dim, dim3 grid, const SweepShape& sh,
   }
 }
 
+// Slots of the maximum wavespeed in a SimCtl for ndim dimensions.
+inline int sim_slots(int ndim) { return ndim == 1 ? 3 : 2; }
+
+// begin (nullable): the sweep begins step k of a simulation.
+struct SimBegin {
+  fl::SimCtl* sim;
+  const fl_sim_params* p;
+  int64_t k;
+};
+
 template <typename T>
 int launch_sweep_t(const fl_context* ctx, const fl_field* in, const fl_field* out, int dim,
                    const fl_scheme* s, double dtdh, const fl::StepCtl* ctl,
-                   unsigned long long* ws_out, hipStream_t stream) {
+                   unsigned long long* ws_out, const SimBegin* begin, hipStream_t stream) {
   dim3 grid;
   SweepShape sh{false, ctx->tuning.x_block, 1};
   if (in->ndim == 1) {
@@ -340,7 +350,18 @@ int launch_sweep_t(const fl_context* ctx, const fl_field* in, const fl_field* ou
     sh = pick_shape<T>(ctx, dim, in->n[0], in->n[1], 1);
     grid = shape_grid(sh, dim, in->n[0], in->n[1], 1);
   }
-  const fl::SweepArgs<T> a = make_args<T>(ctx, in, out, s, dtdh, ctl, ws_out, sh.rows);
+  fl::SweepArgs<T> a = make_args<T>(ctx, in, out, s, dtdh, ctl, ws_out, sh.rows);
+  if (begin) {
+    const int n = sim_slots(in->ndim);
+    a.sim = begin->sim;
+    a.sim_half = (int)(begin->k & 1);
+    a.sim_ws = (int)(begin->k % n);
+    a.sim_zero = (int)((begin->k + n - 1) % n);
+    a.cfl = begin->p->cfl;
+    a.dh = begin->p->dh;
+    a.sim_time = begin->p->sim_time;
+    a.max_iters = (long long)begin->p->max_iters;
+  }
   if (std::is_same<T, double>::value && fast_numerics(s))
     launch_flux_t<T, true>(s->flux, in->ndim, dim, grid, sh, a, stream);
   else
@@ -353,8 +374,25 @@ int launch_sweep(const fl_context* ctx, const fl_field* in, const fl_field* out,
                  const fl_scheme* s, double dtdh, const fl::StepCtl* ctl,
                  unsigned long long* ws_out, hipStream_t stream) {
   if (in->dtype == FL_F64)
-    return launch_sweep_t<double>(ctx, in, out, dim, s, dtdh, ctl, ws_out, stream);
-  return launch_sweep_t<float>(ctx, in, out, dim, s, dtdh, ctl, ws_out, stream);
+    return launch_sweep_t<double>(ctx, in, out, dim, s, dtdh, ctl, ws_out, nullptr, stream);
+  return launch_sweep_t<float>(ctx, in, out, dim, s, dtdh, ctl, ws_out, nullptr, stream);
+}
+
+int launch_sim_step(const fl_context* ctx, const fl_field* state, const fl_field* work,
+                    const fl_scheme* s, const fl_sim_params* p, fl::SimCtl* sim, int64_t k,
+                    hipStream_t stream) {
+  const SimBegin begin = {sim, p, k};
+  unsigned long long* next = &sim->ws[(k + 1) % sim_slots(state->ndim)];
+  const bool one = state->ndim == 1;
+  const fl_field* src = one && (k & 1) ? work : state;
+  const fl_field* dst = one && (k & 1) ? state : work;
+  const int rc = state->dtype == FL_F64
+                     ? launch_sweep_t<double>(ctx, src, dst, 0, s, 1.0, nullptr,
+                                              one ? next : nullptr, &begin, stream)
+                     : launch_sweep_t<float>(ctx, src, dst, 0, s, 1.0, nullptr,
+                                             one ? next : nullptr, &begin, stream);
+  if (rc || one) return rc;
+  return launch_sweep(ctx, work, state, 1, s, 1.0, &sim->c, next, stream);
 }
 
 // Both materials' sweeps of dimension `dim` in one launch: in[m] -> out[m]
@@ -638,6 +676,19 @@ int simulate_persist1d(fl_context* c, fl_field* state, fl_field* work, const fl_
 
 }  // namespace
 
+namespace {
+
+void drop_sim_graphs(fl_context* c) {
+  for (int g = 0; g < 2; ++g) {
+    if (c->sim_exec[g]) (void)hipGraphExecDestroy(c->sim_exec[g]);
+    if (c->sim_graph[g]) (void)hipGraphDestroy(c->sim_graph[g]);
+    c->sim_exec[g] = nullptr;
+    c->sim_graph[g] = nullptr;
+  }
+}
+
+}  // namespace
+
 extern "C" {
 
 const char* fl_status_string(int status) {
@@ -669,6 +720,8 @@ int fl_ctx_create(int device, fl_context** out) {
   (void)resolve_tuning(nullptr, &c->tuning, c->shape);
   hipError_t e = hipMalloc((void**)&c->ctl, sizeof(fl::StepCtl));
   if (e == hipSuccess) e = hipMalloc((void**)&c->ws_tmp, sizeof(unsigned long long));
+  if (e == hipSuccess) e = hipMalloc((void**)&c->sim, sizeof(fl::SimCtl));
+  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_sim, sizeof(fl::SimCtl), 0);
   if (e == hipSuccess) e = hipMalloc((void**)&c->partial, sizeof(double) * kSumBlocks * 4);
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_ctl, sizeof(fl::StepCtl), 0);
   if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_partial, sizeof(double) * kSumBlocks * 4, 0);
@@ -692,13 +745,12 @@ int fl_ctx_destroy(fl_context* c) {
   DeviceGuard g(c->device);
   if (c->ctl) (void)hipFree(c->ctl);
   if (c->ws_tmp) (void)hipFree(c->ws_tmp);
+  if (c->sim) (void)hipFree(c->sim);
+  if (c->host_sim) (void)hipHostFree(c->host_sim);
   if (c->partial) (void)hipFree(c->partial);
   if (c->host_ctl) (void)hipHostFree(c->host_ctl);
   if (c->host_partial) (void)hipHostFree(c->host_partial);
-  if (c->sim_exec) (void)hipGraphExecDestroy(c->sim_exec);
-  if (c->sim_graph) (void)hipGraphDestroy(c->sim_graph);
-  if (c->sim_exec_run) (void)hipGraphExecDestroy(c->sim_exec_run);
-  if (c->sim_graph_run) (void)hipGraphDestroy(c->sim_graph_run);
+  drop_sim_graphs(c);
   if (c->cap_stream) (void)hipStreamDestroy(c->cap_stream);
   if (c->eik) (void)hipFree(c->eik);
   if (c->host_eik) (void)hipHostFree(c->host_eik);
@@ -993,34 +1045,23 @@ int fl_simulate(fl_context* c, fl_field* state, fl_field* work, const fl_scheme*
     }
   }
 
-  hipLaunchKernelGGL(fl::init_control_kernel, dim3(1), dim3(1), 0, st, c->ctl);
-  rc = launch_max_ws(state, s, &c->ctl->ws_bits[0], st);
+  hipLaunchKernelGGL(fl::init_sim_kernel, dim3(1), dim3(1), 0, st, c->sim);
+  rc = launch_max_ws(state, s, &c->sim->ws[0], st);
   if (rc) return rc;
 
   // Steps are launched in batches; between batches the host reads the control
-  // block once to stop when the loop condition fails.  With graphs on, runs
-  // of kSimGraphSteps steps and pairs of steps (both parities) are captured
-  // once and replayed, the runs while a batch has that many steps left (one
-  // host launch per run instead of per pair: small grids' steps are shorter
-  // than a graph launch); a step past the stop condition does nothing, so an
-  // odd batch may run one step more.
-  const int64_t kBatch = 256;
-  constexpr int kSimGraphSteps = 16;
+  // words once to stop when the loop condition fails.  With graphs on, a run
+  // of kSimGraphSteps steps and the steps that a loop of max_iters leaves over
+  // are captured and replayed (one host launch per graph, about 1 us less per
+  // kernel on the device): at once for loops of kSimGraphMin steps or more,
+  // from the second call of the same loop on for shorter ones, which cost
+  // less than their capture.  A step past the stop condition does nothing.
+  constexpr int kSimGraphSteps = 18;  // a multiple of both slot cycles (2 and 3)
+  constexpr int64_t kSimGraphMin = 4 * kSimGraphSteps;
+  constexpr int64_t kBatch = 14 * kSimGraphSteps;
+  const int64_t left_over = p->max_iters % kSimGraphSteps;
   int64_t launched = 0;
-  fl_field a = *state, b = *work;
-  auto one_step = [&](int parity, hipStream_t sx) -> int {
-    hipLaunchKernelGGL(fl::step_control_kernel, dim3(1), dim3(1), 0, sx, c->ctl, parity,
-                       p->cfl, p->dh, p->sim_time, (long long)p->max_iters);
-    unsigned long long* ws_next = &c->ctl->ws_bits[parity ^ 1];
-    if (state->ndim == 1) {
-      const fl_field* src = parity ? &b : &a;
-      const fl_field* dst = parity ? &a : &b;
-      return launch_sweep(c, src, dst, 0, s, 1.0, c->ctl, ws_next, sx);
-    }
-    int r = launch_sweep(c, &a, &b, 0, s, 1.0, c->ctl, nullptr, sx);
-    if (!r) r = launch_sweep(c, &b, &a, 1, s, 1.0, c->ctl, ws_next, sx);
-    return r;
-  };
+  bool graphs = false;
   if (c->use_graphs) {
     SimGraphKey key;
     memset(&key, 0, sizeof(key));
@@ -1037,66 +1078,55 @@ int fl_simulate(fl_context* c, fl_field* state, fl_field* work, const fl_scheme*
     key.max_iters = p->max_iters;
     key.tuning = c->tuning;
     for (int d = 0; d < 2; ++d) key.shape[d] = c->shape[d];
-    if (!c->sim_exec || !c->sim_exec_run || memcmp(&key, &c->sim_key, sizeof(key)) != 0) {
-      if (c->sim_exec) (void)hipGraphExecDestroy(c->sim_exec);
-      if (c->sim_graph) (void)hipGraphDestroy(c->sim_graph);
-      if (c->sim_exec_run) (void)hipGraphExecDestroy(c->sim_exec_run);
-      if (c->sim_graph_run) (void)hipGraphDestroy(c->sim_graph_run);
-      c->sim_exec = c->sim_exec_run = nullptr;
-      c->sim_graph = c->sim_graph_run = nullptr;
-      // captures `steps` steps (even) into *graph and instantiates *exec
-      auto capture = [&](int steps, hipGraph_t* graph, hipGraphExec_t* exec) -> int {
-        FL_HIP(hipStreamBeginCapture(c->cap_stream, hipStreamCaptureModeThreadLocal));
-        int r = FL_OK;
-        for (int k = 0; k < steps && !r; ++k) r = one_step(k & 1, c->cap_stream);
-        hipGraph_t gr = nullptr;
-        const hipError_t e = hipStreamEndCapture(c->cap_stream, &gr);
-        if (r) {
-          if (gr) (void)hipGraphDestroy(gr);
-          return r;
-        }
-        if (e != hipSuccess)
-          return fail(FL_ERR_HIP, "step graph capture failed: %s", hipGetErrorString(e));
-        *graph = gr;
-        FL_HIP(hipGraphInstantiate(exec, gr, nullptr, nullptr, 0));
-        return FL_OK;
-      };
-      if ((rc = capture(2, &c->sim_graph, &c->sim_exec))) return rc;
-      if ((rc = capture(kSimGraphSteps, &c->sim_graph_run, &c->sim_exec_run))) return rc;
+    const bool again = memcmp(&key, &c->sim_key, sizeof(key)) == 0;
+    if (!again) {
+      drop_sim_graphs(c);
       c->sim_key = key;
     }
+    graphs = again || p->max_iters >= kSimGraphMin;
+    const int64_t steps[2] = {p->max_iters >= kSimGraphSteps ? kSimGraphSteps : 0, left_over};
+    for (int g = 0; graphs && g < 2; ++g) {
+      if (c->sim_exec[g] || !steps[g]) continue;
+      FL_HIP(hipStreamBeginCapture(c->cap_stream, hipStreamCaptureModeThreadLocal));
+      for (int64_t k = 0; k < steps[g] && !rc; ++k)
+        rc = launch_sim_step(c, state, work, s, p, c->sim, k, c->cap_stream);
+      hipGraph_t gr = nullptr;
+      const hipError_t e = hipStreamEndCapture(c->cap_stream, &gr);
+      if (rc) {
+        if (gr) (void)hipGraphDestroy(gr);
+        return rc;
+      }
+      if (e != hipSuccess)
+        return fail(FL_ERR_HIP, "step graph capture failed: %s", hipGetErrorString(e));
+      c->sim_graph[g] = gr;
+      FL_HIP(hipGraphInstantiate(&c->sim_exec[g], gr, nullptr, nullptr, 0));
+    }
   }
-  while (launched < p->max_iters) {
-    const int64_t nb = (p->max_iters - launched) < kBatch ? (p->max_iters - launched) : kBatch;
-    if (c->use_graphs) {
-      int64_t k = 0;
+  do {
+    const int64_t nb = std::min<int64_t>(p->max_iters - launched, kBatch);
+    int64_t k = 0;
+    if (graphs) {
       for (; k + kSimGraphSteps <= nb; k += kSimGraphSteps)
-        FL_HIP(hipGraphLaunch(c->sim_exec_run, st));
-      for (; k < nb; k += 2) FL_HIP(hipGraphLaunch(c->sim_exec, st));
-    } else {
-      for (int64_t k = 0; k < nb; ++k) {
-        rc = one_step((int)((launched + k) & 1), st);
-        if (rc) return rc;
+        FL_HIP(hipGraphLaunch(c->sim_exec[0], st));
+      if (nb - k == left_over && left_over) {
+        FL_HIP(hipGraphLaunch(c->sim_exec[1], st));
+        k = nb;
       }
     }
+    for (; k < nb; ++k)
+      if ((rc = launch_sim_step(c, state, work, s, p, c->sim, launched + k, st))) return rc;
     launched += nb;
-    FL_HIP(hipMemcpyAsync(c->host_ctl, c->ctl, sizeof(fl::StepCtl), hipMemcpyDeviceToHost, st));
+    FL_HIP(hipMemcpyAsync(c->host_sim, c->sim, sizeof(fl::SimCtl), hipMemcpyDeviceToHost, st));
     FL_HIP(hipStreamSynchronize(st));
-    if (!c->host_ctl->active) break;
-  }
-  if (launched == 0) {
-    // max_iters == 0: no step ran; the result is the freshly initialised
-    // control block (t = 0, no iterations) with the initial max wavespeed.
-    FL_HIP(hipMemcpyAsync(c->host_ctl, c->ctl, sizeof(fl::StepCtl), hipMemcpyDeviceToHost, st));
-    FL_HIP(hipStreamSynchronize(st));
-  }
-  const fl::StepCtl hc = *c->host_ctl;
+  } while (launched < p->max_iters && c->host_sim->c.active);
+  const fl::SimCtl hs = *c->host_sim;
+  const fl::StepCtl hc = hs.c;
   if (state->ndim == 1 && (hc.iters & 1)) {
     const int64_t bytes = cell_count(state) * 3 * (state->dtype == FL_F64 ? 8 : 4);
     FL_HIP(hipMemcpyAsync(state->data, work->data, (size_t)bytes, hipMemcpyDeviceToDevice, st));
     FL_HIP(hipStreamSynchronize(st));
   }
-  const double final_ws = bits_to_double(hc.ws_bits[hc.iters & 1]);
+  const double final_ws = bits_to_double(hs.ws[hc.iters % sim_slots(state->ndim)]);
   if (result) {
     result->run_time = hc.t;
     result->iters = hc.iters;

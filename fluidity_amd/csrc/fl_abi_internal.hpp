@@ -18,7 +18,7 @@
 #define FL_VLC_KERNELS 1
 #endif
 
-// What a captured fl_simulate step pair depends on (compared bytewise).
+// What a captured run of fl_simulate's steps depends on (compared bytewise).
 struct SimGraphKey {
   void* a;
   void* b;
@@ -38,8 +38,10 @@ enum : int { kShapeRule = 0, kShapeTuning = 1, kShapeCell = 2 };
 
 struct fl_context {
   int device;
-  fl::StepCtl* ctl;            // device control block of fl_simulate
+  fl::StepCtl* ctl;            // device control block of the two-material loop
   unsigned long long* ws_tmp;  // device scratch for fl_max_wavespeed
+  fl::SimCtl* sim;             // device control words of fl_simulate's launched steps
+  fl::SimCtl* host_sim;        // pinned host mirror of sim
   double* partial;             // device partial sums, kSumBlocks * 4
   fl::StepCtl* host_ctl;       // pinned host mirror of ctl
   double* host_partial;        // pinned host mirror of partial
@@ -49,15 +51,13 @@ struct fl_context {
   int32_t shape[2];            // kShape* of the x and the y sweep
   hipEvent_t step_ev;          // fl_mm_simulate: the step's control block is on the host
   int64_t eik_sweeps;          // sweeps the last eikonal solve took (first batch size)
-  int use_graphs;              // fl_simulate replays a captured pair of steps
+  int use_graphs;              // fl_simulate replays captured runs of steps
                                // (small 1D grids: runs the persistent loop)
   fl::PersistCtl* pctl;        // device control words of the persistent 1D loop
   fl::PersistCtl* host_pctl;   // pinned host mirror of pctl
   hipStream_t cap_stream;      // capture stream of that graph
-  hipGraph_t sim_graph;        // a pair of steps (both parities)
-  hipGraphExec_t sim_exec;
-  hipGraph_t sim_graph_run;    // kSimGraphSteps steps
-  hipGraphExec_t sim_exec_run;
+  hipGraph_t sim_graph[2];     // a run of kSimGraphSteps steps, and the steps left over
+  hipGraphExec_t sim_exec[2];
   SimGraphKey sim_key;
 };
 
@@ -120,6 +120,11 @@ int64_t cell_count(const fl_field* f);
 int launch_sweep(const fl_context* ctx, const fl_field* in, const fl_field* out, int dim,
                  const fl_scheme* s, double dtdh, const fl::StepCtl* ctl,
                  unsigned long long* ws_out, hipStream_t stream);
+// Step k of a simulation on state -> work (-> state in 2D): the sweeps, the
+// first of which takes dt from the maximum in sim.
+int launch_sim_step(const fl_context* ctx, const fl_field* state, const fl_field* work,
+                    const fl_scheme* s, const fl_sim_params* p, fl::SimCtl* sim, int64_t k,
+                    hipStream_t stream);
 // Both materials' sweeps of dimension `dim` in one launch; ctl (nullable)
 // as in launch_sweep.
 int launch_sweep2(const fl_context* ctx, const fl_field* const in[2], const fl_field* const out[2],

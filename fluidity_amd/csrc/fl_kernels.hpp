@@ -24,6 +24,23 @@ struct StepCtl {
   int pad;
 };
 
+// Device-resident control of fl_simulate's launched steps.  The first sweep of
+// step k takes dt from the maximum itself (sweep_begin), so a step is its
+// sweeps and nothing else: every workgroup reads t[k & 1], iters[k & 1] and
+// the maximum ws[k % n] (n = 2 slots on 2D grids, 3 on 1D ones, where one
+// sweep reads the maximum and reduces the next) and computes the same dt; the
+// first workgroup writes the other halves, the block that the step's second
+// sweep reads and the zero of a slot that nobody reads or reduces into in
+// this sweep.
+struct SimCtl {
+  StepCtl c;         // dt, dtdh, active of the step; t and iters after it
+  double t[2];       // run time before step k in t[k & 1]
+  long long iters[2];
+  // maximum wavespeeds as bits, on a cache line that no sweep reads dt from
+  // while others reduce into it
+  alignas(128) unsigned long long ws[3];
+};
+
 // Control words of the persistent 1D step loop (persist1d_kernel): the
 // fused wavespeed maxima in three slots (step k reads slot k % 3, reduces into
 // (k + 1) % 3 and clears (k + 2) % 3), run time and iteration count in two
@@ -55,6 +72,13 @@ struct SweepArgs {
   int pad;
   T dtdh_host;         // used when ctl == nullptr
   const StepCtl* ctl;  // nullable: provides dtdh and the active flag
+  // nullable: the first sweep of a step of fl_simulate, which turns the
+  // maximum into dt (ctl unused)
+  SimCtl* sim;
+  int sim_half, sim_ws, sim_zero;  // k & 1, the slot read, the slot cleared
+  int pad2;
+  double cfl, dh, sim_time;
+  long long max_iters;
   unsigned long long* ws_out;  // nullable: fused max wavespeed (bit pattern)
 };
 
@@ -133,6 +157,7 @@ __global__ void zero_u64_kernel(unsigned long long* p);
 __global__ void step_control_kernel(StepCtl* ctl, int parity, double cfl, double dh,
                                     double sim_time, long long max_iters);
 __global__ void init_control_kernel(StepCtl* ctl);
+__global__ void init_sim_kernel(SimCtl* sim);
 __global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh);
 template <typename T, int FLUX>
 __global__ void persist1d_kernel(SweepArgs<T> a_ab, SweepArgs<T> a_ba, PersistCtl* pc,

@@ -1,8 +1,8 @@
 // fl_noalloc.hip -- fl_simulate_noalloc: the device step loop of fl_simulate
 // for callers that cannot allocate device or pinned memory (serving loops,
 // harnesses that forbid hipMalloc).  It takes no context: its only scratch,
-// the step-control block that the kernels read dt/dh from and reduce the
-// fused CFL maximum into, lives in a file-scope device array, one copy per
+// the control words that the kernels take dt/dh from and reduce the fused CFL
+// maximum into, lives in a file-scope device array, one copy per
 // GPU, held until the process ends.
 #include <hip/hip_runtime.h>
 
@@ -16,22 +16,22 @@ using namespace fl::abi;
 
 namespace {
 
-// Room for one step-control block (fl::StepCtl, 48 bytes).  The loop needs
+// Room for one simulation's control words (fl::SimCtl, 256 bytes).  The loop needs
 // exactly one whatever the grid size, so no grid is too large for it; every
 // call on a device shares that device's copy.
 constexpr size_t kScratchBytes = 256;
-static_assert(sizeof(fl::StepCtl) <= kScratchBytes, "step-control block must fit the scratch");
+static_assert(sizeof(fl::SimCtl) <= kScratchBytes, "the control words must fit the scratch");
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mu;
-fl::StepCtl* scratch_ptr[kMaxDevices];  // device address of `scratch` per device
+fl::SimCtl* scratch_ptr[kMaxDevices];  // device address of `scratch` per device
 
 // The device address of this device's `scratch` (looked up once per device,
 // with that device current).  In host code the array's name is only a
 // host-side handle: kernels and copies take this address.
-int scratch_of(int dev, fl::StepCtl** out) {
+int scratch_of(int dev, fl::SimCtl** out) {
   if (dev < 0 || dev >= kMaxDevices)
     return fail(FL_ERR_UNSUPPORTED, "device %d: at most %d devices", dev, kMaxDevices);
   std::lock_guard<std::mutex> lock(scratch_mu);
@@ -41,7 +41,7 @@ int scratch_of(int dev, fl::StepCtl** out) {
     if (e != hipSuccess || !p)
       return fail(FL_ERR_HIP, "hipGetSymbolAddress(scratch) failed on device %d: %s", dev,
                   hipGetErrorString(e));
-    scratch_ptr[dev] = (fl::StepCtl*)p;
+    scratch_ptr[dev] = (fl::SimCtl*)p;
   }
   *out = scratch_ptr[dev];
   return FL_OK;
@@ -69,46 +69,35 @@ int fl_simulate_noalloc(const fl_tuning* tuning, fl_field* state, fl_field* work
   memset(&c, 0, sizeof(c));
   FL_HIP(hipGetDevice(&c.device));
   if ((rc = resolve_tuning(tuning, &c.tuning, c.shape))) return rc;
-  fl::StepCtl* ctl = nullptr;
-  if ((rc = scratch_of(c.device, &ctl))) return rc;
+  fl::SimCtl* sim = nullptr;
+  if ((rc = scratch_of(c.device, &sim))) return rc;
   hipStream_t st = (hipStream_t)stream;
 
-  hipLaunchKernelGGL(fl::init_control_kernel, dim3(1), dim3(1), 0, st, ctl);
-  if ((rc = launch_max_ws(state, s, &ctl->ws_bits[0], st))) return rc;
-  // Steps in batches; the host reads the control block once per batch into a
+  hipLaunchKernelGGL(fl::init_sim_kernel, dim3(1), dim3(1), 0, st, sim);
+  if ((rc = launch_max_ws(state, s, &sim->ws[0], st))) return rc;
+  // Steps in batches; the host reads the control words once per batch into a
   // stack copy and stops when the loop condition fails.  Steps past it do
-  // nothing (their kernels read the inactive flag).
+  // nothing.
   const int64_t kBatch = 256;
-  fl_field a = *state, b = *work;
-  fl::StepCtl hc;
-  memset(&hc, 0, sizeof(hc));
+  fl::SimCtl hs;
+  memset(&hs, 0, sizeof(hs));
   int64_t launched = 0;
   do {
     const int64_t left = p->max_iters - launched;
     const int64_t nb = left < kBatch ? left : kBatch;
-    for (int64_t k = 0; k < nb; ++k) {
-      const int parity = (int)((launched + k) & 1);
-      hipLaunchKernelGGL(fl::step_control_kernel, dim3(1), dim3(1), 0, st, ctl, parity, p->cfl,
-                         p->dh, p->sim_time, (long long)p->max_iters);
-      unsigned long long* ws_next = &ctl->ws_bits[parity ^ 1];
-      if (state->ndim == 1) {
-        rc = launch_sweep(&c, parity ? &b : &a, parity ? &a : &b, 0, s, 1.0, ctl, ws_next, st);
-      } else {
-        rc = launch_sweep(&c, &a, &b, 0, s, 1.0, ctl, nullptr, st);
-        if (!rc) rc = launch_sweep(&c, &b, &a, 1, s, 1.0, ctl, ws_next, st);
-      }
-      if (rc) return rc;
-    }
+    for (int64_t k = 0; k < nb; ++k)
+      if ((rc = launch_sim_step(&c, state, work, s, p, sim, launched + k, st))) return rc;
     launched += nb;
-    FL_HIP(hipMemcpyAsync(&hc, ctl, sizeof(hc), hipMemcpyDeviceToHost, st));
+    FL_HIP(hipMemcpyAsync(&hs, sim, sizeof(hs), hipMemcpyDeviceToHost, st));
     FL_HIP(hipStreamSynchronize(st));
-  } while (launched < p->max_iters && hc.active);
+  } while (launched < p->max_iters && hs.c.active);
+  const fl::StepCtl hc = hs.c;
   if (state->ndim == 1 && (hc.iters & 1)) {
     const int64_t bytes = cell_count(state) * 3 * (state->dtype == FL_F64 ? 8 : 4);
     FL_HIP(hipMemcpyAsync(state->data, work->data, (size_t)bytes, hipMemcpyDeviceToDevice, st));
     FL_HIP(hipStreamSynchronize(st));
   }
-  const double final_ws = bits_to_double(hc.ws_bits[hc.iters & 1]);
+  const double final_ws = bits_to_double(hs.ws[hc.iters % (state->ndim == 1 ? 3 : 2)]);
   if (result) {
     result->run_time = hc.t;
     result->iters = hc.iters;

@@ -359,6 +359,12 @@ __global__ void init_control_kernel(StepCtl* ctl) {
   ctl->pad = 0;
 }
 
+__global__ void init_sim_kernel(SimCtl* sim) {
+  const SimCtl zero = {};
+  *sim = zero;
+  sim->c.active = 1;
+}
+
 // ---------------------------------------------------------------------------
 // FP64 conservation sums (per component), used beside the FP32 bulk path
 // ---------------------------------------------------------------------------

@@ -372,8 +372,46 @@ __device__ __forceinline__ void ws_fold(const T* u, const SweepArgs<T>& a,
   }
 }
 
+// One step of Parameters::update_time_delta / dt_dh / update_simulation_info
+// (simulator/parameters.hpp:60-99) and the loop condition of
+// SimulatorImpl::simulate (simulator/simulator_impl.hpp:235), by every
+// workgroup of the step's first sweep; `writer` (one workgroup's first thread)
+// publishes it.  False: the loop has ended.  A control kernel between the
+// steps took 4.4 us of a 64^2 step of 18.
 template <typename T>
-__device__ __forceinline__ bool sweep_dtdh(const SweepArgs<T>& a, T& dtdh) {
+__device__ __forceinline__ bool sweep_begin(const SweepArgs<T>& a, bool writer, T& dtdh) {
+  SimCtl* const sim = a.sim;
+  const int h = a.sim_half;
+  const double t = sim->t[h];
+  const long long it = sim->iters[h];
+  const double maxws = __longlong_as_double((long long)sim->ws[a.sim_ws]);
+  const bool active = t < a.sim_time && it < a.max_iters;
+  const double dt = a.cfl * a.dh / maxws;
+  const double r = dt / a.dh;
+  if (writer) {
+    const double tn = active ? t + dt : t;
+    const long long in = active ? it + 1 : it;
+    sim->t[h ^ 1] = tn;
+    sim->iters[h ^ 1] = in;
+    sim->c.t = tn;
+    sim->c.iters = in;
+    sim->c.active = active ? 1 : 0;
+    if (active) {
+      sim->c.dt = dt;
+      sim->c.dtdh = r;
+      sim->ws[a.sim_zero] = 0ull;
+    }
+  }
+  dtdh = (T)r;
+  return active;
+}
+
+// FIRST: an x or 1D sweep, which may begin a step; writer as in sweep_begin.
+template <bool FIRST, typename T>
+__device__ __forceinline__ bool sweep_dtdh(const SweepArgs<T>& a, bool writer, T& dtdh) {
+  if constexpr (FIRST) {
+    if (a.sim) return sweep_begin(a, writer, dtdh);
+  }
   if (a.ctl) {
     if (!a.ctl->active) return false;
     dtdh = (T)a.ctl->dtdh;
@@ -414,7 +452,7 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, int64_t bx, 
   T* const sG = sL + S * (int)blockDim.x;        // [S][B]
 
   T dtdh;
-  if (!sweep_dtdh(a, dtdh)) return;
+  if (!sweep_dtdh<true>(a, bx == 0 && by == 0 && threadIdx.x == 0, dtdh)) return;
   const T half_dtdh = T(0.5) * dtdh;
   const T dhdt = T(1) / dtdh;
 
@@ -624,7 +662,7 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, int64_t bx, 
   T* const ring = sK + W;                        // [B / 64][kYRing][S][64]
 
   T dtdh;
-  if (!sweep_dtdh(a, dtdh)) return;
+  if (!sweep_dtdh<false>(a, false, dtdh)) return;
   const T half_dtdh = T(0.5) * dtdh;
   const T dhdt = T(1) / dtdh;
 
@@ -893,6 +931,28 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// sweep_begin for a staged tile, and the barrier after its staging: the last
+// wave, which stages one row only, reads the control words and divides while
+// the others stage (in every wave the two FP64 divisions were a tenth of the
+// FP32 tile's instructions).
+template <typename T>
+__device__ __forceinline__ bool cell_begin(const SweepArgs<T>& a, int w, int t, bool writer,
+                                           T& dtdh) {
+  __shared__ T s_dtdh;
+  __shared__ int s_active;
+  if (w == kCellWaves - 1) {
+    T r = T(0);
+    const bool active = sweep_begin(a, writer && t == 0, r);
+    if (t == 0) {
+      s_dtdh = r;
+      s_active = active ? 1 : 0;
+    }
+  }
+  __syncthreads();
+  dtdh = s_dtdh;
+  return s_active != 0;
+}
+
 // x sweep of columns [62 bx, 62 bx + 62) of rows [kCellWaves by, kCellWaves
 // (by + 1)).  Lanes 0 and 63 hold the columns beside them, whose face states
 // the tile's outer faces need.  Called by every thread of a workgroup of
@@ -903,12 +963,15 @@ __device__ __forceinline__ void cell_x_tile(const SweepArgs<T>& a, int64_t bx, i
   constexpr bool F = UseFast<T, FAST>::value;
   const int limiter = VLC ? int(kLimVanLeer) : a.limiter;
   const int form = VLC ? int(kFormCons) : a.form;
-  T dtdh;
-  if (!sweep_dtdh(a, dtdh)) return;
-  const T half_dtdh = T(0.5) * dtdh;
-  const T dhdt = T(1) / dtdh;
   const int t = (int)(threadIdx.x & 63);
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // read ahead of the tile, used after its staging
+  T dtdh = a.dtdh_host;
+  int active = 1;
+  if (a.ctl) {
+    active = a.ctl->active;
+    dtdh = (T)a.ctl->dtdh;
+  }
   extern __shared__ __align__(16) unsigned char fl_c_lds[];
   T* const sP = reinterpret_cast<T*>(fl_c_lds);  // [NW + 6][kCellCols]
   T* const sVX = sP + (NW + 6) * kCellCols;      // [NW][kCellCols]
@@ -925,7 +988,14 @@ __device__ __forceinline__ void cell_x_tile(const SweepArgs<T>& a, int64_t bx, i
   issue_at<T, S>(a, row, fy, ll, Ql);
   issue_at<T, S>(a, row, fy, lr, Qr);
   cell_stage<T, F>(a, xc, yb, w, t, row, fy, lc, sP, sVX, sVY, u0);
-  __syncthreads();
+  if (a.sim) {
+    if (!cell_begin(a, w, t, bx == 0 && by == 0, dtdh)) return;
+  } else {
+    __syncthreads();
+    if (!active) return;
+  }
+  const T half_dtdh = T(0.5) * dtdh;
+  const T dhdt = T(1) / dtdh;
   unsigned long long wsmax = 0ull;
   if (r < a.ny) {  // uniform over the wave
     const T chi = cell_chi<T, F>(a, w, t, sP, sVX, sVY);
@@ -964,12 +1034,15 @@ __device__ __forceinline__ void cell_y_tile(const SweepArgs<T>& a, int64_t bx, i
   constexpr bool F = UseFast<T, FAST>::value;
   const int limiter = VLC ? int(kLimVanLeer) : a.limiter;
   const int form = VLC ? int(kFormCons) : a.form;
-  T dtdh;
-  if (!sweep_dtdh(a, dtdh)) return;
-  const T half_dtdh = T(0.5) * dtdh;
-  const T dhdt = T(1) / dtdh;
   const int t = (int)(threadIdx.x & 63);
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // read ahead of the tile, used after its staging
+  T dtdh = a.dtdh_host;
+  int active = 1;
+  if (a.ctl) {
+    active = a.ctl->active;
+    dtdh = (T)a.ctl->dtdh;
+  }
   extern __shared__ __align__(16) unsigned char fl_c_lds[];
   T* const sP = reinterpret_cast<T*>(fl_c_lds);  // as in cell_x_tile
   T* const sVX = sP + (NW + 6) * kCellCols;
@@ -987,6 +1060,9 @@ __device__ __forceinline__ void cell_y_tile(const SweepArgs<T>& a, int64_t bx, i
   issue_near<T, S>(a, r - 1, lc, Ql);
   issue_near<T, S>(a, r + 1, lc, Qr);
   __syncthreads();
+  if (!active) return;
+  const T half_dtdh = T(0.5) * dtdh;
+  const T dhdt = T(1) / dtdh;
   T R[S], L[S], G[S];
   const bool live = r <= a.ny;  // uniform over the wave; row ny is the ghost above the grid
   if (live) {

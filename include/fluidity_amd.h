@@ -218,9 +218,9 @@ int fl_simulate_noalloc(const fl_tuning* tuning, fl_field* state, fl_field* work
                         const fl_scheme* scheme, const fl_sim_params* params,
                         fl_sim_result* result, void* stream);
 
-/* fl_simulate captures a pair of steps (control kernel + sweeps, both
- * parities) in a hipGraph on first use for a given grid, scheme, parameters
- * and tuning, and replays it (default); a 1D line of at most 2^16 cells
+/* fl_simulate captures runs of steps in hipGraphs for a given grid, scheme,
+ * parameters and tuning and replays them (default): at once for loops of 72
+ * steps or more, from the second call on for shorter ones; a 1D line of at most 2^16 cells
  * (exact FP64 or FP32) instead runs the whole loop in one cooperative launch
  * with a grid barrier per step.  enable = 0 launches every kernel. */
 int fl_ctx_set_graphs(fl_context* ctx, int enable);
