@@ -55,6 +55,7 @@ struct fl_context {
                                // (small 1D grids: runs the persistent loop)
   fl::PersistCtl* pctl;        // device control words of the persistent 1D loop
   fl::PersistCtl* host_pctl;   // pinned host mirror of pctl
+  unsigned long long* words;   // its workgroups' exchange, 3 slots
   hipStream_t cap_stream;      // capture stream of that graph
   hipGraph_t sim_graph[2];     // a run of kSimGraphSteps steps, and the steps left over
   hipGraphExec_t sim_exec[2];

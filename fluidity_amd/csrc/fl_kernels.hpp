@@ -41,18 +41,15 @@ struct SimCtl {
   alignas(128) unsigned long long ws[3];
 };
 
-// Control words of the persistent 1D step loop (persist1d_kernel): the
-// fused wavespeed maxima in three slots (step k reads slot k % 3, reduces into
-// (k + 1) % 3 and clears (k + 2) % 3), run time and iteration count in two
-// (step k reads k % 2, writes (k + 1) % 2), the last dt, the grid-barrier
-// counter of the launch and a timeout flag.
+// Loop state of the persistent 1D step loop (persist1d_kernel) between its
+// launches, and its timeout flag.
 struct PersistCtl {
-  unsigned long long ws[3];
-  unsigned long long t[2];  // run time as bits
-  long long iters[2];
-  double dt;
-  unsigned int bar;
+  unsigned long long ws;  // maximum wavespeed of the state as bits
+  double t;
+  long long iters;
+  double dt;              // last step's
   int err;
+  int pad;
 };
 
 template <typename T>
@@ -119,6 +116,14 @@ constexpr int kCellYCols = 64, kCellYRows = kCellWaves - 2;
 // unseen (two rounds of the blocks the device holds).
 constexpr unsigned kCellFewBlocks = 1024;
 
+// Persistent 1D loop: cells of a wave's segment (4 lanes on either side hold
+// the neighbours'), waves of a workgroup, workgroups and the words each
+// publishes per step (the maximum, and 3 values of 4 cells at either end).
+constexpr int kPersistCells = 56;
+constexpr int kPersistMaxWaves = 16;
+constexpr int kPersistMaxGroups = 4 * 64;
+constexpr int kPersistWords = 25;
+
 // Standalone wavespeed max: at most kMaxWsBlocks workgroups of kMaxBlock
 // threads, each thread loading kMaxWsUnroll cells per iteration.
 constexpr int kMaxWsBlocks = 512;
@@ -159,10 +164,11 @@ __global__ void step_control_kernel(StepCtl* ctl, int parity, double cfl, double
 __global__ void init_control_kernel(StepCtl* ctl);
 __global__ void init_sim_kernel(SimCtl* sim);
 __global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh);
-template <typename T, int FLUX>
-__global__ void persist1d_kernel(SweepArgs<T> a_ab, SweepArgs<T> a_ba, PersistCtl* pc,
-                                 double cfl, double dh, double sim_time, long long max_iters,
-                                 long long k0, long long nsteps, unsigned int spin_limit);
-__global__ void persist_init_kernel(PersistCtl* pc, const unsigned long long* ws0);
-__global__ void persist_bar_reset_kernel(PersistCtl* pc);
+template <typename T, int FLUX, bool FAST, bool VLC>
+__global__ void persist1d_kernel(SweepArgs<T> a, PersistCtl* pc, unsigned long long* words,
+                                 int nseg, double cfl, double dh, double sim_time,
+                                 long long max_iters, long long nsteps, int first,
+                                 unsigned int spin_limit);
+__global__ void persist_init_kernel(PersistCtl* pc, unsigned long long* words, int count,
+                                    int first);
 }  // namespace fl

@@ -9,12 +9,21 @@
 //     v_rsq_f64 (FP32: v_sqrt_f32);
 //   - the van Leer slope is its closed form: with r = b/f,
 //     (b + f)/2 * 2 min(r, 1)/(1 + r) equals b when 0 < r <= 1 and f when
-//     r > 1, i.e. minmod(b, f), so it needs no division at all;
-//   - multiply-adds contract to FMAs.
+//     r > 1, i.e. minmod(b, f), the median of b, f and 0: no division and no
+//     branch (FP64 four v_min/v_max, FP32 one v_med3);
+//   - an ideal gas's shock speed a sqrt(1 + q (p*/p - 1)) is one root of
+//     gamma/rho (p + q (p* - p)), without the quotient;
+//   - multiply-adds are FMAs, written out: the compiler contracts within a
+//     basic block only, so left to it the rounding would depend on the kernel
+//     that a formula is inlined into, and the step loops, batches and launch
+//     shapes would differ in their last bits.
 // Results differ from the reference's in the last bits of each operation; the
 // FP64 fast path is held to 1e-12 relative L-inf of the reference's results
 // over a 100-step run.  FP32 uses these forms always.  Branches (limiter
 // signs, flattening threshold, HLLC wave ordering) are the reference's.
+// Measured (FP64 HLLC, 4096^2, 4 steps): 2950 us with the quotient forms the
+// compiler contracted, 2950 us with these: the same speed, with bits that no
+// longer depend on the kernel.
 #pragma once
 
 #include "fl_numerics.hpp"
@@ -69,8 +78,22 @@ template <typename T> __device__ __forceinline__ T div(T a, T b) { return a * rc
 // the comparison-based fl::smin/smax only in which operand a NaN or a signed
 // zero leaves: a NaN operand yields the other one, as std::min(max, NaN) and
 // std::max(0, NaN) do where the reference uses them to clamp.
-template <typename T> __device__ __forceinline__ T mn(T a, T b) { return __builtin_fmin(a, b); }
-template <typename T> __device__ __forceinline__ T mx(T a, T b) { return __builtin_fmax(a, b); }
+__device__ __forceinline__ double mn(double a, double b) { return __builtin_fmin(a, b); }
+__device__ __forceinline__ double mx(double a, double b) { return __builtin_fmax(a, b); }
+__device__ __forceinline__ float mn(float a, float b) { return __builtin_fminf(a, b); }
+__device__ __forceinline__ float mx(float a, float b) { return __builtin_fmaxf(a, b); }
+
+// a b + c with one rounding.
+__device__ __forceinline__ double fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// minmod(a, b): the median of a, b and 0.
+__device__ __forceinline__ double minmod(double a, double b) {
+  return fast::mx(fast::mn(a, b), fast::mn(fast::mx(a, b), 0.0));
+}
+__device__ __forceinline__ float minmod(float a, float b) {
+  return __builtin_amdgcn_fmed3f(a, b, 0.0f);
+}
 
 // Primitive quantities and 1/rho of one conservative state.
 template <typename T, int ND> struct PrimR {
@@ -79,19 +102,20 @@ template <typename T, int ND> struct PrimR {
   T rinv;
 };
 
-template <typename T, int ND>
+// FIRST: the velocity component whose square is rounded before the others'
+// are added to it (the last, unless said otherwise).
+template <typename T, int ND, int FIRST = ND - 1>
 __device__ __forceinline__ PrimR<T, ND> prim_of(const T* U, const Material<T>& m) {
-#pragma clang fp contract(fast)
   PrimR<T, ND> w;
   w.rinv = fast::rcp(U[0]);
-  T sum = T(0);
 #pragma unroll
-  for (int i = 0; i < ND; ++i) {
-    w.vel[i] = U[2 + i] * w.rinv;
-    sum += w.vel[i] * w.vel[i];
-  }
-  w.p = m.gm1 * (U[1] - T(0.5) * U[0] * sum);
-  if (m.corr) w.p = w.p - m.gpinf;
+  for (int i = 0; i < ND; ++i) w.vel[i] = U[2 + i] * w.rinv;
+  T sum = w.vel[FIRST] * w.vel[FIRST];
+#pragma unroll
+  for (int i = ND - 1; i >= 0; --i)
+    if (i != FIRST) sum = fast::fma(w.vel[i], w.vel[i], sum);
+  const T e = fast::fma(T(-0.5) * U[0], sum, U[1]);
+  w.p = m.corr ? fast::fma(m.gm1, e, -m.gpinf) : m.gm1 * e;
   return w;
 }
 
@@ -106,17 +130,15 @@ __device__ __forceinline__ Prim<T, ND> as_prim(const PrimR<T, ND>& w) {
 
 template <typename T>
 __device__ __forceinline__ T sound_speed(T p, T rinv, const Material<T>& m) {
-#pragma clang fp contract(fast)
   if (m.stiff) return fast::sqt(m.gamma * (p + m.p_inf) * rinv);
   return fast::sqt(m.gamma * p * rinv);
 }
 
 template <typename T, int ND, int D>
 __device__ __forceinline__ void euler_flux(const T* U, const PrimR<T, ND>& w, T* F) {
-#pragma clang fp contract(fast)
   const T v = w.vel[D];
   F[0] = U[2 + D];
-  F[2 + D] = U[2 + D] * v + w.p;
+  F[2 + D] = fast::fma(U[2 + D], v, w.p);
   F[1] = v * (U[1] + w.p);
 #pragma unroll
   for (int o = 0; o < ND; ++o)
@@ -134,7 +156,6 @@ __device__ __forceinline__ T max_wavespeed(const PrimR<T, ND>& w, const Material
 // Superbee's limit (superbee_limiter.hpp:72-89) of the ratio a / b.
 template <typename T>
 __device__ __forceinline__ T superbee(T a, T b) {
-#pragma clang fp contract(fast)
   const T r = fast::div(a, b);
   if (r <= T(0) || b == T(0)) return T(0);
   if (r <= T(0.5)) return T(2) * r;
@@ -147,17 +168,14 @@ __device__ __forceinline__ T superbee(T a, T b) {
 // (van_leer_limiter.hpp:65-74) in closed form: minmod(back, fwrd).
 template <typename T>
 __device__ __forceinline__ T slope_cons(int limiter, T back, T fwrd) {
-#pragma clang fp contract(fast)
   if (limiter == kLimSuperbee) return (back + fwrd) * T(0.5) * fast::superbee(back, fwrd);
-  if (!(back * fwrd > T(0))) return T(0);
-  return (fabs(back) <= fabs(fwrd)) ? back : fwrd;
+  return fast::minmod(back, fwrd);
 }
 
 // Primitive form: the limit of the primitive differences (rb, rf) scales the
 // average of the conservative ones (limiting/limiter.hpp:79-97).
 template <typename T>
 __device__ __forceinline__ T slope_prim(int limiter, T back, T fwrd, T rb, T rf) {
-#pragma clang fp contract(fast)
   const T avg = (back + fwrd) * T(0.5);
   if (limiter == kLimSuperbee) return avg * fast::superbee(rb, rf);
   if (!(rb * rf > T(0))) return T(0);
@@ -169,7 +187,6 @@ __device__ __forceinline__ T slope_prim(int limiter, T back, T fwrd, T rb, T rf)
 template <typename T>
 __device__ __forceinline__ T chi_factor(T p_pprev, T p_prev, T p_next, T p_nnext, T v_prev,
                                         T v_next, const Material<T>& m) {
-#pragma clang fp contract(fast)
   const T u_factor = v_prev - v_next;
   const T dp = fabs(p_next - p_prev);
   T pmin = fast::mn(p_next, p_prev);
@@ -180,7 +197,7 @@ __device__ __forceinline__ T chi_factor(T p_pprev, T p_prev, T p_next, T p_nnext
   const bool flatten = u_factor > T(0) && pmin >= T(0) && dp > T(0.33) * pmin;
   if (!flatten) return T(1);
   const T z = fast::div(dp, T(fabs(p_nnext - p_pprev)));
-  const T temp = T(1) - (z - T(0.75)) * T(10);
+  const T temp = fast::fma(T(0.75) - z, T(10), T(1));
   return fast::mn(T(1), fast::mx(T(0), temp));
 }
 
@@ -190,7 +207,6 @@ template <typename T, int ND, int D>
 __device__ __forceinline__ void evolve_faces(const T* um, const T* u0, const T* up, T chi,
                                              T half_dtdh, int limiter, int form,
                                              const Material<T>& m, T* R, T* L) {
-#pragma clang fp contract(fast)
   constexpr int S = 2 + ND;
   T rb[S], rf[S];
   if (form == kFormPrim) {
@@ -215,84 +231,106 @@ __device__ __forceinline__ void evolve_faces(const T* um, const T* u0, const T* 
     const T fwrd = up[k] - u0[k];
     const T lim = (form == kFormPrim) ? fast::slope_prim(limiter, back, fwrd, rb[k], rf[k])
                                       : fast::slope_cons(limiter, back, fwrd);
-    const T delta = lim * cscale;
-    plus[k] = u0[k] + delta;
-    minus[k] = u0[k] - delta;
+    plus[k] = fast::fma(lim, cscale, u0[k]);
+    minus[k] = fast::fma(-lim, cscale, u0[k]);
   }
-  T fm[S], fp[S];
   const PrimR<T, ND> wmi = fast::prim_of<T, ND>(minus, m);
   const PrimR<T, ND> wpl = fast::prim_of<T, ND>(plus, m);
-  fast::euler_flux<T, ND, D>(minus, wmi, fm);
-  fast::euler_flux<T, ND, D>(plus, wpl, fp);
+  // F(minus) - F(plus)
+  const T vm = wmi.vel[D], vp = wpl.vel[D];
+  T df[S];
+  df[0] = minus[2 + D] - plus[2 + D];
+  df[1] = fast::fma(vm, minus[1] + wmi.p, -(vp * (plus[1] + wpl.p)));
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+    df[2 + i] = i == D ? fast::fma(minus[2 + D], vm, wmi.p) - fast::fma(plus[2 + D], vp, wpl.p)
+                       : fast::fma(minus[2 + i], vm, -(plus[2 + i] * vp));
+  // FP32 rounds the increment of one of the two states first (x: R, y: L), as
+  // FP32 results always have; FP64 rounds once
+  constexpr bool f64 = sizeof(T) == 8;
 #pragma unroll
   for (int k = 0; k < S; ++k) {
-    const T dflux = (fm[k] - fp[k]) * half_dtdh;
-    R[k] = plus[k] + dflux;
-    L[k] = minus[k] + dflux;
+    R[k] = f64 || D == 1 ? fast::fma(df[k], half_dtdh, plus[k]) : plus[k] + df[k] * half_dtdh;
+    L[k] = f64 || D == 0 ? fast::fma(df[k], half_dtdh, minus[k]) : minus[k] + df[k] * half_dtdh;
   }
 }
 
+// u + side * (the sound speed, or the shock's where p* > p), side = -1 or +1.
+// The ideal gas's FP64 form has no quotient; FP32 keeps the one it has, whose
+// reciprocal and root are one instruction each.
 template <typename T>
-__device__ __forceinline__ T hllc_wavespeed(T u, T p, T pstar, T sound, const Material<T>& m) {
-#pragma clang fp contract(fast)
-  if (pstar <= p) return u + sound;
-  if (m.corr) return u + sound * fast::sqt(T(1) + m.q * (fast::div(pstar + m.p_inf, p + m.p_inf) - T(1)));
-  return u + sound * fast::sqt(T(1) + m.q * (fast::div(pstar, p) - T(1)));
+__device__ __forceinline__ T hllc_wavespeed(T u, T p, T rinv, T pstar, T sound, T side,
+                                            const Material<T>& m) {
+  if (pstar <= p) return u + side * sound;
+  if (m.corr)
+    return u + side * (sound * fast::sqt(fast::fma(
+                                   m.q, fast::div(pstar + m.p_inf, p + m.p_inf) - T(1), T(1))));
+  if (sizeof(T) == 4 || m.stiff)
+    return u + side * (sound * fast::sqt(fast::fma(m.q, fast::div(pstar, p) - T(1), T(1))));
+  return u + side * fast::sqt(m.gamma * rinv * fast::fma(m.q, pstar - p, p));
 }
 
 // HLLC (flux_method/flux_hllc.hpp:82-245), as fl::hllc_flux.
 template <typename T, int ND, int D>
 __device__ __forceinline__ void hllc_flux(const T* ul, const T* ur, const Material<T>& m,
                                           T* F) {
-#pragma clang fp contract(fast)
   constexpr int S = 2 + ND;
-  const PrimR<T, ND> wl = fast::prim_of<T, ND>(ul, m);
+  // (the left state of an FP32 x face sums its squares from vel[0], as FP32
+  // results always have)
+  const PrimR<T, ND> wl = fast::prim_of<T, ND, sizeof(T) == 4 && D == 0 ? 0 : ND - 1>(ul, m);
   const PrimR<T, ND> wr = fast::prim_of<T, ND>(ur, m);
   const T al = fast::sound_speed(wl.p, wl.rinv, m);
   const T ar = fast::sound_speed(wr.p, wr.rinv, m);
   const T vl = wl.vel[D], vr = wr.vel[D];
-  const T p_pvrs = T(0.5) * ((wl.p + wr.p) - (T(0.25) * (vr - vl) * (ur[0] + ul[0]) * (al + ar)));
+  const T p_pvrs =
+      T(0.5) * fast::fma(T(-0.25) * fast::fma(ur[2 + D], wr.rinv, -vl) * (ur[0] + ul[0]), al + ar,
+                         wl.p + wr.p);
   const T p_star = m.corr ? fast::mx(-m.p_inf, p_pvrs) : fast::mx(T(0), p_pvrs);
 
-  const T wsl = fast::hllc_wavespeed(vl, wl.p, p_star, -al, m);
+  const T wsl = fast::hllc_wavespeed(vl, wl.p, wl.rinv, p_star, al, T(-1), m);
   if (T(0) <= wsl) {
     fast::euler_flux<T, ND, D>(ul, wl, F);
     return;
   }
-  const T wsr = fast::hllc_wavespeed(vr, wr.p, p_star, ar, m);
+  const T wsr = fast::hllc_wavespeed(vr, wr.p, wr.rinv, p_star, ar, T(1), m);
   if (T(0) >= wsr) {
     fast::euler_flux<T, ND, D>(ur, wr, F);
     return;
   }
   const T factorl = ul[0] * (wsl - vl);
   const T factorr = ur[0] * (wsr - vr);
-  const T ws_star = fast::div(wr.p - wl.p + vl * factorl - vr * factorr, factorl - factorr);
+  const T ws_star = fast::div(fast::fma(-vr, factorr, fast::fma(vl, factorl, wr.p - wl.p)),
+                              fast::fma(ul[0], wsl - vl, -factorr));
 
   const bool left = T(0) <= ws_star;
   const T* st = left ? ul : ur;
   const PrimR<T, ND>& w = left ? wl : wr;
   const T ws = left ? wsl : wsr;
-  T f[S];
-  fast::euler_flux<T, ND, D>(st, w, f);
   const T state_factor = ws - w.vel[D];
   // 1/(ws - ws_star) and 1/state_factor from one reciprocal of their product
   const T rr = fast::rcp((ws - ws_star) * state_factor);
   const T scale_factor = state_factor * state_factor * rr;
   const T inv_sf = (ws - ws_star) * rr;
-  T us[S];
+  // star state minus state
+  T d[S];
 #pragma unroll
-  for (int k = 0; k < S; ++k) us[k] = st[k] * scale_factor;
-  us[2 + D] = ws_star * st[0] * scale_factor;
-  us[1] = scale_factor *
-          (st[1] + st[0] * (ws_star - w.vel[D]) * (ws_star + w.p * w.rinv * inv_sf));
+  for (int k = 0; k < S; ++k) d[k] = fast::fma(st[k], scale_factor, -st[k]);
+  d[2 + D] = fast::fma(ws_star * st[0], scale_factor, -st[2 + D]);
+  d[1] = fast::fma(scale_factor,
+                   fast::fma(st[0] * (ws_star - w.vel[D]),
+                             fast::fma(w.p * w.rinv, inv_sf, ws_star), st[1]),
+                   -st[1]);
 #pragma unroll
-  for (int k = 0; k < S; ++k) F[k] = f[k] + (us[k] - st[k]) * ws;
+  for (int i = 0; i < ND; ++i)
+    F[2 + i] = i == D ? fast::fma(d[2 + D], ws, fast::fma(st[2 + D], w.vel[D], w.p))
+                      : fast::fma(st[2 + i], w.vel[D], d[2 + i] * ws);
+  F[0] = fast::fma(d[0], ws, st[2 + D]);
+  F[1] = fast::fma(w.vel[D], st[1] + w.p, d[1] * ws);
 }
 
 template <typename T, int ND, int D>
 __device__ __forceinline__ void force_flux(const T* ul, const T* ur, T dtdh, T dhdt,
                                            const Material<T>& m, T* F) {
-#pragma clang fp contract(fast)
   constexpr int S = 2 + ND;
   const PrimR<T, ND> wl = fast::prim_of<T, ND>(ul, m);
   const PrimR<T, ND> wr = fast::prim_of<T, ND>(ur, m);
@@ -300,21 +338,21 @@ __device__ __forceinline__ void force_flux(const T* ul, const T* ur, T dtdh, T d
   fast::euler_flux<T, ND, D>(ul, wl, fl);
   fast::euler_flux<T, ND, D>(ur, wr, fr);
 #pragma unroll
-  for (int k = 0; k < S; ++k) uri[k] = (ul[k] + ur[k] + (fl[k] - fr[k]) * dtdh) * T(0.5);
+  for (int k = 0; k < S; ++k)
+    uri[k] = fast::fma(fl[k] - fr[k], dtdh, ul[k] + ur[k]) * T(0.5);
   const PrimR<T, ND> wri = fast::prim_of<T, ND>(uri, m);
   T fri[S];
   fast::euler_flux<T, ND, D>(uri, wri, fri);
 #pragma unroll
   for (int k = 0; k < S; ++k) {
-    const T lf = (fl[k] + fr[k] + (ul[k] - ur[k]) * dhdt) * T(0.5);
-    F[k] = (lf + fri[k]) * T(0.5);
+    const T lf2 = fast::fma(ul[k] - ur[k], dhdt, fl[k] + fr[k]);
+    F[k] = fast::fma(T(0.5), lf2, fri[k]) * T(0.5);
   }
 }
 
 template <typename T, int ND, int D>
 __device__ __forceinline__ void lax_friedrichs_flux(const T* ul, const T* ur, T dhdt,
                                                     const Material<T>& m, T* F) {
-#pragma clang fp contract(fast)
   constexpr int S = 2 + ND;
   const PrimR<T, ND> wl = fast::prim_of<T, ND>(ul, m);
   const PrimR<T, ND> wr = fast::prim_of<T, ND>(ur, m);
@@ -322,13 +360,13 @@ __device__ __forceinline__ void lax_friedrichs_flux(const T* ul, const T* ur, T 
   fast::euler_flux<T, ND, D>(ul, wl, fl);
   fast::euler_flux<T, ND, D>(ur, wr, fr);
 #pragma unroll
-  for (int k = 0; k < S; ++k) F[k] = (fl[k] + fr[k] + (ul[k] - ur[k]) * dhdt) * T(0.5);
+  for (int k = 0; k < S; ++k)
+    F[k] = fast::fma(ul[k] - ur[k], dhdt, fl[k] + fr[k]) * T(0.5);
 }
 
 template <typename T, int ND, int D>
 __device__ __forceinline__ void richtmyer_flux(const T* ul, const T* ur, T dtdh,
                                                const Material<T>& m, T* F) {
-#pragma clang fp contract(fast)
   constexpr int S = 2 + ND;
   const PrimR<T, ND> wl = fast::prim_of<T, ND>(ul, m);
   const PrimR<T, ND> wr = fast::prim_of<T, ND>(ur, m);
@@ -336,7 +374,8 @@ __device__ __forceinline__ void richtmyer_flux(const T* ul, const T* ur, T dtdh,
   fast::euler_flux<T, ND, D>(ul, wl, fl);
   fast::euler_flux<T, ND, D>(ur, wr, fr);
 #pragma unroll
-  for (int k = 0; k < S; ++k) uri[k] = (ul[k] + ur[k] + (fl[k] - fr[k]) * dtdh) * T(0.5);
+  for (int k = 0; k < S; ++k)
+    uri[k] = fast::fma(fl[k] - fr[k], dtdh, ul[k] + ur[k]) * T(0.5);
   const PrimR<T, ND> wri = fast::prim_of<T, ND>(uri, m);
   fast::euler_flux<T, ND, D>(uri, wri, F);
 }

@@ -94,7 +94,7 @@ class SplitSolver:
 
     def set_graphs(self, enable: bool) -> None:
         """simulate() replays hipGraphs of steps (default; a 1D line of at
-        most 2^16 cells runs the whole loop in one cooperative launch) or
+        most 229376 cells runs the whole loop in one launch) or
         launches every kernel."""
         N.check(N.lib.fl_ctx_set_graphs(self.ctx.handle, 1 if enable else 0))
 

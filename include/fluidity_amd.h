@@ -220,9 +220,9 @@ int fl_simulate_noalloc(const fl_tuning* tuning, fl_field* state, fl_field* work
 
 /* fl_simulate captures runs of steps in hipGraphs for a given grid, scheme,
  * parameters and tuning and replays them (default): at once for loops of 72
- * steps or more, from the second call on for shorter ones; a 1D line of at most 2^16 cells
- * (exact FP64 or FP32) instead runs the whole loop in one cooperative launch
- * with a grid barrier per step.  enable = 0 launches every kernel. */
+ * steps or more, from the second call on for shorter ones; a 1D line of at
+ * most 229376 cells instead runs the whole loop in one (cooperative) launch.
+ * enable = 0 launches every kernel. */
 int fl_ctx_set_graphs(fl_context* ctx, int enable);
 
 /* FP64 sums of each conserved component over the grid (synchronises
