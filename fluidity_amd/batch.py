@@ -3,7 +3,7 @@
 A batch advances many independent grids together, each with its own
 material, CFL dt and stop condition, as a host loop of the reference's
 ``SimulatorImpl.simulate`` (simulator/simulator_impl.hpp:222-258) over the
-problems would, but in one persistent launch per sweep phase with the steps
+problems would, but in one launch per sweep phase with the steps
 replayed from a hipGraph.  Grids are device tensors as in ``euler.grid_field``.
 """
 from __future__ import annotations

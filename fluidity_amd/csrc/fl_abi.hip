@@ -570,7 +570,7 @@ namespace {
 // Longer lines take the launched sweeps: past a workgroup of 16 waves on every
 // CU a step is more arithmetic than exchange.
 constexpr int64_t kPersistMaxCells =
-    (int64_t)fl::kPersistCells * fl::kPersistMaxWaves * fl::kPersistMaxGroups;
+    (int64_t)fl::kLineCells * fl::kPersistMaxWaves * fl::kPersistMaxGroups;
 constexpr int64_t kPersistChunk = 1 << 16;     // steps per launch (then the host looks)
 // Polls before a workgroup gives up (each is a load from device memory: a
 // fraction of a second in all, against a few microseconds per step).
@@ -612,7 +612,7 @@ PersistShape persist_shape(const fl_field* f, const fl_scheme* s) {
   sh.kernel = f->dtype == FL_F32 ? persist_kernel_for<float, false>(s->flux, vlc)
               : fast_numerics(s) ? persist_kernel_for<double, true>(s->flux, vlc)
                                  : persist_kernel_for<double, false>(s->flux, vlc);
-  int nseg = (int)((f->n[0] + fl::kPersistCells - 1) / fl::kPersistCells);
+  int nseg = (int)((f->n[0] + fl::kLineCells - 1) / fl::kLineCells);
   const int spread = (nseg + fl::kPersistMaxGroups - 1) / fl::kPersistMaxGroups;
   const int waves = nseg <= 8 ? nseg : std::max(4, spread);
   const int groups = (nseg + waves - 1) / waves;

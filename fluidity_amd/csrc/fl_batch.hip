@@ -4,12 +4,12 @@
 // replayed: the control kernel (one thread per problem: dt from the problem's
 // fused maximum wavespeed, its run time and iteration count, as
 // Parameters::update_time_delta / dt_dh / update_simulation_info,
-// simulator/parameters.hpp:60-99), then one persistent launch per sweep
-// phase.  Phase 0 runs the x sweep of every 2D problem and the whole step of
-// every 1D problem; phase 1 runs the y sweep of every 2D problem.  The
-// workgroups of a phase take tiles from a shared counter (largest tiles
-// first), so problems of very different sizes share one launch and the
-// machine stays busy to the end of the phase.  Tile bodies are those of the
+// simulator/parameters.hpp:60-99), then one launch per sweep phase.  Phase 0
+// runs the x sweep of every 2D problem and the whole step of every 1D problem;
+// phase 1 runs the y sweep of every 2D problem.  Problems of very different
+// sizes share a phase's list of tiles, largest problems first: cell-parallel
+// tiles, one per workgroup, or marching tiles, which persistent workgroups
+// take from a counter.  1D problems run register tiles in either.  Tile bodies are those of the
 // single-grid sweeps (fl_sweep_tiles.hpp), so every problem's result is the
 // single-grid result bit for bit.
 #include "fl_batch.hpp"
@@ -63,9 +63,33 @@ __global__ void reset_counters_kernel(Counters* cnt) {
   cnt->next[1] = 0;
 }
 
-// Persistent sweep phase.  timing != 0 runs every tile state -> work with a
-// fixed dt/dh and no wavespeed output (launch-shape measurement; the states
-// are not modified).
+// Sweep arguments of a problem in a phase (ND = 1 or 2: of which kind it is).
+// timing != 0 runs every tile state -> work with a fixed dt/dh and no
+// wavespeed output (launch-shape measurement; the states are not modified).
+template <typename T, int ND, int PHASE>
+__device__ __forceinline__ SweepArgs<T> phase_args(const Prob<T>& P, int timing, T timing_dtdh) {
+  SweepArgs<T> a = P.x;
+  a.ws_out = nullptr;
+  if (PHASE == 1) a.rows_per_block = P.rows_y;
+  if (timing) {
+    a.ctl = nullptr;
+    a.dtdh_host = timing_dtdh;
+  } else if (PHASE == 1) {
+    a.in = P.x.out;
+    a.out = const_cast<T*>(P.x.in);
+    a.ws_out = &P.ctl->ws_bits[P.ctl->iters & 1];
+  } else if (ND == 1) {
+    const long long it = P.ctl->iters;  // already advanced by this step's control
+    if ((it - 1) & 1) {                 // odd steps run work -> state
+      a.in = P.x.out;
+      a.out = const_cast<T*>(P.x.in);
+    }
+    a.ws_out = &P.ctl->ws_bits[it & 1];
+  }
+  return a;
+}
+
+// Persistent sweep phase: marching tiles, taken from the phase's counter.
 // FAST: the fast FP64 numerics (FP32 has its own forms); VLC: every problem
 // limits with van Leer in conservative form (fixed at compile time, as in
 // the single-grid sweeps).
@@ -82,38 +106,32 @@ phase_kernel(const Prob<T>* __restrict__ probs, const Tile* __restrict__ tiles, 
     if (tile >= ntiles) break;
     const Tile td = tiles[tile];
     const Prob<T>& P = probs[td.prob];
-    SweepArgs<T> a = P.x;
-    if (timing) {
-      a.ctl = nullptr;
-      a.dtdh_host = timing_dtdh;
-      a.ws_out = nullptr;
-    }
-    if (PHASE == 0) {
-      if (P.nd == 1) {
-        if (!timing) {
-          const long long it = P.ctl->iters;  // already advanced by this step's control
-          if ((it - 1) & 1) {                 // odd steps run work -> state
-            a.in = P.x.out;
-            a.out = const_cast<T*>(P.x.in);
-          }
-          a.ws_out = &P.ctl->ws_bits[it & 1];
-        }
-        sweep_x_tile<T, 1, FLUX, FAST, VLC>(a, td.bx, 0);
-      } else {
-        a.ws_out = nullptr;
-        sweep_x_tile<T, 2, FLUX, FAST, VLC>(a, td.bx, td.by);
-      }
-    } else {
-      a.rows_per_block = P.rows_y;
-      if (!timing) {
-        a.in = P.x.out;
-        a.out = const_cast<T*>(P.x.in);
-        a.ws_out = &P.ctl->ws_bits[P.ctl->iters & 1];
-      }
-      sweep_y_tile<T, FLUX, FAST, VLC>(a, td.bx, td.by);
-    }
+    if (PHASE == 1)
+      sweep_y_tile<T, FLUX, FAST, VLC>(phase_args<T, 2, 1>(P, timing, timing_dtdh), td.bx, td.by);
+    else if (P.nd == 1)
+      line_tile<T, FLUX, FAST, VLC>(phase_args<T, 1, 0>(P, timing, timing_dtdh), td.bx);
+    else
+      sweep_x_tile<T, 2, FLUX, FAST, VLC>(phase_args<T, 2, 0>(P, timing, timing_dtdh), td.bx,
+                                          td.by);
     __syncthreads();  // the next tile reuses the LDS
   }
+}
+
+// Sweep phase of cell-parallel tiles, one per workgroup (32 lines of up to
+// 65536 cells beside 16 planes of up to 1024^2: 275 -> 175 us a phase; a line
+// marched eight segments of 254 cells one after the other, 120 us when alone).
+template <typename T, int FLUX, int PHASE, bool FAST, bool VLC>
+__global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(4)))
+cell_phase_kernel(const Prob<T>* __restrict__ probs, const Tile* __restrict__ tiles, int timing,
+                  T timing_dtdh) {
+  const Tile td = tiles[blockIdx.x];
+  const Prob<T>& P = probs[td.prob];
+  if (PHASE == 1)
+    cell_y_tile<T, FLUX, FAST, VLC>(phase_args<T, 2, 1>(P, timing, timing_dtdh), td.bx, td.by);
+  else if (P.nd == 1)
+    line_tile<T, FLUX, FAST, VLC>(phase_args<T, 1, 0>(P, timing, timing_dtdh), td.bx);
+  else
+    cell_x_tile<T, FLUX, FAST, VLC>(phase_args<T, 2, 0>(P, timing, timing_dtdh), td.bx, td.by);
 }
 
 // 1D problems that ran an odd number of steps hold their result in the work
@@ -163,15 +181,16 @@ __global__ void __launch_bounds__(256) sums_kernel(const Prob<T>* __restrict__ p
   }
 }
 
-#define FL_BATCH_PHASES(T, FAST, VLC)                                                    \
-  template __global__ void phase_kernel<T, kFluxHllc, 0, FAST, VLC>(                        \
-      const Prob<T>*, const Tile*, int, Counters*, int, T);                                  \
-  template __global__ void phase_kernel<T, kFluxHllc, 1, FAST, VLC>(                        \
-      const Prob<T>*, const Tile*, int, Counters*, int, T);                                  \
-  template __global__ void phase_kernel<T, kFluxForce, 0, FAST, VLC>(                       \
-      const Prob<T>*, const Tile*, int, Counters*, int, T);                                  \
-  template __global__ void phase_kernel<T, kFluxForce, 1, FAST, VLC>(                       \
-      const Prob<T>*, const Tile*, int, Counters*, int, T);
+#define FL_BATCH_PHASE(T, FLUX, PHASE, FAST, VLC)                                  \
+  template __global__ void phase_kernel<T, FLUX, PHASE, FAST, VLC>(                \
+      const Prob<T>*, const Tile*, int, Counters*, int, T);                        \
+  template __global__ void cell_phase_kernel<T, FLUX, PHASE, FAST, VLC>(           \
+      const Prob<T>*, const Tile*, int, T);
+#define FL_BATCH_PHASES(T, FAST, VLC)          \
+  FL_BATCH_PHASE(T, kFluxHllc, 0, FAST, VLC)   \
+  FL_BATCH_PHASE(T, kFluxHllc, 1, FAST, VLC)   \
+  FL_BATCH_PHASE(T, kFluxForce, 0, FAST, VLC)  \
+  FL_BATCH_PHASE(T, kFluxForce, 1, FAST, VLC)
 #define FL_BATCH_INST(T)                                                                     \
   FL_BATCH_PHASES(T, false, false)                                                           \
   FL_BATCH_PHASES(T, false, true)                                                            \

@@ -19,7 +19,9 @@ struct Prob {
   int rows_y;
 };
 
-// A tile of one sweep phase: problem index and tile coordinates.
+// A tile of one sweep phase: problem index and tile coordinates (a marching or
+// cell-parallel tile of a 2D problem; by = 0 and the workgroup's segments bx
+// of a 1D one).
 struct Tile {
   int prob;
   int bx;
@@ -49,6 +51,9 @@ __global__ void reset_counters_kernel(Counters* cnt);
 template <typename T, int FLUX, int PHASE, bool FAST, bool VLC>
 __global__ void phase_kernel(const Prob<T>* probs, const Tile* tiles, int ntiles, Counters* cnt,
                              int timing, T timing_dtdh);
+template <typename T, int FLUX, int PHASE, bool FAST, bool VLC>
+__global__ void cell_phase_kernel(const Prob<T>* probs, const Tile* tiles, int timing,
+                                  T timing_dtdh);
 template <typename T>
 __global__ void finish_kernel(const Prob<T>* probs, int nprob, int dir);
 template <typename T>

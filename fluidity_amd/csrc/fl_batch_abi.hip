@@ -33,7 +33,8 @@ struct fl_batch {
   double* sums;              // [nprob * 4] (device)
   double* host_sums;         // pinned mirror
   fl_tuning tuning;
-  int grid[2];               // persistent workgroups per phase
+  bool cell[2];              // per phase: cell-parallel tiles (tuning unused)
+  int grid[2];               // workgroups per phase
   hipStream_t cap_stream;    // stream used to capture the step graph
   hipGraph_t graph;
   hipGraphExec_t exec;
@@ -45,10 +46,6 @@ struct fl_batch {
 namespace {
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// Segments of B-2 cells a 1D tile marches (loads of the next segments overlap
-// the current one).
-constexpr int kSegments1D = 8;
 
 bool valid_width(int b) { return b >= 64 && b <= fl::kMaxBlock && (b % 64) == 0; }
 
@@ -85,21 +82,23 @@ void build_tiles(const fl_batch* b, const fl_tuning& t, std::vector<bt::Tile>& t
   });
   t0.clear();
   t1.clear();
+  const int line = (b->cell[0] ? fl::kCellWaves : t.x_block / 64) * fl::kLineCells;
   for (int p : order) {
     const fl_field& f = b->problems[p].state;
     const int64_t nx = f.n[0];
     if (f.ndim == 1) {
-      for (int64_t bx = 0; bx < ceil_div(ceil_div(nx, t.x_block - 2), kSegments1D); ++bx)
-        t0.push_back({p, (int)bx, 0, 0});
-    } else {
-      const int64_t ny = f.n[1];
-      const int64_t gx = ceil_div(nx, t.x_block - 2), gy = ceil_div(ny, tile_rows(ny, t.x_rows));
-      for (int64_t by = 0; by < gy; ++by)
-        for (int64_t bx = 0; bx < gx; ++bx) t0.push_back({p, (int)bx, (int)by, 0});
-      const int64_t hx = ceil_div(nx, t.y_block), hy = ceil_div(ny, tile_rows(ny, t.y_rows));
-      for (int64_t by = 0; by < hy; ++by)
-        for (int64_t bx = 0; bx < hx; ++bx) t1.push_back({p, (int)bx, (int)by, 0});
+      for (int64_t bx = 0; bx < ceil_div(nx, line); ++bx) t0.push_back({p, (int)bx, 0, 0});
+      continue;
     }
+    const int64_t ny = f.n[1];
+    const int64_t gx = ceil_div(nx, b->cell[0] ? fl::kCellXCols : t.x_block - 2);
+    const int64_t gy = ceil_div(ny, b->cell[0] ? fl::kCellXRows : tile_rows(ny, t.x_rows));
+    for (int64_t by = 0; by < gy; ++by)
+      for (int64_t bx = 0; bx < gx; ++bx) t0.push_back({p, (int)bx, (int)by, 0});
+    const int64_t hx = ceil_div(nx, b->cell[1] ? fl::kCellYCols : t.y_block);
+    const int64_t hy = ceil_div(ny, b->cell[1] ? fl::kCellYRows : tile_rows(ny, t.y_rows));
+    for (int64_t by = 0; by < hy; ++by)
+      for (int64_t bx = 0; bx < hx; ++bx) t1.push_back({p, (int)bx, (int)by, 0});
   }
 }
 
@@ -124,12 +123,12 @@ std::vector<bt::Prob<T>> make_probs(const fl_batch* b, const fl_tuning& t) {
     a.form = q.scheme.form;
     a.bcx = q.scheme.bc[0];
     a.bcy = q.state.ndim > 1 ? q.scheme.bc[1] : 0;
-    a.rows_per_block = q.state.ndim > 1 ? (int)tile_rows(a.ny, t.x_rows) : kSegments1D;
+    a.rows_per_block = (int)tile_rows(a.ny, t.x_rows);
     a.ctl = b->ctls + p;
     a.ws_out = nullptr;
     P.ctl = b->ctls + p;
     P.nd = q.state.ndim;
-    P.rows_y = (int)tile_rows(q.state.ndim > 1 ? q.state.n[1] : 1, t.y_rows);
+    P.rows_y = (int)tile_rows(a.ny, t.y_rows);
   }
   return v;
 }
@@ -158,6 +157,30 @@ const void* phase_kernel_ptr(const fl_batch* b, int phase) {
                 : phase_fn_f<float, false, false>(b->flux, phase);
 }
 
+// 2D cells of a batch up to which its phases run cell-parallel tiles unless
+// tuned otherwise.  A step (HLLC, exact | FP32, marching tiles of 256 columns
+// against cell-parallel ones): 16 planes of up to 1024^2, 4.5M cells, 556
+// against 355 us | 303 against 176; 10 planes, 1.4M cells, 516 against 147 |
+// 286 against 84; 200 planes, 36M cells, 2517 against 2559 | 998 against 1321.
+// The marching tiles of a few large planes are too few to fill the device,
+// and short ones pay their warm-up rows; past the limit they are many and
+// tall.  The two lines cross at 19M cells in FP64, 17M in FP32.
+constexpr int64_t kBatchCellMax = 1 << 24;
+
+// Launch shapes of a batch that was not tuned.
+fl_tuning rule_shape(fl_batch* b) {
+  int64_t cells = 0;
+  for (const fl_batch_problem& q : b->problems)
+    if (q.state.ndim > 1) cells += q.state.n[0] * q.state.n[1];
+  b->cell[0] = b->cell[1] = cells <= kBatchCellMax;
+  fl_tuning t;
+  t.x_block = 256;
+  t.x_rows = 32;
+  t.y_block = 256;
+  t.y_rows = 64;
+  return t;
+}
+
 // Uploads the problem table and tile lists of tuning t; sizes the persistent
 // grids.  Synchronous (the host vectors are staging).
 int apply_tuning(fl_batch* b, const fl_tuning& t) {
@@ -184,6 +207,10 @@ int apply_tuning(fl_batch* b, const fl_tuning& t) {
   FL_HIP(hipGetDeviceProperties(&prop, b->device));
   for (int ph = 0; ph < 2; ++ph) {
     const int B = ph ? t.y_block : t.x_block;
+    if (b->cell[ph]) {
+      b->grid[ph] = b->ntiles[ph];
+      continue;
+    }
     int per_cu = 0;
     FL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &per_cu, phase_kernel_ptr(b, ph), B,
@@ -201,16 +228,29 @@ template <typename T, int FLUX, bool FAST, bool VLC>
 void launch_phases_v(const fl_batch* b, hipStream_t st, int timing, double timing_dtdh,
                      int only_phase) {
   const bt::Prob<T>* probs = (const bt::Prob<T>*)b->probs;
-  if (only_phase != 1 && b->ntiles[0] > 0)
-    hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 0, FAST, VLC>), dim3(b->grid[0]),
-                       dim3(b->tuning.x_block), fl::x_tile_lds_bytes(b->tuning.x_block, 4, sizeof(T)),
-                       st, probs, (const bt::Tile*)b->tiles[0],
-                       b->ntiles[0], b->cnt, timing, (T)timing_dtdh);
-  if (only_phase != 0 && b->ntiles[1] > 0)
-    hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 1, FAST, VLC>), dim3(b->grid[1]),
-                       dim3(b->tuning.y_block), fl::y_tile_lds_bytes(b->tuning.y_block, sizeof(T)),
-                       st, probs, (const bt::Tile*)b->tiles[1],
-                       b->ntiles[1], b->cnt, timing, (T)timing_dtdh);
+  const dim3 cell_block(64 * fl::kCellWaves);
+  const size_t cell_lds = fl::cell_tile_lds_bytes(sizeof(T));
+  if (only_phase != 1 && b->ntiles[0] > 0) {
+    const bt::Tile* tiles = b->tiles[0];
+    if (b->cell[0])
+      hipLaunchKernelGGL((bt::cell_phase_kernel<T, FLUX, 0, FAST, VLC>), dim3(b->grid[0]),
+                         cell_block, cell_lds, st, probs, tiles, timing, (T)timing_dtdh);
+    else
+      hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 0, FAST, VLC>), dim3(b->grid[0]),
+                         dim3(b->tuning.x_block),
+                         fl::x_tile_lds_bytes(b->tuning.x_block, 4, sizeof(T)), st, probs, tiles,
+                         b->ntiles[0], b->cnt, timing, (T)timing_dtdh);
+  }
+  if (only_phase != 0 && b->ntiles[1] > 0) {
+    const bt::Tile* tiles = b->tiles[1];
+    if (b->cell[1])
+      hipLaunchKernelGGL((bt::cell_phase_kernel<T, FLUX, 1, FAST, VLC>), dim3(b->grid[1]),
+                         cell_block, cell_lds, st, probs, tiles, timing, (T)timing_dtdh);
+    else
+      hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 1, FAST, VLC>), dim3(b->grid[1]),
+                         dim3(b->tuning.y_block), fl::y_tile_lds_bytes(b->tuning.y_block, sizeof(T)),
+                         st, probs, tiles, b->ntiles[1], b->cnt, timing, (T)timing_dtdh);
+  }
 }
 
 template <typename T, int FLUX>
@@ -350,12 +390,13 @@ int fl_batch_create(fl_context* c, const fl_batch_problem* problems, int nprob, 
   b->graph = nullptr;
   b->exec = nullptr;
   b->graph_ok = false;
-  // capacity: the finest tiling the tuning limits allow (64-lane tiles, 1 row)
+  // capacity: the finest tiling the tuning limits allow (64-lane tiles, 1 row;
+  // the cell-parallel tiles are as wide and higher)
   int64_t c0 = 0, c1 = 0;
   for (int p = 0; p < nprob; ++p) {
     const fl_field& f = problems[p].state;
     const int64_t ny = f.ndim > 1 ? f.n[1] : 1;
-    c0 += ceil_div(f.n[0], 62) * ny;
+    c0 += ceil_div(f.n[0], f.ndim > 1 ? 62 : fl::kLineCells) * ny;
     if (f.ndim > 1) c1 += ceil_div(f.n[0], 64) * ny;
   }
   b->cap[0] = c0;
@@ -384,11 +425,7 @@ int fl_batch_create(fl_context* c, const fl_batch_problem* problems, int nprob, 
     hp[p].sim_time = problems[p].params.sim_time;
     hp[p].max_iters = problems[p].params.max_iters;
   }
-  fl_tuning t;
-  t.x_block = 256;
-  t.x_rows = 32;
-  t.y_block = 256;
-  t.y_rows = 64;
+  const fl_tuning t = rule_shape(b);
   int rc = FL_OK;
   e = hipMemcpy(b->params, hp.data(), sizeof(bt::Params) * nprob, hipMemcpyHostToDevice);
   if (e != hipSuccess) rc = fail(FL_ERR_HIP, "hipMemcpy failed: %s", hipGetErrorString(e));
@@ -424,6 +461,7 @@ int fl_batch_set_tuning(fl_batch* b, const fl_tuning* t) {
     return fail(FL_ERR_ARGUMENT, "rows per tile must be in [1, 4096]");
   DeviceGuard g(b->device);
   FL_HIP(hipDeviceSynchronize());  // tables in use by queued steps
+  b->cell[0] = b->cell[1] = false;
   return apply_tuning(b, n);
 }
 
@@ -459,17 +497,17 @@ int fl_batch_autotune(fl_batch* b, int reps, fl_tuning* chosen, void* stream) {
   int rc = FL_OK;
   for (int ph = 0; ph < 2 && !rc; ++ph) {
     float best_ms = 1e30f;
+    bool best_cell = false;
     for (int w : widths) {
       const int* rows = ph ? yrows : xrows;
       const int nr = ph ? 4 : 5;
-      for (int k = 0; k < nr && !rc; ++k) {
+      // k = -1, once: the cell-parallel tiles
+      for (int k = w == widths[0] ? -1 : 0; k < nr && !rc; ++k) {
         fl_tuning t = best;
-        if (ph == 0) {
-          t.x_block = w;
-          t.x_rows = rows[k];
-        } else {
-          t.y_block = w;
-          t.y_rows = rows[k];
+        b->cell[ph] = k < 0;
+        if (k >= 0) {
+          (ph ? t.y_block : t.x_block) = w;
+          (ph ? t.y_rows : t.x_rows) = rows[k];
         }
         if ((rc = apply_tuning(b, t))) break;
         if (b->ntiles[ph] == 0) break;
@@ -487,9 +525,11 @@ int fl_batch_autotune(fl_batch* b, int reps, fl_tuning* chosen, void* stream) {
         if (!rc && total < best_ms) {
           best_ms = total;
           best = t;
+          best_cell = k < 0;
         }
       }
     }
+    b->cell[ph] = best_cell;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

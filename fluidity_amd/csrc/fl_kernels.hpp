@@ -119,7 +119,7 @@ constexpr unsigned kCellFewBlocks = 1024;
 // Persistent 1D loop: cells of a wave's segment (4 lanes on either side hold
 // the neighbours'), waves of a workgroup, workgroups and the words each
 // publishes per step (the maximum, and 3 values of 4 cells at either end).
-constexpr int kPersistCells = 56;
+constexpr int kLineCells = 56;
 constexpr int kPersistMaxWaves = 16;
 constexpr int kPersistMaxGroups = 4 * 64;
 constexpr int kPersistWords = 25;

@@ -3,7 +3,7 @@
 // The reference's loop (simulator/simulator_impl.hpp:235-252) on a line of at
 // most kPersistMaxCells cells.  A step there is latency: one cell's dependent
 // arithmetic, and the exchange of the maximum wavespeed and of the segments'
-// edges.  The line is cut into segments of at most kPersistCells cells, one
+// edges.  The line is cut into segments of at most kLineCells cells, one
 // per wave; a lane holds its cell in registers for the whole loop, and four
 // lanes on either side hold the neighbours' cells, so a step reads and writes
 // no state.  Neighbours in a wave pass through DPP moves, waves of a workgroup
@@ -32,25 +32,6 @@ namespace {
 
 constexpr int kPolls = kPersistMaxGroups / 64;  // maxima a lane polls
 constexpr unsigned long long kEmpty = ~0ull;  // a NaN that no published word keeps
-
-// The value of the lane above (t + 1) or below (t - 1); 0 past the ends.
-template <int CTRL>
-__device__ __forceinline__ unsigned dpp32(unsigned v) {
-  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = dpp32<CTRL>((unsigned)b), hi = dpp32<CTRL>((unsigned)(b >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __uint_as_float(dpp32<CTRL>(__float_as_uint(v)));
-}
-constexpr int kWaveShl = 0x130, kWaveShr = 0x138;  // DPP wave_shl:1, wave_shr:1
-template <typename T> __device__ __forceinline__ T above(T v) { return dpp<kWaveShl>(v); }
-template <typename T> __device__ __forceinline__ T below(T v) { return dpp<kWaveShr>(v); }
 
 // Maximum over the wave, in every lane.
 template <int CTRL, int ROWS>
@@ -296,27 +277,8 @@ persist1d_kernel(SweepArgs<T> a, PersistCtl* pc, unsigned long long* words, int 
       if (a.bcx == kBcReflective && flip) reflect<T, 1>(u, 0);
     }
     // ---- the step
-    const Prim<T, 1> pw = prim_sel<F, T, 1>(u, a.mat);
-    const T pa = above(pw.p), pb = below(pw.p);
-    const T paa = above(pa), pbb = below(pb);
-    const T K = chi_sel<F>(pbb, pb, pa, paa, below(pw.vel[0]), above(pw.vel[0]), a.mat);
-    const int sx = signum(pa - pb);
-    const T Ka = above(K), Kb = below(K);
-    const T Kn = sx > 0 ? Ka : (sx < 0 ? Kb : K);
-    const T chi = min_sel<F>(Limits<T>::max(), min_sel<F>(K, Kn));
-    T um[S], up[S], R[S], L[S], Lr[S], Gf[S];
-#pragma unroll
-    for (int c = 0; c < S; ++c) {
-      um[c] = below(u[c]);
-      up[c] = above(u[c]);
-    }
-    evolve_sel<F, T, 1, 0>(um, u, up, chi, half_dtdh, limiter, form, a.mat, R, L);
-#pragma unroll
-    for (int c = 0; c < S; ++c) Lr[c] = above(L[c]);
-    flux_sel<F, T, 1, 0, FLUX>(R, Lr, dtdh, dhdt, a.mat, Gf);
     T o[S];
-#pragma unroll
-    for (int c = 0; c < S; ++c) o[c] = u[c] + (below(Gf[c]) - Gf[c]) * dtdh;
+    line_step<T, FLUX, F>(u, dtdh, half_dtdh, dhdt, limiter, form, a.mat, o);
     ws = 0ull;
     if (own) {
 #pragma unroll

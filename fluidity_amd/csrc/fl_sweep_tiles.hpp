@@ -1098,4 +1098,86 @@ __device__ __forceinline__ void cell_y_tile(const SweepArgs<T>& a, int64_t bx, i
   if (a.ws_out) block_atomic_max(wsmax, a.ws_out, gridDim.x > kCellFewBlocks);
 }
 
+// ---------------------------------------------------------------------------
+// a segment of a 1D line in one wave's registers
+// ---------------------------------------------------------------------------
+
+// The value of the lane above (t + 1) or below (t - 1); 0 past the ends.
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp32(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = dpp32<CTRL>((unsigned)b), hi = dpp32<CTRL>((unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __uint_as_float(dpp32<CTRL>(__float_as_uint(v)));
+}
+constexpr int kWaveShl = 0x130, kWaveShr = 0x138;  // DPP wave_shl:1, wave_shr:1
+template <typename T> __device__ __forceinline__ T above(T v) { return dpp<kWaveShl>(v); }
+template <typename T> __device__ __forceinline__ T below(T v) { return dpp<kWaveShr>(v); }
+
+
+// One step of the cells that a wave's lanes hold in order: o is the new state
+// of lanes 4 to 59, which have the stencil's four cells on either side.
+template <typename T, int FLUX, bool F>
+__device__ __forceinline__ void line_step(const T* u, T dtdh, T half_dtdh, T dhdt, int limiter,
+                                          int form, const Material<T>& m, T* o) {
+  constexpr int S = 3;
+  const Prim<T, 1> pw = prim_sel<F, T, 1>(u, m);
+  const T pa = above(pw.p), pb = below(pw.p);
+  const T paa = above(pa), pbb = below(pb);
+  const T K = chi_sel<F>(pbb, pb, pa, paa, below(pw.vel[0]), above(pw.vel[0]), m);
+  const int sx = signum(pa - pb);
+  const T Ka = above(K), Kb = below(K);
+  const T Kn = sx > 0 ? Ka : (sx < 0 ? Kb : K);
+  const T chi = min_sel<F>(Limits<T>::max(), min_sel<F>(K, Kn));
+  T um[S], up[S], R[S], L[S], Lr[S], G[S];
+#pragma unroll
+  for (int c = 0; c < S; ++c) {
+    um[c] = below(u[c]);
+    up[c] = above(u[c]);
+  }
+  evolve_sel<F, T, 1, 0>(um, u, up, chi, half_dtdh, limiter, form, m, R, L);
+#pragma unroll
+  for (int c = 0; c < S; ++c) Lr[c] = above(L[c]);
+  flux_sel<F, T, 1, 0, FLUX>(R, Lr, dtdh, dhdt, m, G);
+#pragma unroll
+  for (int c = 0; c < S; ++c) o[c] = u[c] + (below(G[c]) - G[c]) * dtdh;
+}
+
+// The 1D sweep of one segment of kLineCells cells per wave, segments bx W to
+// bx W + W - 1 of the line, W = blockDim.x / 64.  Nothing is marched and no
+// LDS is used but for the maximum: a segment is one load and one cell's
+// arithmetic.
+template <typename T, int FLUX, bool FAST, bool VLC>
+__device__ __forceinline__ void line_tile(const SweepArgs<T>& a, int64_t bx) {
+  constexpr int S = 3;
+  constexpr bool F = UseFast<T, FAST>::value;
+  const int t = (int)(threadIdx.x & 63);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t x = (bx * (blockDim.x >> 6) + w) * kLineCells - 4 + t;
+  Pending<T, S> Q;
+  issue_load<T, 1>(a, x, 0, Q);
+  T dtdh = a.dtdh_host;
+  if (a.ctl) {
+    if (!a.ctl->active) return;
+    dtdh = (T)a.ctl->dtdh;
+  }
+  T u[S], o[S];
+  take<T, 1>(Q, u);
+  line_step<T, FLUX, F>(u, dtdh, T(0.5) * dtdh, T(1) / dtdh, VLC ? int(kLimVanLeer) : a.limiter,
+                        VLC ? int(kFormCons) : a.form, a.mat, o);
+  unsigned long long wsmax = 0ull;
+  if (t >= 4 && t < 4 + kLineCells && x < a.nx) {
+    store_cell<T, S>(a.out, x, a.es, a.cs, o);
+    if (a.ws_out) ws_fold<F, T, 1>(o, a, wsmax);
+  }
+  if (a.ws_out) block_atomic_max(wsmax, a.ws_out, gridDim.x > kCellFewBlocks);
+}
+
 }  // namespace fl

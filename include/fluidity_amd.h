@@ -282,9 +282,8 @@ int fl_write_results_separate_raw(fl_context* ctx, const fl_field* state,
 /* ---- batched problems -------------------------------------------------------
  * Many independent grids of uneven size (1D and 2D, each with its own
  * material, CFL dt and stop condition) advanced together: one step is a
- * control kernel plus one persistent launch per sweep phase whose workgroups
- * take tiles from a shared counter; steps are captured once in a hipGraph and
- * replayed.  Each problem's result is bit-identical to fl_simulate on that
+ * control kernel plus one launch per sweep phase over the tiles of all
+ * problems; steps are captured once in a hipGraph and replayed.  Each problem's result is bit-identical to fl_simulate on that
  * problem alone.  The batch as a whole replaces a host loop of
  * SimulatorImpl::simulate calls (simulator/simulator_impl.hpp:222-258), one
  * per problem, with Parameters::update_time_delta / dt_dh per problem
@@ -304,8 +303,10 @@ typedef struct fl_batch_problem {
 int fl_batch_create(fl_context* ctx, const fl_batch_problem* problems, int nprob,
                     fl_batch** batch, void* stream);
 int fl_batch_destroy(fl_batch* batch);
-/* Tile shapes of the two sweep phases (x_block/x_rows: x tiles of 2D problems
- * and 1D tiles; y_block/y_rows: y tiles).  Zeros keep the current values. */
+/* Marching tiles of the given shapes in the two sweep phases (x_block/x_rows:
+ * x tiles of 2D problems, x_block also the width of 1D tiles; y_block/y_rows:
+ * y tiles).  Zeros keep the current values.  Without this call a batch of up
+ * to 2^24 2D cells runs cell-parallel tiles, and the values are unused. */
 int fl_batch_set_tuning(fl_batch* batch, const fl_tuning* tuning);
 int fl_batch_get_tuning(const fl_batch* batch, fl_tuning* tuning);
 /* Times every candidate tile shape of each phase on this batch (`reps` timed
