@@ -152,6 +152,7 @@ fl::SweepArgs<T> make_args(const fl_context* ctx, const fl_field* in, const fl_f
   a.dtdh_host = (T)dtdh;
   a.ctl = ctl;
   a.ws_out = ws_out;
+  a.wide = wide_cells(a);
   (void)ctx;
   return a;
 }
@@ -183,13 +184,15 @@ struct SweepShape {
 
 // Cells (of all grids of the launch) up to which the cell-parallel sweeps are
 // the faster ones.
-template <typename T> constexpr int64_t kCellMax = 5 << 17;
-template <> constexpr int64_t kCellMax<float> = 3 << 19;
+template <typename T> constexpr int64_t kCellMax = 5 << 19;
+template <> constexpr int64_t kCellMax<float> = 5 << 20;
 
 // Launch shape of the sweep of dimension dim over ngrids grids of nx x ny
 // cells.  By rule: small grids go cell-parallel (a 64^2 FP64 sweep takes 7 us
-// against 16 (x) and 21 us (y) marching; 512^2 17 against 19 and 22; 1024^2
-// 46 and 51 against 41 and 45).  Larger ones march, x in 128-lane workgroups of
+// against 16 (x) and 21 us (y) marching; a step of 1024^2 101 against 124,
+// 3861x515 161 against 176, 2048^2 312 against 284; FP32 3861x515 82 against
+// 117, 2048^2 146 against 159, 4096^2 544 against 419: the line is where the
+// two cross).  Larger ones march, x in 128-lane workgroups of
 // about 10500 waves and y in 64-lane ones of about 4096 in all: fewer, taller
 // tiles end unevenly, shorter ones pay more warm-up rows (FP64 x at 2048^2: 8
 // rows 133 us, 32 rows 186 us; y at 4096^2: 64 rows 441 us, 22 rows 455 us).
@@ -224,23 +227,31 @@ dim3 shape_grid(const SweepShape& sh, int dim, int64_t nx, int64_t ny, int ngrid
               (unsigned)((ny + sh.rows - 1) / sh.rows), ngrids);
 }
 
-template <typename T, int FLUX, bool FAST, bool VLC>
-void launch_flux_v(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a,
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
+void launch_flux_w(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a,
                    hipStream_t stream) {
   const int B = sh.block;
   if (sh.cell) {
-    auto k = dim == 0 ? fl::cell_x_kernel<T, FLUX, FAST, VLC> : fl::cell_y_kernel<T, FLUX, FAST, VLC>;
+    auto k = dim == 0 ? fl::cell_x_kernel<T, FLUX, FAST, VLC, WIDE>
+                      : fl::cell_y_kernel<T, FLUX, FAST, VLC, WIDE>;
     hipLaunchKernelGGL(k, grid, dim3(64 * fl::kCellWaves), fl::cell_tile_lds_bytes(sizeof(T)),
                        stream, a, a);
   } else if (ndim == 1)
-    hipLaunchKernelGGL((fl::sweep_x_kernel<T, 1, FLUX, FAST, VLC>), grid, dim3(B),
+    hipLaunchKernelGGL((fl::sweep_x_kernel<T, 1, FLUX, FAST, VLC, false>), grid, dim3(B),
                        fl::x_tile_lds_bytes(B, 3, sizeof(T)), stream, a);
   else if (dim == 0)
-    hipLaunchKernelGGL((fl::sweep_x_kernel<T, 2, FLUX, FAST, VLC>), grid, dim3(B),
+    hipLaunchKernelGGL((fl::sweep_x_kernel<T, 2, FLUX, FAST, VLC, WIDE>), grid, dim3(B),
                        fl::x_tile_lds_bytes(B, 4, sizeof(T)), stream, a);
   else
-    hipLaunchKernelGGL((fl::sweep_y_kernel<T, FLUX, FAST, VLC>), grid, dim3(B),
+    hipLaunchKernelGGL((fl::sweep_y_kernel<T, FLUX, FAST, VLC, WIDE>), grid, dim3(B),
                        fl::y_tile_lds_bytes(B, sizeof(T)), stream, a);
+}
+
+template <typename T, int FLUX, bool FAST, bool VLC>
+void launch_flux_v(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a,
+                   hipStream_t stream) {
+  if (a.wide) launch_flux_w<T, FLUX, FAST, VLC, true>(ndim, dim, grid, sh, a, stream);
+  else launch_flux_w<T, FLUX, FAST, VLC, false>(ndim, dim, grid, sh, a, stream);
 }
 
 // One sweep kernel of flux FLUX: the 1D sweep, or the x or y sweep of a 2D grid.
@@ -262,8 +273,8 @@ inline bool fast_numerics(const fl_scheme* s) { return s->numerics == FL_NUMERIC
 // Workgroups of B lanes of one sweep kernel that a CU holds at once.
 template <typename T, int FLUX, bool FAST, bool VLC>
 const void* sweep_kernel_2d(int dim) {
-  return dim == 0 ? reinterpret_cast<const void*>(&fl::sweep_x_kernel<T, 2, FLUX, FAST, VLC>)
-                  : reinterpret_cast<const void*>(&fl::sweep_y_kernel<T, FLUX, FAST, VLC>);
+  return dim == 0 ? reinterpret_cast<const void*>(&fl::sweep_x_kernel<T, 2, FLUX, FAST, VLC, false>)
+                  : reinterpret_cast<const void*>(&fl::sweep_y_kernel<T, FLUX, FAST, VLC, false>);
 }
 
 template <typename T, int FLUX, bool FAST>
@@ -399,23 +410,33 @@ int launch_sim_step(const fl_context* ctx, const fl_field* state, const fl_field
 // with scheme s[m].  The two grids share shape, layout and dtype; the flux
 // methods must be equal (the launch instantiates one), else each grid is
 // swept on its own.
-template <typename T, int FLUX, bool FAST, bool VLC>
-void launch_flux2_v(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a0,
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
+void launch_flux2_w(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a0,
                     const fl::SweepArgs<T>& a1, hipStream_t stream) {
   const int B = sh.block;
   if (sh.cell) {
-    auto k = dim == 0 ? fl::cell_x_kernel<T, FLUX, FAST, VLC> : fl::cell_y_kernel<T, FLUX, FAST, VLC>;
+    auto k = dim == 0 ? fl::cell_x_kernel<T, FLUX, FAST, VLC, WIDE>
+                      : fl::cell_y_kernel<T, FLUX, FAST, VLC, WIDE>;
     hipLaunchKernelGGL(k, grid, dim3(64 * fl::kCellWaves), fl::cell_tile_lds_bytes(sizeof(T)),
                        stream, a0, a1);
   } else if (ndim == 1)
-    hipLaunchKernelGGL((fl::sweep_x2_kernel<T, 1, FLUX, FAST, VLC>), grid, dim3(B),
+    hipLaunchKernelGGL((fl::sweep_x2_kernel<T, 1, FLUX, FAST, VLC, false>), grid, dim3(B),
                        fl::x_tile_lds_bytes(B, 3, sizeof(T)), stream, a0, a1);
   else if (dim == 0)
-    hipLaunchKernelGGL((fl::sweep_x2_kernel<T, 2, FLUX, FAST, VLC>), grid, dim3(B),
+    hipLaunchKernelGGL((fl::sweep_x2_kernel<T, 2, FLUX, FAST, VLC, WIDE>), grid, dim3(B),
                        fl::x_tile_lds_bytes(B, 4, sizeof(T)), stream, a0, a1);
   else
-    hipLaunchKernelGGL((fl::sweep_y2_kernel<T, FLUX, FAST, VLC>), grid, dim3(B),
+    hipLaunchKernelGGL((fl::sweep_y2_kernel<T, FLUX, FAST, VLC, WIDE>), grid, dim3(B),
                        fl::y_tile_lds_bytes(B, sizeof(T)), stream, a0, a1);
+}
+
+template <typename T, int FLUX, bool FAST, bool VLC>
+void launch_flux2_v(int ndim, int dim, dim3 grid, const SweepShape& sh, const fl::SweepArgs<T>& a0,
+                    const fl::SweepArgs<T>& a1, hipStream_t stream) {
+  if (a0.wide && a1.wide)
+    launch_flux2_w<T, FLUX, FAST, VLC, true>(ndim, dim, grid, sh, a0, a1, stream);
+  else
+    launch_flux2_w<T, FLUX, FAST, VLC, false>(ndim, dim, grid, sh, a0, a1, stream);
 }
 
 // fast: the fast FP64 numerics (FP64 only; the FP32 kernels have their own)
@@ -859,7 +880,7 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
       }
     }
     // the cell-parallel kernel, on grids where it can be the faster one
-    if (in->ndim == 2 && !rc && in->n[0] * in->n[1] <= 4 * kCellMax<float>) {
+    if (in->ndim == 2 && !rc && in->n[0] * in->n[1] <= 2 * kCellMax<float>) {
       float total = 0.0f;
       c->shape[dim] = kShapeCell;
       rc = timed(dim, &total);

@@ -104,6 +104,12 @@ inline fl::Material<T> make_material(const fl_scheme* s) {
   return m;
 }
 
+// SweepArgs::wide of a 2D sweep's arguments.
+template <typename T>
+inline int wide_cells(const fl::SweepArgs<T>& a) {
+  return a.es == 4 && a.cs == 1 && ((uintptr_t)a.in | (uintptr_t)a.out) % 16 == 0;
+}
+
 double bits_to_double(unsigned long long b);
 // `t` (nullable: all defaults) with zeros replaced by the built-in launch
 // shapes, validated, into *out; shape[d] becomes kShapeTuning where t names a

@@ -91,9 +91,9 @@ __device__ __forceinline__ SweepArgs<T> phase_args(const Prob<T>& P, int timing,
 
 // Persistent sweep phase: marching tiles, taken from the phase's counter.
 // FAST: the fast FP64 numerics (FP32 has its own forms); VLC: every problem
-// limits with van Leer in conservative form (fixed at compile time, as in
-// the single-grid sweeps).
-template <typename T, int FLUX, int PHASE, bool FAST, bool VLC>
+// limits with van Leer in conservative form; WIDE: every 2D problem is
+// SweepArgs::wide (fixed at compile time, as in the single-grid sweeps).
+template <typename T, int FLUX, int PHASE, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(SweepWaves<T>::value)))
 phase_kernel(const Prob<T>* __restrict__ probs, const Tile* __restrict__ tiles, int ntiles,
              Counters* __restrict__ cnt, int timing, T timing_dtdh) {
@@ -107,11 +107,11 @@ phase_kernel(const Prob<T>* __restrict__ probs, const Tile* __restrict__ tiles, 
     const Tile td = tiles[tile];
     const Prob<T>& P = probs[td.prob];
     if (PHASE == 1)
-      sweep_y_tile<T, FLUX, FAST, VLC>(phase_args<T, 2, 1>(P, timing, timing_dtdh), td.bx, td.by);
+      sweep_y_tile<T, FLUX, FAST, VLC, WIDE>(phase_args<T, 2, 1>(P, timing, timing_dtdh), td.bx, td.by);
     else if (P.nd == 1)
       line_tile<T, FLUX, FAST, VLC>(phase_args<T, 1, 0>(P, timing, timing_dtdh), td.bx);
     else
-      sweep_x_tile<T, 2, FLUX, FAST, VLC>(phase_args<T, 2, 0>(P, timing, timing_dtdh), td.bx,
+      sweep_x_tile<T, 2, FLUX, FAST, VLC, WIDE>(phase_args<T, 2, 0>(P, timing, timing_dtdh), td.bx,
                                           td.by);
     __syncthreads();  // the next tile reuses the LDS
   }
@@ -120,18 +120,18 @@ phase_kernel(const Prob<T>* __restrict__ probs, const Tile* __restrict__ tiles, 
 // Sweep phase of cell-parallel tiles, one per workgroup (32 lines of up to
 // 65536 cells beside 16 planes of up to 1024^2: 275 -> 175 us a phase; a line
 // marched eight segments of 254 cells one after the other, 120 us when alone).
-template <typename T, int FLUX, int PHASE, bool FAST, bool VLC>
+template <typename T, int FLUX, int PHASE, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(4)))
 cell_phase_kernel(const Prob<T>* __restrict__ probs, const Tile* __restrict__ tiles, int timing,
                   T timing_dtdh) {
   const Tile td = tiles[blockIdx.x];
   const Prob<T>& P = probs[td.prob];
   if (PHASE == 1)
-    cell_y_tile<T, FLUX, FAST, VLC>(phase_args<T, 2, 1>(P, timing, timing_dtdh), td.bx, td.by);
+    cell_y_tile<T, FLUX, FAST, VLC, WIDE>(phase_args<T, 2, 1>(P, timing, timing_dtdh), td.bx, td.by);
   else if (P.nd == 1)
     line_tile<T, FLUX, FAST, VLC>(phase_args<T, 1, 0>(P, timing, timing_dtdh), td.bx);
   else
-    cell_x_tile<T, FLUX, FAST, VLC>(phase_args<T, 2, 0>(P, timing, timing_dtdh), td.bx, td.by);
+    cell_x_tile<T, FLUX, FAST, VLC, WIDE>(phase_args<T, 2, 0>(P, timing, timing_dtdh), td.bx, td.by);
 }
 
 // 1D problems that ran an odd number of steps hold their result in the work
@@ -181,16 +181,19 @@ __global__ void __launch_bounds__(256) sums_kernel(const Prob<T>* __restrict__ p
   }
 }
 
-#define FL_BATCH_PHASE(T, FLUX, PHASE, FAST, VLC)                                  \
-  template __global__ void phase_kernel<T, FLUX, PHASE, FAST, VLC>(                \
-      const Prob<T>*, const Tile*, int, Counters*, int, T);                        \
-  template __global__ void cell_phase_kernel<T, FLUX, PHASE, FAST, VLC>(           \
+#define FL_BATCH_PHASE(T, FLUX, PHASE, FAST, VLC, WIDE)                             \
+  template __global__ void phase_kernel<T, FLUX, PHASE, FAST, VLC, WIDE>(        \
+      const Prob<T>*, const Tile*, int, Counters*, int, T);                      \
+  template __global__ void cell_phase_kernel<T, FLUX, PHASE, FAST, VLC, WIDE>(   \
       const Prob<T>*, const Tile*, int, T);
-#define FL_BATCH_PHASES(T, FAST, VLC)          \
-  FL_BATCH_PHASE(T, kFluxHllc, 0, FAST, VLC)   \
-  FL_BATCH_PHASE(T, kFluxHllc, 1, FAST, VLC)   \
-  FL_BATCH_PHASE(T, kFluxForce, 0, FAST, VLC)  \
-  FL_BATCH_PHASE(T, kFluxForce, 1, FAST, VLC)
+#define FL_BATCH_PHASES_W(T, FAST, VLC, WIDE)        \
+  FL_BATCH_PHASE(T, kFluxHllc, 0, FAST, VLC, WIDE)   \
+  FL_BATCH_PHASE(T, kFluxHllc, 1, FAST, VLC, WIDE)   \
+  FL_BATCH_PHASE(T, kFluxForce, 0, FAST, VLC, WIDE)  \
+  FL_BATCH_PHASE(T, kFluxForce, 1, FAST, VLC, WIDE)
+#define FL_BATCH_PHASES(T, FAST, VLC)      \
+  FL_BATCH_PHASES_W(T, FAST, VLC, false)   \
+  FL_BATCH_PHASES_W(T, FAST, VLC, true)
 #define FL_BATCH_INST(T)                                                                     \
   FL_BATCH_PHASES(T, false, false)                                                           \
   FL_BATCH_PHASES(T, false, true)                                                            \

@@ -41,6 +41,7 @@ struct fl_batch {
   bool graph_ok;
   bool vlc;                  // every problem: van Leer, conservative form
   bool fast;                 // FP64 batch in the fast numerics
+  bool wide;                 // every 2D problem: SweepArgs::wide
 };
 
 namespace {
@@ -103,8 +104,9 @@ void build_tiles(const fl_batch* b, const fl_tuning& t, std::vector<bt::Tile>& t
 }
 
 template <typename T>
-std::vector<bt::Prob<T>> make_probs(const fl_batch* b, const fl_tuning& t) {
+std::vector<bt::Prob<T>> make_probs(fl_batch* b, const fl_tuning& t) {
   std::vector<bt::Prob<T>> v(b->nprob);
+  b->wide = true;
   for (int p = 0; p < b->nprob; ++p) {
     const fl_batch_problem& q = b->problems[p];
     bt::Prob<T>& P = v[p];
@@ -126,6 +128,8 @@ std::vector<bt::Prob<T>> make_probs(const fl_batch* b, const fl_tuning& t) {
     a.rows_per_block = (int)tile_rows(a.ny, t.x_rows);
     a.ctl = b->ctls + p;
     a.ws_out = nullptr;
+    a.wide = wide_cells(a);
+    b->wide = b->wide && (a.wide || q.state.ndim < 2);
     P.ctl = b->ctls + p;
     P.nd = q.state.ndim;
     P.rows_y = (int)tile_rows(a.ny, t.y_rows);
@@ -134,27 +138,30 @@ std::vector<bt::Prob<T>> make_probs(const fl_batch* b, const fl_tuning& t) {
 }
 
 template <typename T, int FLUX, bool FAST, bool VLC>
-const void* phase_fn(int phase) {
-  return phase ? reinterpret_cast<const void*>(&bt::phase_kernel<T, FLUX, 1, FAST, VLC>)
-               : reinterpret_cast<const void*>(&bt::phase_kernel<T, FLUX, 0, FAST, VLC>);
+const void* phase_fn(int phase, bool wide) {
+  if (wide)
+    return phase ? reinterpret_cast<const void*>(&bt::phase_kernel<T, FLUX, 1, FAST, VLC, true>)
+                 : reinterpret_cast<const void*>(&bt::phase_kernel<T, FLUX, 0, FAST, VLC, true>);
+  return phase ? reinterpret_cast<const void*>(&bt::phase_kernel<T, FLUX, 1, FAST, VLC, false>)
+               : reinterpret_cast<const void*>(&bt::phase_kernel<T, FLUX, 0, FAST, VLC, false>);
 }
 
 template <typename T, bool FAST, bool VLC>
-const void* phase_fn_f(int flux, int phase) {
-  return flux == FL_FLUX_HLLC ? phase_fn<T, fl::kFluxHllc, FAST, VLC>(phase)
-                              : phase_fn<T, fl::kFluxForce, FAST, VLC>(phase);
+const void* phase_fn_f(const fl_batch* b, int phase) {
+  return b->flux == FL_FLUX_HLLC ? phase_fn<T, fl::kFluxHllc, FAST, VLC>(phase, b->wide)
+                                 : phase_fn<T, fl::kFluxForce, FAST, VLC>(phase, b->wide);
 }
 
 const void* phase_kernel_ptr(const fl_batch* b, int phase) {
   if (b->dtype == FL_F64) {
     if (b->fast)
-      return b->vlc ? phase_fn_f<double, true, true>(b->flux, phase)
-                    : phase_fn_f<double, true, false>(b->flux, phase);
-    return b->vlc ? phase_fn_f<double, false, true>(b->flux, phase)
-                  : phase_fn_f<double, false, false>(b->flux, phase);
+      return b->vlc ? phase_fn_f<double, true, true>(b, phase)
+                    : phase_fn_f<double, true, false>(b, phase);
+    return b->vlc ? phase_fn_f<double, false, true>(b, phase)
+                  : phase_fn_f<double, false, false>(b, phase);
   }
-  return b->vlc ? phase_fn_f<float, false, true>(b->flux, phase)
-                : phase_fn_f<float, false, false>(b->flux, phase);
+  return b->vlc ? phase_fn_f<float, false, true>(b, phase)
+                : phase_fn_f<float, false, false>(b, phase);
 }
 
 // 2D cells of a batch up to which its phases run cell-parallel tiles unless
@@ -224,8 +231,8 @@ int apply_tuning(fl_batch* b, const fl_tuning& t) {
   return FL_OK;
 }
 
-template <typename T, int FLUX, bool FAST, bool VLC>
-void launch_phases_v(const fl_batch* b, hipStream_t st, int timing, double timing_dtdh,
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
+void launch_phases_w(const fl_batch* b, hipStream_t st, int timing, double timing_dtdh,
                      int only_phase) {
   const bt::Prob<T>* probs = (const bt::Prob<T>*)b->probs;
   const dim3 cell_block(64 * fl::kCellWaves);
@@ -233,10 +240,10 @@ void launch_phases_v(const fl_batch* b, hipStream_t st, int timing, double timin
   if (only_phase != 1 && b->ntiles[0] > 0) {
     const bt::Tile* tiles = b->tiles[0];
     if (b->cell[0])
-      hipLaunchKernelGGL((bt::cell_phase_kernel<T, FLUX, 0, FAST, VLC>), dim3(b->grid[0]),
+      hipLaunchKernelGGL((bt::cell_phase_kernel<T, FLUX, 0, FAST, VLC, WIDE>), dim3(b->grid[0]),
                          cell_block, cell_lds, st, probs, tiles, timing, (T)timing_dtdh);
     else
-      hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 0, FAST, VLC>), dim3(b->grid[0]),
+      hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 0, FAST, VLC, WIDE>), dim3(b->grid[0]),
                          dim3(b->tuning.x_block),
                          fl::x_tile_lds_bytes(b->tuning.x_block, 4, sizeof(T)), st, probs, tiles,
                          b->ntiles[0], b->cnt, timing, (T)timing_dtdh);
@@ -244,13 +251,20 @@ void launch_phases_v(const fl_batch* b, hipStream_t st, int timing, double timin
   if (only_phase != 0 && b->ntiles[1] > 0) {
     const bt::Tile* tiles = b->tiles[1];
     if (b->cell[1])
-      hipLaunchKernelGGL((bt::cell_phase_kernel<T, FLUX, 1, FAST, VLC>), dim3(b->grid[1]),
+      hipLaunchKernelGGL((bt::cell_phase_kernel<T, FLUX, 1, FAST, VLC, WIDE>), dim3(b->grid[1]),
                          cell_block, cell_lds, st, probs, tiles, timing, (T)timing_dtdh);
     else
-      hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 1, FAST, VLC>), dim3(b->grid[1]),
+      hipLaunchKernelGGL((bt::phase_kernel<T, FLUX, 1, FAST, VLC, WIDE>), dim3(b->grid[1]),
                          dim3(b->tuning.y_block), fl::y_tile_lds_bytes(b->tuning.y_block, sizeof(T)),
                          st, probs, tiles, b->ntiles[1], b->cnt, timing, (T)timing_dtdh);
   }
+}
+
+template <typename T, int FLUX, bool FAST, bool VLC>
+void launch_phases_v(const fl_batch* b, hipStream_t st, int timing, double timing_dtdh,
+                     int only_phase) {
+  if (b->wide) launch_phases_w<T, FLUX, FAST, VLC, true>(b, st, timing, timing_dtdh, only_phase);
+  else launch_phases_w<T, FLUX, FAST, VLC, false>(b, st, timing, timing_dtdh, only_phase);
 }
 
 template <typename T, int FLUX>
@@ -375,6 +389,7 @@ int fl_batch_create(fl_context* c, const fl_batch_problem* problems, int nprob, 
   b->dtype = dtype;
   b->flux = flux;
   b->fast = dtype == FL_F64 && problems[0].scheme.numerics == FL_NUMERICS_FAST;
+  b->wide = false;
   b->vlc = FL_VLC_KERNELS != 0;
   for (int p = 0; p < nprob; ++p)
     b->vlc = b->vlc && problems[p].scheme.limiter == FL_LIMITER_VAN_LEER &&

@@ -66,7 +66,7 @@ struct SweepArgs {
   int limiter, form;
   int bcx, bcy;
   int rows_per_block;  // row chunk marched by one workgroup
-  int pad;
+  int wide;            // 2D: both grids AoS, every cell at a multiple of 16 bytes
   T dtdh_host;         // used when ctl == nullptr
   const StepCtl* ctl;  // nullable: provides dtdh and the active flag
   // nullable: the first sweep of a step of fl_simulate, which turns the
@@ -131,17 +131,20 @@ constexpr int kMaxWsUnroll = 4;
 
 }  // namespace fl
 
-// Kernels defined in fl_sweep.hip (explicitly instantiated there).
+// Kernels defined in fl_sweep.hip (explicitly instantiated there).  WIDE:
+// every grid of the launch is SweepArgs::wide.
 namespace fl {
-template <typename T, int ND, int FLUX, bool FAST, bool VLC> __global__ void sweep_x_kernel(SweepArgs<T> a);
-template <typename T, int FLUX, bool FAST, bool VLC> __global__ void sweep_y_kernel(SweepArgs<T> a);
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int ND, int FLUX, bool FAST, bool VLC, bool WIDE>
+__global__ void sweep_x_kernel(SweepArgs<T> a);
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
+__global__ void sweep_y_kernel(SweepArgs<T> a);
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void cell_x_kernel(SweepArgs<T> a0, SweepArgs<T> a1);
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void cell_y_kernel(SweepArgs<T> a0, SweepArgs<T> a1);
-template <typename T, int ND, int FLUX, bool FAST, bool VLC>
+template <typename T, int ND, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void sweep_x2_kernel(SweepArgs<T> a0, SweepArgs<T> a1);
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void sweep_y2_kernel(SweepArgs<T> a0, SweepArgs<T> a1);
 template <typename T, int ND, bool FAST>
 __global__ void max_wavespeed2_kernel(const T* in0, const T* in1, int64_t es0, int64_t cs0,

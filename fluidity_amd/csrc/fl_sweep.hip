@@ -30,55 +30,55 @@ __device__ __forceinline__ void tile_of_block(int64_t& bx, int64_t& by) {
 
 // VLC: van Leer in conservative form, fixed at compile time (the launcher
 // picks these kernels when the scheme says so).
-template <typename T, int ND, int FLUX, bool FAST, bool VLC>
+template <typename T, int ND, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(SweepWavesOf<T, FAST>::value)))
 sweep_x_kernel(SweepArgs<T> a) {
   int64_t bx, by;
   tile_of_block(bx, by);
-  sweep_x_tile<T, ND, FLUX, FAST, VLC>(a, bx, by);
+  sweep_x_tile<T, ND, FLUX, FAST, VLC, WIDE>(a, bx, by);
 }
 
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(SweepWavesOf<T, FAST>::value)))
 sweep_y_kernel(SweepArgs<T> a) {
   int64_t bx, by;
   tile_of_block(bx, by);
-  sweep_y_tile<T, FLUX, FAST, VLC>(a, bx, by);
+  sweep_y_tile<T, FLUX, FAST, VLC, WIDE>(a, bx, by);
 }
 
 // Cell-parallel sweeps of small grids (cell_x_tile, cell_y_tile), of one grid
 // or of two of one shape (blockIdx.y selects the grid), one tile per
 // workgroup, tiles numbered along x first.
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(4)))
 cell_x_kernel(SweepArgs<T> a0, SweepArgs<T> a1) {
   const unsigned nbx = (unsigned)((a0.nx + kCellXCols - 1) / kCellXCols);
-  cell_x_tile<T, FLUX, FAST, VLC>(blockIdx.y ? a1 : a0, blockIdx.x % nbx, blockIdx.x / nbx);
+  cell_x_tile<T, FLUX, FAST, VLC, WIDE>(blockIdx.y ? a1 : a0, blockIdx.x % nbx, blockIdx.x / nbx);
 }
 
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(64 * kCellWaves) __attribute__((amdgpu_waves_per_eu(4)))
 cell_y_kernel(SweepArgs<T> a0, SweepArgs<T> a1) {
   const unsigned nbx = (unsigned)((a0.nx + kCellYCols - 1) / kCellYCols);
-  cell_y_tile<T, FLUX, FAST, VLC>(blockIdx.y ? a1 : a0, blockIdx.x % nbx, blockIdx.x / nbx);
+  cell_y_tile<T, FLUX, FAST, VLC, WIDE>(blockIdx.y ? a1 : a0, blockIdx.x % nbx, blockIdx.x / nbx);
 }
 
 // The same sweeps over two grids of one shape in one launch (the two
 // materials of a two-material step): blockIdx.z selects the grid.
-template <typename T, int ND, int FLUX, bool FAST, bool VLC>
+template <typename T, int ND, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(SweepWaves<T>::value)))
 sweep_x2_kernel(SweepArgs<T> a0, SweepArgs<T> a1) {
   int64_t bx, by;
   tile_of_block(bx, by);
-  sweep_x_tile<T, ND, FLUX, FAST, VLC>(blockIdx.z ? a1 : a0, bx, by);
+  sweep_x_tile<T, ND, FLUX, FAST, VLC, WIDE>(blockIdx.z ? a1 : a0, bx, by);
 }
 
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(SweepWaves<T>::value)))
 sweep_y2_kernel(SweepArgs<T> a0, SweepArgs<T> a1) {
   int64_t bx, by;
   tile_of_block(bx, by);
-  sweep_y_tile<T, FLUX, FAST, VLC>(blockIdx.z ? a1 : a0, bx, by);
+  sweep_y_tile<T, FLUX, FAST, VLC, WIDE>(blockIdx.z ? a1 : a0, bx, by);
 }
 
 // ---------------------------------------------------------------------------
@@ -303,10 +303,13 @@ __global__ void __launch_bounds__(kMaxBlock) component_sums_kernel(const T* __re
 // explicit instantiations (launched from fl_abi.cpp)
 // ---------------------------------------------------------------------------
 
-#define FL_INST_SWEEPS2_V(T, FLUX, FAST, VLC)                                               \
-  template __global__ void sweep_x2_kernel<T, 1, FLUX, FAST, VLC>(SweepArgs<T>, SweepArgs<T>); \
-  template __global__ void sweep_x2_kernel<T, 2, FLUX, FAST, VLC>(SweepArgs<T>, SweepArgs<T>); \
-  template __global__ void sweep_y2_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>, SweepArgs<T>);
+#define FL_INST_SWEEPS2_W(T, FLUX, FAST, VLC, WIDE)                                               \
+  template __global__ void sweep_x2_kernel<T, 2, FLUX, FAST, VLC, WIDE>(SweepArgs<T>, SweepArgs<T>); \
+  template __global__ void sweep_y2_kernel<T, FLUX, FAST, VLC, WIDE>(SweepArgs<T>, SweepArgs<T>);
+#define FL_INST_SWEEPS2_V(T, FLUX, FAST, VLC)                                                      \
+  template __global__ void sweep_x2_kernel<T, 1, FLUX, FAST, VLC, false>(SweepArgs<T>, SweepArgs<T>); \
+  FL_INST_SWEEPS2_W(T, FLUX, FAST, VLC, false)                                                     \
+  FL_INST_SWEEPS2_W(T, FLUX, FAST, VLC, true)
 #define FL_INST_SWEEPS2(T, FLUX) FL_INST_SWEEPS2_V(T, FLUX, false, false)
 
 FL_INST_SWEEPS2(double, kFluxHllc)
@@ -342,12 +345,15 @@ FL_INST_MAXWS2(double)
 FL_INST_MAXWS2(float)
 FL_INST_MAXWS2_F(double, true)
 
-#define FL_SWEEPS_V(T, FLUX, FAST, VLC)                                          \
-  template __global__ void sweep_x_kernel<T, 1, FLUX, FAST, VLC>(SweepArgs<T>);  \
-  template __global__ void sweep_x_kernel<T, 2, FLUX, FAST, VLC>(SweepArgs<T>);  \
-  template __global__ void sweep_y_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>);     \
-  template __global__ void cell_x_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>, SweepArgs<T>); \
-  template __global__ void cell_y_kernel<T, FLUX, FAST, VLC>(SweepArgs<T>, SweepArgs<T>);
+#define FL_SWEEPS_W(T, FLUX, FAST, VLC, WIDE)                                                   \
+  template __global__ void sweep_x_kernel<T, 2, FLUX, FAST, VLC, WIDE>(SweepArgs<T>);           \
+  template __global__ void sweep_y_kernel<T, FLUX, FAST, VLC, WIDE>(SweepArgs<T>);              \
+  template __global__ void cell_x_kernel<T, FLUX, FAST, VLC, WIDE>(SweepArgs<T>, SweepArgs<T>); \
+  template __global__ void cell_y_kernel<T, FLUX, FAST, VLC, WIDE>(SweepArgs<T>, SweepArgs<T>);
+#define FL_SWEEPS_V(T, FLUX, FAST, VLC)                                                \
+  template __global__ void sweep_x_kernel<T, 1, FLUX, FAST, VLC, false>(SweepArgs<T>); \
+  FL_SWEEPS_W(T, FLUX, FAST, VLC, false)                                               \
+  FL_SWEEPS_W(T, FLUX, FAST, VLC, true)
 #define FL_SWEEPS(T, FLUX, FAST) FL_SWEEPS_V(T, FLUX, FAST, false)
 
 #define FL_INST_SWEEPS(T)                                                      \

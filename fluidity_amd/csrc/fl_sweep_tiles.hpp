@@ -176,7 +176,31 @@ __device__ __forceinline__ int map_row(int y, int ny, int kind, bool& flip) {
   return y < 0 ? -y - 1 : 2 * ny - 1 - y;
 }
 
+// 16 bytes of a cell.
+template <typename T>
+using Wide = T __attribute__((ext_vector_type(16 / sizeof(T))));
+
+// WIDE: the grid is AoS and aligned (SweepArgs::wide), and a cell's components
+// go 16 bytes a load and store; one by one each of them touches every line of
+// the row again.  A step (HLLC, AoS, one by one | wide): FP32 1500x900 80.4 |
+// 62.0 us, 4096^2 494 | 431; FP64 4096^2 exact 972 | 976, fast 755 | 722.  It
+// is a parameter of the kernels: tested in them it cost the SoA sweeps 2 to 8
+// percent.
 template <typename T, int S>
+__device__ __forceinline__ void load_wide(const char* row, uint32_t off, T* u) {
+  constexpr int N = 16 / sizeof(T);
+  static_assert(S % N == 0);
+  asm volatile("" : "+s"(row));
+#pragma unroll
+  for (int k = 0; k < S; k += N) {
+    const Wide<T> v = *(const __attribute__((address_space(1))) Wide<T>*)(
+        (const __attribute__((address_space(1))) char*)row + off + k * sizeof(T));
+#pragma unroll
+    for (int j = 0; j < N; ++j) u[k + j] = v[j];
+  }
+}
+
+template <typename T, int S, bool WIDE>
 __device__ __forceinline__ void issue_row(const SweepArgs<T>& a, int64_t y, const LaneCol& lc,
                                           Pending<T, S>& q) {
   bool fy = false;
@@ -188,21 +212,38 @@ __device__ __forceinline__ void issue_row(const SweepArgs<T>& a, int64_t y, cons
   // load is a scalar base plus a 32-bit lane offset.
   uint32_t off = lc.off;
   asm volatile("" : "+v"(off));
+  if constexpr (WIDE) {
+    load_wide<T, S>(row, off, q.u);
+  } else {
 #pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const char* base = row + k * a.cs * (int64_t)sizeof(T);
-    asm volatile("" : "+s"(base));
-    q.u[k] = *(const __attribute__((address_space(1))) T*)(
-        (const __attribute__((address_space(1))) char*)base + off);
+    for (int k = 0; k < S; ++k) {
+      const char* base = row + k * a.cs * (int64_t)sizeof(T);
+      asm volatile("" : "+s"(base));
+      q.u[k] = *(const __attribute__((address_space(1))) T*)(
+          (const __attribute__((address_space(1))) char*)base + off);
+    }
   }
   q.flip = lc.flip | (fy ? 2 : 0);
 }
 
-template <typename T, int S>
+template <typename T, int S, bool WIDE>
 __device__ __forceinline__ void store_row(const SweepArgs<T>& a, int64_t y, uint32_t off,
                                           const T* u) {
   char* row = (char*)a.out + y * a.nx * a.es * (int64_t)sizeof(T);
   asm volatile("" : "+v"(off));
+  if constexpr (WIDE) {
+    constexpr int N = 16 / sizeof(T);
+    asm volatile("" : "+s"(row));
+#pragma unroll
+    for (int k = 0; k < S; k += N) {
+      Wide<T> v;
+#pragma unroll
+      for (int j = 0; j < N; ++j) v[j] = u[k + j];
+      *(__attribute__((address_space(1))) Wide<T>*)(
+          (__attribute__((address_space(1))) char*)row + off + k * sizeof(T)) = v;
+    }
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < S; ++k) {
     char* base = row + k * a.cs * (int64_t)sizeof(T);
@@ -430,7 +471,7 @@ __device__ __forceinline__ bool sweep_dtdh(const SweepArgs<T>& a, bool writer, T
 // is rows_per_block consecutive segments of B-2 cells, starting at segment
 // bx rows_per_block, marched like rows.  Every thread of the workgroup must
 // call it with the same arguments.
-template <typename T, int ND, int FLUX, bool FAST = false, bool VLC = false>
+template <typename T, int ND, int FLUX, bool FAST, bool VLC, bool WIDE>
 __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, int64_t bx, int64_t by) {
   constexpr int S = 2 + ND;
   constexpr bool F = UseFast<T, FAST>::value;
@@ -504,7 +545,7 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, int64_t bx, 
   const LaneCol lc = lane_col(a, c), lh = lane_col(a, hcol);
   const uint32_t out_off = col_off(a, c);
   auto issue = [&](int64_t x, int64_t r, const LaneCol& l, Pending<T, S>& q) {
-    if constexpr (ND == 2) issue_row<T, S>(a, r, l, q);
+    if constexpr (ND == 2) issue_row<T, S, WIDE>(a, r, l, q);
     else issue_load<T, ND>(a, x, r, q);
   };
   constexpr int PF = PrefetchXOf<T, FAST>::value;
@@ -622,7 +663,7 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, int64_t bx, 
       T o[S];
 #pragma unroll
       for (int k = 0; k < S; ++k) o[k] = U0[k] + (sG[k * B + t - 1] - G[k]) * dtdh;
-      if constexpr (ND == 2) store_row<T, S>(a, jo, out_off, o);
+      if constexpr (ND == 2) store_row<T, S, WIDE>(a, jo, out_off, o);
       else store_cell<T, S>(a.out, jo * a.nx + cr, a.es, a.cs, o);
       if (a.ws_out) {
         ws_fold<F, T, ND>(o, a, wsmax);
@@ -639,7 +680,7 @@ __device__ __forceinline__ void sweep_x_tile(const SweepArgs<T>& a, int64_t bx, 
 
 // One y-sweep tile: columns [bx B, (bx+1) B) of rows [by rows_per_block,
 // (by+1) rows_per_block), B = blockDim.x.  Workgroup-uniform arguments.
-template <typename T, int FLUX, bool FAST = false, bool VLC = false>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, int64_t bx, int64_t by) {
   constexpr int ND = 2, S = 4;
   constexpr bool F = UseFast<T, FAST>::value;
@@ -703,8 +744,8 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, int64_t bx, 
   Pending<T, S> Qs[PF], Hs[PF];
 #pragma unroll
   for (int i = 0; i < PF; ++i) {
-    issue_row<T, S>(a, min(rbeg + i, rlast), lc, Qs[i]);
-    issue_row<T, S>(a, min(rbeg + i, rlast), lh, Hs[i]);
+    issue_row<T, S, WIDE>(a, min(rbeg + i, rlast), lc, Qs[i]);
+    issue_row<T, S, WIDE>(a, min(rbeg + i, rlast), lh, Hs[i]);
   }
   // ring slot of row r: (r - rbeg) mod kYRing, advanced per row
   int slot = 0;
@@ -726,10 +767,10 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, int64_t bx, 
     }
     T un[S];
     take<T, ND>(Q, un);
-    issue_row<T, S>(a, min(r + PF, rlast), lc, Q);
+    issue_row<T, S, WIDE>(a, min(r + PF, rlast), lc, Q);
     T uh[S];
     take<T, ND>(H, uh);
-    issue_row<T, S>(a, min(r + PF, rlast), lh, H);
+    issue_row<T, S, WIDE>(a, min(r + PF, rlast), lh, H);
 #pragma unroll
     for (int k = 0; k < S; ++k) ring_t[(slot * S + k) * 64] = un[k];
     const Prim<T, ND> w = prim_sel<F, T, ND>(un, a.mat);
@@ -791,7 +832,7 @@ __device__ __forceinline__ void sweep_y_tile(const SweepArgs<T>& a, int64_t bx, 
           T o[S];
 #pragma unroll
           for (int k = 0; k < S; ++k) o[k] = um[k] + (Gprev[k] - G[k]) * dtdh;
-          store_row<T, S>(a, jo, out_off, o);
+          store_row<T, S, WIDE>(a, jo, out_off, o);
           if (a.ws_out) {
             ws_fold<F, T, ND>(o, a, wsmax);
           }
@@ -834,29 +875,33 @@ __device__ __forceinline__ const char* row_ptr(const SweepArgs<T>& a, int64_t y,
 
 // Issues the loads of a lane's cell of the row at `row` (row_ptr), each a
 // scalar base plus a 32-bit lane offset as in issue_row.
-template <typename T, int S>
+template <typename T, int S, bool WIDE>
 __device__ __forceinline__ void issue_at(const SweepArgs<T>& a, const char* row, int flip,
                                          const LaneCol& lc, Pending<T, S>& q) {
   uint32_t off = lc.off;
   asm volatile("" : "+v"(off));
+  if constexpr (WIDE) {
+    load_wide<T, S>(row, off, q.u);
+  } else {
 #pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const char* base = row;
-    asm volatile("" : "+s"(base));
-    q.u[k] = *(const __attribute__((address_space(1))) T*)(
-        (const __attribute__((address_space(1))) char*)base + off);
-    row += a.csb;
+    for (int k = 0; k < S; ++k) {
+      const char* base = row;
+      asm volatile("" : "+s"(base));
+      q.u[k] = *(const __attribute__((address_space(1))) T*)(
+          (const __attribute__((address_space(1))) char*)base + off);
+      row += a.csb;
+    }
   }
   q.flip = lc.flip | flip;
 }
 
 // issue_at of row y.
-template <typename T, int S>
+template <typename T, int S, bool WIDE>
 __device__ __forceinline__ void issue_near(const SweepArgs<T>& a, int64_t y, const LaneCol& lc,
                                            Pending<T, S>& q) {
   int flip;
   const char* row = row_ptr(a, y, flip);
-  issue_at<T, S>(a, row, flip, lc, q);
+  issue_at<T, S, WIDE>(a, row, flip, lc, q);
 }
 
 // Stages the primitives that the flattening factors of rows yb .. yb +
@@ -865,19 +910,19 @@ __device__ __forceinline__ void issue_near(const SweepArgs<T>& a, int64_t y, con
 // kHalo columns on either side of the rows.  Wave w stages its own row yb + w
 // (its first byte `row`), whose states it keeps in u0, and one of the six
 // rows above and below (w < 6) or the halo cells (w = 6).
-template <typename T, bool F>
+template <typename T, bool F, bool WIDE>
 __device__ __forceinline__ void cell_stage(const SweepArgs<T>& a, int64_t xc, int64_t yb, int w,
                                            int t, const char* row, int flip, const LaneCol& lc,
                                            T* sP, T* sVX, T* sVY, T* u0) {
   constexpr int S = 4, ND = 2, NW = kCellWaves, PW = kCellCols;
   static_assert(NW >= 7 && 6 * NW <= 64, "one wave stages the halo cells");
   Pending<T, S> Q, H;
-  issue_at<T, S>(a, row, flip, lc, Q);
+  issue_at<T, S, WIDE>(a, row, flip, lc, Q);
   const int j = t / 6, h = t - 6 * j;       // halo cell of this lane (w = 6)
   const int hcol = h < kHalo ? h : 64 + h;  // its column in the staged row
   const bool halo = w == 6 && j < NW;
   const int q2 = w < 3 ? w : NW + w;        // second staged row of this wave (w < 6)
-  if (w < 6) issue_near<T, S>(a, yb - 3 + q2, lc, H);
+  if (w < 6) issue_near<T, S, WIDE>(a, yb - 3 + q2, lc, H);
   else if (halo) issue_load<T, ND>(a, xc - kHalo + hcol, yb + j, H);
   take<T, ND>(Q, u0);
   {
@@ -957,7 +1002,7 @@ __device__ __forceinline__ bool cell_begin(const SweepArgs<T>& a, int w, int t, 
 // (by + 1)).  Lanes 0 and 63 hold the columns beside them, whose face states
 // the tile's outer faces need.  Called by every thread of a workgroup of
 // kCellWaves waves.
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __device__ __forceinline__ void cell_x_tile(const SweepArgs<T>& a, int64_t bx, int64_t by) {
   constexpr int ND = 2, S = 4, NW = kCellWaves;
   constexpr bool F = UseFast<T, FAST>::value;
@@ -985,9 +1030,9 @@ __device__ __forceinline__ void cell_x_tile(const SweepArgs<T>& a, int64_t bx, i
   const char* row = row_ptr(a, r, fy);
   Pending<T, S> Ql, Qr;
   T u0[S];
-  issue_at<T, S>(a, row, fy, ll, Ql);
-  issue_at<T, S>(a, row, fy, lr, Qr);
-  cell_stage<T, F>(a, xc, yb, w, t, row, fy, lc, sP, sVX, sVY, u0);
+  issue_at<T, S, WIDE>(a, row, fy, ll, Ql);
+  issue_at<T, S, WIDE>(a, row, fy, lr, Qr);
+  cell_stage<T, F, WIDE>(a, xc, yb, w, t, row, fy, lc, sP, sVX, sVY, u0);
   if (a.sim) {
     if (!cell_begin(a, w, t, bx == 0 && by == 0, dtdh)) return;
   } else {
@@ -1018,7 +1063,7 @@ __device__ __forceinline__ void cell_x_tile(const SweepArgs<T>& a, int64_t bx, i
       T o[S];
 #pragma unroll
       for (int k = 0; k < S; ++k) o[k] = u0[k] + (sX[k * 64 + t - 1] - G[k]) * dtdh;
-      store_row<T, S>(a, r, col_off(a, c), o);
+      store_row<T, S, WIDE>(a, r, col_off(a, c), o);
       if (a.ws_out) ws_fold<F, T, ND>(o, a, wsmax);
     }
   }
@@ -1028,7 +1073,7 @@ __device__ __forceinline__ void cell_x_tile(const SweepArgs<T>& a, int64_t bx, i
 // y sweep of columns [64 bx, 64 bx + 64) of rows [(kCellWaves - 2) by,
 // (kCellWaves - 2) (by + 1)).  Waves 0 and kCellWaves - 1 hold the rows beside
 // them.  Called as cell_x_tile.
-template <typename T, int FLUX, bool FAST, bool VLC>
+template <typename T, int FLUX, bool FAST, bool VLC, bool WIDE>
 __device__ __forceinline__ void cell_y_tile(const SweepArgs<T>& a, int64_t bx, int64_t by) {
   constexpr int ND = 2, S = 4, NW = kCellWaves;
   constexpr bool F = UseFast<T, FAST>::value;
@@ -1056,9 +1101,9 @@ __device__ __forceinline__ void cell_y_tile(const SweepArgs<T>& a, int64_t bx, i
   const char* row = row_ptr(a, r, fy);
   Pending<T, S> Ql, Qr;
   T u0[S];
-  cell_stage<T, F>(a, xc, yb, w, t, row, fy, lc, sP, sVX, sVY, u0);
-  issue_near<T, S>(a, r - 1, lc, Ql);
-  issue_near<T, S>(a, r + 1, lc, Qr);
+  cell_stage<T, F, WIDE>(a, xc, yb, w, t, row, fy, lc, sP, sVX, sVY, u0);
+  issue_near<T, S, WIDE>(a, r - 1, lc, Ql);
+  issue_near<T, S, WIDE>(a, r + 1, lc, Qr);
   __syncthreads();
   if (!active) return;
   const T half_dtdh = T(0.5) * dtdh;
@@ -1092,7 +1137,7 @@ __device__ __forceinline__ void cell_y_tile(const SweepArgs<T>& a, int64_t bx, i
     T o[S];
 #pragma unroll
     for (int k = 0; k < S; ++k) o[k] = u0[k] + (G[k] - sX[(w * S + k) * 64 + t]) * dtdh;
-    store_row<T, S>(a, r, col_off(a, c), o);
+    store_row<T, S, WIDE>(a, r, col_off(a, c), o);
     if (a.ws_out) ws_fold<F, T, ND>(o, a, wsmax);
   }
   if (a.ws_out) block_atomic_max(wsmax, a.ws_out, gridDim.x > kCellFewBlocks);

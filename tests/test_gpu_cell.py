@@ -60,7 +60,7 @@ def test_rule_sweeps_bitwise(E, oracle, case, dim):
     assert np.array_equal(_bits(_host(b, layout)), _bits(ref))
 
 
-@pytest.mark.parametrize("shape", [(640, 1024), (641, 1024)])  # the rule's line for FP64
+@pytest.mark.parametrize("shape", [(2560, 1024), (2561, 1024)])  # the rule's line for FP64
 def test_rule_line_matches_marching_loop(E, shape):
     """The step loop (fused CFL maximum included) on either side of the rule's
     line equals the loop with a caller's marching shapes bit for bit."""
@@ -75,3 +75,26 @@ def test_rule_line_matches_marching_loop(E, shape):
         out.append((_bits(_host(a, 1)), r.run_time, r.max_wavespeed))
     assert np.array_equal(out[0][0], out[1][0])
     assert out[0][1:] == out[1][1:]
+
+
+@pytest.mark.parametrize("shape,tuning", [((70, 130), None), ((70, 130), dict(x_block=64, x_rows=8,
+                                                                              y_block=128, y_rows=16))])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=str)
+def test_unaligned_aos_matches_aligned(E, shape, tuning, dtype):
+    """An AoS grid whose cells are not at multiples of 16 bytes takes the
+    loads of single components, with the same bits: state, work or both."""
+    n = shape[0] * shape[1] * 4
+    U = cons_field("smooth", shape, seed=9)
+    out = []
+    for off_state, off_work in ((0, 0), (1, 0), (0, 1), (1, 1)):
+        bufs = [torch.zeros(n + 4, dtype=dtype, device="cuda") for _ in range(2)]
+        a, b = (q[o:o + n].view(*shape, 4) for q, o in zip(bufs, (off_state, off_work)))
+        a.copy_(_dev(U, 0, dtype))
+        solver = E.SplitSolver(E.Scheme(bc=(1, 2, 0)), layout=0)
+        if tuning:
+            solver.set_tuning(**tuning)
+        r = solver.simulate(a, b, 0.9, 1.0 / shape[1], max_iters=4)
+        out.append((_bits(_host(a, 0)), r.run_time))
+        assert all(float(q[o + n:].abs().sum()) == 0.0 for q, o in zip(bufs, (off_state, off_work)))
+    for o in out[1:]:
+        assert np.array_equal(o[0], out[0][0]) and o[1] == out[0][1]
