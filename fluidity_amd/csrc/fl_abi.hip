@@ -204,7 +204,9 @@ SweepShape pick_shape(const fl_context* ctx, int dim, int64_t nx, int64_t ny, in
     const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
     return {false, B, fit_rows(dim ? tu.y_rows : tu.x_rows, ngrids * bands, ny, B)};
   }
-  if (ctx->shape[dim] == kShapeCell || nx * ny * ngrids <= kCellMax<T>) return {true, 0, 0};
+  // kShapeCell was measured on one grid; two of them may be past the line
+  if ((ctx->shape[dim] == kShapeCell && ngrids == 1) || nx * ny * ngrids <= kCellMax<T>)
+    return {true, 0, 0};
   const int B = dim ? 64 : 128;
   const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
   const int64_t waves = ngrids * bands * (B / 64) * ny;  // of one-row tiles

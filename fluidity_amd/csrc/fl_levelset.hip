@@ -169,45 +169,6 @@ __global__ void velocity_kernel(const double* __restrict__ phi0, const double* _
   V[i] = v;
 }
 
-// Both level sets' speeds in one pass (the two-material step's
-// velocity_kernel with target 0 and target 1): V_m = u.n_m of the material
-// present, with the same expressions per target.
-template <int ND>
-__global__ void velocity2_kernel(const double* __restrict__ phi0, const double* __restrict__ phi1,
-                                 StateView u0, StateView u1, Grid g, double dh,
-                                 double* __restrict__ V0, double* __restrict__ V1) {
-  const int64_t i = gid();
-  if (i >= g.nx * g.ny) return;
-  const int64_t x = i % g.nx, y = i / g.nx;
-  // the first material whose phi <= 0 (both values loaded up front)
-  // (bitwise ors: no short circuit that would move the second load after
-  // the first test)
-  const double p0 = phi0[i], p1 = phi1[i];
-  keep(p0);
-  keep(p1);
-  const bool in0 = ((int)(p0 <= 0.0) | (int)(p0 <= -0.0)) != 0;
-  const bool in1 = ((int)(p1 <= 0.0) | (int)(p1 <= -0.0)) != 0;
-  const int m = in0 ? 0 : (in1 ? 1 : -1);
-  double v0 = 0.0, v1 = 0.0;
-  if (m >= 0) {
-    double n0[2], n1[2];
-    norm_at<ND>(phi0, g, x, y, dh, n0);
-    norm_at<ND>(phi1, g, x, y, dh, n1);
-    double u[2 + ND];
-    load_state_i<2 + ND>(m == 0 ? u0 : u1, i, u);
-    double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      s0 += (u[2 + d] / u[0]) * n0[d];
-      s1 += (u[2 + d] / u[0]) * n1[d];
-    }
-    v0 = s0;
-    v1 = s1;
-  }
-  V0[i] = v0;
-  V1[i] = v1;
-}
-
 __global__ void project2_kernel(double* __restrict__ phi0, double* __restrict__ phi1,
                                 int64_t count) {
   const int64_t i = gid();
@@ -225,40 +186,66 @@ __global__ void project2_kernel(double* __restrict__ phi0, double* __restrict__ 
 __device__ __forceinline__ double smin(double a, double b) { return (b < a) ? b : a; }
 __device__ __forceinline__ double smax(double a, double b) { return (a < b) ? b : a; }
 
-// HJWeno5::diff (scheme/stencils/weno_hj_5.hpp:97-143), std::pow(x, 2) as x*x.
-// FAST: the fast FP64 numerics (four refined reciprocals instead of the
-// correctly rounded quotients).
+// HJWeno5::diff (scheme/stencils/weno_hj_5.hpp:97-143), std::pow(x, 2) as x*x:
+// the candidate derivatives (6 times them) of the differences d1..d5 from the
+// upwind end, and their weighted mean.  dmax = max |d|, whose square is the
+// maximum of the squares.  FAST: the fast FP64 numerics (FMAs, and four
+// refined reciprocals instead of the correctly rounded quotients).
+struct Weno {
+  double d1, d2, d3, d4, d5, phi_1, phi_2, phi_3;
+};
+
 template <bool FAST>
-__device__ __forceinline__ double weno_diff(double d1, double d2, double d3, double d4,
-                                            double d5) {
-  const double phi_1 = 2.0 * d1 - 7.0 * d2 + 11.0 * d3;
-  const double phi_2 = -d2 + 5.0 * d3 + 2.0 * d4;
-  const double phi_3 = 2.0 * d3 + 5.0 * d4 - d5;
+__device__ __forceinline__ Weno weno_of(double d1, double d2, double d3, double d4, double d5) {
+  Weno w = {d1, d2, d3, d4, d5, 0.0, 0.0, 0.0};
+  if (FAST) {
+    w.phi_1 = fast::fma(11.0, d3, fast::fma(-7.0, d2, d1 + d1));
+    w.phi_2 = fast::fma(2.0, d4, fast::fma(5.0, d3, -d2));
+    w.phi_3 = fast::fma(5.0, d4, fast::fma(2.0, d3, -d5));
+  } else {
+    w.phi_1 = 2.0 * d1 - 7.0 * d2 + 11.0 * d3;
+    w.phi_2 = -d2 + 5.0 * d3 + 2.0 * d4;
+    w.phi_3 = 2.0 * d3 + 5.0 * d4 - d5;
+  }
+  return w;
+}
+
+template <bool FAST>
+__device__ __forceinline__ double weno_mean(const Weno& w, double dmax) {
+  const double d1 = w.d1, d2 = w.d2, d3 = w.d3, d4 = w.d4, d5 = w.d5;
   const double f1 = 13.0 / 12.0;
   const double f2 = 1.0 / 4.0;
+  if (FAST) {
+    const double s11 = fast::fma(-2.0, d2, d1 + d3);
+    const double s12 = fast::fma(3.0, d3, fast::fma(-4.0, d2, d1));
+    const double s21 = fast::fma(-2.0, d3, d2 + d4), s22 = d2 - d4;
+    const double s31 = fast::fma(-2.0, d4, d3 + d5);
+    const double s32 = fast::fma(3.0, d3, fast::fma(-4.0, d4, d5));
+    const double e = fast::fma(10.0e-6 * dmax, dmax, 10.0e-99);
+    const double a1e = fast::fma(f1 * s11, s11, fast::fma(f2 * s12, s12, e));
+    const double a2e = fast::fma(f1 * s21, s21, fast::fma(f2 * s22, s22, e));
+    const double a3e = fast::fma(f1 * s31, s31, fast::fma(f2 * s32, s32, e));
+    // the quotients as products with refined reciprocals; a*e^2 >= 1e-196
+    // and the weight sum <= 6e196 keep every reciprocal in the normal range
+    const double w_1 = 0.1 * fast::rcp(a1e * a1e);
+    const double w_2 = 0.6 * fast::rcp(a2e * a2e);
+    const double w_3 = 0.3 * fast::rcp(a3e * a3e);
+    const double num = fast::fma(w_1, w.phi_1, fast::fma(w_2, w.phi_2, w_3 * w.phi_3));
+    return num * fast::rcp((w_1 + w_2 + w_3) * 6.0);
+  }
   const double s11 = d1 - 2.0 * d2 + d3, s12 = d1 - 4.0 * d2 + 3.0 * d3;
   const double s21 = d2 - 2.0 * d3 + d4, s22 = d2 - d4;
   const double s31 = d3 - 2.0 * d4 + d5, s32 = 3.0 * d3 - 4.0 * d4 + d5;
   double alpha_1 = f1 * (s11 * s11) + f2 * (s12 * s12);
   double alpha_2 = f1 * (s21 * s21) + f2 * (s22 * s22);
   double alpha_3 = f1 * (s31 * s31) + f2 * (s32 * s32);
-  const double e =
-      10.0e-6 * smax(smax(smax(smax(d1 * d1, d2 * d2), d3 * d3), d4 * d4), d5 * d5) + 10.0e-99;
+  const double e = 10.0e-6 * (dmax * dmax) + 10.0e-99;
   const double a1e = alpha_1 + e, a2e = alpha_2 + e, a3e = alpha_3 + e;
-  if (FAST) {
-    // the quotients as products with refined reciprocals; a*e*^2 >= 1e-196
-    // and the weight sum <= 6e196 keep every reciprocal in the normal range
-    alpha_1 = 0.1 * fast::rcp(a1e * a1e);
-    alpha_2 = 0.6 * fast::rcp(a2e * a2e);
-    alpha_3 = 0.3 * fast::rcp(a3e * a3e);
-    const double w_denom = (alpha_1 + alpha_2 + alpha_3) * 6.0;
-    return (alpha_1 * phi_1 + alpha_2 * phi_2 + alpha_3 * phi_3) * fast::rcp(w_denom);
-  }
   alpha_1 = 0.1 / (a1e * a1e);
   alpha_2 = 0.6 / (a2e * a2e);
   alpha_3 = 0.3 / (a3e * a3e);
   const double w_denom = (alpha_1 + alpha_2 + alpha_3) * 6.0;
-  return (alpha_1 * phi_1 + alpha_2 * phi_2 + alpha_3 * phi_3) / w_denom;
+  return (alpha_1 * w.phi_1 + alpha_2 * w.phi_2 + alpha_3 * w.phi_3) / w_denom;
 }
 
 // Mirrored index within a line of n cells (32-bit; n < 2^30).
@@ -271,14 +258,13 @@ __device__ __forceinline__ int mirror32(int i, int n) {
 // L = V * H(phi) (levelset_hamiltonian.hpp:63-98, godunov_upwind.hpp:94-166).
 // h1 = 1 / dh, computed once by the caller (the same IEEE quotient).  ND =
 // g.nd; the 7-cell stencils of all dimensions are loaded before any is used.
-// xin / yin: every cell of the stencil in x / y lies inside the grid (the
-// caller's workgroup-uniform test), so the mirror index math is skipped.
-template <int ND, bool FAST>
-__device__ double ls_rhs(const double* __restrict__ phi, const Grid& g, int x, int y, double v,
-                         double h1, bool xin, bool yin) {
-  double result = 0.0;
+// ls_stencil: xin / yin: every cell of the stencil in x / y lies inside the
+// grid (the caller's workgroup-uniform test), so the mirror index math is
+// skipped.
+template <int ND>
+__device__ __forceinline__ void ls_stencil(const double* __restrict__ phi, const Grid& g, int x,
+                                           int y, bool xin, bool yin, double (*fs)[7]) {
   const int nx = (int)g.nx, ny = (int)g.ny;
-  double fs[ND][7];
   {
     const double* row = phi + (int64_t)y * nx;
     if (xin) {
@@ -298,32 +284,55 @@ __device__ double ls_rhs(const double* __restrict__ phi, const Grid& g, int x, i
       for (int k = -3; k <= 3; ++k) fs[ND - 1][k + 3] = phi[(int64_t)mirror32(y + k, ny) * nx + x];
     }
   }
-  // A stencil whose cells all hold the centre's bit pattern (the clamped
-  // values outside the reinitialised band) has every difference +0: each
-  // one-sided WENO derivative is then 0 / (6 * 10^195) = +0 and the Godunov
-  // sum is +0, so L = v * sqrt(+0) = v * 0 exactly.  A wave whose cells are
-  // all such skips the WENO arithmetic; the others take it.
-  bool flat = isfinite(fs[0][3]);
-#pragma unroll
-  for (int d = 0; d < ND; ++d)
-#pragma unroll
-    for (int k = 0; k < 7; ++k)
-      flat = flat && __double_as_longlong(fs[d][k]) == __double_as_longlong(fs[0][3]);
-  if (__all(flat)) return v * 0.0;
+}
+
+template <int ND, bool FAST>
+__device__ __forceinline__ double ls_rhs(const double (*fs)[7], double v, double h1) {
+  double D[ND][6], inner[ND], dmax = 0.0;
+  bool calm = true;  // every difference finite, no product of the weights overflows
 #pragma unroll
   for (int d = 0; d < ND; ++d) {
-    const double* f = fs[d];
-    const double bd = weno_diff<FAST>(h1 * (f[1] - f[0]), h1 * (f[2] - f[1]), h1 * (f[3] - f[2]),
-                                h1 * (f[4] - f[3]), h1 * (f[5] - f[4]));
-    const double fd = weno_diff<FAST>(h1 * (f[6] - f[5]), h1 * (f[5] - f[4]), h1 * (f[4] - f[3]),
-                                h1 * (f[3] - f[2]), h1 * (f[2] - f[1]));
-    double back, fwrd;
-    if (v <= 0.0) {
-      back = smax(bd, 0.0);
-      fwrd = smin(fd, 0.0);
-    } else {
-      back = smin(bd, 0.0);
-      fwrd = smax(fd, 0.0);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) D[d][k] = h1 * (fs[d][k + 1] - fs[d][k]);
+    inner[d] = fast::mx(fast::mx(fabs(D[d][1]), fabs(D[d][2])),
+                        fast::mx(fabs(D[d][3]), fabs(D[d][4])));
+    dmax = fast::mx(dmax, fast::mx(inner[d], fast::mx(fabs(D[d][0]), fabs(D[d][5]))));
+    const double sum = ((D[d][0] + D[d][1]) + (D[d][2] + D[d][3])) + (D[d][4] + D[d][5]);
+    calm = calm && fabs(sum) < 1.0e41;  // false for a NaN, which mx passes over
+  }
+  calm = calm && dmax < 1.0e40;
+  // A stencil of one value (the clamped ones outside the reinitialised band)
+  // has every difference +0: each one-sided WENO derivative is then 0 / (6 *
+  // 10^195) = +0 and the Godunov sum is +0, so L = v * sqrt(+0) = v * 0
+  // exactly.  A wave whose cells are all such skips the WENO arithmetic; the
+  // others take it.
+  if (__all(calm && dmax == 0.0)) return v * 0.0;
+  const bool up = v <= 0.0;
+  double result = 0.0;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    // Of each one-sided derivative Godunov's sum keeps one sign: positive
+    // backward and negative forward ones for v <= 0, the others for v > 0.
+    // The derivative is a mean of its three candidates with positive weights,
+    // so where these all have the other sign it contributes the square of 0,
+    // and a wave of such cells leaves it out: away from kinks that is one of
+    // the two.
+    const Weno b = weno_of<FAST>(D[d][0], D[d][1], D[d][2], D[d][3], D[d][4]);
+    const Weno w = weno_of<FAST>(D[d][5], D[d][4], D[d][3], D[d][2], D[d][1]);
+    const double lo_b = fast::mn(fast::mn(b.phi_1, b.phi_2), b.phi_3);
+    const double hi_b = fast::mx(fast::mx(b.phi_1, b.phi_2), b.phi_3);
+    const double lo_w = fast::mn(fast::mn(w.phi_1, w.phi_2), w.phi_3);
+    const double hi_w = fast::mx(fast::mx(w.phi_1, w.phi_2), w.phi_3);
+    const bool no_b = calm && (up ? hi_b <= 0.0 : lo_b >= 0.0);
+    const bool no_w = calm && (up ? lo_w >= 0.0 : hi_w <= 0.0);
+    double back = 0.0, fwrd = 0.0;
+    if (!__all(no_b)) {
+      const double bd = weno_mean<FAST>(b, fast::mx(fabs(D[d][0]), inner[d]));
+      back = up ? smax(bd, 0.0) : smin(bd, 0.0);
+    }
+    if (!__all(no_w)) {
+      const double fd = weno_mean<FAST>(w, fast::mx(fabs(D[d][5]), inner[d]));
+      fwrd = up ? smin(fd, 0.0) : smax(fd, 0.0);
     }
     result += smax(back * back, fwrd * fwrd);
   }
@@ -336,6 +345,13 @@ __device__ double ls_rhs(const double* __restrict__ phi, const Grid& g, int x, i
 //  stage 2: out = (1/3) phi_n + (2 (1/3)) (s2 - dt L(s2))
 // Launched on a (ceil(nx / blockDim.x), min(ny, 65535)) grid; rows stride by
 // gridDim.y.
+__device__ __forceinline__ double rk3_last(double phi_n, double s2, double dtl) {
+  const double fact_13 = 1.0 / 3.0;
+  const double fact_23 = 2.0 * fact_13;
+  const double s3 = s2 - dtl;
+  return (fact_13 * phi_n) + (fact_23 * s3);
+}
+
 template <int ND, bool FAST>
 __device__ __forceinline__ void rk3_stage_body(int stage, const double* __restrict__ phi_n,
                                                const double* __restrict__ src,
@@ -348,16 +364,15 @@ __device__ __forceinline__ void rk3_stage_body(int stage, const double* __restri
   for (int y = blockIdx.y; y < g.ny; y += gridDim.y) {
     const int64_t i = (int64_t)y * g.nx + x;
     const bool yin = y >= 3 && y + 3 < g.ny;
-    const double l = ls_rhs<ND, FAST>(src, g, x, y, V[i], h1, xin, yin);
+    double fs[ND][7];
+    ls_stencil<ND>(src, g, x, y, xin, yin, fs);
+    const double l = ls_rhs<ND, FAST>(fs, V[i], h1);
     if (stage == 0) {
       out[i] = phi_n[i] - dt * l;
     } else if (stage == 1) {
-      out[i] = 0.75 * phi_n[i] + 0.25 * (src[i] - dt * l);
+      out[i] = 0.75 * phi_n[i] + 0.25 * (fs[0][3] - dt * l);
     } else {
-      const double fact_13 = 1.0 / 3.0;
-      const double fact_23 = 2.0 * fact_13;
-      const double s3 = src[i] - dt * l;
-      out[i] = (fact_13 * phi_n[i]) + (fact_23 * s3);
+      out[i] = rk3_last(phi_n[i], fs[0][3], dt * l);
     }
   }
 }
@@ -373,13 +388,175 @@ __global__ void rk3_stage_kernel(int stage, const double* __restrict__ phi_n,
   rk3_stage_body<ND, false>(stage, phi_n, src, V, g, dt, h1, out);
 }
 
-// The same stage of two level sets' advection in one launch (blockIdx.z
-// selects the job), dt in device memory; FAST: the fast FP64 numerics.
+// The RK3 stages of two level sets.  A wave marches down `rows` rows of 64
+// columns, four waves to a workgroup one below the other: a stage reads each
+// cell's seven rows, and from a register window they are one load a cell (with
+// a workgroup per row the seven rows came to seven XCDs' L2s), and the tiles
+// of an XCD are neighbours.  FP64 instructions bound it (350 a cell with one
+// of the two WENO derivatives, 71% of the issue slots): a stage of two
+// 2048x1024 level sets 74 -> 56 us, with the speeds computed in it 102 -> 71,
+// with the projection 87 -> 58.  Four waves a SIMD (128 registers) spill: 77
+// and 67 us.
+struct LsTile {
+  int x, y0, y1;  // this lane's column, the wave's rows
+  bool xin;       // workgroup-uniform: every stencil of the tile lies inside in x
+};
+
+__device__ __forceinline__ LsTile ls_tile(const Grid& g, int rows) {
+  // workgroups go to the 8 XCDs in turn; each XCD takes consecutive tiles
+  const int total = (int)(gridDim.x * gridDim.y), id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  const int base = total / 8, extra = total % 8, xcd = id % 8;
+  const int tile = xcd * base + (xcd < extra ? xcd : extra) + id / 8;
+  const int bx = tile % (int)gridDim.x, by = tile / (int)gridDim.x;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  LsTile t;
+  t.x = bx * 64 + (int)(threadIdx.x & 63);
+  t.y0 = (by * 4 + w) * rows;
+  t.y1 = t.y0 + rows < (int)g.ny ? t.y0 + rows : (int)g.ny;
+  t.xin = bx > 0 && bx * 64 + 67 <= (int)g.nx;
+  return t;
+}
+
+// One level set's stencil window down a column: rows y - 3 .. y + 3 in fs[ND -
+// 1], the row's neighbours in fs[0].
+template <int ND>
+struct LsWindow {
+  double fs[ND][7];
+  const double* __restrict__ phi;
+
+  __device__ __forceinline__ double at(const Grid& g, int x, int y) const {
+    return phi[(int64_t)mirror32(y, (int)g.ny) * g.nx + x];
+  }
+  // before the first row y0
+  __device__ __forceinline__ void start(const double* p, const Grid& g, int x, int y0) {
+    phi = p;
+    if (ND > 1) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) fs[ND - 1][k + 1] = at(g, x, y0 - 3 + k);
+    }
+  }
+  __device__ __forceinline__ void step(const Grid& g, int x, int y, bool xin) {
+    if (ND > 1) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) fs[ND - 1][k] = fs[ND - 1][k + 1];
+      fs[ND - 1][6] = at(g, x, y + 3);
+    }
+    const double* row = phi + (int64_t)y * g.nx;
+#pragma unroll
+    for (int k = -3; k <= 3; ++k) {
+      if (ND > 1 && k == 0) fs[0][3] = fs[ND - 1][3];
+      else fs[0][k + 3] = row[xin ? x + k : mirror32(x + k, (int)g.nx)];
+    }
+  }
+};
+
+// MultidimIterator::norm from the window: the mirrored neighbours of norm_at
+// are the stencil's.
+template <int ND>
+__device__ __forceinline__ void norm_of(const double (*fs)[7], double dh, double* nrm) {
+  const double fact = 0.5 / dh;
+  double mag = 0.0;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    nrm[d] = fact * (fs[d][4] - fs[d][2]);
+    mag += nrm[d] * nrm[d];
+  }
+  if (__all(mag == 0.0)) {
+#pragma unroll
+    for (int d = 0; d < ND; ++d) nrm[d] = 0.0;
+    return;
+  }
+  const double s = sqrt(mag);
+#pragma unroll
+  for (int d = 0; d < ND; ++d) nrm[d] = (mag == 0.0) ? 0.0 : nrm[d] / s;
+}
+
+// Stages 0 to 2 of one level set (blockIdx.z selects the job), speeds given.
 template <int ND, bool FAST>
-__global__ void rk3_stage2_kernel(int stage, Rk3Job j0, Rk3Job j1, Grid g,
-                                  const double* dt_dev, double h1) {
+__global__ void __launch_bounds__(256) rk3_stage2_kernel(int stage, Rk3Job j0, Rk3Job j1, Grid g,
+                                                         int rows, const double* dt_dev,
+                                                         double h1) {
   const Rk3Job j = blockIdx.z ? j1 : j0;
-  rk3_stage_body<ND, FAST>(stage, j.phi_n, j.src, j.V, g, *dt_dev, h1, j.out);
+  const LsTile t = ls_tile(g, rows);
+  const double dt = *dt_dev;
+  if (t.x >= g.nx) return;
+  LsWindow<ND> win;
+  win.start(j.src, g, t.x, t.y0);
+  for (int y = t.y0; y < t.y1; ++y) {
+    const int64_t i = (int64_t)y * g.nx + t.x;
+    win.step(g, t.x, y, t.xin);
+    const double v = j.V[i], n = stage ? j.phi_n[i] : 0.0;
+    const double s = win.fs[0][3], dtl = dt * ls_rhs<ND, FAST>(win.fs, v, h1);
+    j.out[i] = stage == 0   ? s - dtl
+               : stage == 1 ? 0.75 * n + 0.25 * (s - dtl)
+                            : rk3_last(n, s, dtl);
+  }
+}
+
+// The first and last stages of a two-material step, both level sets of a cell
+// in one thread, with what the step does to them before and after: the first
+// computes the speeds V_m = u . n_m of the material present (velocity_kernel
+// with target 0 and target 1) from the neighbours that the stencil holds
+// anyway, the last projects (project2_kernel).  As passes of their own these
+// two took 28 and 12 us of a 2048x1024 step, most of it memory.
+template <int ND, bool FAST>
+__global__ void __launch_bounds__(256) rk3_first2_kernel(Rk3Job j0, Rk3Job j1, double* V0,
+                                                         double* V1, StateView u0, StateView u1,
+                                                         Grid g, int rows, const double* dt_dev,
+                                                         double dh, double h1) {
+  const LsTile t = ls_tile(g, rows);
+  const double dt = *dt_dev;
+  if (t.x >= g.nx) return;
+  LsWindow<ND> w0, w1;
+  w0.start(j0.src, g, t.x, t.y0);
+  w1.start(j1.src, g, t.x, t.y0);
+  for (int y = t.y0; y < t.y1; ++y) {
+    const int64_t i = (int64_t)y * g.nx + t.x;
+    w0.step(g, t.x, y, t.xin);
+    w1.step(g, t.x, y, t.xin);
+    const double p0 = w0.fs[0][3], p1 = w1.fs[0][3];
+    const bool in0 = p0 <= 0.0, in1 = p1 <= 0.0;
+    double v0 = 0.0, v1 = 0.0;
+    if (in0 || in1) {
+      double u[2 + ND], n0[2], n1[2];
+      load_state_i<2 + ND>(in0 ? u0 : u1, i, u);
+      norm_of<ND>(w0.fs, dh, n0);
+      norm_of<ND>(w1.fs, dh, n1);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        const double ud = u[2 + d] / u[0];
+        v0 += ud * n0[d];
+        v1 += ud * n1[d];
+      }
+    }
+    V0[i] = v0;
+    V1[i] = v1;
+    j0.out[i] = p0 - dt * ls_rhs<ND, FAST>(w0.fs, v0, h1);
+    j1.out[i] = p1 - dt * ls_rhs<ND, FAST>(w1.fs, v1, h1);
+  }
+}
+
+template <int ND, bool FAST>
+__global__ void __launch_bounds__(256) rk3_last2_kernel(Rk3Job j0, Rk3Job j1, Grid g, int rows,
+                                                        const double* dt_dev, double h1) {
+  const LsTile t = ls_tile(g, rows);
+  const double dt = *dt_dev;
+  if (t.x >= g.nx) return;
+  LsWindow<ND> w0, w1;
+  w0.start(j0.src, g, t.x, t.y0);
+  w1.start(j1.src, g, t.x, t.y0);
+  for (int y = t.y0; y < t.y1; ++y) {
+    const int64_t i = (int64_t)y * g.nx + t.x;
+    w0.step(g, t.x, y, t.xin);
+    w1.step(g, t.x, y, t.xin);
+    const double v0 = j0.V[i], v1 = j1.V[i], n0 = j0.phi_n[i], n1 = j1.phi_n[i];
+    const double p0 = rk3_last(n0, w0.fs[0][3], dt * ls_rhs<ND, FAST>(w0.fs, v0, h1));
+    const double p1 = rk3_last(n1, w1.fs[0][3], dt * ls_rhs<ND, FAST>(w1.fs, v1, h1));
+    const double avg = 0.5 * (p0 + p1);
+    const double a = p0 - avg;
+    j0.out[i] = a;
+    j1.out[i] = -a;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1087,15 +1264,19 @@ __global__ void combine_kernel(const double* __restrict__ phi0, StateView u0, St
   store_state<S>(out, i, s);
 }
 
+#define FL_LS_RK3(ND, FAST)                                                                   \
+  template __global__ void rk3_first2_kernel<ND, FAST>(Rk3Job, Rk3Job, double*, double*,       \
+                                                       StateView, StateView, Grid, int,        \
+                                                       const double*, double, double);         \
+  template __global__ void rk3_last2_kernel<ND, FAST>(Rk3Job, Rk3Job, Grid, int,               \
+                                                      const double*, double);                  \
+  template __global__ void rk3_stage2_kernel<ND, FAST>(int, Rk3Job, Rk3Job, Grid, int,         \
+                                                       const double*, double);
 #define FL_LS_INST(ND)                                                                       \
   template __global__ void velocity_kernel<ND>(const double*, const double*, StateView,      \
                                                StateView, int, Grid, double, int, double*); \
-  template __global__ void velocity2_kernel<ND>(const double*, const double*, StateView,     \
-                                                StateView, Grid, double, double*, double*); \
-  template __global__ void rk3_stage2_kernel<ND, false>(int, Rk3Job, Rk3Job, Grid,            \
-                                                        const double*, double);              \
-  template __global__ void rk3_stage2_kernel<ND, true>(int, Rk3Job, Rk3Job, Grid,             \
-                                                       const double*, double);               \
+  FL_LS_RK3(ND, false)                                                                        \
+  FL_LS_RK3(ND, true)                                                                         \
   template __global__ void rk3_stage_kernel<ND>(int, const double*, const double*,            \
                                                 const double*, Grid, double, const double*,  \
                                                 double, double*);                            \

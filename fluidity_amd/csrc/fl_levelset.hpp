@@ -85,9 +85,6 @@ __global__ void project_n_kernel(PhiSet ps, int64_t count);
 template <int ND>
 __global__ void velocity_kernel(const double* phi0, const double* phi1, StateView u0,
                                 StateView u1, int nmat, Grid g, double dh, int target, double* V);
-template <int ND>
-__global__ void velocity2_kernel(const double* phi0, const double* phi1, StateView u0,
-                                 StateView u1, Grid g, double dh, double* V0, double* V1);
 __global__ void project2_kernel(double* phi0, double* phi1, int64_t count);
 // One level set's RK3 stage: phi_n, the stage source, the speed and the output.
 struct Rk3Job {
@@ -96,9 +93,18 @@ struct Rk3Job {
   const double* V;
   double* out;
 };
+// Launched on (ceil(nx / 64), ceil(ny / (4 rows))) workgroups of 256 threads
+// (rk3_stage2_kernel: z = 2, a level set each).
 template <int ND, bool FAST>
-__global__ void rk3_stage2_kernel(int stage, Rk3Job j0, Rk3Job j1, Grid g, const double* dt_dev,
+__global__ void rk3_stage2_kernel(int stage, Rk3Job j0, Rk3Job j1, Grid g, int rows,
+                                  const double* dt_dev, double h1);
+template <int ND, bool FAST>
+__global__ void rk3_first2_kernel(Rk3Job j0, Rk3Job j1, double* V0, double* V1, StateView u0,
+                                  StateView u1, Grid g, int rows, const double* dt_dev, double dh,
                                   double h1);
+template <int ND, bool FAST>
+__global__ void rk3_last2_kernel(Rk3Job j0, Rk3Job j1, Grid g, int rows, const double* dt_dev,
+                                 double h1);
 template <int ND>
 __global__ void rk3_stage_kernel(int stage, const double* phi_n, const double* src,
                                  const double* V, Grid g, double dt, const double* dt_dev,

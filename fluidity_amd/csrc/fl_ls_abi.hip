@@ -92,22 +92,6 @@ int launch_velocity(int nmat, const double* const* phis, const fl_field* states,
   return FL_OK;
 }
 
-// Both level sets' speeds from the level sets phis and the two states.
-int launch_velocity2(double* const* phis, const fl_field& s0, const fl_field& s1,
-                     const ls::Grid& g, double dh, double* const* V, hipStream_t st) {
-  const dim3 grid = grid_for(g.nx * g.ny);
-  if (g.nd == 1)
-    hipLaunchKernelGGL(ls::velocity2_kernel<1>, grid, dim3(kBlock), 0, st,
-                       (const double*)phis[0], (const double*)phis[1], view_of(&s0),
-                       view_of(&s1), g, dh, V[0], V[1]);
-  else
-    hipLaunchKernelGGL(ls::velocity2_kernel<2>, grid, dim3(kBlock), 0, st,
-                       (const double*)phis[0], (const double*)phis[1], view_of(&s0),
-                       view_of(&s1), g, dh, V[0], V[1]);
-  FL_HIP(hipGetLastError());
-  return FL_OK;
-}
-
 // RK3: phi -> s1 -> s2 -> out, s1/s2 in work.  dt_dev (nullable): dt in
 // device memory, used instead of dt.
 int launch_advect(const double* phi, const double* V, const ls::Grid& g, double dt, double dh,
@@ -128,29 +112,73 @@ int launch_advect(const double* phi, const double* V, const ls::Grid& g, double 
   return FL_OK;
 }
 
+// Rows a wave of the two-level-set stages marches: as many as leave 16384 waves
+// of 64 columns in the launch, at most 8 (at least what keeps the launch's y
+// extent below 65536).  A stage at 2048x1024 with 4096, 8192, 16384, 65536
+// waves: 68, 61, 56, 62 us.
+int march_rows(const ls::Grid& g, int jobs) {
+  const int64_t rows = (g.nx + 63) / 64 * g.ny * jobs / 16384;
+  const int64_t least = (g.ny + 4 * 65535 - 1) / (4 * 65535);
+  return (int)std::max(std::max<int64_t>(1, least), std::min<int64_t>(rows, 8));
+}
+dim3 march_grid(const ls::Grid& g, int rows, int jobs) {
+  return dim3((unsigned)((g.nx + 63) / 64), (unsigned)((g.ny + 4 * rows - 1) / (4 * rows)), jobs);
+}
+
+struct Rk3Jobs { ls::Rk3Job j[3][2]; };
+Rk3Jobs rk3_jobs(double* const cur[2], double* const V[2], const ls::Grid& g, double* const out[2],
+                 double* work) {
+  const int64_t cells = g.nx * g.ny;
+  Rk3Jobs r;
+  for (int m = 0; m < 2; ++m) {
+    double* s1 = work + m * cells;
+    double* s2 = work + (2 + m) * cells;
+    r.j[0][m] = {cur[m], cur[m], V[m], s1};
+    r.j[1][m] = {cur[m], s1, V[m], s2};
+    r.j[2][m] = {cur[m], s2, V[m], out[m]};
+  }
+  return r;
+}
+
+void launch_rk3_stage2(int stage, const Rk3Jobs& r, const ls::Grid& g, const double* dt_dev,
+                       double h1, bool fast, hipStream_t st) {
+  auto k = g.nd == 1 ? (fast ? ls::rk3_stage2_kernel<1, true> : ls::rk3_stage2_kernel<1, false>)
+                     : (fast ? ls::rk3_stage2_kernel<2, true> : ls::rk3_stage2_kernel<2, false>);
+  const int rows = march_rows(g, 2);
+  hipLaunchKernelGGL(k, march_grid(g, rows, 2), dim3(256), 0, st, stage, r.j[stage][0],
+                     r.j[stage][1], g, rows, dt_dev, h1);
+}
+
 // RK3 of both level sets, each stage of both in one launch: cur[m] -> out[m]
 // with speeds V[m], dt in device memory; work holds 4 cells of scratch.
 // fast: the fast FP64 numerics in the WENO derivatives.
 int launch_advect2(double* const cur[2], double* const V[2], const ls::Grid& g, double dh,
                    double* const out[2], double* work, const double* dt_dev, bool fast,
                    hipStream_t st) {
-  const int64_t cells = g.nx * g.ny;
-  double* s1[2] = {work, work + cells};
-  double* s2[2] = {work + 2 * cells, work + 3 * cells};
-  const dim3 grid((unsigned)((g.nx + kBlock - 1) / kBlock),
-                  (unsigned)(g.ny < 65535 ? g.ny : 65535), 2);
-  const double h1 = 1.0 / dh;
-  auto k = g.nd == 1 ? (fast ? ls::rk3_stage2_kernel<1, true> : ls::rk3_stage2_kernel<1, false>)
-                     : (fast ? ls::rk3_stage2_kernel<2, true> : ls::rk3_stage2_kernel<2, false>);
-  ls::Rk3Job j[3][2];
-  for (int m = 0; m < 2; ++m) {
-    j[0][m] = {cur[m], cur[m], V[m], s1[m]};
-    j[1][m] = {cur[m], s1[m], V[m], s2[m]};
-    j[2][m] = {cur[m], s2[m], V[m], out[m]};
-  }
+  const Rk3Jobs r = rk3_jobs(cur, V, g, out, work);
   for (int stage = 0; stage < 3; ++stage)
-    hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, st, stage, j[stage][0], j[stage][1], g, dt_dev,
-                       h1);
+    launch_rk3_stage2(stage, r, g, dt_dev, 1.0 / dh, fast, st);
+  FL_HIP(hipGetLastError());
+  return FL_OK;
+}
+
+// The same with the speeds V[m] computed from the states on the way, and the
+// result projected: three launches for a two-material step's level sets.
+int launch_advance2(double* const cur[2], double* const V[2], const fl_field& s0,
+                    const fl_field& s1, const ls::Grid& g, double dh, double* const out[2],
+                    double* work, const double* dt_dev, bool fast, hipStream_t st) {
+  const Rk3Jobs r = rk3_jobs(cur, V, g, out, work);
+  const double h1 = 1.0 / dh;
+  const int rows = march_rows(g, 1);
+  const dim3 grid = march_grid(g, rows, 1);
+  auto first = g.nd == 1 ? (fast ? ls::rk3_first2_kernel<1, true> : ls::rk3_first2_kernel<1, false>)
+                         : (fast ? ls::rk3_first2_kernel<2, true> : ls::rk3_first2_kernel<2, false>);
+  auto last = g.nd == 1 ? (fast ? ls::rk3_last2_kernel<1, true> : ls::rk3_last2_kernel<1, false>)
+                        : (fast ? ls::rk3_last2_kernel<2, true> : ls::rk3_last2_kernel<2, false>);
+  hipLaunchKernelGGL(first, grid, dim3(256), 0, st, r.j[0][0], r.j[0][1], V[0], V[1], view_of(&s0),
+                     view_of(&s1), g, rows, dt_dev, dh, h1);
+  launch_rk3_stage2(1, r, g, dt_dev, h1, fast, st);
+  hipLaunchKernelGGL(last, grid, dim3(256), 0, st, r.j[2][0], r.j[2][1], g, rows, dt_dev, h1);
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
@@ -865,9 +893,9 @@ int fl_mm_simulate(fl_context* c, fl_material* mats, int nmat, const fl_sim_para
     // level sets: speeds from the old level sets and new states (both in one
     // pass), advection with the device dt, projection, reinitialisation every
     // `every` steps
-    if ((rc = launch_velocity2(cur, mats[0].state, mats[1].state, g, dh, w.V, st))) return rc;
-    if ((rc = launch_advect2(cur, w.V, g, dh, nxt, w.adv, &ctl->dt, fast, st))) return rc;
-    if ((rc = launch_project(nxt[0], nxt[1], cells, st))) return rc;
+    if ((rc = launch_advance2(cur, w.V, mats[0].state, mats[1].state, g, dh, nxt, w.adv, &ctl->dt,
+                              fast, st)))
+      return rc;
     const bool reinit = (it % every) == every - 1;
     if (reinit) {  // both level sets in one solve, written back into cur[m]
       ls::EikJobs ej;
