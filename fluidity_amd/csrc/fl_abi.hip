@@ -886,7 +886,8 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
       float total = 0.0f;
       c->shape[dim] = kShapeCell;
       rc = timed(dim, &total);
-      if (!rc && total >= best_ms) c->shape[dim] = kShapeTuning;
+      // the best of many marching shapes is a lucky one when they are about equal
+      if (!rc && total >= 1.05f * best_ms) c->shape[dim] = kShapeTuning;
     }
   }
   (void)hipEventDestroy(e0);

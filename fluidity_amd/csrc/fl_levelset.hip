@@ -571,57 +571,55 @@ __device__ __forceinline__ EikJob eik_job(const EikJobs& js) {
   return blockIdx.z ? js.j[1] : js.j[0];
 }
 
+// Tiles of the eikonal solve: W cells x H rows, one per workgroup of
+// kEikThreads threads (512 cells of a line).
+template <int ND>
+struct EikTile {
+  static constexpr int W = eik_tile_w(ND), H = eik_tile_h(ND);
+  static constexpr int RW = W + 2 * kEikSteps, RH = ND == 1 ? 1 : H + 2 * kEikSteps;
+  static constexpr int R = RW * RH;  // cells of a tile with its halo
+  static constexpr int P = (R + kEikThreads - 1) / kEikThreads;
+};
+
 // Sources (fast_iterative_init, scheme/cuda/fast_iterative_method.cuh:48-85):
 // a cell beside a sign change with the smaller |phi|; distance |phi| there.
 // info = source | (signum(phi) + 1) << 1.  Both Jacobi buffers start equal.
-__global__ void eik_init_kernel(EikJobs jobs, Grid g) {
-  const int64_t i = gid();
-  if (i >= g.nx * g.ny) return;
+// src[t] = tile t holds a source; the control words are cleared.  Launched on
+// (tiles per row, min(tile rows, 65535)) workgroups; tile rows stride by
+// gridDim.y.
+template <int ND>
+__global__ void __launch_bounds__(kEikThreads) eik_init_kernel(EikJobs jobs, Grid g,
+                                                               int64_t trows) {
   const EikJob J = eik_job(jobs);
   const double* __restrict__ phi = J.phi;
-  double* __restrict__ d = J.d[0];
-  double* __restrict__ d1 = J.d[1];
-  uint8_t* __restrict__ info = J.info;
-  const int64_t x = i % g.nx, y = i / g.nx;
-  const double c = phi[i];
-  // the four axis neighbours (those past the edge, or in y on a 1D grid,
-  // read the cell itself and do not count), loaded together
-  const bool ok[4] = {x + 1 < g.nx, x > 0, g.nd > 1 && y + 1 < g.ny, g.nd > 1 && y > 0};
-  const int64_t nb[4] = {i + 1, i - 1, i + g.nx, i - g.nx};
-  double o[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) o[k] = phi[ok[k] ? nb[k] : i];
-  int source = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    if (ok[k] && signum(c) != signum(o[k]) && fabs(c) < fabs(o[k])) source = 1;
-  info[i] = (uint8_t)(source | ((signum(c) + 1) << 1));
-  const double v = source ? fabs(c) : DBL_MAX;
-  d[i] = v;
-  d1[i] = v;
-}
-
-// Tiles of the eikonal sweeps: kEikTileW cells x kEikTileH rows, one per
-// workgroup of kEikTileW * kEikTileH threads.  src[t] = the tile holds a
-// source.  Launched on (tiles per row, min(tile rows, 65535)) workgroups; tile
-// rows stride by gridDim.y.
-__device__ __forceinline__ void eik_cell_of(int64_t tr, int64_t& x, int64_t& y) {
-  x = (int64_t)blockIdx.x * kEikTileW + (threadIdx.x % kEikTileW);
-  y = tr * kEikTileH + (threadIdx.x / kEikTileW);
-}
-
-__global__ void __launch_bounds__(kEikTileW * kEikTileH) eik_tile_src_kernel(
-    EikJobs jobs, Grid g, int64_t trows) {
-  const EikJob J = eik_job(jobs);
-  const uint8_t* __restrict__ info = J.info;
-  uint8_t* __restrict__ src = J.src;
-  const int64_t segs = gridDim.x;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    const EikCtl zero = {};
+    *J.ctl = zero;
+  }
   for (int64_t tr = blockIdx.y; tr < trows; tr += gridDim.y) {
-    int64_t x, y;
-    eik_cell_of(tr, x, y);
-    const int has = (x < g.nx && y < g.ny) ? (info[y * g.nx + x] & 1) : 0;
-    const int any = __syncthreads_or(has);
-    if (threadIdx.x == 0) src[tr * segs + blockIdx.x] = (uint8_t)(any != 0);
+    const int64_t x = (int64_t)blockIdx.x * EikTile<ND>::W + threadIdx.x % EikTile<ND>::W;
+    const int64_t y = tr * EikTile<ND>::H + threadIdx.x / EikTile<ND>::W;
+    int source = 0;
+    if (x < g.nx && y < g.ny) {
+      const int64_t i = y * g.nx + x;
+      const double c = phi[i];
+      // the four axis neighbours (those past the edge, or in y on a 1D grid,
+      // read the cell itself and do not count), loaded together
+      const bool ok[4] = {x + 1 < g.nx, x > 0, ND > 1 && y + 1 < g.ny, ND > 1 && y > 0};
+      const int64_t nb[4] = {i + 1, i - 1, i + g.nx, i - g.nx};
+      double o[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = phi[ok[k] ? nb[k] : i];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (ok[k] && signum(c) != signum(o[k]) && fabs(c) < fabs(o[k])) source = 1;
+      J.info[i] = (uint8_t)(source | ((signum(c) + 1) << 1));
+      const double v = source ? fabs(c) : DBL_MAX;
+      J.d[0][i] = v;
+      J.d[1][i] = v;
+    }
+    const int any = __syncthreads_or(source);
+    if (threadIdx.x == 0) J.src[tr * gridDim.x + blockIdx.x] = (uint8_t)(any != 0);
   }
 }
 
@@ -655,119 +653,155 @@ __global__ void eik_tile_act_kernel(EikJobs jobs, int64_t trows, int64_t segs, i
   if (a) J.list[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)t;
 }
 
-// Neighbour distance v (info byte inf) seen from a cell with sign bits sc:
-// negated across the interface unless not yet reached.
-__device__ __forceinline__ double eik_nbr_v(double v, uint8_t inf, uint8_t sc) {
-  return ((inf & 6) == sc || v == DBL_MAX) ? v : -v;
+// Neighbour distance v seen from a cell on the same or the other side: negated
+// across the interface unless not yet reached.
+__device__ __forceinline__ double eik_nbr_v(double v, bool same) {
+  return (same || v == DBL_MAX) ? v : -v;
 }
 
-// One thread per job.
-__global__ void eik_ctl_init_kernel(EikJobs jobs, int njobs) {
-  if ((int)threadIdx.x >= njobs) return;
-  EikCtl* c = threadIdx.x ? jobs.j[1].ctl : jobs.j[0].ctl;
-  c->flags[0] = c->flags[1] = c->flags[2] = 0;
-  c->done = 0;
-  c->iters = 0;
-  c->ntiles = 0;
-  c->pad = 0;
-}
-
-// Sweep k of the Godunov eikonal update
-// (scheme/schemes/godunov_upwind_scheme.hpp:37-53, f = 1) restricted to the
-// band: a cell takes q when q < d and q <= limit.  A sweep after one that
-// changed nothing marks the loop done; later sweeps return at once, so a
-// batch of sweeps can be launched ahead of the convergence test.  Every
-// active sweep writes every cell of the active tiles (the others hold their
-// initial value in both buffers), so once converged both buffers agree.
-// Sweep k reads the job's buffer d[k & 1] and writes d[(k + 1) & 1].  Each
-// job has its own control words, so one job's sweeps return at once when it
-// has converged while the other's go on.  Launched on (kEikSweepGroups, 1,
-// jobs) workgroups of kEikTileW * kEikTileH threads that stride over the
-// job's active tiles, one tile per workgroup at a time.
-__global__ void __launch_bounds__(kEikTileW * kEikTileH) eik_sweep_kernel(
-    EikJobs jobs, Grid g, int64_t segs, double dh, double limit, int k) {
+// Sweeps kEikSteps launch .. kEikSteps (launch + 1) - 1 of the Godunov
+// eikonal update (scheme/schemes/godunov_upwind_scheme.hpp:37-53, f = 1)
+// restricted to the band: a cell takes q when q < d and q <= limit.
+//
+// A sweep is a chain of a few hundred cycles on a band of cells, so as a
+// launch of its own it was all launch: 23 sweeps of a 384x192 grid took 82 of
+// a step's 240 us.  Here a workgroup loads a tile and kEikSteps cells around
+// it, and sweeps them kEikSteps times in LDS; what the missing neighbours of
+// the outermost cells spoil moves inwards by one cell a sweep and stops short
+// of the tile, so its cells are those of whole sweeps.  A launch reads the
+// job's buffer d[launch & 1] and writes the active tiles of d[(launch + 1) &
+// 1] (the other tiles hold their initial values in both).
+//
+// flags[launch % 3][s]: sweep s of the launch changed a cell.  After a sweep
+// that changed nothing no other can, so a launch whose predecessor's last
+// sweep changed nothing marks the job done, and later ones return at once: a
+// batch of them can be launched ahead of the convergence test.  Launched on
+// (kEikSweepGroups, 1, jobs) workgroups that stride over the job's active
+// tiles.
+template <int ND>
+__global__ void __launch_bounds__(kEikThreads) eik_sweep_kernel(EikJobs jobs, Grid g,
+                                                                int64_t segs, double dh,
+                                                                double limit, int launch) {
+  using Tile = EikTile<ND>;
+  constexpr int K = kEikSteps, P = Tile::P;
   const EikJob J = eik_job(jobs);
-  const double* __restrict__ d = (k & 1) ? J.d[1] : J.d[0];
-  double* __restrict__ e = (k & 1) ? J.d[0] : J.d[1];
+  const double* __restrict__ d = (launch & 1) ? J.d[1] : J.d[0];
+  double* __restrict__ e = (launch & 1) ? J.d[0] : J.d[1];
   const uint8_t* __restrict__ info = J.info;
   const int* __restrict__ list = J.list;
-  EikCtl* __restrict__ ctl = J.ctl;
+  EikCtl* const ctl = J.ctl;
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-  // the control words, loaded together ((k + 2) % 3 is sweep k-1's flag)
-  const int done = ctl->done, prev_changed = ctl->flags[(k + 2) % 3];
+  // the control words, loaded together ((launch + 2) % 3: the launch before)
+  const int done = ctl->done, prev_changed = ctl->flags[(launch + 2) % 3][K - 1];
   const int ntiles = ctl->ntiles;
   keep(done);
   keep(prev_changed);
   keep(ntiles);
   if (done) return;
-  if (k > 0 && prev_changed == 0) {
+  if (launch > 0 && prev_changed == 0) {
     if (first) ctl->done = 1;
     return;
   }
   if (first) {
-    ctl->flags[(k + 1) % 3] = 0;
-    ctl->iters = k + 1;
+    for (int s = 0; s < K; ++s) ctl->flags[(launch + 1) % 3][s] = 0;
+    ctl->launches = launch + 1;
   }
-  bool changed = false;
+  __shared__ double sd[2][Tile::R];
+  __shared__ uint8_t si[Tile::R];
+  __shared__ unsigned s_changed;
+  if (threadIdx.x == 0) s_changed = 0u;
+  unsigned changed = 0u;  // bit s: sweep s changed a cell of a tile
+  const double fh = 1.0 * dh;
   for (int li = blockIdx.x; li < ntiles; li += gridDim.x) {
     const int64_t t = list[li];
-    const int64_t x = (t % segs) * kEikTileW + (threadIdx.x % kEikTileW);
-    const int64_t y = (t / segs) * kEikTileH + (threadIdx.x / kEikTileW);
-    if (x >= g.nx || y >= g.ny) continue;
-    const int64_t i = y * g.nx + x;
-    const double cur = d[i];
-    double nv = cur;
-    const uint8_t me = info[i];
-    // neighbours loaded together, before the branch (those past the edge
-    // read the cell itself and are replaced by DBL_MAX)
-    const bool okxm = x > 0, okxp = x < g.nx - 1;
-    const bool okym = g.nd > 1 && y > 0, okyp = g.nd > 1 && y < g.ny - 1;
-    const int64_t jxm = okxm ? i - 1 : i, jxp = okxp ? i + 1 : i;
-    const int64_t jym = okym ? i - g.nx : i, jyp = okyp ? i + g.nx : i;
-    const double dxm = d[jxm], dxp = d[jxp], dym = d[jym], dyp = d[jyp];
-    const uint8_t ixm = info[jxm], ixp = info[jxp], iym = info[jym], iyp = info[jyp];
-    keep(dxm);
-    keep(dxp);
-    keep(dym);
-    keep(dyp);
-    keep((int)(ixm | (ixp << 8) | (iym << 16) | (iyp << 24)));
-    if (!(me & 1)) {
-      const uint8_t sc = me & 6;
-      const double fh = 1.0 * dh;
-      const double xm = okxm ? eik_nbr_v(dxm, ixm, sc) : DBL_MAX;
-      const double xp = okxp ? eik_nbr_v(dxp, ixp, sc) : DBL_MAX;
-      const double a = smin(xm, xp);
-      double q;
-      if (g.nd == 1) {
-        q = a + fh;
-      } else {
-        const double ym = okym ? eik_nbr_v(dym, iym, sc) : DBL_MAX;
-        const double yp = okyp ? eik_nbr_v(dyp, iyp, sc) : DBL_MAX;
-        const double b = smin(ym, yp);
-        const double amb = a - b;
-        q = fabs(amb) >= fh ? smin(a, b) + fh
-                            : 0.5 * (a + b + sqrt(2.0 * fh * fh - (amb * amb)));
-      }
-      if (q < cur && q <= limit) {
-        nv = q;
-        changed = true;
+    const int64_t tx = (t % segs) * Tile::W - K;
+    const int64_t ty = ND == 1 ? 0 : (t / segs) * Tile::H - K;
+    double cur[P];
+    int64_t at[P];
+    bool in[P];
+#pragma unroll
+    for (int n = 0; n < P; ++n) {
+      const int c = (int)threadIdx.x + n * kEikThreads;
+      const int64_t x = tx + c % Tile::RW, y = ty + c / Tile::RW;
+      in[n] = c < Tile::R && x >= 0 && x < g.nx && y >= 0 && y < g.ny;
+      at[n] = in[n] ? y * g.nx + x : 0;
+      cur[n] = in[n] ? d[at[n]] : DBL_MAX;
+      const uint8_t me = in[n] ? info[at[n]] : 0;
+      if (c < Tile::R) {
+        sd[0][c] = cur[n];
+        si[c] = me;
       }
     }
-    e[i] = nv;
+    __syncthreads();
+    // per cell: whether it may change, whether it is the tile's, and which of
+    // its neighbours lie on its side (bits 0 to 3: x - 1, x + 1, y - 1, y + 1)
+    bool moves[P], own[P];
+    int same[P];
+#pragma unroll
+    for (int n = 0; n < P; ++n) {
+      const int c = (int)threadIdx.x + n * kEikThreads;
+      const int rx = c % Tile::RW, ry = c / Tile::RW;
+      const bool inner = rx > 0 && rx < Tile::RW - 1 &&
+                         (ND == 1 ? c < Tile::R : ry > 0 && ry < Tile::RH - 1);
+      own[n] = in[n] && rx >= K && rx < Tile::RW - K &&
+               (ND == 1 || (ry >= K && ry < Tile::RH - K));
+      moves[n] = false;
+      same[n] = 0;
+      if (in[n] && inner) {
+        const uint8_t me = si[c], sc = me & 6;
+        moves[n] = !(me & 1);
+        same[n] = ((si[c - 1] & 6) == sc ? 1 : 0) | ((si[c + 1] & 6) == sc ? 2 : 0);
+        if (ND > 1)
+          same[n] |= ((si[c - Tile::RW] & 6) == sc ? 4 : 0) |
+                     ((si[c + Tile::RW] & 6) == sc ? 8 : 0);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < K; ++s) {
+      const double* from = sd[s & 1];
+      double* to = sd[(s + 1) & 1];
+#pragma unroll
+      for (int n = 0; n < P; ++n) {
+        const int c = (int)threadIdx.x + n * kEikThreads;
+        if (moves[n]) {
+          const double a = smin(eik_nbr_v(from[c - 1], same[n] & 1),
+                                eik_nbr_v(from[c + 1], same[n] & 2));
+          double q;
+          if (ND == 1) {
+            q = a + fh;
+          } else {
+            const double b = smin(eik_nbr_v(from[c - Tile::RW], same[n] & 4),
+                                  eik_nbr_v(from[c + Tile::RW], same[n] & 8));
+            const double amb = a - b;
+            q = fabs(amb) >= fh ? smin(a, b) + fh
+                                : 0.5 * (a + b + sqrt(2.0 * fh * fh - (amb * amb)));
+          }
+          if (q < cur[n] && q <= limit) {
+            cur[n] = q;
+            if (own[n]) changed |= 1u << s;
+          }
+        }
+        if (c < Tile::R) to[c] = cur[n];
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int n = 0; n < P; ++n)
+      if (own[n]) e[at[n]] = cur[n];
   }
-  // one store of the change flag per wave
-  const unsigned long long m = __ballot(changed);
-  if (m && (int)(threadIdx.x % 64) == __ffsll((long long)m) - 1) ctl->flags[k % 3] = 1;
+  __syncthreads();
+  if (changed) atomicOr(&s_changed, changed);
+  __syncthreads();
+  if (threadIdx.x < K && (s_changed >> threadIdx.x & 1u)) ctl->flags[launch % 3][threadIdx.x] = 1;
 }
 
-// d = the converged buffer d[iters & 1] of the job; both hold the same
-// values once the loop has converged.
+// d = the buffer that the job's last launch wrote.
 __global__ void eik_finish_kernel(EikJobs jobs, Grid g, double limit, double clamp) {
   const int64_t i = gid();
   if (i >= g.nx * g.ny) return;
   const EikJob J = eik_job(jobs);
   const double* __restrict__ phi = J.phi;
-  const double* __restrict__ d = (J.ctl->iters & 1) ? J.d[1] : J.d[0];
+  const double* __restrict__ d = (J.ctl->launches & 1) ? J.d[1] : J.d[0];
   double* __restrict__ out = J.out;
   uint8_t* __restrict__ band_mask = J.band_mask;
   const int in_band = d[i] <= limit;
@@ -1272,6 +1306,11 @@ __global__ void combine_kernel(const double* __restrict__ phi0, StateView u0, St
                                                       const double*, double);                  \
   template __global__ void rk3_stage2_kernel<ND, FAST>(int, Rk3Job, Rk3Job, Grid, int,         \
                                                        const double*, double);
+#define FL_EIK_INST(ND)                                                                       \
+  template __global__ void eik_init_kernel<ND>(EikJobs, Grid, int64_t);                       \
+  template __global__ void eik_sweep_kernel<ND>(EikJobs, Grid, int64_t, double, double, int);
+FL_EIK_INST(1)
+FL_EIK_INST(2)
 #define FL_LS_INST(ND)                                                                       \
   template __global__ void velocity_kernel<ND>(const double*, const double*, StateView,      \
                                                StateView, int, Grid, double, int, double*); \

@@ -14,7 +14,7 @@ namespace ls = fl::ls;
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kEikBatch = 8;  // eikonal sweeps launched per convergence test
+constexpr int kEikBatch = 3;  // eikonal launches per convergence test
 
 dim3 grid_for(int64_t cells) { return dim3((unsigned)((cells + kBlock - 1) / kBlock)); }
 
@@ -190,8 +190,12 @@ int launch_project(double* phi0, double* phi1, int64_t cells, hipStream_t st) {
   return FL_OK;
 }
 
-int64_t eik_segs(const ls::Grid& g) { return (g.nx + ls::kEikTileW - 1) / ls::kEikTileW; }
-int64_t eik_trows(const ls::Grid& g) { return (g.ny + ls::kEikTileH - 1) / ls::kEikTileH; }
+int64_t eik_segs(const ls::Grid& g) {
+  return (g.nx + ls::eik_tile_w(g.nd) - 1) / ls::eik_tile_w(g.nd);
+}
+int64_t eik_trows(const ls::Grid& g) {
+  return (g.ny + ls::eik_tile_h(g.nd) - 1) / ls::eik_tile_h(g.nd);
+}
 
 // Two distance buffers, the per-cell info bytes, the per-tile source flags
 // and the active-tile list.
@@ -223,28 +227,30 @@ ls::EikJob eik_job(const double* phi, const ls::Grid& g, double* out, uint8_t* b
 
 // Eikonal reinitialisation of njobs (1 or 2) level sets on one grid, every
 // launch covering all jobs; iterations (nullable) receives each job's sweep
-// count.  The host tests convergence after every kEikBatch sweeps.
+// count.  The host tests convergence after every kEikBatch launches.
 int run_reinit(fl_context* c, const ls::EikJobs& jobs, int njobs, const ls::Grid& g, double dh,
                int band, int64_t* iterations, hipStream_t st) {
   const int64_t cells = g.nx * g.ny;
   const int64_t segs = eik_segs(g), trows = eik_trows(g), tiles = segs * trows;
   const double limit = band * dh;
   const double clamp = (band + 1) * dh;
+  constexpr int K = ls::kEikSteps;
   dim3 grid = grid_for(cells);
   grid.z = njobs;
   const dim3 tgrid((unsigned)segs, (unsigned)(trows < 65535 ? trows : 65535), njobs);
-  const dim3 tblock(ls::kEikTileW * ls::kEikTileH);
+  const dim3 block(ls::kEikThreads);
   const dim3 sgrid((unsigned)(tiles < ls::kEikSweepGroups ? tiles : ls::kEikSweepGroups), 1,
                    njobs);
   dim3 agrid = grid_for(tiles);
   agrid.z = njobs;
   // cells within which a source can pull a cell into the band, in tiles
   const int reach = (int)ceil(band * sqrt(2.0)) + 2;
-  const int segs_r = (reach + ls::kEikTileW - 1) / ls::kEikTileW;
-  const int tr_r = g.nd > 1 ? (reach + ls::kEikTileH - 1) / ls::kEikTileH : 0;
-  hipLaunchKernelGGL(ls::eik_init_kernel, grid, dim3(kBlock), 0, st, jobs, g);
-  hipLaunchKernelGGL(ls::eik_tile_src_kernel, tgrid, tblock, 0, st, jobs, g, trows);
-  hipLaunchKernelGGL(ls::eik_ctl_init_kernel, dim3(1), dim3(64), 0, st, jobs, njobs);
+  const int tw = ls::eik_tile_w(g.nd), th = ls::eik_tile_h(g.nd);
+  const int segs_r = (reach + tw - 1) / tw;
+  const int tr_r = g.nd > 1 ? (reach + th - 1) / th : 0;
+  auto init = g.nd == 1 ? ls::eik_init_kernel<1> : ls::eik_init_kernel<2>;
+  auto sweep = g.nd == 1 ? ls::eik_sweep_kernel<1> : ls::eik_sweep_kernel<2>;
+  hipLaunchKernelGGL(init, tgrid, block, 0, st, jobs, g, trows);
   hipLaunchKernelGGL(ls::eik_tile_act_kernel, agrid, dim3(kBlock), 0, st, jobs, trows, segs,
                      tr_r, segs_r);
   FL_HIP(hipGetLastError());
@@ -253,16 +259,15 @@ int run_reinit(fl_context* c, const ls::EikJobs& jobs, int njobs, const ls::Grid
   // reports convergence.
   // The first batch is as long as the context's previous solve took (a
   // level set reinitialised every few steps needs about the same number of
-  // sweeps each time), so that one test usually suffices; sweeps past
-  // convergence return at once.
-  const int64_t max_sweeps = cells + 2;
+  // sweeps each time) and one launch more, so that one test usually suffices;
+  // launches past convergence return at once.
+  const int64_t max_launches = cells / K + 2;
   int64_t launched = 0;
-  int64_t batch = c->eik_sweeps > kEikBatch ? c->eik_sweeps + 1 : kEikBatch;
-  if (batch > max_sweeps) batch = max_sweeps;
+  int64_t batch = std::min(std::max<int64_t>(kEikBatch, c->eik_sweeps / K + 2), max_launches);
+  int64_t sweeps[2] = {0, 0};
   for (;;) {
     for (int64_t b = 0; b < batch; ++b, ++launched)
-      hipLaunchKernelGGL(ls::eik_sweep_kernel, sgrid, tblock, 0, st, jobs, g, segs, dh, limit,
-                         (int)launched);
+      hipLaunchKernelGGL(sweep, sgrid, block, 0, st, jobs, g, segs, dh, limit, (int)launched);
     batch = kEikBatch;
     FL_HIP(hipGetLastError());
     FL_HIP(hipMemcpyAsync(c->host_eik, c->eik, njobs * sizeof(ls::EikCtl),
@@ -270,22 +275,23 @@ int run_reinit(fl_context* c, const ls::EikJobs& jobs, int njobs, const ls::Grid
     FL_HIP(hipStreamSynchronize(st));
     bool converged = true;
     for (int j = 0; j < njobs; ++j) {
+      // the sweeps that changed a cell and the one that did not
       const ls::EikCtl& h = c->host_eik[j];
-      converged = converged && (h.done || h.flags[(h.iters - 1) % 3] == 0);
+      const int* f = h.flags[(h.launches - 1) % 3];
+      converged = converged && f[K - 1] == 0;
+      sweeps[j] = (int64_t)(h.launches - 1) * K + 1;
+      for (int k = 0; k < K; ++k) sweeps[j] += f[k] != 0;
     }
     if (converged) break;
-    if (launched >= max_sweeps)
+    if (launched >= max_launches)
       return fail(FL_ERR_NUMERIC, "eikonal solve did not converge in %lld sweeps",
-                  (long long)launched);
+                  (long long)(launched * K));
   }
-  int64_t took = 0;
-  for (int j = 0; j < njobs; ++j)
-    took = c->host_eik[j].iters > took ? c->host_eik[j].iters : took;
-  c->eik_sweeps = took;
+  c->eik_sweeps = std::max(sweeps[0], sweeps[1]);
   hipLaunchKernelGGL(ls::eik_finish_kernel, grid, dim3(kBlock), 0, st, jobs, g, limit, clamp);
   FL_HIP(hipGetLastError());
   if (iterations)
-    for (int j = 0; j < njobs; ++j) iterations[j] = c->host_eik[j].iters;
+    for (int j = 0; j < njobs; ++j) iterations[j] = sweeps[j];
   return FL_OK;
 }
 
