@@ -341,9 +341,6 @@ void launch_flux_t(int flux, int ndim, int dim, dim3 grid, const SweepShape& sh,
   }
 }
 
-// Slots of the maximum wavespeed in a SimCtl for ndim dimensions.
-inline int sim_slots(int ndim) { return ndim == 1 ? 3 : 2; }
-
 // begin (nullable): the sweep begins step k of a simulation.
 struct SimBegin {
   fl::SimCtl* sim;
@@ -394,18 +391,25 @@ int launch_sweep(const fl_context* ctx, const fl_field* in, const fl_field* out,
 int launch_sim_step(const fl_context* ctx, const fl_field* state, const fl_field* work,
                     const fl_scheme* s, const fl_sim_params* p, fl::SimCtl* sim, int64_t k,
                     hipStream_t stream) {
+  if (state->ndim == 1)
+    return (k & 1) ? launch_sim_step(ctx, work, nullptr, state, s, p, sim, k, stream)
+                   : launch_sim_step(ctx, state, nullptr, work, s, p, sim, k, stream);
+  return launch_sim_step(ctx, state, work, state, s, p, sim, k, stream);
+}
+
+int launch_sim_step(const fl_context* ctx, const fl_field* in, const fl_field* mid,
+                    const fl_field* out, const fl_scheme* s, const fl_sim_params* p,
+                    fl::SimCtl* sim, int64_t k, hipStream_t stream) {
   const SimBegin begin = {sim, p, k};
-  unsigned long long* next = &sim->ws[(k + 1) % sim_slots(state->ndim)];
-  const bool one = state->ndim == 1;
-  const fl_field* src = one && (k & 1) ? work : state;
-  const fl_field* dst = one && (k & 1) ? state : work;
-  const int rc = state->dtype == FL_F64
-                     ? launch_sweep_t<double>(ctx, src, dst, 0, s, 1.0, nullptr,
+  const bool one = in->ndim == 1;
+  unsigned long long* next = &sim->ws[(k + 1) % sim_slots(in->ndim)];
+  const int rc = in->dtype == FL_F64
+                     ? launch_sweep_t<double>(ctx, in, one ? out : mid, 0, s, 1.0, nullptr,
                                               one ? next : nullptr, &begin, stream)
-                     : launch_sweep_t<float>(ctx, src, dst, 0, s, 1.0, nullptr,
+                     : launch_sweep_t<float>(ctx, in, one ? out : mid, 0, s, 1.0, nullptr,
                                              one ? next : nullptr, &begin, stream);
   if (rc || one) return rc;
-  return launch_sweep(ctx, work, state, 1, s, 1.0, &sim->c, next, stream);
+  return launch_sweep(ctx, mid, out, 1, s, 1.0, &sim->c, next, stream);
 }
 
 // Both materials' sweeps of dimension `dim` in one launch: in[m] -> out[m]
@@ -886,8 +890,12 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
       float total = 0.0f;
       c->shape[dim] = kShapeCell;
       rc = timed(dim, &total);
-      // the best of many marching shapes is a lucky one when they are about equal
-      if (!rc && total >= 1.05f * best_ms) c->shape[dim] = kShapeTuning;
+      // the best of many marching shapes is a lucky one when they are about
+      // equal, the more so where a sweep takes 20 us (512^2: 22 against 17 us
+      // in the steps after it)
+      const bool by_rule = in->n[0] * in->n[1] <=
+                           (in->dtype == FL_F64 ? kCellMax<double> : kCellMax<float>);
+      if (!rc && total >= (by_rule ? 1.25f : 1.05f) * best_ms) c->shape[dim] = kShapeTuning;
     }
   }
   (void)hipEventDestroy(e0);

@@ -127,11 +127,18 @@ int64_t cell_count(const fl_field* f);
 int launch_sweep(const fl_context* ctx, const fl_field* in, const fl_field* out, int dim,
                  const fl_scheme* s, double dtdh, const fl::StepCtl* ctl,
                  unsigned long long* ws_out, hipStream_t stream);
+// Slots of SimCtl::ws that the steps of a grid use in turn.
+inline int sim_slots(int ndim) { return ndim == 1 ? 3 : 2; }
 // Step k of a simulation on state -> work (-> state in 2D): the sweeps, the
 // first of which takes dt from the maximum in sim.
 int launch_sim_step(const fl_context* ctx, const fl_field* state, const fl_field* work,
                     const fl_scheme* s, const fl_sim_params* p, fl::SimCtl* sim, int64_t k,
                     hipStream_t stream);
+// The same from in to out, on 2D grids through mid (in 1D unused).  Until the
+// next step's first sweep the step's maximum stays in ws[k % sim_slots].
+int launch_sim_step(const fl_context* ctx, const fl_field* in, const fl_field* mid,
+                    const fl_field* out, const fl_scheme* s, const fl_sim_params* p,
+                    fl::SimCtl* sim, int64_t k, hipStream_t stream);
 // Both materials' sweeps of dimension `dim` in one launch; ctl (nullable)
 // as in launch_sweep.
 int launch_sweep2(const fl_context* ctx, const fl_field* const in[2], const fl_field* const out[2],

@@ -6,6 +6,8 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
+
 #include "fl_abi_internal.hpp"
 #include "fl_adjoint_kernels.hpp"
 
@@ -55,11 +57,10 @@ fl::Material<double> mat64(const fl_scheme* s) {
 int64_t cells_of(const fl_field* f) { return f->n[0] * (f->ndim > 1 ? f->n[1] : 1); }
 int64_t grid_bytes(const fl_field* f) { return cells_of(f) * (2 + f->ndim) * 8; }
 
-int64_t max_faces(const fl_field* f) {
+// Workgroups of the adjoint of the sweep along dimension d.
+int64_t sweep_blocks(const fl_field* f, int d) {
   const int64_t nx = f->n[0], ny = f->ndim > 1 ? f->n[1] : 1;
-  const int64_t fx = (nx + 1) * ny;
-  const int64_t fy = f->ndim > 1 ? nx * (ny + 1) : 0;
-  return fx > fy ? fx : fy;
+  return ceil_div(d ? ny : nx, aj::kAdjCells) * ceil_div(d ? nx : ny, aj::kAdjWaves);
 }
 
 // Scratch of the backward pass for segments of K steps.
@@ -67,20 +68,19 @@ struct AdjLayout {
   double* U;         // K+1 grids: states of the segment
   double* X;         // K grids: x-sweep outputs (2D)
   double* lam[3];    // adjoint ping-pong + adjoint after the y sweep
-  double* contrib;   // faces * 4 * S
-  double* face_g;    // faces * 2
+  double* sums[2];   // per sweep: 2 per workgroup
   double* P;         // (nx+8)(ny+8): pressure within 4 ghost cells
   double* V0;        // same: x velocity
   double* V1;        // same: y velocity
   double* chi;       // (nx+2)(ny+2): flattening factor within 1 ghost cell
-  double* chi_g;     // faces * 2: chi adjoints of each face's two cells
+  double* chi_g;     // (nx+2)(ny+2): its adjoint
   int* rec_k;        // (nx+2)(ny+2): the factor each chi minimum selected
   double* rec_v;     // (nx+2)(ny+2) * 4: its pressure adjoints
   int* any;          // 1: some chi position has a record
-  double* partials;  // 4 slots * 2 * kPartialBlocks: x, y faces; x, y chi
+  double* partials;  // 2 slots * 2 * kPartialBlocks: x, y chi
   aj::StepRec* rec;  // K
   double* acc;       // 2
-  fl::StepCtl* ctl;  // 1
+  fl::SimCtl* sim;   // 1
   int64_t bytes;
 };
 
@@ -93,14 +93,11 @@ AdjLayout adj_layout(void* base, const fl_field* f, int K) {
     return r;
   };
   const int64_t gb = grid_bytes(f);
-  const int S = 2 + f->ndim;
-  const int64_t nf = max_faces(f);
   AdjLayout L;
   L.U = (double*)take(gb * (K + 1));
   L.X = (double*)take(f->ndim > 1 ? gb * K : 8);
   for (int i = 0; i < 3; ++i) L.lam[i] = (double*)take(gb);
-  L.contrib = (double*)take(nf * 4 * S * 8);
-  L.face_g = (double*)take(nf * 2 * 8);
+  for (int d = 0; d < f->ndim; ++d) L.sums[d] = (double*)take(sweep_blocks(f, d) * 2 * 8);
   const int64_t nx = f->n[0], ny = f->ndim > 1 ? f->n[1] : 1;
   const int64_t padded = (nx + 8) * (f->ndim > 1 ? ny + 8 : 1);
   L.P = (double*)take(padded * 8);
@@ -108,14 +105,14 @@ AdjLayout adj_layout(void* base, const fl_field* f, int K) {
   L.V1 = (double*)take(padded * 8);
   const int64_t cpad = (nx + 2) * (f->ndim > 1 ? ny + 2 : 1);
   L.chi = (double*)take(cpad * 8);
-  L.chi_g = (double*)take(nf * 2 * 8);
+  L.chi_g = (double*)take(cpad * 8);
   L.rec_k = (int*)take(cpad * 4);
   L.rec_v = (double*)take(cpad * 4 * 8);
   L.any = (int*)take(4);
-  L.partials = (double*)take(4 * 2 * aj::kPartialBlocks * 8);
+  L.partials = (double*)take(2 * 2 * aj::kPartialBlocks * 8);
   L.rec = (aj::StepRec*)take(sizeof(aj::StepRec) * K);
   L.acc = (double*)take(2 * 8);
-  L.ctl = (fl::StepCtl*)take(sizeof(fl::StepCtl));
+  L.sim = (fl::SimCtl*)take(sizeof(fl::SimCtl));
   L.bytes = off;
   return L;
 }
@@ -143,61 +140,45 @@ aj::AGrid agrid(const fl_field* f, const double* data, const fl_scheme* s) {
 // only the final state is kept (in U[(b-a) & 1]).
 int forward_steps(const fl_context* c, const fl_field* f, const fl_scheme* s, double cfl,
                   double dh, int64_t nsteps, double* Ubase, double* Xbase, aj::StepRec* rec,
-                  fl::StepCtl* ctl, bool keep_all, hipStream_t st) {
+                  fl::SimCtl* sim, bool keep_all, hipStream_t st) {
   const int64_t cells = cells_of(f);
   const int S = 2 + f->ndim;
   const fl::Material<double> m = mat64(s);
-  hipLaunchKernelGGL(fl::init_control_kernel, dim3(1), dim3(1), 0, st, ctl);
+  const fl_sim_params params = {cfl, dh, (double)INFINITY, (int64_t)1 << 62};
+  hipLaunchKernelGGL(fl::init_sim_kernel, dim3(1), dim3(1), 0, st, sim);
+  if (rec)
+    hipLaunchKernelGGL(aj::rec_clear_kernel, dim3((unsigned)ceil_div(nsteps, 256)), dim3(256), 0,
+                       st, rec, nsteps);
   fl_field u0 = with_data(f, Ubase);
-  int rc = launch_max_ws(&u0, s, &ctl->ws_bits[0], st);
+  int rc = launch_max_ws(&u0, s, &sim->ws[0], st);
   if (rc) return rc;
   for (int64_t k = 0; k < nsteps; ++k) {
-    const int parity = (int)(k & 1);
     double* Uk = keep_all ? Ubase + k * cells * S : Ubase + (k & 1) * cells * S;
     double* Un = keep_all ? Ubase + (k + 1) * cells * S : Ubase + ((k + 1) & 1) * cells * S;
-    hipLaunchKernelGGL(fl::step_control_kernel, dim3(1), dim3(1), 0, st, ctl, parity, cfl, dh,
-                       (double)INFINITY, (long long)1 << 62);
-    if (rec) {
-      hipLaunchKernelGGL(aj::record_kernel, dim3(1), dim3(1), 0, st, (const fl::StepCtl*)ctl,
-                         parity, rec + k);
-      const aj::AGrid g = agrid(f, Uk, s);
-      int64_t blocks = ceil_div(cells, 256);
-      if (blocks > 2048) blocks = 2048;
-      if (f->ndim == 1)
-        hipLaunchKernelGGL(aj::argmax_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, st, g, m,
-                           rec + k);
-      else
-        hipLaunchKernelGGL(aj::argmax_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, st, g, m,
-                           rec + k);
-    }
     const fl_field fin = with_data(f, Uk);
     const fl_field fout = with_data(f, Un);
-    unsigned long long* ws_next = &ctl->ws_bits[parity ^ 1];
-    if (f->ndim == 1) {
-      rc = launch_sweep(c, &fin, &fout, 0, s, 1.0, ctl, ws_next, st);
-    } else {
-      double* Xk = keep_all ? Xbase + k * cells * S : Xbase;
-      const fl_field fx = with_data(f, Xk);
-      rc = launch_sweep(c, &fin, &fx, 0, s, 1.0, ctl, nullptr, st);
-      if (!rc) rc = launch_sweep(c, &fx, &fout, 1, s, 1.0, ctl, ws_next, st);
+    const fl_field fx = with_data(f, keep_all && f->ndim > 1 ? Xbase + k * cells * S : Xbase);
+    if ((rc = launch_sim_step(c, &fin, &fx, &fout, s, &params, sim, k, st))) return rc;
+    if (rec) {
+      const aj::AGrid g = agrid(f, Uk, s);
+      const int64_t blocks = std::min<int64_t>(ceil_div(cells, 256), 2048);
+      auto record = f->ndim == 1 ? aj::record_kernel<1> : aj::record_kernel<2>;
+      hipLaunchKernelGGL(record, dim3((unsigned)blocks), dim3(256), 0, st, g, m,
+                         (const fl::SimCtl*)sim, (int)(k % sim_slots(f->ndim)), rec + k);
     }
-    if (rc) return rc;
   }
   FL_HIP(hipGetLastError());
   return FL_OK;
 }
 
-// Adjoint of one sweep: lam_out -> lam_in; the faces' (dt/dh, gamma) sums
-// into `partials`, the flattening factor's gamma sums into `chi_partials`.
+// Adjoint of one sweep: lam_out -> lam_in; its (dt/dh, gamma) sums into
+// L.sums[D], the flattening factor's gamma sums into `chi_partials`.
 template <int ND, int D>
 void sweep_adj(const fl_field* f, const fl_scheme* s, const double* Uin, const double* lam_out,
-               double* lam_in, const aj::StepRec* rec, const AdjLayout& L, double* partials,
-               double* chi_partials, hipStream_t st) {
+               double* lam_in, const aj::StepRec* rec, const AdjLayout& L, double* chi_partials,
+               hipStream_t st) {
   const aj::AGrid g = agrid(f, Uin, s);
   const fl::Material<double> m = mat64(s);
-  const int64_t n = D == 0 ? g.nx : g.ny;
-  const int64_t lines = D == 0 ? g.ny : g.nx;
-  const int64_t nf = (n + 1) * lines;
   const int64_t padded = (g.nx + 8) * (ND > 1 ? g.ny + 8 : 1);
   const int64_t cpad = (g.nx + 2) * (ND > 1 ? g.ny + 2 : 1);
   hipLaunchKernelGGL(aj::prim_pad_kernel<ND>, dim3((unsigned)ceil_div(padded, 256)), dim3(256), 0,
@@ -206,17 +187,13 @@ void sweep_adj(const fl_field* f, const fl_scheme* s, const double* Uin, const d
                      st, g, (const double*)L.P, (const double*)L.V0, (const double*)L.V1, L.chi,
                      L.any);
   const bool force = s->flux == FL_FLUX_FORCE, prim = s->form == FL_FORM_PRIMITIVE;
-  auto face = force ? (prim ? aj::face_adj_kernel<ND, D, fl::kFluxForce, true>
-                            : aj::face_adj_kernel<ND, D, fl::kFluxForce, false>)
-                    : (prim ? aj::face_adj_kernel<ND, D, fl::kFluxHllc, true>
-                            : aj::face_adj_kernel<ND, D, fl::kFluxHllc, false>);
-  hipLaunchKernelGGL(face, dim3((unsigned)ceil_div(nf, 256)), dim3(256), 0, st, g, lam_out, m,
-                     s->limiter, rec, (const double*)L.chi, L.contrib, L.face_g, L.chi_g);
-  hipLaunchKernelGGL(aj::partial_sum_kernel, dim3(aj::kPartialBlocks), dim3(256), 0, st,
-                     (const double*)L.face_g, nf, partials);
-  const int64_t cells = g.nx * g.ny;
-  hipLaunchKernelGGL((aj::gather_adj_kernel<ND, D>), dim3((unsigned)ceil_div(cells, 256)),
-                     dim3(256), 0, st, g, lam_out, lam_in, (const double*)L.contrib);
+  auto sweep = force ? (prim ? aj::sweep_adj_kernel<ND, D, fl::kFluxForce, true>
+                             : aj::sweep_adj_kernel<ND, D, fl::kFluxForce, false>)
+                     : (prim ? aj::sweep_adj_kernel<ND, D, fl::kFluxHllc, true>
+                             : aj::sweep_adj_kernel<ND, D, fl::kFluxHllc, false>);
+  hipLaunchKernelGGL(sweep, dim3((unsigned)sweep_blocks(f, D)), dim3(64 * aj::kAdjWaves), 0, st, g,
+                     lam_out, lam_in, m, s->limiter, rec, (const double*)L.chi, L.chi_g,
+                     L.sums[D]);
   // the flattening factor: the selected factors' pressure adjoints where
   // 0 < chi < 1, then into lambda and the gamma sum
   hipLaunchKernelGGL((aj::chi_adj_kernel<ND, D>), dim3((unsigned)ceil_div(cpad, 256)), dim3(256),
@@ -235,19 +212,25 @@ int backward_step(const fl_field* f, const fl_scheme* s, const AdjLayout& L, int
   const double* Uk = L.U + k * cells * S;
   const aj::StepRec* rec = L.rec + k;
   const fl::Material<double> m = mat64(s);
-  // partial slots (2 * kPartialBlocks each): faces of the sweeps, then their
-  // flattening-factor terms
+  // the sums of the sweeps, then of their flattening-factor terms
   auto slot = [&](int i) { return L.partials + 2 * aj::kPartialBlocks * i; };
+  aj::Partials parts = {};
+  for (int d = 0; d < f->ndim; ++d) {
+    parts.p[d] = L.sums[d];
+    parts.n[d] = (int)sweep_blocks(f, d);
+    parts.p[2 + d] = slot(d);
+    parts.n[2 + d] = aj::kPartialBlocks;
+  }
   if (f->ndim == 1) {
-    sweep_adj<1, 0>(f, s, Uk, lam_next, lam_prev, rec, L, slot(0), slot(1), st);
+    sweep_adj<1, 0>(f, s, Uk, lam_next, lam_prev, rec, L, slot(0), st);
     hipLaunchKernelGGL(aj::finalize_kernel<1>, dim3(1), dim3(256), 0, st, agrid(f, Uk, s), m, rec,
-                       (const double*)L.partials, 2, lam_prev, L.acc);
+                       parts, lam_prev, L.acc);
   } else {
     const double* Xk = L.X + k * cells * S;
-    sweep_adj<2, 1>(f, s, Xk, lam_next, L.lam[2], rec, L, slot(1), slot(3), st);
-    sweep_adj<2, 0>(f, s, Uk, L.lam[2], lam_prev, rec, L, slot(0), slot(2), st);
+    sweep_adj<2, 1>(f, s, Xk, lam_next, L.lam[2], rec, L, slot(1), st);
+    sweep_adj<2, 0>(f, s, Uk, L.lam[2], lam_prev, rec, L, slot(0), st);
     hipLaunchKernelGGL(aj::finalize_kernel<2>, dim3(1), dim3(256), 0, st, agrid(f, Uk, s), m, rec,
-                       (const double*)L.partials, 4, lam_prev, L.acc);
+                       parts, lam_prev, L.acc);
   }
   FL_HIP(hipGetLastError());
   return FL_OK;
@@ -300,13 +283,13 @@ int fl_adj_forward(fl_context* c, fl_field* state, const fl_scheme* s, double cf
   for (int64_t a = 0; a < steps; a += K) {
     const int64_t ns = (steps - a) < K ? (steps - a) : K;
     FL_HIP(hipMemcpyAsync(L.U, ck + (a / K) * gb, gb, hipMemcpyDeviceToDevice, st));
-    if ((rc = forward_steps(c, state, s, cfl, dh, ns, L.U, L.X, nullptr, L.ctl, false, st)))
+    if ((rc = forward_steps(c, state, s, cfl, dh, ns, L.U, L.X, nullptr, L.sim, false, st)))
       return rc;
     const double* fin = L.U + (ns & 1) * cells_of(state) * (2 + state->ndim);
     if ((a + ns) % K == 0)
       FL_HIP(hipMemcpyAsync(ck + ((a + ns) / K) * gb, fin, gb, hipMemcpyDeviceToDevice, st));
     if (a + ns == steps) FL_HIP(hipMemcpyAsync(state->data, fin, gb, hipMemcpyDeviceToDevice, st));
-    FL_HIP(hipMemcpyAsync(c->host_ctl, L.ctl, sizeof(fl::StepCtl), hipMemcpyDeviceToHost, st));
+    FL_HIP(hipMemcpyAsync(c->host_ctl, &L.sim->c, sizeof(fl::StepCtl), hipMemcpyDeviceToHost, st));
     FL_HIP(hipStreamSynchronize(st));
     t += c->host_ctl->t;
     last_dt = c->host_ctl->dt;
@@ -346,7 +329,7 @@ int fl_adj_backward(fl_context* c, fl_field* grad, const fl_scheme* s, double cf
     const int64_t a = sg * K;
     const int64_t ns = (steps - a) < K ? (steps - a) : K;
     FL_HIP(hipMemcpyAsync(L.U, ck + sg * gb, gb, hipMemcpyDeviceToDevice, st));
-    if ((rc = forward_steps(c, grad, s, cfl, dh, ns, L.U, L.X, L.rec, L.ctl, true, st)))
+    if ((rc = forward_steps(c, grad, s, cfl, dh, ns, L.U, L.X, L.rec, L.sim, true, st)))
       return rc;
     for (int64_t k = ns - 1; k >= 0; --k) {
       if ((rc = backward_step(grad, s, L, k, L.lam[cur], L.lam[cur ^ 1], st))) return rc;
@@ -378,7 +361,7 @@ int fl_split_step_vjp(fl_context* c, const fl_field* state, const fl_field* lamb
   const int64_t gb = grid_bytes(state);
   hipLaunchKernelGGL(aj::acc_clear_kernel, dim3(1), dim3(1), 0, st, L.acc);
   FL_HIP(hipMemcpyAsync(L.U, state->data, gb, hipMemcpyDeviceToDevice, st));
-  if ((rc = forward_steps(c, state, s, cfl, dh, 1, L.U, L.X, L.rec, L.ctl, true, st))) return rc;
+  if ((rc = forward_steps(c, state, s, cfl, dh, 1, L.U, L.X, L.rec, L.sim, true, st))) return rc;
   FL_HIP(hipMemcpyAsync(L.lam[0], lambda_next->data, gb, hipMemcpyDeviceToDevice, st));
   if ((rc = backward_step(state, s, L, 0, L.lam[0], L.lam[1], st))) return rc;
   FL_HIP(hipMemcpyAsync(lambda->data, L.lam[1], gb, hipMemcpyDeviceToDevice, st));

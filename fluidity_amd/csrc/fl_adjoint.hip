@@ -6,21 +6,21 @@
 // i-1..i+1 (solver/split_solver.hpp:138-162,
 // reconstruction/muscl_reconstructor.hpp:99-172, flux_method/flux_hllc.hpp).
 // Adjoint of one sweep, given lambda = dLoss/d out:
-//  * face kernel, one thread per face i+1/2: recompute R_i, L_{i+1} and G,
-//    mu = dtdh (lambda_{i+1} - lambda_i) (ghost cells carry no lambda), and
-//    back-propagate mu through HLLC and both evolutions into the adjoints of
-//    the four stencil cells i-1..i+2 (stored per face and slot), of dt/dh and
-//    of gamma (stored per face);
-//  * gather kernel, one thread per cell: lambda_in = lambda + the slot
-//    contributions of every face whose stencil holds the cell, also through
-//    ghost cells (periodic wrap, mirror, reflective flip), in a fixed order;
-//  * the per-face dt/dh and gamma adjoints are summed in a fixed-order
-//    two-level reduction, so the whole adjoint is deterministic.
+//  * sweep kernel, one lane per cell i of a line: recompute R_i, L_i and with
+//    the next lane's L the flux G of face i+1/2, mu = dtdh (lambda_{i+1} -
+//    lambda_i) (ghost cells carry no lambda), back-propagate mu through HLLC
+//    to the face states, theirs of cell i (one of them from the lane before)
+//    through the evolution to the cells i-1..i+1, and add to lambda what the
+//    cells i-1..i+1 pass to cell i, also through ghost cells (mirror,
+//    reflective flip; a periodic line is followed around its ends);
+//  * the dt/dh and gamma adjoints are summed per workgroup, then over the
+//    workgroups, in a fixed order, so the whole adjoint is deterministic.
 // dt = cfl dh / max wavespeed couples the step to the state through the
 // wavespeed of the cell holding the maximum (lowest index among ties); the
 // step's finalize kernel adds that term.
 #include "fl_adjoint.hpp"
 #include "fl_adjoint_kernels.hpp"
+#include "fl_sweep_tiles.hpp"
 
 namespace fl {
 namespace adj {
@@ -104,164 +104,171 @@ __global__ void __launch_bounds__(256) chi_pad_kernel(AGrid g, const double* __r
   chi[q] = c;
 }
 
+// Adjoint of one sweep: a wave takes kAdjCells cells of a line along the sweep
+// and three on either side, one a lane, and neighbours exchange in registers.
 // PRIM: primitive-form limiting (a template parameter, so that the
 // conservative-form kernel carries none of its code).
+//
+// FP64 arithmetic and its latency at two waves a SIMD bound it (240 registers;
+// a 512^2 sweep at three a SIMD 25 us in x and 31 in y, at four, with spills, 38
+// and 44; workgroups of 8 waves 30 and 36, whose last round is a quarter full).
+// With a thread per face, which evolved both cells beside it forward and back
+// and passed its 16 contributions through memory to a kernel that gathered
+// them, it took 33 us, the gather 9 and the sums 5; now 24 us (x) and 29 (y) in
+// all.  In the y sweep a wave's lanes run down a column: its loads touch a
+// line each, which the columns of a workgroup share.
+//
+// chi_g receives the adjoint of every position's flattening factor (indexed as
+// chi_pad; on the lines of the grid), partials the workgroup's sums of the
+// dt/dh and gamma adjoints.
 template <int ND, int D, int FLUX, bool PRIM>
-__global__ void __launch_bounds__(256) face_adj_kernel(AGrid g, const double* __restrict__ lam,
-                                                       Material<double> m, int limiter,
-                                                       const StepRec* __restrict__ rec,
-                                                       const double* __restrict__ chi_pad,
-                                                       double* __restrict__ contrib,
-                                                       double* __restrict__ face_g,
-                                                       double* __restrict__ chi_g) {
+__global__ void __launch_bounds__(64 * kAdjWaves)
+sweep_adj_kernel(AGrid g, const double* __restrict__ lam, double* __restrict__ lam_in,
+                 Material<double> m, int limiter, const StepRec* __restrict__ rec,
+                 const double* __restrict__ chi_pad, double* __restrict__ chi_g,
+                 double* __restrict__ partials) {
   constexpr int S = 2 + ND;
   constexpr int form = PRIM ? kFormPrim : kFormCons;
   const int64_t n = D == 0 ? g.nx : g.ny;          // cells along the sweep
   const int64_t lines = D == 0 ? g.ny : g.nx;
-  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= (n + 1) * lines) return;
-  int64_t i, line;
-  if (D == 0) {
-    i = f % (n + 1) - 1;
-    line = f / (n + 1);
-  } else {
-    i = f / lines - 1;
-    line = f % lines;
-  }
-  auto pos = [&](int64_t k, int64_t& x, int64_t& y) {
-    if (D == 0) {
-      x = k;
-      y = line;
-    } else {
-      x = line;
-      y = k;
-    }
+  const int bc = D == 0 ? g.bcx : g.bcy;
+  const bool ring = bc == kBcPeriodic;
+  // blocks go to the 8 XCDs in turn; each takes neighbouring groups of lines
+  const int64_t total = gridDim.x, xcd = blockIdx.x % 8;
+  const int64_t tile = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
+  const int64_t groups = (lines + kAdjWaves - 1) / kAdjWaves;
+  const int64_t seg = tile / groups;
+  const int t = (int)(threadIdx.x & 63);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t line_of = (tile % groups) * kAdjWaves + w;
+  const bool live = line_of < lines;               // uniform over the wave
+  const int64_t line = live ? line_of : lines - 1;
+  const int64_t j = seg * kAdjCells - kAdjHalo + t;  // this lane's position
+  // the cell it names, and whether it is one of the grid
+  bool flip;
+  const int64_t jc = ghost_index(j, n, bc, flip);
+  const bool cell = ring || (j >= 0 && j < n);
+  const int64_t xi = D == 0 ? jc : line, yi = D == 0 ? line : jc;
+  const int64_t at = (yi * g.nx + xi) * g.es;
+  // flattening factors exist for positions -1 .. n
+  const int64_t jq = ring ? jc : (j < -1 ? -1 : (j > n ? n : j));
+  const int64_t cxw = g.nx + 2;
+  auto chi_at = [&](int64_t p) {
+    const int64_t x = D == 0 ? p : line, y = D == 0 ? line : p;
+    return (ND > 1 ? (y + 1) * cxw : 0) + x + 1;
   };
+  double u0[S], la[S];
+#pragma unroll
+  for (int k = 0; k < S; ++k) u0[k] = g.U[at + k * g.cs];
+#pragma unroll
+  for (int k = 0; k < S; ++k) la[k] = lam[at + k * g.cs];
+  const double chi = chi_pad[chi_at(jq)];
   const double dtdh = rec->dtdh;
   const double half_dtdh = 0.5 * dtdh;
-  double u[4][S];
-  for (int s = 0; s < 4; ++s) {
-    int64_t x, y;
-    pos(i - 1 + s, x, y);
-    load_state<ND>(g, x, y, u[s]);
+  if (flip) reflect<double, ND>(u0, D);
+#pragma unroll
+  for (int k = 0; k < S; ++k) la[k] = cell ? la[k] : 0.0;
+
+  // ---- forward: the face states of this cell, the flux of the face after it
+  double R[S], L[S], G[S];
+  {
+    double um[S], up[S], Lc[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      um[k] = below(u0[k]);
+      up[k] = above(u0[k]);
+    }
+    evolve_faces<double, ND, D>(um, u0, up, chi, half_dtdh, limiter, form, m, R, Lc);
+#pragma unroll
+    for (int k = 0; k < S; ++k) L[k] = above(Lc[k]);
   }
-  int64_t xa, ya, xb, yb;
-  pos(i, xa, ya);
-  pos(i + 1, xb, yb);
-  const int64_t cxw = g.nx + 2;
-  const double chi_a = chi_pad[(ND > 1 ? (ya + 1) * cxw : 0) + xa + 1];
-  const double chi_b = chi_pad[(ND > 1 ? (yb + 1) * cxw : 0) + xb + 1];
-  double R[S], L[S], tmp[S], G[S];
-  evolve_faces<double, ND, D>(u[0], u[1], u[2], chi_a, half_dtdh, limiter, form, m, R, tmp);
-  evolve_faces<double, ND, D>(u[1], u[2], u[3], chi_b, half_dtdh, limiter, form, m, tmp, L);
   if constexpr (FLUX == kFluxHllc) hllc_flux<double, ND, D>(R, L, m, G);
   else force_flux<double, ND, D>(R, L, dtdh, 1.0 / dtdh, m, G);
-  double la[S], lb[S];
+  // ---- the face's adjoint; faces lie after positions -1 .. n - 1
+  const bool face = ring || (j >= -1 && j < n);
+  double mu[S], g_dtdh = 0.0, gR[S], gL[S];
 #pragma unroll
   for (int k = 0; k < S; ++k) {
-    la[k] = 0.0;
-    lb[k] = 0.0;
-  }
-  if (i >= 0) {
-    const double* p = lam + (ya * g.nx + xa) * g.es;
-#pragma unroll
-    for (int k = 0; k < S; ++k) la[k] = p[k * g.cs];
-  }
-  if (i + 1 < n) {
-    const double* p = lam + (yb * g.nx + xb) * g.es;
-#pragma unroll
-    for (int k = 0; k < S; ++k) lb[k] = p[k * g.cs];
-  }
-  double mu[S], g_dtdh = 0.0;
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const double dl = lb[k] - la[k];
+    const double dl = above(la[k]) - la[k];
     mu[k] = dtdh * dl;
     g_dtdh += G[k] * dl;
-  }
-  GMat gm{0.0};
-  double gR[S], gL[S], zero[S];
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
     gR[k] = 0.0;
     gL[k] = 0.0;
-    zero[k] = 0.0;
   }
-  if constexpr (FLUX == kFluxHllc) hllc_adj<ND, D>(R, L, m, mu, gR, gL, gm);
-  else force_adj<ND, D>(R, L, dtdh, m, mu, gR, gL, g_dtdh, gm);
-  double c[4][S];
+  GMat gm_face{0.0};
+  if constexpr (FLUX == kFluxHllc) hllc_adj<ND, D>(R, L, m, mu, gR, gL, gm_face);
+  else force_adj<ND, D>(R, L, dtdh, m, mu, gR, gL, g_dtdh, gm_face);
+  // ---- the cell's adjoint, from the faces after and before it
+  const bool state = ring || (j >= -1 && j <= n);
+  GMat gm_cell{0.0};
+  double g_half = 0.0, g_chi = 0.0, acc[S];
+  {
+    double um[S], up[S], gum[S], gup[S];
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
-#pragma unroll
-    for (int k = 0; k < S; ++k) c[s][k] = 0.0;
-  double g_half = 0.0, g_chi_a = 0.0, g_chi_b = 0.0;
-  evolve_adj<ND, D>(u[0], u[1], u[2], chi_a, half_dtdh, limiter, form, m, gR, zero, c[0], c[1],
-                    c[2], g_half, g_chi_a, gm);
-  evolve_adj<ND, D>(u[1], u[2], u[3], chi_b, half_dtdh, limiter, form, m, zero, gL, c[1], c[2],
-                    c[3], g_half, g_chi_b, gm);
-  chi_g[2 * f] = g_chi_a;      // of cell i (its right face state)
-  chi_g[2 * f + 1] = g_chi_b;  // of cell i + 1 (its left face state)
-  // contributions as planes (slot, component) x faces: coalesced both here and
-  // in the gather
-  const int64_t nf = (n + 1) * lines;
-#pragma unroll
-  for (int s = 0; s < 4; ++s)
-#pragma unroll
-    for (int k = 0; k < S; ++k) contrib[(s * S + k) * nf + f] = c[s][k];
-  face_g[2 * f] = g_dtdh + 0.5 * g_half;
-  face_g[2 * f + 1] = gm.gamma;
-}
-
-// lambda_in = lambda_out + contributions of every face whose stencil holds
-// the cell (directly or as a ghost alias).
-template <int ND, int D>
-__global__ void __launch_bounds__(256) gather_adj_kernel(AGrid g, const double* __restrict__ lam_out,
-                                                         double* __restrict__ lam_in,
-                                                         const double* __restrict__ contrib) {
-  constexpr int S = 2 + ND;
-  const int64_t cell = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cell >= g.nx * g.ny) return;
-  const int64_t x = cell % g.nx, y = cell / g.nx;
-  const int64_t n = D == 0 ? g.nx : g.ny;
-  const int64_t lines = D == 0 ? g.ny : g.nx;
-  const int64_t j = D == 0 ? x : y;
-  const int64_t line = D == 0 ? y : x;
-  const int bc = D == 0 ? g.bcx : g.bcy;
-  double acc[S];
-  const double* lp = lam_out + cell * g.es;
-#pragma unroll
-  for (int k = 0; k < S; ++k) acc[k] = lp[k * g.cs];
-  // virtual positions holding this cell: itself, then ghost aliases
-  int64_t vs[3];
-  int flips[3];
-  int nv = 0;
-  vs[nv] = j;
-  flips[nv++] = 0;
-  if (bc == kBcPeriodic) {
-    if (j >= n - 2) { vs[nv] = j - n; flips[nv++] = 0; }
-    if (j <= 1) { vs[nv] = j + n; flips[nv++] = 0; }
-  } else {
-    const int fl = bc == kBcReflective ? 1 : 0;
-    if (j <= 1) { vs[nv] = -j - 1; flips[nv++] = fl; }
-    if (j >= n - 2) { vs[nv] = 2 * n - 1 - j; flips[nv++] = fl; }
-  }
-  for (int a = 0; a < nv; ++a) {
-    const int64_t v = vs[a];
-    for (int s = 0; s < 4; ++s) {
-      const int64_t i = v + 1 - s;
-      if (i < -1 || i > n - 1) continue;
-      const int64_t f = D == 0 ? line * (n + 1) + (i + 1) : (i + 1) * lines + line;
-      const int64_t nf = (n + 1) * lines;
-#pragma unroll
-      for (int k = 0; k < S; ++k) {
-        const double ck = contrib[(s * S + k) * nf + f];
-        acc[k] += (flips[a] && k == 2 + D) ? -ck : ck;
-      }
+    for (int k = 0; k < S; ++k) {
+      gR[k] = face ? gR[k] : 0.0;
+      gL[k] = below(face ? gL[k] : 0.0);
+      um[k] = below(u0[k]);
+      up[k] = above(u0[k]);
+      acc[k] = 0.0;
+      gum[k] = 0.0;
+      gup[k] = 0.0;
     }
-  }
-  double* o = lam_in + cell * g.es;
+    evolve_adj<ND, D>(um, u0, up, chi, half_dtdh, limiter, form, m, gR, gL, gum, acc, gup, g_half,
+                      g_chi, gm_cell);
 #pragma unroll
-  for (int k = 0; k < S; ++k) o[k * g.cs] = acc[k];
+    for (int k = 0; k < S; ++k)
+      acc[k] = (state ? acc[k] : 0.0) + above(state ? gum[k] : 0.0) + below(state ? gup[k] : 0.0);
+  }
+  // ---- what the ghost cells of the line's ends pass on to the cells they mirror
+  if (!ring && (seg == 0 || (seg + 1) * kAdjCells >= n - 2)) {  // uniform
+    const bool lo = j >= 0 && j <= 1, hi = j >= n - 2 && j < n;
+    const int src_lo = lo ? t - (int)(2 * j + 1) : t;
+    const int src_hi = hi ? t + (int)(2 * (n - j) - 1) : t;
+    double add[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      const double sgn = bc == kBcReflective && k == 2 + D ? -1.0 : 1.0;
+      const double a = __shfl(acc[k], src_lo, 64), b = __shfl(acc[k], src_hi, 64);
+      add[k] = (lo ? sgn * a : 0.0) + (hi ? sgn * b : 0.0);
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k) acc[k] += add[k];
+  }
+  // ---- results: a segment's own cells, and at a line's ends its ghost cells
+  const bool own = live && t >= kAdjHalo && t < kAdjHalo + kAdjCells && j < n;
+  const bool before = live && j == -1, after = live && j == n && t > kAdjHalo &&
+                                                t <= kAdjHalo + kAdjCells;
+  if (own) {
+#pragma unroll
+    for (int k = 0; k < S; ++k) lam_in[at + k * g.cs] = la[k] + acc[k];
+  }
+  if (own || before || after) chi_g[chi_at(j)] = ring && !own ? 0.0 : g_chi;
+  double s0 = 0.0, s1 = 0.0;
+  if (own || (!ring && before)) {
+    s0 += g_dtdh;
+    s1 += gm_face.gamma;
+  }
+  if (own || (!ring && (before || after))) {
+    s0 += 0.5 * g_half;
+    s1 += gm_cell.gamma;
+  }
+  __shared__ double red[2][kAdjWaves];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    s0 += __shfl_xor(s0, off, 64);
+    s1 += __shfl_xor(s1, off, 64);
+  }
+  if (t == 0) {
+    red[0][w] = s0;
+    red[1][w] = s1;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double v = 0.0;
+    for (int i = 0; i < kAdjWaves; ++i) v += red[threadIdx.x][i];
+    partials[2 * blockIdx.x + threadIdx.x] = v;
+  }
 }
 
 // ---- the flattening factor's adjoint ----------------------------------------
@@ -274,9 +281,9 @@ __global__ void __launch_bounds__(256) gather_adj_kernel(AGrid g, const double* 
 
 // At each chi position (the grid padded by one cell) whose chi lies strictly
 // between 0 and 1 (elsewhere the selected factor is clamped or not
-// flattened and carries no gradient): the adjoint of chi, the sum of what the
-// position's right face state (face i+1/2) and left face state (face i-1/2)
-// passed back in sweep dimension D; which factor the minimum selected,
+// flattened and carries no gradient): the adjoint of chi that the position's
+// face states passed back in sweep dimension D; which factor the minimum
+// selected,
 // rec_k = 4 d + (j - c along d) + 1 for K_d(j) (-1: none); and the adjoints
 // of the pressures at j-2, j-1, j+1, j+2 along d (rec_v, 4 per position).
 // *any is set when some position has a record.
@@ -297,17 +304,9 @@ __global__ void __launch_bounds__(256) chi_adj_kernel(AGrid g, const double* __r
   const double cv = chi[q];
   double G = 0.0;
   if (cv > 0.0 && cv < 1.0) {
-    const int64_t n = D == 0 ? g.nx : g.ny;
     const int64_t lines = D == 0 ? g.ny : g.nx;
-    const int64_t i = D == 0 ? x : y;     // along the sweep: -1 .. n
     const int64_t line = D == 0 ? y : x;  // faces exist on interior lines only
-    if (line >= 0 && line < lines) {
-      auto face = [&](int64_t ii) {
-        return D == 0 ? line * (n + 1) + (ii + 1) : (ii + 1) * lines + line;
-      };
-      if (i <= n - 1) G += chi_g[2 * face(i)];
-      if (i >= 0) G += chi_g[2 * face(i - 1) + 1];
-    }
+    if (line >= 0 && line < lines) G = chi_g[q];
   }
   auto at = [&](const double* A, int64_t xx, int64_t yy) {
     return A[(ND > 1 ? (yy + 4) * px : 0) + xx + 4];
@@ -470,47 +469,23 @@ __global__ void __launch_bounds__(256) chi_gather_kernel(AGrid g, Material<doubl
   }
 }
 
-// Per-block sums of the per-face (dt/dh, gamma) adjoints; kPartialBlocks
-// blocks of 256 threads, fixed order.
-__global__ void __launch_bounds__(256) partial_sum_kernel(const double* __restrict__ face_g,
-                                                          int64_t nfaces,
-                                                          double* __restrict__ partials) {
-  __shared__ double s0[256], s1[256];
-  double a0 = 0.0, a1 = 0.0;
-  for (int64_t f = (int64_t)blockIdx.x * 256 + threadIdx.x; f < nfaces;
-       f += (int64_t)kPartialBlocks * 256) {
-    a0 += face_g[2 * f];
-    a1 += face_g[2 * f + 1];
-  }
-  s0[threadIdx.x] = a0;
-  s1[threadIdx.x] = a1;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      s0[threadIdx.x] += s0[threadIdx.x + w];
-      s1[threadIdx.x] += s1[threadIdx.x + w];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    partials[2 * blockIdx.x] = s0[0];
-    partials[2 * blockIdx.x + 1] = s1[0];
-  }
+// Clears the argmax of n records.
+__global__ void rec_clear_kernel(StepRec* rec, int64_t n) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) rec[k].argmax = ~0ull;
 }
 
-// Records this step's max wavespeed and dt/dh from the control block and
-// clears the argmax slot.
-__global__ void record_kernel(const StepCtl* ctl, int parity, StepRec* rec) {
-  rec->maxws_bits = ctl->ws_bits[parity];
-  rec->dtdh = ctl->dtdh;
-  rec->argmax = ~0ull;
-}
-
-// Lowest index of a cell whose wavespeed bits equal the recorded maximum.
+// Records a step's max wavespeed and dt/dh (its input g, the maximum in slot
+// `slot`, its sweeps just run) and the lowest index of a cell whose wavespeed
+// bits equal the maximum.
 template <int ND>
-__global__ void __launch_bounds__(256) argmax_kernel(AGrid g, Material<double> m,
-                                                     StepRec* rec) {
-  const unsigned long long target = rec->maxws_bits;
+__global__ void __launch_bounds__(256) record_kernel(AGrid g, Material<double> m,
+                                                     const SimCtl* sim, int slot, StepRec* rec) {
+  const unsigned long long target = sim->ws[slot];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    rec->maxws_bits = target;
+    rec->dtdh = sim->c.dtdh;
+  }
   unsigned long long best = ~0ull;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < g.nx * g.ny;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -527,22 +502,22 @@ __global__ void __launch_bounds__(256) argmax_kernel(AGrid g, Material<double> m
   if (best != ~0ull) atomicMin(&rec->argmax, best);
 }
 
-// Sums the partials of the step's sweeps (x then y), turns the dt/dh adjoint
+// Sums the partials of the step's sweeps, turns the dt/dh adjoint
 // into the max-wavespeed adjoint (d(dt/dh)/d maxws = -(dt/dh)/maxws), adds
 // that cell's wavespeed adjoint into lambda_n and accumulates the gamma
 // adjoint.  One workgroup of 256 threads.
 template <int ND>
 __global__ void __launch_bounds__(256) finalize_kernel(AGrid g, Material<double> m,
                                                        const StepRec* __restrict__ rec,
-                                                       const double* __restrict__ partials,
-                                                       int nsweeps, double* __restrict__ lam_n,
+                                                       Partials parts,
+                                                       double* __restrict__ lam_n,
                                                        double* __restrict__ acc) {
   __shared__ double s0[256], s1[256];
   double a0 = 0.0, a1 = 0.0;
-  for (int sw = 0; sw < nsweeps; ++sw)
-    for (int b = threadIdx.x; b < kPartialBlocks; b += 256) {
-      a0 += partials[sw * 2 * kPartialBlocks + 2 * b];
-      a1 += partials[sw * 2 * kPartialBlocks + 2 * b + 1];
+  for (int i = 0; i < 4; ++i)
+    for (int b = threadIdx.x; b < parts.n[i]; b += 256) {
+      a0 += parts.p[i][2 * b];
+      a1 += parts.p[i][2 * b + 1];
     }
   s0[threadIdx.x] = a0;
   s1[threadIdx.x] = a1;
@@ -582,17 +557,15 @@ __global__ void acc_clear_kernel(double* acc) {
   acc[1] = 0.0;
 }
 
-#define FL_FACE_INST(ND, D, FLUX, PRIM)                                                     \
-  template __global__ void face_adj_kernel<ND, D, FLUX, PRIM>(                               \
-      AGrid, const double*, Material<double>, int, const StepRec*, const double*, double*,     \
+#define FL_SWEEP_INST(ND, D, FLUX, PRIM)                                                     \
+  template __global__ void sweep_adj_kernel<ND, D, FLUX, PRIM>(                               \
+      AGrid, const double*, double*, Material<double>, int, const StepRec*, const double*,     \
       double*, double*);
 #define FL_ADJ_INST(ND, D)                                                                  \
-  FL_FACE_INST(ND, D, kFluxHllc, false)                                                      \
-  FL_FACE_INST(ND, D, kFluxForce, false)                                                     \
-  FL_FACE_INST(ND, D, kFluxHllc, true)                                                       \
-  FL_FACE_INST(ND, D, kFluxForce, true)                                                      \
-  template __global__ void gather_adj_kernel<ND, D>(AGrid, const double*, double*,           \
-                                                    const double*);                          \
+  FL_SWEEP_INST(ND, D, kFluxHllc, false)                                                     \
+  FL_SWEEP_INST(ND, D, kFluxForce, false)                                                    \
+  FL_SWEEP_INST(ND, D, kFluxHllc, true)                                                      \
+  FL_SWEEP_INST(ND, D, kFluxForce, true)                                                     \
   template __global__ void chi_adj_kernel<ND, D>(AGrid, const double*, const double*,         \
                                                  const double*, const double*, const double*, \
                                                  int*, double*, int*);
@@ -610,12 +583,12 @@ template __global__ void chi_gather_kernel<1>(AGrid, Material<double>, const int
                                               const int*, double*, double*);
 template __global__ void chi_gather_kernel<2>(AGrid, Material<double>, const int*, const double*,
                                               const int*, double*, double*);
-template __global__ void argmax_kernel<1>(AGrid, Material<double>, StepRec*);
-template __global__ void argmax_kernel<2>(AGrid, Material<double>, StepRec*);
+template __global__ void record_kernel<1>(AGrid, Material<double>, const SimCtl*, int, StepRec*);
+template __global__ void record_kernel<2>(AGrid, Material<double>, const SimCtl*, int, StepRec*);
 template __global__ void finalize_kernel<1>(AGrid, Material<double>, const StepRec*,
-                                            const double*, int, double*, double*);
+                                            Partials, double*, double*);
 template __global__ void finalize_kernel<2>(AGrid, Material<double>, const StepRec*,
-                                            const double*, int, double*, double*);
+                                            Partials, double*, double*);
 
 }  // namespace adj
 }  // namespace fl

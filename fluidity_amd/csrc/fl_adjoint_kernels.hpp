@@ -25,15 +25,29 @@ struct StepRec {
 
 constexpr int kPartialBlocks = 256;
 
+// Waves of a sweep workgroup (a line each), the cells of a line that a wave
+// takes, and those on either side that its lanes hold as well: the reverse of
+// the cell before needs that of the face before it, whose left state is that
+// of the cell before that.
+constexpr int kAdjWaves = 4;
+constexpr int kAdjHalo = 3;
+constexpr int kAdjCells = 64 - 2 * kAdjHalo;
+
+// (dt/dh, gamma) sums of a step, up to four lists of pairs.
+struct Partials {
+  const double* p[4];
+  int n[4];
+};
+
 template <int ND>
 __global__ void prim_pad_kernel(AGrid g, Material<double> m, double* P, double* V0, double* V1);
 template <int ND>
 __global__ void chi_pad_kernel(AGrid g, const double* P, const double* V0, const double* V1,
                                double* chi, int* any);
 template <int ND, int D, int FLUX, bool PRIM>
-__global__ void face_adj_kernel(AGrid g, const double* lam, Material<double> m, int limiter,
-                                const StepRec* rec, const double* chi_pad, double* contrib,
-                                double* face_g, double* chi_g);
+__global__ void sweep_adj_kernel(AGrid g, const double* lam, double* lam_in, Material<double> m,
+                                 int limiter, const StepRec* rec, const double* chi_pad,
+                                 double* chi_g, double* partials);
 template <int ND, int D>
 __global__ void chi_adj_kernel(AGrid g, const double* P, const double* V0, const double* V1,
                                const double* chi, const double* chi_g, int* rec_k,
@@ -42,16 +56,13 @@ template <int ND>
 __global__ void chi_gather_kernel(AGrid g, Material<double> m, const int* rec_k,
                                   const double* rec_v, const int* any, double* lam,
                                   double* partials);
-template <int ND, int D>
-__global__ void gather_adj_kernel(AGrid g, const double* lam_out, double* lam_in,
-                                  const double* contrib);
-__global__ void partial_sum_kernel(const double* face_g, int64_t nfaces, double* partials);
-__global__ void record_kernel(const StepCtl* ctl, int parity, StepRec* rec);
+__global__ void rec_clear_kernel(StepRec* rec, int64_t n);
 template <int ND>
-__global__ void argmax_kernel(AGrid g, Material<double> m, StepRec* rec);
+__global__ void record_kernel(AGrid g, Material<double> m, const SimCtl* sim, int slot,
+                              StepRec* rec);
 template <int ND>
 __global__ void finalize_kernel(AGrid g, Material<double> m, const StepRec* rec,
-                                const double* partials, int nsweeps, double* lam_n, double* acc);
+                                Partials parts, double* lam_n, double* acc);
 __global__ void acc_clear_kernel(double* acc);
 
 }  // namespace adj

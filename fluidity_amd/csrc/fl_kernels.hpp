@@ -162,8 +162,6 @@ __global__ void wavespeeds_kernel(const T* in, int64_t es, int64_t cs, int64_t n
                                   Material<double> m64, double* ws);
 __global__ void max_element_kernel(const double* v, int64_t n, unsigned long long* dst);
 __global__ void zero_u64_kernel(unsigned long long* p);
-__global__ void step_control_kernel(StepCtl* ctl, int parity, double cfl, double dh,
-                                    double sim_time, long long max_iters);
 __global__ void init_control_kernel(StepCtl* ctl);
 __global__ void init_sim_kernel(SimCtl* sim);
 __global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh);

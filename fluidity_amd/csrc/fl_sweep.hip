@@ -198,24 +198,6 @@ __global__ void __launch_bounds__(kMaxBlock) max_element_kernel(const double* __
 
 __global__ void zero_u64_kernel(unsigned long long* p) { *p = 0ull; }
 
-// One step of Parameters::update_time_delta / dt_dh / update_simulation_info
-// (simulator/parameters.hpp:60-99) and the loop condition of
-// SimulatorImpl::simulate (simulator/simulator_impl.hpp:235).
-__global__ void step_control_kernel(StepCtl* ctl, int parity, double cfl, double dh,
-                                    double sim_time, long long max_iters) {
-  const bool active = ctl->t < sim_time && ctl->iters < max_iters;
-  if (active) {
-    const double maxws = __longlong_as_double((long long)ctl->ws_bits[parity]);
-    const double dt = cfl * dh / maxws;
-    ctl->dt = dt;
-    ctl->dtdh = dt / dh;
-    ctl->t += dt;
-    ctl->iters += 1;
-    ctl->ws_bits[parity ^ 1] = 0ull;  // target of this step's fused CFL epilogue
-  }
-  ctl->active = active ? 1 : 0;
-}
-
 // dt of a two-material step from the maximum wavespeed reduced into
 // ws_bits[0] over both grids after the ghost states were written (the loop of
 // simulator/multimaterial_simulator.hpp, update_time_delta in
