@@ -751,27 +751,43 @@ int fl_ctx_create(int device, fl_context** out) {
   memset(c, 0, sizeof(*c));
   c->device = device;
   (void)resolve_tuning(nullptr, &c->tuning, c->shape);
-  hipError_t e = hipMalloc((void**)&c->ctl, sizeof(fl::StepCtl));
-  if (e == hipSuccess) e = hipMalloc((void**)&c->ws_tmp, sizeof(unsigned long long));
-  if (e == hipSuccess) e = hipMalloc((void**)&c->sim, sizeof(fl::SimCtl));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_sim, sizeof(fl::SimCtl), 0);
-  if (e == hipSuccess) e = hipMalloc((void**)&c->partial, sizeof(double) * kSumBlocks * 4);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_ctl, sizeof(fl::StepCtl), 0);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_partial, sizeof(double) * kSumBlocks * 4, 0);
-  if (e == hipSuccess) e = hipStreamCreate(&c->cap_stream);
   c->use_graphs = 1;
-  if (e == hipSuccess) e = hipMalloc((void**)&c->eik, 2 * sizeof(fl::ls::EikCtl));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_eik, 2 * sizeof(fl::ls::EikCtl), 0);
+  // one block on the device and one pinned, each part on 256 bytes of its own
+  size_t dev = 0, host = 0;
+  auto part = [](size_t& at, size_t bytes) {
+    const size_t a = at;
+    at += (bytes + 255) & ~(size_t)255;
+    return a;
+  };
+  const size_t sums = sizeof(double) * kSumBlocks * 4;
+  const size_t ctl = part(dev, sizeof(fl::StepCtl)), ws_tmp = part(dev, sizeof(unsigned long long)),
+               sim = part(dev, sizeof(fl::SimCtl)), eik = part(dev, 2 * sizeof(fl::ls::EikCtl)),
+               pctl = part(dev, sizeof(fl::PersistCtl)), partial = part(dev, sums),
+               words = part(dev, sizeof(unsigned long long) * 3 * fl::kPersistWords *
+                                     fl::kPersistMaxGroups);
+  const size_t host_ctl = part(host, sizeof(fl::StepCtl)), host_sim = part(host, sizeof(fl::SimCtl)),
+               host_eik = part(host, 2 * sizeof(fl::ls::EikCtl)),
+               host_pctl = part(host, sizeof(fl::PersistCtl)), host_partial = part(host, sums);
+  hipError_t e = hipMalloc((void**)&c->dev_block, dev);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_block, host, 0);
+  if (e == hipSuccess) e = hipStreamCreate(&c->cap_stream);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&c->step_ev, hipEventDisableTiming);
-  if (e == hipSuccess) e = hipMalloc((void**)&c->pctl, sizeof(fl::PersistCtl));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&c->host_pctl, sizeof(fl::PersistCtl), 0);
-  if (e == hipSuccess)
-    e = hipMalloc((void**)&c->words,
-                  sizeof(unsigned long long) * 3 * fl::kPersistWords * fl::kPersistMaxGroups);
   if (e != hipSuccess) {
     fl_ctx_destroy(c);
     return fail(FL_ERR_HIP, "context allocation failed: %s", hipGetErrorString(e));
   }
+  c->ctl = (fl::StepCtl*)(c->dev_block + ctl);
+  c->ws_tmp = (unsigned long long*)(c->dev_block + ws_tmp);
+  c->sim = (fl::SimCtl*)(c->dev_block + sim);
+  c->eik = (fl::ls::EikCtl*)(c->dev_block + eik);
+  c->pctl = (fl::PersistCtl*)(c->dev_block + pctl);
+  c->partial = (double*)(c->dev_block + partial);
+  c->words = (unsigned long long*)(c->dev_block + words);
+  c->host_ctl = (fl::StepCtl*)(c->host_block + host_ctl);
+  c->host_sim = (fl::SimCtl*)(c->host_block + host_sim);
+  c->host_eik = (fl::ls::EikCtl*)(c->host_block + host_eik);
+  c->host_pctl = (fl::PersistCtl*)(c->host_block + host_pctl);
+  c->host_partial = (double*)(c->host_block + host_partial);
   *out = c;
   return FL_OK;
 }
@@ -779,21 +795,11 @@ int fl_ctx_create(int device, fl_context** out) {
 int fl_ctx_destroy(fl_context* c) {
   if (!c) return FL_OK;
   DeviceGuard g(c->device);
-  if (c->ctl) (void)hipFree(c->ctl);
-  if (c->ws_tmp) (void)hipFree(c->ws_tmp);
-  if (c->sim) (void)hipFree(c->sim);
-  if (c->host_sim) (void)hipHostFree(c->host_sim);
-  if (c->partial) (void)hipFree(c->partial);
-  if (c->host_ctl) (void)hipHostFree(c->host_ctl);
-  if (c->host_partial) (void)hipHostFree(c->host_partial);
   drop_sim_graphs(c);
   if (c->cap_stream) (void)hipStreamDestroy(c->cap_stream);
-  if (c->eik) (void)hipFree(c->eik);
-  if (c->host_eik) (void)hipHostFree(c->host_eik);
   if (c->step_ev) (void)hipEventDestroy(c->step_ev);
-  if (c->pctl) (void)hipFree(c->pctl);
-  if (c->host_pctl) (void)hipHostFree(c->host_pctl);
-  if (c->words) (void)hipFree(c->words);
+  if (c->dev_block) (void)hipFree(c->dev_block);
+  if (c->host_block) (void)hipHostFree(c->host_block);
   delete c;
   return FL_OK;
 }

@@ -38,6 +38,8 @@ enum : int { kShapeRule = 0, kShapeTuning = 1, kShapeCell = 2 };
 
 struct fl_context {
   int device;
+  char* dev_block;             // the device memory of the pointers below
+  char* host_block;            // the pinned memory of the host mirrors
   fl::StepCtl* ctl;            // device control block of the two-material loop
   unsigned long long* ws_tmp;  // device scratch for fl_max_wavespeed
   fl::SimCtl* sim;             // device control words of fl_simulate's launched steps
