@@ -199,14 +199,16 @@ template <> constexpr int64_t kCellMax<float> = 5 << 20;
 template <typename T>
 SweepShape pick_shape(const fl_context* ctx, int dim, int64_t nx, int64_t ny, int ngrids) {
   const fl_tuning& tu = ctx->tuning;
-  if (ctx->shape[dim] == kShapeTuning) {
+  const bool few = nx * ny * ngrids <= kCellMax<T>;
+  // kShapeCell was measured on one grid; two of them may be past the line, and
+  // then take the fastest marching shape of that measurement
+  if (ctx->shape[dim] == kShapeTuning ||
+      (ctx->shape[dim] == kShapeCell && ngrids > 1 && !few)) {
     const int B = dim ? tu.y_block : tu.x_block;
     const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
     return {false, B, fit_rows(dim ? tu.y_rows : tu.x_rows, ngrids * bands, ny, B)};
   }
-  // kShapeCell was measured on one grid; two of them may be past the line
-  if ((ctx->shape[dim] == kShapeCell && ngrids == 1) || nx * ny * ngrids <= kCellMax<T>)
-    return {true, 0, 0};
+  if (ctx->shape[dim] == kShapeCell || few) return {true, 0, 0};
   const int B = dim ? 64 : 128;
   const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
   const int64_t waves = ngrids * bands * (B / 64) * ny;  // of one-row tiles

@@ -162,9 +162,13 @@ __global__ void wavespeeds_kernel(const T* in, int64_t es, int64_t cs, int64_t n
                                   Material<double> m64, double* ws);
 __global__ void max_element_kernel(const double* v, int64_t n, unsigned long long* dst);
 __global__ void zero_u64_kernel(unsigned long long* p);
-__global__ void init_control_kernel(StepCtl* ctl);
 __global__ void init_sim_kernel(SimCtl* sim);
-__global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh);
+// Counts that a two-material step clears for the next one (nullable).
+struct MmCounts {
+  int* p[4];
+};
+__global__ void mm_init_kernel(StepCtl* ctl, MmCounts counts);
+__global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh, MmCounts counts);
 template <typename T, int FLUX, bool FAST, bool VLC>
 __global__ void persist1d_kernel(SweepArgs<T> a, PersistCtl* pc, unsigned long long* words,
                                  int nseg, double cfl, double dh, double sim_time,

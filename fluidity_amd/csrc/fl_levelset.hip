@@ -931,25 +931,14 @@ __device__ void interp_state(const StateView& v, const Grid& g, int64_t x, int64
   }
 }
 
-// RiemannGFM<3>::invoke (ghost_fluid/riemann_ghost_fluid.hpp:50-195) at an
-// inside-interfacial cell i = (x, y) of material m: p = phi_m[i], po =
-// phi_o[i].  Writes star[i] and sets has_star[i] when the cell takes a star
-// state.
+// RiemannGFM<3>::invoke (ghost_fluid/riemann_ghost_fluid.hpp:50-195): the star
+// state of material m at an interfacial cell (x, y), p = phi_m there.
 template <int ND>
-__device__ __forceinline__ void star_cell(const double* __restrict__ phi_m, double po,
-                                          const StateView& um, const StateView& uo,
-                                          const Eos& em, const Eos& eo, const Grid& g, double dh,
-                                          int64_t x, int64_t y, int64_t i, double p,
-                                          double* __restrict__ star,
-                                          uint8_t* __restrict__ has_star) {
+__device__ __forceinline__ void star_state(const double* __restrict__ phi_m, const StateView& um,
+                                           const StateView& uo, const Eos& em, const Eos& eo,
+                                           const Grid& g, double dh, int64_t x, int64_t y,
+                                           double p, double* out) {
   constexpr int S = 2 + ND;
-  for (int d = 0; d < ND; ++d) {
-    const int64_t dx = (d == 0), dy = (d == 1);
-    if (phi_at1<ND>(phi_m, g, x - dx, y - dy) == 0.0 || phi_at1<ND>(phi_m, g, x + dx, y + dy) == 0.0)
-      return;
-  }
-  const uint8_t mo = mask_value(po, dh);
-  if (!((mo & 16) || (mo & 4))) return;
   double nrm[2] = {0.0, 0.0};
   norm_at<ND>(phi_m, g, x, y, dh, nrm);
   const double abs_phi = fabs(p);
@@ -986,8 +975,34 @@ __device__ __forceinline__ void star_cell(const double* __restrict__ phi_m, doub
   const double vs_n = Ws[2];
 #pragma unroll
   for (int d = 0; d < ND; ++d) Ws[2 + d] = vl[d] + (vs_n - vl_n) * nrm[d];
-  double out[S];
   prim_to_cons<ND>(Ws, em, out);
+}
+
+// The other material beside an inside-interfacial cell: po = phi_o there.
+__device__ __forceinline__ bool star_other(double po, double dh) {
+  const uint8_t mo = mask_value(po, dh);
+  return (mo & 16) || (mo & 4);
+}
+
+// At an inside-interfacial cell i = (x, y) of material m, p = phi_m[i], po =
+// phi_o[i]: writes star[i] and sets has_star[i] when the cell takes a star
+// state.
+template <int ND>
+__device__ __forceinline__ void star_cell(const double* __restrict__ phi_m, double po,
+                                          const StateView& um, const StateView& uo,
+                                          const Eos& em, const Eos& eo, const Grid& g, double dh,
+                                          int64_t x, int64_t y, int64_t i, double p,
+                                          double* __restrict__ star,
+                                          uint8_t* __restrict__ has_star) {
+  constexpr int S = 2 + ND;
+  for (int d = 0; d < ND; ++d) {
+    const int64_t dx = (d == 0), dy = (d == 1);
+    if (phi_at1<ND>(phi_m, g, x - dx, y - dy) == 0.0 || phi_at1<ND>(phi_m, g, x + dx, y + dy) == 0.0)
+      return;
+  }
+  if (!star_other(po, dh)) return;
+  double out[S];
+  star_state<ND>(phi_m, um, uo, em, eo, g, dh, x, y, p, out);
 #pragma unroll
   for (int k = 0; k < S; ++k) star[i * S + k] = out[k];
   has_star[i] = 1;
@@ -1008,31 +1023,6 @@ __global__ void gfm_star_kernel(const double* __restrict__ phi_m, const double* 
   const double p = phi_m[i];
   if (!(mask_value(p, dh) & 8)) return;
   star_cell<ND>(phi_m, phi_o[i], um, uo, em, eo, g, dh, x, y, i, p, star, has_star);
-}
-
-// Star states of both materials of a two-material step in one pass: thread i
-// tests cell i for both, from one load of each level set; both band-list
-// counts are zeroed.
-template <int ND>
-__global__ void gfm_star2_kernel(const double* __restrict__ phi0, const double* __restrict__ phi1,
-                                 StateView u0, StateView u1, Eos e0, Eos e1, Grid g, double dh,
-                                 double* __restrict__ star0, double* __restrict__ star1,
-                                 uint8_t* __restrict__ has0, uint8_t* __restrict__ has1,
-                                 int* __restrict__ count0, int* __restrict__ count1) {
-  const int64_t i = gid();
-  if (i >= g.nx * g.ny) return;
-  if (i == 0) {
-    *count0 = 0;
-    *count1 = 0;
-  }
-  const int64_t x = i % g.nx, y = i / g.nx;
-  const double p0 = phi0[i], p1 = phi1[i];
-  has0[i] = 0;
-  has1[i] = 0;
-  if (mask_value(p0, dh) & 8)
-    star_cell<ND>(phi0, p1, u0, u1, e0, e1, g, dh, x, y, i, p0, star0, has0);
-  if (mask_value(p1, dh) & 8)
-    star_cell<ND>(phi1, p0, u1, u0, e1, e0, g, dh, x, y, i, p1, star1, has1);
 }
 
 // Star states of material m among ms.nmat materials (one thread per cell):
@@ -1118,22 +1108,24 @@ __device__ __forceinline__ int in_band(double p, double upper) {
 // written: the band cells and their neighbours (a band cell reads itself and
 // its upwind neighbours).  Band cells 0 < phi <= upper are appended to `list`
 // in no particular order: each band cell's update is independent of the
-// others within a sweep.
+// others within a sweep.  pc: phi at the cell; zero: it is 0 at a neighbour.
 template <int ND>
 __device__ __forceinline__ void band_flags(const double* __restrict__ phi_m, double upper,
                                            const Grid& g, int64_t x, int64_t y, int64_t i,
-                                           bool& band, bool& needed) {
+                                           bool& band, bool& needed, double& pc, bool& zero) {
   // neighbours past the edge read the cell itself, which adds nothing to
   // `needed`; the loads are unconditional so that they are issued together
-  const double pc = phi_m[i];
+  pc = phi_m[i];
   const double pxm = phi_m[x > 0 ? i - 1 : i];
   const double pxp = phi_m[x < g.nx - 1 ? i + 1 : i];
   const int b = in_band(pc, upper);
   int n = b | in_band(pxm, upper) | in_band(pxp, upper);
+  zero = pxm == 0.0 || pxp == 0.0;
   if (ND > 1) {
     const double pym = phi_m[y > 0 ? i - g.nx : i];
     const double pyp = phi_m[y < g.ny - 1 ? i + g.nx : i];
     n |= in_band(pym, upper) | in_band(pyp, upper);
+    zero = zero || pym == 0.0 || pyp == 0.0;
   }
   band = b != 0;
   needed = n != 0;
@@ -1183,8 +1175,9 @@ __global__ void gfm_band_seed_kernel(const double* __restrict__ phi_m, double up
   const int64_t i = gid();
   if (i >= g.nx * g.ny) return;
   const int64_t x = i % g.nx, y = i / g.nx;
-  bool band, needed;
-  band_flags<ND>(phi_m, upper, g, x, y, i, band, needed);
+  bool band, needed, zero;
+  double p;
+  band_flags<ND>(phi_m, upper, g, x, y, i, band, needed, p, zero);
   list_append(band, i, list, count);
   if (needed) band_seed_cell<ND>(um, star, has_star, g, x, y, i, A, B);
 }
@@ -1199,13 +1192,72 @@ __global__ void gfm_band_seed2_kernel(ExtrapJob j0, ExtrapJob j1, double upper,
   const int64_t i = gid();
   if (i >= g.nx * g.ny) return;
   const int64_t x = i % g.nx, y = i / g.nx;
-  bool band0, needed0, band1, needed1;
-  band_flags<ND>(j0.phi, upper, g, x, y, i, band0, needed0);
-  band_flags<ND>(j1.phi, upper, g, x, y, i, band1, needed1);
+  bool band0, needed0, band1, needed1, zero0, zero1;
+  double p0, p1;
+  band_flags<ND>(j0.phi, upper, g, x, y, i, band0, needed0, p0, zero0);
+  band_flags<ND>(j1.phi, upper, g, x, y, i, band1, needed1, p1, zero1);
   list_append(band0, i, j0.list, j0.count);
   list_append(band1, i, j1.list, j1.count);
   if (needed0) band_seed_cell<ND>(j0.um, star0, has0, g, x, y, i, j0.A, j0.B);
   if (needed1) band_seed_cell<ND>(j1.um, star1, has1, g, x, y, i, j1.A, j1.B);
+}
+
+// The two-material step's seeds: both materials' bands as in
+// gfm_band_seed2_kernel with their own states, and the lists of the cells that
+// take star states, which gfm_star_list_kernel then computes.  A star state
+// is a chain of some thirty divisions and roots at the few cells of the
+// interface: computed by the threads of a pass over the grid, both materials'
+// one after the other, the pass took 36 us at 2048x1024 and 15 at 384x192
+// (and the seeds 21 and 6); a launch over the listed cells takes 8 and 7 (and
+// this one 24 and 7).
+template <int ND>
+__global__ void gfm_seed2_kernel(ExtrapJob j0, ExtrapJob j1, double upper, StarJob s0, StarJob s1,
+                                 Grid g, double dh) {
+  const int64_t i = gid();
+  if (i >= g.nx * g.ny) return;
+  const int64_t x = i % g.nx, y = i / g.nx;
+  bool band0, needed0, band1, needed1, zero0, zero1;
+  double p0, p1;
+  band_flags<ND>(j0.phi, upper, g, x, y, i, band0, needed0, p0, zero0);
+  band_flags<ND>(j1.phi, upper, g, x, y, i, band1, needed1, p1, zero1);
+  list_append(band0, i, j0.list, j0.count);
+  list_append(band1, i, j1.list, j1.count);
+  list_append((mask_value(p0, dh) & 8) && !zero0 && star_other(p1, dh), i, s0.list, s0.count);
+  list_append((mask_value(p1, dh) & 8) && !zero1 && star_other(p0, dh), i, s1.list, s1.count);
+  constexpr int S = 2 + ND;
+  double u[S];
+  if (needed0) {
+    load_state_i<S>(j0.um, i, u);
+#pragma unroll
+    for (int k = 0; k < S; ++k) j0.A[i * S + k] = j0.B[i * S + k] = u[k];
+  }
+  if (needed1) {
+    load_state_i<S>(j1.um, i, u);
+#pragma unroll
+    for (int k = 0; k < S; ++k) j1.A[i * S + k] = j1.B[i * S + k] = u[k];
+  }
+}
+
+// Star states of the listed cells into both Jacobi buffers, a material per
+// blockIdx.y.
+template <int ND>
+__global__ void __launch_bounds__(64) gfm_star_list_kernel(ExtrapJob j0, ExtrapJob j1, StarJob s0,
+                                                           StarJob s1, Eos e0, Eos e1, Grid g,
+                                                           double dh) {
+  constexpr int S = 2 + ND;
+  const bool second = blockIdx.y != 0;
+  const ExtrapJob j = second ? j1 : j0;
+  const StarJob sj = second ? s1 : s0;
+  const StateView uo = second ? j0.um : j1.um;
+  const Eos em = second ? e1 : e0, eo = second ? e0 : e1;
+  const int n = *sj.count;
+  for (int k = (int)(blockIdx.x * 64 + threadIdx.x); k < n; k += (int)gridDim.x * 64) {
+    const int64_t i = sj.list[k];
+    double out[S];
+    star_state<ND>(j.phi, j.um, uo, em, eo, g, dh, i % g.nx, i / g.nx, j.phi[i], out);
+#pragma unroll
+    for (int c = 0; c < S; ++c) j.A[i * S + c] = j.B[i * S + c] = out[c];
+  }
 }
 
 __global__ void count_clear_kernel(int* count) { *count = 0; }
@@ -1328,9 +1380,10 @@ FL_EIK_INST(2)
   template __global__ void gfm_band_seed_kernel<ND>(const double*, double, StateView,       \
                                                     const double*, const uint8_t*, Grid,      \
                                                     double*, double*, int*, int*);            \
-  template __global__ void gfm_star2_kernel<ND>(const double*, const double*, StateView,     \
-                                                StateView, Eos, Eos, Grid, double, double*,  \
-                                                double*, uint8_t*, uint8_t*, int*, int*);    \
+  template __global__ void gfm_seed2_kernel<ND>(ExtrapJob, ExtrapJob, double, StarJob,       \
+                                                StarJob, Grid, double);                       \
+  template __global__ void gfm_star_list_kernel<ND>(ExtrapJob, ExtrapJob, StarJob, StarJob,  \
+                                                    Eos, Eos, Grid, double);                  \
   template __global__ void gfm_band_seed2_kernel<ND>(ExtrapJob, ExtrapJob, double,          \
                                                      const double*, const double*,           \
                                                      const uint8_t*, const uint8_t*, Grid);  \

@@ -356,21 +356,16 @@ void band_seed(const ls::ExtrapJob& j, const double* star, const uint8_t* has,
                        extrap_upper(dh), j.um, star, has, g, j.A, j.B, j.list, j.count);
 }
 
-// Star states of both materials (each from the same level sets and states)
-// and zeroed band-list counts of both jobs.
-void launch_star2(double* const cur[2], const fl_material* mats, const ls::Grid& g, double dh,
-                  const MmGhost& w, const ls::ExtrapJob jobs[2], hipStream_t st) {
-  const dim3 grid = grid_for(g.nx * g.ny);
-  const ls::StateView u0 = view_of(&mats[0].state), u1 = view_of(&mats[1].state);
-  const ls::Eos e0 = eos_of(&mats[0].scheme), e1 = eos_of(&mats[1].scheme);
-  if (g.nd == 1)
-    hipLaunchKernelGGL(ls::gfm_star2_kernel<1>, grid, dim3(kBlock), 0, st,
-                       (const double*)cur[0], (const double*)cur[1], u0, u1, e0, e1, g, dh,
-                       w.star[0], w.star[1], w.has[0], w.has[1], jobs[0].count, jobs[1].count);
-  else
-    hipLaunchKernelGGL(ls::gfm_star2_kernel<2>, grid, dim3(kBlock), 0, st,
-                       (const double*)cur[0], (const double*)cur[1], u0, u1, e0, e1, g, dh,
-                       w.star[0], w.star[1], w.has[0], w.has[1], jobs[0].count, jobs[1].count);
+// Ghost seeds of both materials of a two-material step: the bands, and the
+// star states at the interface from the same data (every count must be zero).
+void launch_seed2(const ls::ExtrapJob jobs[2], const ls::StarJob stars[2], const fl_material* mats,
+                  const ls::Grid& g, double dh, hipStream_t st) {
+  auto seed = g.nd == 1 ? ls::gfm_seed2_kernel<1> : ls::gfm_seed2_kernel<2>;
+  auto star = g.nd == 1 ? ls::gfm_star_list_kernel<1> : ls::gfm_star_list_kernel<2>;
+  hipLaunchKernelGGL(seed, grid_for(g.nx * g.ny), dim3(kBlock), 0, st, jobs[0], jobs[1],
+                     extrap_upper(dh), stars[0], stars[1], g, dh);
+  hipLaunchKernelGGL(star, dim3(128, 2), dim3(64), 0, st, jobs[0], jobs[1], stars[0], stars[1],
+                     eos_of(&mats[0].scheme), eos_of(&mats[1].scheme), g, dh);
 }
 
 // Band seeds of both materials (the jobs' counts must be zero).
@@ -516,7 +511,7 @@ int mm_simulate_n(fl_context* c, fl_material* mats, int nmat, const fl_sim_param
   };
   const dim3 grid = grid_for(cells);
   fl::StepCtl* ctl = c->ctl;
-  hipLaunchKernelGGL(fl::init_control_kernel, dim3(1), dim3(1), 0, st, ctl);
+  hipLaunchKernelGGL(fl::mm_init_kernel, dim3(1), dim3(1), 0, st, ctl, fl::MmCounts{});
   FL_HIP(hipGetLastError());
   while (t < p->sim_time && it < p->max_iters) {
     ls::ExtrapJob jobs[ls::kMaxMat];
@@ -544,7 +539,8 @@ int mm_simulate_n(fl_context* c, fl_material* mats, int nmat, const fl_sim_param
     FL_HIP(hipGetLastError());
     for (int m = 0; m < nmat; ++m)
       if ((rc = launch_max_ws(&mats[m].state, &mats[m].scheme, &ctl->ws_bits[0], st))) return rc;
-    hipLaunchKernelGGL(fl::mm_control_kernel, dim3(1), dim3(1), 0, st, ctl, p->cfl, dh);
+    hipLaunchKernelGGL(fl::mm_control_kernel, dim3(1), dim3(1), 0, st, ctl, p->cfl, dh,
+                       fl::MmCounts{});
     FL_HIP(hipGetLastError());
     FL_HIP(hipMemcpyAsync(c->host_ctl, ctl, sizeof(fl::StepCtl), hipMemcpyDeviceToHost, st));
     FL_HIP(hipEventRecord(c->step_ev, st));
@@ -846,7 +842,17 @@ int fl_mm_simulate(fl_context* c, fl_material* mats, int nmat, const fl_sim_para
   // condition and to stop on a NaN or vacuum maximum, as the reference loop
   // does, before the level sets move.
   fl::StepCtl* ctl = c->ctl;
-  hipLaunchKernelGGL(fl::init_control_kernel, dim3(1), dim3(1), 0, st, ctl);
+  // the lists of star cells in the scratch that holds star states when there
+  // are more materials; their counts and the bands' are cleared by the step's
+  // control kernel
+  ls::StarJob stars[2];
+  fl::MmCounts counts;
+  for (int m = 0; m < 2; ++m) {
+    stars[m] = {(int*)w.star[m], (int*)w.has[m]};
+    counts.p[m] = stars[m].count;
+    counts.p[2 + m] = extrap_job(cur[m], view_of(&mats[m].state), g, w.extrap[m]).count;
+  }
+  hipLaunchKernelGGL(fl::mm_init_kernel, dim3(1), dim3(1), 0, st, ctl, counts);
   FL_HIP(hipGetLastError());
   while (t < p->sim_time && it < p->max_iters) {
     // ghost cells: star states of both materials from the same data, then
@@ -854,16 +860,14 @@ int fl_mm_simulate(fl_context* c, fl_material* mats, int nmat, const fl_sim_para
     ls::ExtrapJob jobs[2];
     for (int m = 0; m < 2; ++m)
       jobs[m] = extrap_job(cur[m], view_of(&mats[m].state), g, w.extrap[m]);
-    const MmGhost gw = {{w.star[0], w.star[1]}, {w.has[0], w.has[1]}};
-    launch_star2(cur, mats, g, dh, gw, jobs, st);
-    band_seed2(jobs, gw, g, dh, st);
+    launch_seed2(jobs, stars, mats, g, dh, st);
     extrap_sweeps(jobs[0], jobs[1], 2, g, dh, sweeps, st);
     FL_HIP(hipGetLastError());
     // dt from the maximum wavespeed over both grids (ws_bits[0] is clear)
     if ((rc = launch_max_ws2(&mats[0].state, &mats[1].state, &mats[0].scheme, &mats[1].scheme,
                              &ctl->ws_bits[0], st)))
       return rc;
-    hipLaunchKernelGGL(fl::mm_control_kernel, dim3(1), dim3(1), 0, st, ctl, p->cfl, dh);
+    hipLaunchKernelGGL(fl::mm_control_kernel, dim3(1), dim3(1), 0, st, ctl, p->cfl, dh, counts);
     FL_HIP(hipGetLastError());
     FL_HIP(hipMemcpyAsync(c->host_ctl, ctl, sizeof(fl::StepCtl), hipMemcpyDeviceToHost, st));
     FL_HIP(hipEventRecord(c->step_ev, st));

@@ -198,6 +198,12 @@ __global__ void __launch_bounds__(kMaxBlock) max_element_kernel(const double* __
 
 __global__ void zero_u64_kernel(unsigned long long* p) { *p = 0ull; }
 
+__device__ __forceinline__ void clear_counts(const MmCounts& counts) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (counts.p[i]) *counts.p[i] = 0;
+}
+
 // dt of a two-material step from the maximum wavespeed reduced into
 // ws_bits[0] over both grids after the ghost states were written (the loop of
 // simulator/multimaterial_simulator.hpp, update_time_delta in
@@ -205,7 +211,8 @@ __global__ void zero_u64_kernel(unsigned long long* p) { *p = 0ull; }
 // iteration count.  The maximum moves to ws_bits[1] (reported) and ws_bits[0]
 // is cleared for the next step.  A NaN, infinite or non-positive maximum
 // leaves dt, t and iters unchanged and clears `active`, which the sweeps read.
-__global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh) {
+__global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh, MmCounts counts) {
+  clear_counts(counts);
   const unsigned long long bits = ctl->ws_bits[0];
   const double maxws = __longlong_as_double((long long)bits);
   ctl->ws_bits[1] = bits;
@@ -221,7 +228,8 @@ __global__ void mm_control_kernel(StepCtl* ctl, double cfl, double dh) {
   ctl->active = ok ? 1 : 0;
 }
 
-__global__ void init_control_kernel(StepCtl* ctl) {
+__global__ void mm_init_kernel(StepCtl* ctl, MmCounts counts) {
+  clear_counts(counts);
   ctl->ws_bits[0] = 0ull;
   ctl->ws_bits[1] = 0ull;
   ctl->dt = 0.0;
