@@ -73,7 +73,6 @@ struct AdjLayout {
   double* V0;        // same: x velocity
   double* V1;        // same: y velocity
   double* chi;       // (nx+2)(ny+2): flattening factor within 1 ghost cell
-  double* chi_g;     // (nx+2)(ny+2): its adjoint
   int* rec_k;        // (nx+2)(ny+2): the factor each chi minimum selected
   double* rec_v;     // (nx+2)(ny+2) * 4: its pressure adjoints
   int* any;          // 1: some chi position has a record
@@ -105,7 +104,6 @@ AdjLayout adj_layout(void* base, const fl_field* f, int K) {
   L.V1 = (double*)take(padded * 8);
   const int64_t cpad = (nx + 2) * (f->ndim > 1 ? ny + 2 : 1);
   L.chi = (double*)take(cpad * 8);
-  L.chi_g = (double*)take(cpad * 8);
   L.rec_k = (int*)take(cpad * 4);
   L.rec_v = (double*)take(cpad * 4 * 8);
   L.any = (int*)take(4);
@@ -192,14 +190,11 @@ void sweep_adj(const fl_field* f, const fl_scheme* s, const double* Uin, const d
                      : (prim ? aj::sweep_adj_kernel<ND, D, fl::kFluxHllc, true>
                              : aj::sweep_adj_kernel<ND, D, fl::kFluxHllc, false>);
   hipLaunchKernelGGL(sweep, dim3((unsigned)sweep_blocks(f, D)), dim3(64 * aj::kAdjWaves), 0, st, g,
-                     lam_out, lam_in, m, s->limiter, rec, (const double*)L.chi, L.chi_g,
-                     L.sums[D]);
-  // the flattening factor: the selected factors' pressure adjoints where
-  // 0 < chi < 1, then into lambda and the gamma sum
-  hipLaunchKernelGGL((aj::chi_adj_kernel<ND, D>), dim3((unsigned)ceil_div(cpad, 256)), dim3(256),
-                     0, st, g, (const double*)L.P, (const double*)L.V0, (const double*)L.V1,
-                     (const double*)L.chi, (const double*)L.chi_g, L.rec_k, L.rec_v, L.any);
-  hipLaunchKernelGGL(aj::chi_gather_kernel<ND>, dim3(aj::kPartialBlocks), dim3(256), 0, st, g, m,
+                     lam_out, lam_in, m, s->limiter, rec, (const double*)L.chi,
+                     (const double*)L.P, (const double*)L.V0, (const double*)L.V1, L.rec_k, L.rec_v,
+                     L.any, L.sums[D]);
+  // the flattening factors' pressure adjoints into lambda and the gamma sum
+  hipLaunchKernelGGL((aj::chi_gather_kernel<ND, D>), dim3(aj::kPartialBlocks), dim3(256), 0, st, g, m,
                      (const int*)L.rec_k, (const double*)L.rec_v, (const int*)L.any, lam_in,
                      chi_partials);
 }

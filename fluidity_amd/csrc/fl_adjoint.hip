@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(256) chi_pad_kernel(AGrid g, const double* __r
   const int64_t px = g.nx + 8;
   const int64_t cx = g.nx + 2, cy = ND > 1 ? g.ny + 2 : 1;
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q == 0) *any = 0;  // chi_adj_kernel's record flag, read by chi_gather_kernel
+  if (q == 0) *any = 0;  // the record flag, read by chi_gather_kernel
   if (q >= cx * cy) return;
   const int64_t x = q % cx - 1, y = ND > 1 ? q / cx - 1 : 0;
   auto at = [&](const double* A, int64_t xx, int64_t yy) {
@@ -104,6 +104,92 @@ __global__ void __launch_bounds__(256) chi_pad_kernel(AGrid g, const double* __r
   chi[q] = c;
 }
 
+// ---- the flattening factor's adjoint ----------------------------------------
+// chi_v of a cell (chi_pad_kernel) is the smallest of the flattening factors
+// K_d(j) of the cell and of its neighbour on the higher-pressure side in each
+// dimension d; where the selected factor is flattened and not clamped,
+// K = 1 - (z - 0.75) / 0.1 with z = |p(j+1) - p(j-1)| / |p(j+2) - p(j-2)|
+// along d carries the gradient (muscl_reconstructor.hpp:59-87); the
+// flattening test, the neighbour and the minimum are branches.
+
+// At a chi position q = (x, y) (of the grid padded by one cell) whose chi lies
+// strictly between 0 and 1 (elsewhere the selected factor is clamped or not
+// flattened and carries no gradient), G being the adjoint of chi that the
+// position's face states passed back: which factor the minimum selected,
+// rec_k = 4 d + (j - c along d) + 1 for K_d(j) (-1: none); and the adjoints
+// of the pressures at j-2, j-1, j+1, j+2 along d (rec_v, 4 per position).
+// *any is set when some position has a record.
+template <int ND>
+__device__ void chi_record(const AGrid& g, const double* __restrict__ P,
+                           const double* __restrict__ V0, const double* __restrict__ V1, int64_t x,
+                           int64_t y, int64_t q, double G, int* __restrict__ rec_k,
+                           double* __restrict__ rec_v, int* __restrict__ any) {
+  const int64_t px = g.nx + 8;
+  auto at = [&](const double* A, int64_t xx, int64_t yy) {
+    return A[(ND > 1 ? (yy + 4) * px : 0) + xx + 4];
+  };
+  const Material<double> no_shift{};
+  auto chi_d = [&](int64_t xx, int64_t yy, int d) {
+    const int64_t dx = (d == 0), dy = (d == 1);
+    const double* V = d == 0 ? V0 : V1;
+    return chi_factor<double>(at(P, xx - 2 * dx, yy - 2 * dy), at(P, xx - dx, yy - dy),
+                              at(P, xx + dx, yy + dy), at(P, xx + 2 * dx, yy + 2 * dy),
+                              at(V, xx - dx, yy - dy), at(V, xx + dx, yy + dy), no_shift);
+  };
+  int best = -1;
+  {
+    // the selection of chi_pad_kernel: smin(chi, smin(K(c), K(c + s)))
+    double c = DBL_MAX;
+    for (int d = 0; d < ND; ++d) {
+      const int64_t dx = (d == 0), dy = (d == 1);
+      const int sign = signum(at(P, x + dx, y + dy) - at(P, x - dx, y - dy));
+      const double k0 = chi_d(x, y, d);
+      const double k1 = chi_d(x + sign * dx, y + sign * dy, d);
+      double mv = k0;
+      int sel = 4 * d + 1;
+      if (k1 < k0) {
+        mv = k1;
+        sel = 4 * d + sign + 1;
+      }
+      if (mv < c) {
+        c = mv;
+        best = sel;
+      }
+    }
+  }
+  if (best >= 0) {
+    const int d = best / 4, jo = best % 4 - 1;
+    const int64_t dx = (d == 0), dy = (d == 1);
+    const int64_t jx = x + jo * dx, jy = y + jo * dy;
+    const double* V = d == 0 ? V0 : V1;
+    const double p_pp = at(P, jx - 2 * dx, jy - 2 * dy), p_p = at(P, jx - dx, jy - dy);
+    const double p_n = at(P, jx + dx, jy + dy), p_nn = at(P, jx + 2 * dx, jy + 2 * dy);
+    const double u_factor = at(V, jx - dx, jy - dy) - at(V, jx + dx, jy + dy);
+    const double dp = fabs(p_n - p_p);
+    const double pmin = smin(p_n, p_p);
+    const bool flatten = u_factor > 0.0 && dv(dp, pmin) > 0.33;
+    const double den = fabs(p_nn - p_pp);
+    if (flatten && den > 0.0) {
+      const double z = dv(dp, den);
+      const double temp = 1.0 - dv(z - 0.75, 0.85 - 0.75);
+      if (temp > 0.0 && temp < 1.0) {
+        const double g_z = -G / (0.85 - 0.75);
+        const double g_dp = g_z / den;
+        const double g_den = -g_z * z / den;
+        const double sn = (double)signum(p_n - p_p), snn = (double)signum(p_nn - p_pp);
+        rec_v[4 * q + 0] = -g_den * snn;  // p(j-2)
+        rec_v[4 * q + 1] = -g_dp * sn;    // p(j-1)
+        rec_v[4 * q + 2] = g_dp * sn;     // p(j+1)
+        rec_v[4 * q + 3] = g_den * snn;   // p(j+2)
+        rec_k[q] = best;
+        *any = 1;
+        return;
+      }
+    }
+  }
+  rec_k[q] = -1;
+}
+
 // Adjoint of one sweep: a wave takes kAdjCells cells of a line along the sweep
 // and three on either side, one a lane, and neighbours exchange in registers.
 // PRIM: primitive-form limiting (a template parameter, so that the
@@ -118,14 +204,16 @@ __global__ void __launch_bounds__(256) chi_pad_kernel(AGrid g, const double* __r
 // all.  In the y sweep a wave's lanes run down a column: its loads touch a
 // line each, which the columns of a workgroup share.
 //
-// chi_g receives the adjoint of every position's flattening factor (indexed as
-// chi_pad; on the lines of the grid), partials the workgroup's sums of the
-// dt/dh and gamma adjoints.
+// rec_k, rec_v and any receive the records of the flattening factors
+// (chi_record) at the positions of the grid's lines, partials the workgroup's
+// sums of the dt/dh and gamma adjoints.
 template <int ND, int D, int FLUX, bool PRIM>
-__global__ void __launch_bounds__(64 * kAdjWaves)
+__global__ void __launch_bounds__(64 * kAdjWaves) __attribute__((amdgpu_waves_per_eu(2)))
 sweep_adj_kernel(AGrid g, const double* __restrict__ lam, double* __restrict__ lam_in,
                  Material<double> m, int limiter, const StepRec* __restrict__ rec,
-                 const double* __restrict__ chi_pad, double* __restrict__ chi_g,
+                 const double* __restrict__ chi_pad, const double* __restrict__ P,
+                 const double* __restrict__ V0, const double* __restrict__ V1,
+                 int* __restrict__ rec_k, double* __restrict__ rec_v, int* __restrict__ any,
                  double* __restrict__ partials) {
   constexpr int S = 2 + ND;
   constexpr int form = PRIM ? kFormPrim : kFormCons;
@@ -243,7 +331,6 @@ sweep_adj_kernel(AGrid g, const double* __restrict__ lam, double* __restrict__ l
 #pragma unroll
     for (int k = 0; k < S; ++k) lam_in[at + k * g.cs] = la[k] + acc[k];
   }
-  if (own || before || after) chi_g[chi_at(j)] = ring && !own ? 0.0 : g_chi;
   double s0 = 0.0, s1 = 0.0;
   if (own || (!ring && before)) {
     s0 += g_dtdh;
@@ -269,108 +356,14 @@ sweep_adj_kernel(AGrid g, const double* __restrict__ lam, double* __restrict__ l
     for (int i = 0; i < kAdjWaves; ++i) v += red[threadIdx.x][i];
     partials[2 * blockIdx.x + threadIdx.x] = v;
   }
-}
-
-// ---- the flattening factor's adjoint ----------------------------------------
-// chi_v of a cell (chi_pad_kernel) is the smallest of the flattening factors
-// K_d(j) of the cell and of its neighbour on the higher-pressure side in each
-// dimension d; where the selected factor is flattened and not clamped,
-// K = 1 - (z - 0.75) / 0.1 with z = |p(j+1) - p(j-1)| / |p(j+2) - p(j-2)|
-// along d carries the gradient (muscl_reconstructor.hpp:59-87); the
-// flattening test, the neighbour and the minimum are branches.
-
-// At each chi position (the grid padded by one cell) whose chi lies strictly
-// between 0 and 1 (elsewhere the selected factor is clamped or not
-// flattened and carries no gradient): the adjoint of chi that the position's
-// face states passed back in sweep dimension D; which factor the minimum
-// selected,
-// rec_k = 4 d + (j - c along d) + 1 for K_d(j) (-1: none); and the adjoints
-// of the pressures at j-2, j-1, j+1, j+2 along d (rec_v, 4 per position).
-// *any is set when some position has a record.
-template <int ND, int D>
-__global__ void __launch_bounds__(256) chi_adj_kernel(AGrid g, const double* __restrict__ P,
-                                                      const double* __restrict__ V0,
-                                                      const double* __restrict__ V1,
-                                                      const double* __restrict__ chi,
-                                                      const double* __restrict__ chi_g,
-                                                      int* __restrict__ rec_k,
-                                                      double* __restrict__ rec_v,
-                                                      int* __restrict__ any) {
-  const int64_t px = g.nx + 8;
-  const int64_t cx = g.nx + 2, cy = ND > 1 ? g.ny + 2 : 1;
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= cx * cy) return;
-  const int64_t x = q % cx - 1, y = ND > 1 ? q / cx - 1 : 0;
-  const double cv = chi[q];
-  double G = 0.0;
-  if (cv > 0.0 && cv < 1.0) {
-    const int64_t lines = D == 0 ? g.ny : g.nx;
-    const int64_t line = D == 0 ? y : x;  // faces exist on interior lines only
-    if (line >= 0 && line < lines) G = chi_g[q];
+  if (own || before || after) {
+    const int64_t q = chi_at(j);
+    const double G = ring && !own ? 0.0 : g_chi;
+    if (chi > 0.0 && chi < 1.0 && G != 0.0)
+      chi_record<ND>(g, P, V0, V1, D == 0 ? j : line, D == 0 ? line : j, q, G, rec_k, rec_v, any);
+    else
+      rec_k[q] = -1;
   }
-  auto at = [&](const double* A, int64_t xx, int64_t yy) {
-    return A[(ND > 1 ? (yy + 4) * px : 0) + xx + 4];
-  };
-  const Material<double> no_shift{};
-  auto chi_d = [&](int64_t xx, int64_t yy, int d) {
-    const int64_t dx = (d == 0), dy = (d == 1);
-    const double* V = d == 0 ? V0 : V1;
-    return chi_factor<double>(at(P, xx - 2 * dx, yy - 2 * dy), at(P, xx - dx, yy - dy),
-                              at(P, xx + dx, yy + dy), at(P, xx + 2 * dx, yy + 2 * dy),
-                              at(V, xx - dx, yy - dy), at(V, xx + dx, yy + dy), no_shift);
-  };
-  int best = -1;
-  if (G != 0.0) {
-    // the selection of chi_pad_kernel: smin(chi, smin(K(c), K(c + s)))
-    double c = DBL_MAX;
-    for (int d = 0; d < ND; ++d) {
-      const int64_t dx = (d == 0), dy = (d == 1);
-      const int sign = signum(at(P, x + dx, y + dy) - at(P, x - dx, y - dy));
-      const double k0 = chi_d(x, y, d);
-      const double k1 = chi_d(x + sign * dx, y + sign * dy, d);
-      double mv = k0;
-      int sel = 4 * d + 1;
-      if (k1 < k0) {
-        mv = k1;
-        sel = 4 * d + sign + 1;
-      }
-      if (mv < c) {
-        c = mv;
-        best = sel;
-      }
-    }
-  }
-  if (best >= 0) {
-    const int d = best / 4, jo = best % 4 - 1;
-    const int64_t dx = (d == 0), dy = (d == 1);
-    const int64_t jx = x + jo * dx, jy = y + jo * dy;
-    const double* V = d == 0 ? V0 : V1;
-    const double p_pp = at(P, jx - 2 * dx, jy - 2 * dy), p_p = at(P, jx - dx, jy - dy);
-    const double p_n = at(P, jx + dx, jy + dy), p_nn = at(P, jx + 2 * dx, jy + 2 * dy);
-    const double u_factor = at(V, jx - dx, jy - dy) - at(V, jx + dx, jy + dy);
-    const double dp = fabs(p_n - p_p);
-    const double pmin = smin(p_n, p_p);
-    const bool flatten = u_factor > 0.0 && dv(dp, pmin) > 0.33;
-    const double den = fabs(p_nn - p_pp);
-    if (flatten && den > 0.0) {
-      const double z = dv(dp, den);
-      const double temp = 1.0 - dv(z - 0.75, 0.85 - 0.75);
-      if (temp > 0.0 && temp < 1.0) {
-        const double g_z = -G / (0.85 - 0.75);
-        const double g_dp = g_z / den;
-        const double g_den = -g_z * z / den;
-        const double sn = (double)signum(p_n - p_p), snn = (double)signum(p_nn - p_pp);
-        rec_v[4 * q + 0] = -g_den * snn;  // p(j-2)
-        rec_v[4 * q + 1] = -g_dp * sn;    // p(j-1)
-        rec_v[4 * q + 2] = g_dp * sn;     // p(j+1)
-        rec_v[4 * q + 3] = g_den * snn;   // p(j+2)
-        rec_k[q] = best;
-        *any = 1;
-        return;
-      }
-    }
-  }
-  rec_k[q] = -1;
 }
 
 // Positions within 4 ghost cells of a line of n cells whose ghost rule maps
@@ -402,7 +395,7 @@ __device__ __forceinline__ int alias_positions(int64_t x, int64_t n, int bc, int
 // kPartialBlocks workgroups of 256 threads stride over the cells, so the sums
 // have a fixed order; with no record at all (*any == 0) they only write
 // zeros.
-template <int ND>
+template <int ND, int D>
 __global__ void __launch_bounds__(256) chi_gather_kernel(AGrid g, Material<double> m,
                                                          const int* __restrict__ rec_k,
                                                          const double* __restrict__ rec_v,
@@ -429,7 +422,9 @@ __global__ void __launch_bounds__(256) chi_gather_kernel(AGrid g, Material<doubl
             // pressure at c + jo + k, k in {-2, -1, 1, 2}: here t = jo + k
             for (int t = -3; t <= 3; ++t) {
               const int64_t qx = ax[a] - t * dx, qy = ay[b] - t * dy;
-              if (qx < -1 || qx > g.nx || (ND > 1 && (qy < -1 || qy > g.ny))) continue;
+              // records lie on the grid's lines along D, and a cell past their ends
+              if (D == 0 ? qx < -1 || qx > g.nx : qx < 0 || qx >= g.nx) continue;
+              if (ND > 1 && (D == 1 ? qy < -1 || qy > g.ny : qy < 0 || qy >= g.ny)) continue;
               const int64_t qc = (ND > 1 ? (qy + 1) * cx : 0) + qx + 1;
               const int r = rec_k[qc];
               if (r < 0 || r / 4 != d) continue;
@@ -560,15 +555,14 @@ __global__ void acc_clear_kernel(double* acc) {
 #define FL_SWEEP_INST(ND, D, FLUX, PRIM)                                                     \
   template __global__ void sweep_adj_kernel<ND, D, FLUX, PRIM>(                               \
       AGrid, const double*, double*, Material<double>, int, const StepRec*, const double*,     \
-      double*, double*);
+      const double*, const double*, const double*, int*, double*, int*, double*);
 #define FL_ADJ_INST(ND, D)                                                                  \
   FL_SWEEP_INST(ND, D, kFluxHllc, false)                                                     \
   FL_SWEEP_INST(ND, D, kFluxForce, false)                                                    \
   FL_SWEEP_INST(ND, D, kFluxHllc, true)                                                      \
   FL_SWEEP_INST(ND, D, kFluxForce, true)                                                     \
-  template __global__ void chi_adj_kernel<ND, D>(AGrid, const double*, const double*,         \
-                                                 const double*, const double*, const double*, \
-                                                 int*, double*, int*);
+  template __global__ void chi_gather_kernel<ND, D>(AGrid, Material<double>, const int*,      \
+                                                    const double*, const int*, double*, double*);
 
 FL_ADJ_INST(1, 0)
 FL_ADJ_INST(2, 0)
@@ -579,10 +573,6 @@ template __global__ void chi_pad_kernel<1>(AGrid, const double*, const double*, 
                                            double*, int*);
 template __global__ void chi_pad_kernel<2>(AGrid, const double*, const double*, const double*,
                                            double*, int*);
-template __global__ void chi_gather_kernel<1>(AGrid, Material<double>, const int*, const double*,
-                                              const int*, double*, double*);
-template __global__ void chi_gather_kernel<2>(AGrid, Material<double>, const int*, const double*,
-                                              const int*, double*, double*);
 template __global__ void record_kernel<1>(AGrid, Material<double>, const SimCtl*, int, StepRec*);
 template __global__ void record_kernel<2>(AGrid, Material<double>, const SimCtl*, int, StepRec*);
 template __global__ void finalize_kernel<1>(AGrid, Material<double>, const StepRec*,

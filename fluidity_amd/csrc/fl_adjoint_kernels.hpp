@@ -47,12 +47,9 @@ __global__ void chi_pad_kernel(AGrid g, const double* P, const double* V0, const
 template <int ND, int D, int FLUX, bool PRIM>
 __global__ void sweep_adj_kernel(AGrid g, const double* lam, double* lam_in, Material<double> m,
                                  int limiter, const StepRec* rec, const double* chi_pad,
-                                 double* chi_g, double* partials);
+                                 const double* P, const double* V0, const double* V1, int* rec_k,
+                                 double* rec_v, int* any, double* partials);
 template <int ND, int D>
-__global__ void chi_adj_kernel(AGrid g, const double* P, const double* V0, const double* V1,
-                               const double* chi, const double* chi_g, int* rec_k,
-                               double* rec_v, int* any);
-template <int ND>
 __global__ void chi_gather_kernel(AGrid g, Material<double> m, const int* rec_k,
                                   const double* rec_v, const int* any, double* lam,
                                   double* partials);
