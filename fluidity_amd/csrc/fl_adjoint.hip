@@ -195,13 +195,14 @@ __device__ void chi_record(const AGrid& g, const double* __restrict__ P,
 // PRIM: primitive-form limiting (a template parameter, so that the
 // conservative-form kernel carries none of its code).
 //
-// FP64 arithmetic and its latency at two waves a SIMD bound it (240 registers;
-// a 512^2 sweep at three a SIMD 25 us in x and 31 in y, at four, with spills, 38
-// and 44; workgroups of 8 waves 30 and 36, whose last round is a quarter full).
+// FP64 arithmetic and its latency at two waves a SIMD bound it (182 registers
+// and more; a 512^2 sweep at three a SIMD 26 us in x and 32 in y, at four, with
+// spills, 38 and 44; workgroups of 8 waves 30 and 36, whose last round is a
+// quarter full).
 // With a thread per face, which evolved both cells beside it forward and back
 // and passed its 16 contributions through memory to a kernel that gathered
-// them, it took 33 us, the gather 9 and the sums 5; now 24 us (x) and 29 (y) in
-// all.  In the y sweep a wave's lanes run down a column: its loads touch a
+// them, it took 33 us, the gather 9, the sums 5 and the flattening factors'
+// records 4; now 25 us (x) and 29 (y) in all.  In the y sweep a wave's lanes run down a column: its loads touch a
 // line each, which the columns of a workgroup share.
 //
 // rec_k, rec_v and any receive the records of the flattening factors
