@@ -9,9 +9,11 @@
 // phase 1 runs the y sweep of every 2D problem.  Problems of very different
 // sizes share a phase's list of tiles, largest problems first: cell-parallel
 // tiles, one per workgroup, or marching tiles, which persistent workgroups
-// take from a counter.  1D problems run register tiles in either.  Tile bodies are those of the
-// single-grid sweeps (fl_sweep_tiles.hpp), so every problem's result is the
-// single-grid result bit for bit.
+// take from a counter.  1D problems run register tiles (one segment a wave)
+// beside the first and marching ones (eight segments in turn) beside the
+// second.  Tile bodies are those of the single-grid sweeps
+// (fl_sweep_tiles.hpp), so every problem's result is the single-grid result
+// bit for bit.
 #include "fl_batch.hpp"
 #include "fl_sweep_tiles.hpp"
 
@@ -109,7 +111,8 @@ phase_kernel(const Prob<T>* __restrict__ probs, const Tile* __restrict__ tiles, 
     if (PHASE == 1)
       sweep_y_tile<T, FLUX, FAST, VLC, WIDE>(phase_args<T, 2, 1>(P, timing, timing_dtdh), td.bx, td.by);
     else if (P.nd == 1)
-      line_tile<T, FLUX, FAST, VLC>(phase_args<T, 1, 0>(P, timing, timing_dtdh), td.bx);
+      sweep_x_tile<T, 1, FLUX, FAST, VLC, false>(phase_args<T, 1, 0>(P, timing, timing_dtdh),
+                                                 td.bx, 0);
     else
       sweep_x_tile<T, 2, FLUX, FAST, VLC, WIDE>(phase_args<T, 2, 0>(P, timing, timing_dtdh), td.bx,
                                           td.by);
