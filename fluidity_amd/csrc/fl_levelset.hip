@@ -584,7 +584,7 @@ struct EikTile {
 // Sources (fast_iterative_init, scheme/cuda/fast_iterative_method.cuh:48-85):
 // a cell beside a sign change with the smaller |phi|; distance |phi| there.
 // info = source | (signum(phi) + 1) << 1.  Both Jacobi buffers start equal.
-// src[t] = tile t holds a source; the control words are cleared.  Launched on
+// tile[t] = whether tile t holds a source; the control words are cleared.  Launched on
 // (tiles per row, min(tile rows, 65535)) workgroups; tile rows stride by
 // gridDim.y.
 template <int ND>
@@ -619,38 +619,47 @@ __global__ void __launch_bounds__(kEikThreads) eik_init_kernel(EikJobs jobs, Gri
       J.d[1][i] = v;
     }
     const int any = __syncthreads_or(source);
-    if (threadIdx.x == 0) J.src[tr * gridDim.x + blockIdx.x] = (uint8_t)(any != 0);
+    if (threadIdx.x == 0) J.tile[tr * gridDim.x + blockIdx.x] = any ? kEikSource : 0u;
   }
 }
 
-// Tile t is active when some tile within `tr_r` tile rows and `segs_r`
-// tiles of it holds a source; the active tiles are appended to the job's
-// list (one atomicAdd per wave; ctl->ntiles starts at zero).  A cell's
-// distance grows by at least dh/sqrt(2) per axis step from the nearest
-// source (the Godunov update q >= min(a, b) + dh/sqrt(2)), so a cell farther
-// than band * sqrt(2) steps from every source never enters the band and
-// tiles without such cells can be skipped by every sweep.
+// Tile t is active when some tile within `tr_r` tile rows and `segs_r` (each
+// at least 1 where there are neighbours) tiles of it holds a source; the
+// active tiles are appended to the job's list (one atomicAdd per wave;
+// ctl->appended starts at zero).  A cell's distance grows by at least
+// dh/sqrt(2) per axis step from the nearest source (the Godunov update q >=
+// min(a, b) + dh/sqrt(2)), so from sources beside the interface of a distance
+// function no cell farther than band * sqrt(2) steps enters the band and the
+// other tiles are never visited.  Where phi is steep or jumps, a neighbour
+// across the interface enters with a large negated distance and the band
+// reaches farther: the sweeps add the tiles that it runs into.
 __global__ void eik_tile_act_kernel(EikJobs jobs, int64_t trows, int64_t segs, int tr_r,
                                     int segs_r) {
   const int64_t t = gid();
   if (t >= trows * segs) return;
   const EikJob J = eik_job(jobs);
-  const uint8_t* __restrict__ src = J.src;
+  const unsigned* src = J.tile;
   const int64_t y = t / segs, sx = t % segs;
   const int64_t y0 = y - tr_r < 0 ? 0 : y - tr_r, y1 = y + tr_r >= trows ? trows - 1 : y + tr_r;
   const int64_t s0 = sx - segs_r < 0 ? 0 : sx - segs_r;
   const int64_t s1 = sx + segs_r >= segs ? segs - 1 : sx + segs_r;
-  uint8_t a = 0;
+  unsigned a = 0u;
   for (int64_t yy = y0; yy <= y1 && !a; ++yy)
-    for (int64_t ss = s0; ss <= s1; ++ss) a |= src[yy * segs + ss];
+    for (int64_t ss = s0; ss <= s1; ++ss) a |= src[yy * segs + ss] & kEikSource;
   const unsigned long long m = __ballot(a != 0);
   if (!m) return;
   const int lane = (int)(threadIdx.x % 64);
   const int leader = __ffsll((long long)m) - 1;
   int base = 0;
-  if (lane == leader) base = atomicAdd(&J.ctl->ntiles, __popcll(m));
+  if (lane == leader) {
+    atomicAdd(&J.ctl->ntiles[0], __popcll(m));
+    base = atomicAdd(&J.ctl->appended, __popcll(m));
+  }
   base = __shfl(base, leader, 64);
-  if (a) J.list[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)t;
+  if (a) {
+    J.list[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)t;
+    atomicOr(&J.tile[t], kEikActive);
+  }
 }
 
 // Neighbour distance v seen from a cell on the same or the other side: negated
@@ -671,6 +680,11 @@ __device__ __forceinline__ double eik_nbr_v(double v, bool same) {
 // of the tile, so its cells are those of whole sweeps.  A launch reads the
 // job's buffer d[launch & 1] and writes the active tiles of d[(launch + 1) &
 // 1] (the other tiles hold their initial values in both).
+//
+// A cell changes only in the sweep after a neighbour did, so the changes of a
+// launch lie within kEikSteps cells of those of the last sweep of the launch
+// before: where these come that near to a tile's edge, the tile beyond it is on
+// the list from the next launch on.
 //
 // flags[launch % 3][s]: sweep s of the launch changed a cell.  After a sweep
 // that changed nothing no other can, so a launch whose predecessor's last
@@ -693,7 +707,7 @@ __global__ void __launch_bounds__(kEikThreads) eik_sweep_kernel(EikJobs jobs, Gr
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
   // the control words, loaded together ((launch + 2) % 3: the launch before)
   const int done = ctl->done, prev_changed = ctl->flags[(launch + 2) % 3][K - 1];
-  const int ntiles = ctl->ntiles;
+  const int ntiles = ctl->ntiles[launch & 1];
   keep(done);
   keep(prev_changed);
   keep(ntiles);
@@ -705,6 +719,7 @@ __global__ void __launch_bounds__(kEikThreads) eik_sweep_kernel(EikJobs jobs, Gr
   if (first) {
     for (int s = 0; s < K; ++s) ctl->flags[(launch + 1) % 3][s] = 0;
     ctl->launches = launch + 1;
+    atomicMax(&ctl->ntiles[(launch + 1) & 1], ntiles);
   }
   __shared__ double sd[2][Tile::R];
   __shared__ uint8_t si[Tile::R];
@@ -736,7 +751,7 @@ __global__ void __launch_bounds__(kEikThreads) eik_sweep_kernel(EikJobs jobs, Gr
     // per cell: whether it may change, whether it is the tile's, and which of
     // its neighbours lie on its side (bits 0 to 3: x - 1, x + 1, y - 1, y + 1)
     bool moves[P], own[P];
-    int same[P];
+    int same[P], toward = 0;  // edges near a change of the last sweep, as bits of `same`
 #pragma unroll
     for (int n = 0; n < P; ++n) {
       const int c = (int)threadIdx.x + n * kEikThreads;
@@ -778,7 +793,14 @@ __global__ void __launch_bounds__(kEikThreads) eik_sweep_kernel(EikJobs jobs, Gr
           }
           if (q < cur[n] && q <= limit) {
             cur[n] = q;
-            if (own[n]) changed |= 1u << s;
+            if (own[n]) {
+              changed |= 1u << s;
+              if (s == K - 1) {
+                const int rx = c % Tile::RW, ry = c / Tile::RW;
+                toward |= (rx < 2 * K ? 1 : 0) | (rx >= Tile::RW - 2 * K ? 2 : 0);
+                if (ND > 1) toward |= (ry < 2 * K ? 4 : 0) | (ry >= Tile::RH - 2 * K ? 8 : 0);
+              }
+            }
           }
         }
         if (c < Tile::R) to[c] = cur[n];
@@ -788,6 +810,23 @@ __global__ void __launch_bounds__(kEikThreads) eik_sweep_kernel(EikJobs jobs, Gr
 #pragma unroll
     for (int n = 0; n < P; ++n)
       if (own[n]) e[at[n]] = cur[n];
+    if (__any(toward)) {
+      // a neighbour a lane: 3 x 3 tiles, or 3 of a line
+      const int lane = (int)(threadIdx.x % 64), kx = lane % 3 - 1, ky = ND == 1 ? 0 : lane / 3 - 1;
+      const bool lo_x = __any(toward & 1), hi_x = __any(toward & 2);
+      const bool lo_y = __any(toward & 4), hi_y = __any(toward & 8);
+      const int64_t sx = t % segs + kx, sy = ND == 1 ? 0 : t / segs + ky;
+      if (lane < (ND == 1 ? 3 : 9) && (kx == 0 || (kx < 0 ? lo_x : hi_x)) &&
+          (ky == 0 || (ky < 0 ? lo_y : hi_y)) && sx >= 0 && sx < segs && sy >= 0 &&
+          sy < (ND == 1 ? 1 : (g.ny + Tile::H - 1) / Tile::H)) {
+        unsigned* const word = &J.tile[sy * segs + sx];
+        if (!(*word & kEikActive) && !(atomicOr(word, kEikActive) & kEikActive)) {
+          const int at_end = atomicAdd(&ctl->appended, 1);
+          J.list[at_end] = (int)(sy * segs + sx);
+          atomicMax(&ctl->ntiles[(launch + 1) & 1], at_end + 1);
+        }
+      }
+    }
   }
   __syncthreads();
   if (changed) atomicOr(&s_changed, changed);

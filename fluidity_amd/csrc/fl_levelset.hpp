@@ -34,12 +34,16 @@ constexpr int kEikThreads = 512;
 constexpr int eik_tile_w(int nd) { return nd == 1 ? kEikThreads : 32; }
 constexpr int eik_tile_h(int nd) { return kEikThreads / eik_tile_w(nd); }
 
+// Bits of a tile: it holds a source; it is on the list.
+constexpr unsigned kEikSource = 1u, kEikActive = 2u;
+
 // Control words of the eikonal Jacobi loop.
 struct EikCtl {
   int flags[3][kEikSteps];  // by launch % 3: sweep s of the launch changed a cell
   int done;
-  int launches;  // launches that swept
-  int ntiles;    // entries of the job's active-tile list
+  int launches;   // launches that swept
+  int appended;   // entries of the job's active-tile list
+  int ntiles[2];  // those that a launch visits, by launch & 1
 };
 
 // One eikonal reinitialisation: the level set in, its two Jacobi distance
@@ -49,8 +53,8 @@ struct EikJob {
   const double* phi;
   double* d[2];
   uint8_t* info;
-  uint8_t* src;   // per tile: holds a source
-  int* list;      // the tiles a sweep visits, in no particular order
+  unsigned* tile;  // per tile: kEikSource | kEikActive
+  int* list;       // the tiles a sweep visits, in no particular order
   EikCtl* ctl;
   double* out;
   uint8_t* band_mask;  // nullable

@@ -197,12 +197,12 @@ int64_t eik_trows(const ls::Grid& g) {
   return (g.ny + ls::eik_tile_h(g.nd) - 1) / ls::eik_tile_h(g.nd);
 }
 
-// Two distance buffers, the per-cell info bytes, the per-tile source flags
-// and the active-tile list.
+// Two distance buffers, the per-cell info bytes, the tiles' bits and the
+// active-tile list.
 int64_t reinit_work_bytes(const ls::Grid& g) {
   const int64_t cells = g.nx * g.ny;
   const int64_t tiles = eik_segs(g) * eik_trows(g);
-  return 2 * align256(cells * 8) + align256(cells) + align256(tiles) + align256(tiles * 4);
+  return 2 * align256(cells * 8) + align256(cells) + 2 * align256(tiles * 4);
 }
 
 // One reinitialisation job: phi in, out (and the nullable band mask) out,
@@ -217,8 +217,8 @@ ls::EikJob eik_job(const double* phi, const ls::Grid& g, double* out, uint8_t* b
   j.d[0] = (double*)w;
   j.d[1] = (double*)(w + align256(cells * 8));
   j.info = (uint8_t*)(w + 2 * align256(cells * 8));
-  j.src = j.info + align256(cells);
-  j.list = (int*)(j.src + align256(tiles));
+  j.tile = (unsigned*)(j.info + align256(cells));
+  j.list = (int*)((char*)j.tile + align256(tiles * 4));
   j.ctl = ctl;
   j.out = out;
   j.band_mask = band_mask;
@@ -243,7 +243,9 @@ int run_reinit(fl_context* c, const ls::EikJobs& jobs, int njobs, const ls::Grid
                    njobs);
   dim3 agrid = grid_for(tiles);
   agrid.z = njobs;
-  // cells within which a source can pull a cell into the band, in tiles
+  // cells within which a source whose distance is at most dh pulls a cell into
+  // the band, in tiles (at least one: the sweeps themselves add what a larger
+  // distance, negated across the interface, reaches)
   const int reach = (int)ceil(band * sqrt(2.0)) + 2;
   const int tw = ls::eik_tile_w(g.nd), th = ls::eik_tile_h(g.nd);
   const int segs_r = (reach + tw - 1) / tw;
