@@ -8,6 +8,7 @@
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -35,20 +36,43 @@ int fail(int status, const char* fmt, ...) {
 
 bool valid_block(int b) { return b >= 64 && b <= fl::kMaxBlock && (b % 64) == 0; }
 
-int resolve_tuning(const fl_tuning* t, fl_tuning* out, int32_t* shape) {
-  fl_tuning n;
-  if (t && (t->x_block || t->x_rows)) shape[0] = kShapeTuning;
-  if (t && (t->y_block || t->y_rows)) shape[1] = kShapeTuning;
-  n.x_block = t && t->x_block ? t->x_block : 256;
-  n.x_rows = t && t->x_rows ? t->x_rows : 32;
-  n.y_block = t && t->y_block ? t->y_block : 256;
-  n.y_rows = t && t->y_rows ? t->y_rows : 64;
-  if (!valid_block(n.x_block) || !valid_block(n.y_block))
-    return fail(FL_ERR_ARGUMENT, "block widths must be multiples of 64 in [64, %d]", fl::kMaxBlock);
-  if (n.x_rows < 1 || n.x_rows > 4096 || n.y_rows < 1 || n.y_rows > 4096)
-    return fail(FL_ERR_ARGUMENT, "rows per workgroup must be in [1, 4096]");
-  *out = n;
+int take_tuning(const fl_tuning* t, fl_tuning* tuning, int32_t* shape) {
+  const int32_t block[2] = {t->x_block, t->y_block}, rows[2] = {t->x_rows, t->y_rows};
+  int32_t* const block_out[2] = {&tuning->x_block, &tuning->y_block};
+  int32_t* const rows_out[2] = {&tuning->x_rows, &tuning->y_rows};
+  for (int d = 0; d < 2; ++d) {
+    if (block[d] && !valid_block(block[d]))
+      return fail(FL_ERR_ARGUMENT, "block widths must be multiples of 64 in [64, %d]",
+                  fl::kMaxBlock);
+    if (rows[d] != FL_ROWS_RULE && (rows[d] < -4096 || rows[d] > 4096))
+      return fail(FL_ERR_ARGUMENT, "rows per workgroup must be in [1, 4096]");
+  }
+  for (int d = 0; d < 2; ++d) {
+    if (block[d]) *block_out[d] = block[d];
+    if (rows[d] == FL_ROWS_RULE) {
+      shape[d] = kShapeRule;
+    } else if (block[d] || rows[d]) {
+      shape[d] = rows[d] < 0 ? kShapeCell : kShapeTuning;
+      if (rows[d]) *rows_out[d] = abs(rows[d]);
+    }
+  }
   return FL_OK;
+}
+
+int resolve_tuning(const fl_tuning* t, fl_tuning* out, int32_t* shape) {
+  *out = {256, 32, 256, 64};
+  shape[0] = shape[1] = kShapeRule;
+  return t ? take_tuning(t, out, shape) : FL_OK;
+}
+
+fl_tuning tuning_of(const fl_tuning& tuning, const int32_t* shape) {
+  fl_tuning t = tuning;
+  int32_t* const rows[2] = {&t.x_rows, &t.y_rows};
+  for (int d = 0; d < 2; ++d) {
+    if (shape[d] == kShapeRule) *rows[d] = FL_ROWS_RULE;
+    if (shape[d] == kShapeCell) *rows[d] = -*rows[d];
+  }
+  return t;
 }
 
 int check_field(const fl_field* f, const char* name) {
@@ -808,23 +832,12 @@ int fl_ctx_destroy(fl_context* c) {
 
 int fl_ctx_set_tuning(fl_context* c, const fl_tuning* t) {
   if (!c || !t) return fail(FL_ERR_ARGUMENT, "NULL context or tuning");
-  fl_tuning n = c->tuning;
-  if (t->x_block) n.x_block = t->x_block;
-  if (t->x_rows) n.x_rows = t->x_rows;
-  if (t->y_block) n.y_block = t->y_block;
-  if (t->y_rows) n.y_rows = t->y_rows;
-  int32_t unused[2];
-  int rc = resolve_tuning(&n, &n, unused);
-  if (rc) return rc;
-  c->tuning = n;
-  if (t->x_block || t->x_rows) c->shape[0] = kShapeTuning;
-  if (t->y_block || t->y_rows) c->shape[1] = kShapeTuning;
-  return FL_OK;
+  return take_tuning(t, &c->tuning, c->shape);
 }
 
 int fl_ctx_get_tuning(const fl_context* c, fl_tuning* t) {
   if (!c || !t) return fail(FL_ERR_ARGUMENT, "NULL context or tuning");
-  *t = c->tuning;
+  *t = tuning_of(c->tuning, c->shape);
   return FL_OK;
 }
 
@@ -911,7 +924,7 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
   c->tuning = rc ? saved : best;
   if (rc)
     for (int d = 0; d < 2; ++d) c->shape[d] = saved_shape[d];
-  if (!rc && chosen) *chosen = best;
+  if (!rc && chosen) *chosen = tuning_of(c->tuning, c->shape);
   return rc;
 }
 

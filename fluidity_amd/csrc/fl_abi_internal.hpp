@@ -33,7 +33,7 @@ struct SimGraphKey {
 
 // Where the launch shape of a 2D sweep (x, y) comes from: the built-in rule
 // on the grid, the march heights and widths in `tuning`, or the cell-parallel
-// kernel (the autotuner's choice).
+// kernel (the rows of a caller's or the autotuner's tuning say which).
 enum : int { kShapeRule = 0, kShapeTuning = 1, kShapeCell = 2 };
 
 struct fl_context {
@@ -113,10 +113,14 @@ inline int wide_cells(const fl::SweepArgs<T>& a) {
 }
 
 double bits_to_double(unsigned long long b);
-// `t` (nullable: all defaults) with zeros replaced by the built-in launch
-// shapes, validated, into *out; shape[d] becomes kShapeTuning where t names a
-// width or height of that sweep.
+// Validates `t` and sets the march heights and widths in *tuning and the
+// source of each sweep's shape that it names; a sweep with zeros only keeps
+// what it has.
+int take_tuning(const fl_tuning* t, fl_tuning* tuning, int32_t* shape);
+// The built-in launch shapes, and on them `t` (nullable).
 int resolve_tuning(const fl_tuning* t, fl_tuning* out, int32_t* shape);
+// The fl_tuning that take_tuning makes these of.
+fl_tuning tuning_of(const fl_tuning& tuning, const int32_t* shape);
 int check_pair(const fl_field* in, const fl_field* out);
 int check_field(const fl_field* f, const char* name);
 int check_scheme(const fl_scheme* s, int ndim);

@@ -53,8 +53,6 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // there made a step of 512 problems 1231 -> 1476 us.
 constexpr int kSegments1D = 8;
 
-bool valid_width(int b) { return b >= 64 && b <= fl::kMaxBlock && (b % 64) == 0; }
-
 // Height of the x or y tiles of a 2D problem with ny rows: the tuning's base
 // height, doubled (up to 8x) while the problem still gives at least
 // kMinRowTiles tiles per column band.  Tall problems pay the warm-up rows of
@@ -180,18 +178,19 @@ const void* phase_kernel_ptr(const fl_batch* b, int phase) {
 // tall.  The two lines cross at 19M cells in FP64, 17M in FP32.
 constexpr int64_t kBatchCellMax = 1 << 24;
 
-// Launch shapes of a batch that was not tuned.
-fl_tuning rule_shape(fl_batch* b) {
+// The rule: whether a batch that was not tuned runs cell-parallel tiles.
+bool cell_by_rule(const fl_batch* b) {
   int64_t cells = 0;
   for (const fl_batch_problem& q : b->problems)
     if (q.state.ndim > 1) cells += q.state.n[0] * q.state.n[1];
-  b->cell[0] = b->cell[1] = cells <= kBatchCellMax;
-  fl_tuning t;
-  t.x_block = 256;
-  t.x_rows = 32;
-  t.y_block = 256;
-  t.y_rows = 64;
-  return t;
+  return cells <= kBatchCellMax;
+}
+
+// What the batch runs, as a caller's tuning.
+fl_tuning batch_tuning(const fl_batch* b) {
+  const int32_t shape[2] = {b->cell[0] ? kShapeCell : kShapeTuning,
+                            b->cell[1] ? kShapeCell : kShapeTuning};
+  return tuning_of(b->tuning, shape);
 }
 
 // Uploads the problem table and tile lists of tuning t; sizes the persistent
@@ -446,7 +445,8 @@ int fl_batch_create(fl_context* c, const fl_batch_problem* problems, int nprob, 
     hp[p].sim_time = problems[p].params.sim_time;
     hp[p].max_iters = problems[p].params.max_iters;
   }
-  const fl_tuning t = rule_shape(b);
+  const fl_tuning t = {256, 32, 256, 64};
+  b->cell[0] = b->cell[1] = cell_by_rule(b);
   int rc = FL_OK;
   e = hipMemcpy(b->params, hp.data(), sizeof(bt::Params) * nprob, hipMemcpyHostToDevice);
   if (e != hipSuccess) rc = fail(FL_ERR_HIP, "hipMemcpy failed: %s", hipGetErrorString(e));
@@ -472,23 +472,19 @@ int fl_batch_destroy(fl_batch* b) {
 int fl_batch_set_tuning(fl_batch* b, const fl_tuning* t) {
   if (!b || !t) return fail(FL_ERR_ARGUMENT, "NULL batch or tuning");
   fl_tuning n = b->tuning;
-  if (t->x_block) n.x_block = t->x_block;
-  if (t->x_rows) n.x_rows = t->x_rows;
-  if (t->y_block) n.y_block = t->y_block;
-  if (t->y_rows) n.y_rows = t->y_rows;
-  if (!valid_width(n.x_block) || !valid_width(n.y_block))
-    return fail(FL_ERR_ARGUMENT, "block widths must be multiples of 64 in [64, %d]", fl::kMaxBlock);
-  if (n.x_rows < 1 || n.x_rows > 4096 || n.y_rows < 1 || n.y_rows > 4096)
-    return fail(FL_ERR_ARGUMENT, "rows per tile must be in [1, 4096]");
+  int32_t shape[2] = {kShapeTuning, kShapeTuning};
+  const int rc = take_tuning(t, &n, shape);
+  if (rc) return rc;
   DeviceGuard g(b->device);
   FL_HIP(hipDeviceSynchronize());  // tables in use by queued steps
-  b->cell[0] = b->cell[1] = false;
+  for (int ph = 0; ph < 2; ++ph)
+    b->cell[ph] = shape[ph] == kShapeCell || (shape[ph] == kShapeRule && cell_by_rule(b));
   return apply_tuning(b, n);
 }
 
 int fl_batch_get_tuning(const fl_batch* b, fl_tuning* t) {
   if (!b || !t) return fail(FL_ERR_ARGUMENT, "NULL batch or tuning");
-  *t = b->tuning;
+  *t = batch_tuning(b);
   return FL_OK;
 }
 
@@ -556,7 +552,7 @@ int fl_batch_autotune(fl_batch* b, int reps, fl_tuning* chosen, void* stream) {
   (void)hipEventDestroy(e1);
   if (!rc) rc = apply_tuning(b, best);
   if (!rc) launch_finish(b, st, 1);
-  if (!rc && chosen) *chosen = best;
+  if (!rc && chosen) *chosen = batch_tuning(b);
   return rc;
 }
 

@@ -24,6 +24,7 @@ FL_FLUX_HLLC, FL_FLUX_FORCE, FL_FLUX_LAX_FRIEDRICHS, FL_FLUX_RICHTMYER = 0, 1, 2
 FL_EOS_IDEAL, FL_EOS_STIFF, FL_EOS_STIFF_CORRECTED = 0, 1, 2
 FL_NUMERICS_EXACT, FL_NUMERICS_FAST = 0, 1
 FL_BC_TRANSMISSIVE, FL_BC_REFLECTIVE, FL_BC_PERIODIC = 0, 1, 2
+FL_ROWS_RULE = -65536  # Tuning rows: the kernel by the grid's size (negative: cell-parallel)
 
 EXPORTED = [
     "fl_status_string", "fl_last_error", "fl_version", "fl_ctx_create", "fl_ctx_destroy",

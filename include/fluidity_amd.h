@@ -115,12 +115,18 @@ typedef struct fl_sim_result {
   double  max_wavespeed; /* max wavespeed of the final state */
 } fl_sim_result;
 
-/* Launch geometry; zeros select the built-in defaults. */
+/* Launch geometry; zeros select the built-in defaults, or keep what is set
+ * where something is.  The rows of a sweep say which kernel runs it on a 2D
+ * grid: r in 1..4096 marches r rows per workgroup; -r is the cell-parallel
+ * sweep, which takes a tile at once (the march of r rows where it does not
+ * apply); FL_ROWS_RULE chooses by the grid's size, as a context does before
+ * anything is set.  A block alone means a march. */
+#define FL_ROWS_RULE (-65536)
 typedef struct fl_tuning {
   int32_t x_block;    /* lanes per x-sweep workgroup (64..256, multiple of 64) */
-  int32_t x_rows;     /* rows marched per x-sweep workgroup                   */
+  int32_t x_rows;     /* rows of an x-sweep workgroup                         */
   int32_t y_block;    /* lanes per y-sweep workgroup (64..256, multiple of 64) */
-  int32_t y_rows;     /* rows marched per y-sweep workgroup                   */
+  int32_t y_rows;     /* rows of a y-sweep workgroup                          */
 } fl_tuning;
 
 typedef struct fl_context fl_context;
@@ -136,13 +142,16 @@ const char* fl_version(void);
 int fl_ctx_create(int device, fl_context** ctx);
 int fl_ctx_destroy(fl_context* ctx);
 int fl_ctx_set_tuning(fl_context* ctx, const fl_tuning* tuning);
+/* What is set, as fl_ctx_set_tuning of this or another context and
+ * fl_simulate_noalloc take it. */
 int fl_ctx_get_tuning(const fl_context* ctx, fl_tuning* tuning);
 /* Launch-shape autotuner: times every candidate (block width 64/128/256 x
  * rows per workgroup: 8..128 and the heights that make a launch fill whole
- * rounds of the workgroups the device holds at once) of each sweep on this
- * grid (in -> work, a fixed small dt/dh; `in` is not modified), keeps the
- * fastest in the context and returns it.  Synchronises.  Replaces the fixed
- * thread_sizes()/block_sizes() (solver/split_solver.hpp:117-125). */
+ * rounds of the workgroups the device holds at once; on grids of up to 10
+ * million cells the cell-parallel sweep) of each sweep on this grid (in ->
+ * work, a fixed small dt/dh; `in` is not modified), keeps the fastest in the
+ * context and returns it as fl_ctx_get_tuning does.  Synchronises.  Replaces
+ * the fixed thread_sizes()/block_sizes() (solver/split_solver.hpp:117-125). */
 int fl_ctx_autotune(fl_context* ctx, const fl_field* in, const fl_field* work,
                     const fl_scheme* scheme, int reps, fl_tuning* chosen, void* stream);
 
@@ -303,14 +312,17 @@ typedef struct fl_batch_problem {
 int fl_batch_create(fl_context* ctx, const fl_batch_problem* problems, int nprob,
                     fl_batch** batch, void* stream);
 int fl_batch_destroy(fl_batch* batch);
-/* Marching tiles of the given shapes in the two sweep phases (x_block/x_rows:
- * x tiles of 2D problems, x_block also the width of 1D tiles; y_block/y_rows:
- * y tiles).  Zeros keep the current values.  Without this call a batch of up
- * to 2^24 2D cells runs cell-parallel tiles, and the values are unused. */
+/* Tiles of the two sweep phases: marching tiles of the given shapes
+ * (x_block/x_rows: x tiles of 2D problems, x_block also the width of 1D tiles;
+ * y_block/y_rows: y tiles), or with negative rows cell-parallel tiles, which a
+ * batch of up to 2^24 2D cells has from the start (FL_ROWS_RULE). */
 int fl_batch_set_tuning(fl_batch* batch, const fl_tuning* tuning);
+/* What is set, as fl_batch_set_tuning takes it (negative rows: cell-parallel
+ * tiles). */
 int fl_batch_get_tuning(const fl_batch* batch, fl_tuning* tuning);
 /* Times every candidate tile shape of each phase on this batch (`reps` timed
- * launches each, states untouched) and keeps the fastest.  Synchronises. */
+ * launches each, states untouched), keeps the fastest and returns it as
+ * fl_batch_get_tuning does.  Synchronises. */
 int fl_batch_autotune(fl_batch* batch, int reps, fl_tuning* chosen, void* stream);
 /* Restarts every problem's clock and iteration count from its current state. */
 int fl_batch_reset(fl_batch* batch, void* stream);
