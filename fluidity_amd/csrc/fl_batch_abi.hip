@@ -472,8 +472,9 @@ int fl_batch_destroy(fl_batch* b) {
 int fl_batch_set_tuning(fl_batch* b, const fl_tuning* t) {
   if (!b || !t) return fail(FL_ERR_ARGUMENT, "NULL batch or tuning");
   fl_tuning n = b->tuning;
-  int32_t shape[2] = {kShapeTuning, kShapeTuning};
-  const int rc = take_tuning(t, &n, shape);
+  int32_t shape[2] = {b->cell[0] ? kShapeCell : kShapeTuning,
+                      b->cell[1] ? kShapeCell : kShapeTuning};
+  const int rc = take_tuning(t, &n, shape);  // a phase with zeros only keeps its tiles
   if (rc) return rc;
   DeviceGuard g(b->device);
   FL_HIP(hipDeviceSynchronize());  // tables in use by queued steps

@@ -107,3 +107,21 @@ def test_batch_tuning_round_trip():
     c = batch()
     _set(c, t)
     assert _tuple(c.get_tuning()) == _tuple(t)
+
+
+def test_batch_zeros_keep_each_phase():
+    """All zeros, or the values of one phase alone, leave the tiles of the
+    phases they do not name as they are."""
+    from fluidity_amd import batch as B
+    from fluidity_amd import euler as E
+    b = B.Batch([{"U": _grid((40, 60)), "scheme": E.Scheme(), "cfl": 0.8, "dh": 1.0 / 60}], layout=1)
+    fresh = _tuple(b.get_tuning())
+    assert fresh[1] < 0 and fresh[3] < 0
+    b.set_tuning()
+    assert _tuple(b.get_tuning()) == fresh
+    b.set_tuning(x_block=64, x_rows=8)
+    assert _tuple(b.get_tuning()) == (64, 8) + fresh[2:]
+    b.set_tuning(y_block=64, y_rows=16)
+    assert _tuple(b.get_tuning()) == (64, 8, 64, 16)
+    b.set_tuning()
+    assert _tuple(b.get_tuning()) == (64, 8, 64, 16)
