@@ -34,6 +34,7 @@ struct fl_batch {
   double* host_sums;         // pinned mirror
   fl_tuning tuning;
   bool cell[2];              // per phase: cell-parallel tiles (tuning unused)
+  bool tables_ok;            // the device tables are those of tuning and cell
   int grid[2];               // workgroups per phase
   hipStream_t cap_stream;    // stream used to capture the step graph
   hipGraph_t graph;
@@ -193,9 +194,10 @@ fl_tuning batch_tuning(const fl_batch* b) {
   return tuning_of(b->tuning, shape);
 }
 
-// Uploads the problem table and tile lists of tuning t; sizes the persistent
-// grids.  Synchronous (the host vectors are staging).
-int apply_tuning(fl_batch* b, const fl_tuning& t) {
+// Uploads the problem table and tile lists of tuning t and the phases' kinds
+// in b->cell; sizes the persistent grids.  Synchronous (the host vectors are
+// staging).
+int upload_tables(fl_batch* b, const fl_tuning& t) {
   std::vector<bt::Tile> t0, t1;
   build_tiles(b, t, t0, t1);
   if ((int64_t)t0.size() > b->cap[0] || (int64_t)t1.size() > b->cap[1])
@@ -231,8 +233,23 @@ int apply_tuning(fl_batch* b, const fl_tuning& t) {
     if (per_cu < 1) per_cu = 1;
     b->grid[ph] = per_cu * prop.multiProcessorCount;
   }
-  b->tuning = t;
+  return FL_OK;
+}
+
+// Tuning t and the phases' kinds `cell` for the steps that follow.  After an
+// error the batch keeps what it had, and the next step uploads that again.
+int apply_tuning(fl_batch* b, const fl_tuning& t, const bool cell[2]) {
+  const bool had[2] = {b->cell[0], b->cell[1]};
   b->graph_ok = false;
+  b->tables_ok = false;
+  for (int ph = 0; ph < 2; ++ph) b->cell[ph] = cell[ph];
+  const int rc = upload_tables(b, t);
+  if (rc) {
+    for (int ph = 0; ph < 2; ++ph) b->cell[ph] = had[ph];
+    return rc;
+  }
+  b->tuning = t;
+  b->tables_ok = true;
   return FL_OK;
 }
 
@@ -446,11 +463,11 @@ int fl_batch_create(fl_context* c, const fl_batch_problem* problems, int nprob, 
     hp[p].max_iters = problems[p].params.max_iters;
   }
   const fl_tuning t = {256, 32, 256, 64};
-  b->cell[0] = b->cell[1] = cell_by_rule(b);
+  const bool cell[2] = {cell_by_rule(b), cell_by_rule(b)};
   int rc = FL_OK;
   e = hipMemcpy(b->params, hp.data(), sizeof(bt::Params) * nprob, hipMemcpyHostToDevice);
   if (e != hipSuccess) rc = fail(FL_ERR_HIP, "hipMemcpy failed: %s", hipGetErrorString(e));
-  if (!rc) rc = apply_tuning(b, t);
+  if (!rc) rc = apply_tuning(b, t, cell);
   if (!rc) rc = reset(b, (hipStream_t)stream);
   if (rc) {
     release(b);
@@ -478,9 +495,10 @@ int fl_batch_set_tuning(fl_batch* b, const fl_tuning* t) {
   if (rc) return rc;
   DeviceGuard g(b->device);
   FL_HIP(hipDeviceSynchronize());  // tables in use by queued steps
+  bool cell[2];
   for (int ph = 0; ph < 2; ++ph)
-    b->cell[ph] = shape[ph] == kShapeCell || (shape[ph] == kShapeRule && cell_by_rule(b));
-  return apply_tuning(b, n);
+    cell[ph] = shape[ph] == kShapeCell || (shape[ph] == kShapeRule && cell_by_rule(b));
+  return apply_tuning(b, n, cell);
 }
 
 int fl_batch_get_tuning(const fl_batch* b, fl_tuning* t) {
@@ -500,34 +518,38 @@ int fl_batch_autotune(fl_batch* b, int reps, fl_tuning* chosen, void* stream) {
   if (reps < 1 || reps > 100) return fail(FL_ERR_ARGUMENT, "reps %d out of [1, 100]", reps);
   DeviceGuard g(b->device);
   hipStream_t st = (hipStream_t)stream;
-  // The timing launches use the work buffers as output: move 1D results that
-  // live there into the state buffers first and back afterwards.
-  launch_finish(b, st, 0);
-  FL_HIP(hipStreamSynchronize(st));  // the tables are rewritten below
   static const int widths[] = {64, 128, 256};
   static const int xrows[] = {4, 8, 16, 32, 64};
   static const int yrows[] = {16, 32, 64, 128};
-  hipEvent_t e0, e1;
+  hipEvent_t e0, e1 = nullptr;
   FL_HIP(hipEventCreate(&e0));
-  FL_HIP(hipEventCreate(&e1));
-  const double dtdh = 1e-3;
-  fl_tuning best = b->tuning;
   int rc = FL_OK;
+  if (hipEventCreate(&e1) != hipSuccess) rc = fail(FL_ERR_HIP, "hipEventCreate");
+  // The timing launches use the work buffers as output: move 1D results that
+  // live there into the state buffers first and back afterwards.
+  launch_finish(b, st, 0);
+  if (!rc && hipStreamSynchronize(st) != hipSuccess)  // the tables are rewritten below
+    rc = fail(FL_ERR_HIP, "hipStreamSynchronize");
+  const double dtdh = 1e-3;
+  const fl_tuning saved = b->tuning;
+  const bool saved_cell[2] = {b->cell[0], b->cell[1]};
+  fl_tuning best = b->tuning;
+  bool best_cell[2] = {b->cell[0], b->cell[1]};
   for (int ph = 0; ph < 2 && !rc; ++ph) {
     float best_ms = 1e30f;
-    bool best_cell = false;
     for (int w : widths) {
       const int* rows = ph ? yrows : xrows;
       const int nr = ph ? 4 : 5;
       // k = -1, once: the cell-parallel tiles
       for (int k = w == widths[0] ? -1 : 0; k < nr && !rc; ++k) {
         fl_tuning t = best;
-        b->cell[ph] = k < 0;
+        bool cell[2] = {best_cell[0], best_cell[1]};
+        cell[ph] = k < 0;
         if (k >= 0) {
           (ph ? t.y_block : t.x_block) = w;
           (ph ? t.y_rows : t.x_rows) = rows[k];
         }
-        if ((rc = apply_tuning(b, t))) break;
+        if ((rc = apply_tuning(b, t, cell))) break;
         if (b->ntiles[ph] == 0) break;
         float total = 0.0f;
         for (int r = 0; r <= reps && !rc; ++r) {  // r = 0 warms up
@@ -543,16 +565,20 @@ int fl_batch_autotune(fl_batch* b, int reps, fl_tuning* chosen, void* stream) {
         if (!rc && total < best_ms) {
           best_ms = total;
           best = t;
-          best_cell = k < 0;
+          best_cell[ph] = k < 0;
         }
       }
     }
-    b->cell[ph] = best_cell;
   }
   (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  if (!rc) rc = apply_tuning(b, best);
-  if (!rc) launch_finish(b, st, 1);
+  if (e1) (void)hipEventDestroy(e1);
+  if (!rc) rc = apply_tuning(b, best, best_cell);
+  if (rc) {  // as before the call: the next step uploads the tables again
+    b->tuning = saved;
+    for (int ph = 0; ph < 2; ++ph) b->cell[ph] = saved_cell[ph];
+    b->tables_ok = false;
+  }
+  launch_finish(b, st, 1);
   if (!rc && chosen) *chosen = batch_tuning(b);
   return rc;
 }
@@ -562,6 +588,10 @@ int fl_batch_step(fl_batch* b, int64_t steps, int use_graph, void* stream) {
   if (steps < 0) return fail(FL_ERR_ARGUMENT, "steps < 0");
   DeviceGuard g(b->device);
   hipStream_t st = (hipStream_t)stream;
+  if (!b->tables_ok) {  // a call that was to change them failed
+    const int rc = apply_tuning(b, b->tuning, b->cell);
+    if (rc) return rc;
+  }
   if (!use_graph) {
     for (int64_t k = 0; k < steps; ++k) {
       int rc = launch_step(b, st);

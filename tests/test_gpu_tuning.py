@@ -125,3 +125,49 @@ def test_batch_zeros_keep_each_phase():
     assert _tuple(b.get_tuning()) == (64, 8, 64, 16)
     b.set_tuning()
     assert _tuple(b.get_tuning()) == (64, 8, 64, 16)
+
+
+def _hip():
+    for line in open("/proc/self/maps"):
+        if "libamdhip64.so" in line:
+            return C.CDLL(line.split()[-1])
+    raise RuntimeError("no HIP runtime in this process")
+
+
+def test_batch_survives_a_failed_autotune():
+    """While a stream captures in global mode the uploads of the autotuner are
+    refused: the call fails, and the steps after it are those of the tiles that
+    the batch had, its 1D problems (here after an odd step count) included."""
+    from fluidity_amd import batch as B
+    from fluidity_amd import euler as E
+    from fluidity_amd import native as N
+
+    def batch():
+        return B.Batch([{"U": _grid(s, 4), "scheme": E.Scheme(), "cfl": 0.8, "dh": 1.0 / s[-1]}
+                        for s in ((90, 130), (333,), (64, 64))], layout=1)
+    hip = _hip()
+    ref = batch()
+    ref.step(7)
+    for tuning in (None, dict(x_block=64, x_rows=8, y_block=64, y_rows=16)):
+        b = batch()
+        if tuning:
+            b.set_tuning(**tuning)
+        had = _tuple(b.get_tuning())
+        b.step(3)
+        torch.cuda.synchronize()
+        stream, graph = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+        assert hip.hipStreamBeginCapture(stream, 0) == 0
+        with pytest.raises(N.FluidityError):
+            b.autotune(reps=1)
+        hip.hipStreamEndCapture(stream, C.byref(graph))
+        if graph:
+            hip.hipGraphDestroy(graph)
+        hip.hipStreamDestroy(stream)
+        hip.hipGetLastError()
+        assert _tuple(b.get_tuning()) == had
+        b.step(4)
+        got, want = b.finish(), ref.finish()
+        for i in range(3):
+            assert torch.equal(b.state(i), ref.state(i))
+            assert (got[i].iters, got[i].run_time) == (want[i].iters, want[i].run_time) == (7, want[i].run_time)
