@@ -210,6 +210,8 @@ struct SweepShape {
 // the faster ones.
 template <typename T> constexpr int64_t kCellMax = 5 << 19;
 template <> constexpr int64_t kCellMax<float> = 5 << 20;
+// Cells up to which the autotuner tries them, and a caller's tuning gets them.
+constexpr int64_t kCellTryMax = 10 << 20;
 
 // Launch shape of the sweep of dimension dim over ngrids grids of nx x ny
 // cells.  By rule: small grids go cell-parallel (a 64^2 FP64 sweep takes 7 us
@@ -224,15 +226,20 @@ template <typename T>
 SweepShape pick_shape(const fl_context* ctx, int dim, int64_t nx, int64_t ny, int ngrids) {
   const fl_tuning& tu = ctx->tuning;
   const bool few = nx * ny * ngrids <= kCellMax<T>;
-  // kShapeCell was measured on one grid; two of them may be past the line, and
-  // then take the fastest marching shape of that measurement
-  if (ctx->shape[dim] == kShapeTuning ||
-      (ctx->shape[dim] == kShapeCell && ngrids > 1 && !few)) {
+  // kShapeCell holds for one grid up to the size that it was measured at (a
+  // 4096^2 sweep in the shapes tuned at 256^2: FP32 629 us cell-parallel, 535
+  // marching); past it, and for two grids past the line, the tuning's march is
+  // the fastest one of that measurement
+  const int64_t measured = ctx->cell_cells[dim];
+  const bool cell =
+      ctx->shape[dim] == kShapeCell &&
+      (few || (ngrids == 1 && nx * ny <= (measured ? measured : kCellTryMax)));
+  if (ctx->shape[dim] != kShapeRule && !cell) {
     const int B = dim ? tu.y_block : tu.x_block;
     const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
     return {false, B, fit_rows(dim ? tu.y_rows : tu.x_rows, ngrids * bands, ny, B)};
   }
-  if (ctx->shape[dim] == kShapeCell || few) return {true, 0, 0};
+  if (cell || few) return {true, 0, 0};
   const int B = dim ? 64 : 128;
   const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
   const int64_t waves = ngrids * bands * (B / 64) * ny;  // of one-row tiles
@@ -832,7 +839,11 @@ int fl_ctx_destroy(fl_context* c) {
 
 int fl_ctx_set_tuning(fl_context* c, const fl_tuning* t) {
   if (!c || !t) return fail(FL_ERR_ARGUMENT, "NULL context or tuning");
-  return take_tuning(t, &c->tuning, c->shape);
+  const int rc = take_tuning(t, &c->tuning, c->shape);
+  if (rc) return rc;
+  if (t->x_block || t->x_rows) c->cell_cells[0] = 0;
+  if (t->y_block || t->y_rows) c->cell_cells[1] = 0;
+  return FL_OK;
 }
 
 int fl_ctx_get_tuning(const fl_context* c, fl_tuning* t) {
@@ -860,6 +871,7 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
   FL_HIP(hipEventCreate(&e1));
   const fl_tuning saved = c->tuning;
   const int32_t saved_shape[2] = {c->shape[0], c->shape[1]};
+  const int64_t saved_cells[2] = {c->cell_cells[0], c->cell_cells[1]};
   fl_tuning best = c->tuning;
   // the sweep with the context's current shape: milliseconds over reps launches
   auto timed = [&](int dim, float* total) -> int {
@@ -907,23 +919,25 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
       }
     }
     // the cell-parallel kernel, on grids where it can be the faster one
-    if (in->ndim == 2 && !rc && in->n[0] * in->n[1] <= 2 * kCellMax<float>) {
+    if (in->ndim == 2 && !rc && in->n[0] * in->n[1] <= kCellTryMax) {
       float total = 0.0f;
       c->shape[dim] = kShapeCell;
+      c->cell_cells[dim] = in->n[0] * in->n[1];
       rc = timed(dim, &total);
       // the best of many marching shapes is a lucky one when they are about
       // equal, the more so where a sweep takes 20 us (512^2: 22 against 17 us
       // in the steps after it)
-      const bool by_rule = in->n[0] * in->n[1] <=
-                           (in->dtype == FL_F64 ? kCellMax<double> : kCellMax<float>);
-      if (!rc && total >= (by_rule ? 1.25f : 1.05f) * best_ms) c->shape[dim] = kShapeTuning;
+      const bool small = in->n[0] * in->n[1] <= (1 << 20);
+      if (!rc && total >= (small ? 1.25f : 1.05f) * best_ms) c->shape[dim] = kShapeTuning;
     }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   c->tuning = rc ? saved : best;
-  if (rc)
-    for (int d = 0; d < 2; ++d) c->shape[d] = saved_shape[d];
+  for (int d = 0; rc && d < 2; ++d) {
+    c->shape[d] = saved_shape[d];
+    c->cell_cells[d] = saved_cells[d];
+  }
   if (!rc && chosen) *chosen = tuning_of(c->tuning, c->shape);
   return rc;
 }
@@ -1140,7 +1154,10 @@ int fl_simulate(fl_context* c, fl_field* state, fl_field* work, const fl_scheme*
     key.sim_time = p->sim_time;
     key.max_iters = p->max_iters;
     key.tuning = c->tuning;
-    for (int d = 0; d < 2; ++d) key.shape[d] = c->shape[d];
+    for (int d = 0; d < 2; ++d) {
+      key.shape[d] = c->shape[d];
+      key.cell_cells[d] = c->cell_cells[d];
+    }
     const bool again = memcmp(&key, &c->sim_key, sizeof(key)) == 0;
     if (!again) {
       drop_sim_graphs(c);

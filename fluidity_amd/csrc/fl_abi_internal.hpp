@@ -29,6 +29,7 @@ struct SimGraphKey {
   int64_t max_iters;
   fl_tuning tuning;
   int32_t shape[2];
+  int64_t cell_cells[2];
 };
 
 // Where the launch shape of a 2D sweep (x, y) comes from: the built-in rule
@@ -51,6 +52,7 @@ struct fl_context {
   fl::ls::EikCtl* host_eik;    // pinned host mirror of eik
   fl_tuning tuning;
   int32_t shape[2];            // kShape* of the x and the y sweep
+  int64_t cell_cells[2];       // kShapeCell: cells of the grid it was measured on (0: none)
   hipEvent_t step_ev;          // fl_mm_simulate: the step's control block is on the host
   int64_t eik_sweeps;          // sweeps the last eikonal solve took (first batch size)
   int use_graphs;              // fl_simulate replays captured runs of steps
