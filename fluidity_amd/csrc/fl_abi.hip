@@ -206,26 +206,59 @@ struct SweepShape {
   int rows;   // rows per workgroup of the march
 };
 
-// Cells (of all grids of the launch) up to which the cell-parallel sweeps are
-// the faster ones.
-template <typename T> constexpr int64_t kCellMax = 5 << 19;
-template <> constexpr int64_t kCellMax<float> = 5 << 20;
+// Cells up to which the cell-parallel sweeps of one grid are the faster ones,
+// and of the two grids of a launch together.  A step, cell-parallel against a
+// round of marching tiles: FP64 exact 1200x1207 111 | 115 us, 1400^2 143 | 146,
+// 1500x1507 165 | 158, 2048^2 298 | 274; fast 1200x1207 88 | 88, 1500x1507 125 |
+// 118; FP32 1200x1207 61 | 61, 1400^2 77 | 76, 1500x1507 85 | 78, 2048^2 141 |
+// 117.  (Two grids march at two waves per SIMD in FP64: their line is farther.)
+constexpr int64_t kCellMax = 7 << 18;
+template <typename T> constexpr int64_t kCellMaxTwo = 5 << 19;
+template <> constexpr int64_t kCellMaxTwo<float> = 5 << 20;
 // Cells up to which the autotuner tries them, and a caller's tuning gets them.
 constexpr int64_t kCellTryMax = 10 << 20;
 
+// Marching shape of a sweep by rule: tiles of one height that fill whole rounds
+// of the workgroups that the device holds at once (`waves` per SIMD of 1024),
+// so that the launch ends evenly, as tall as one round makes them but at most
+// kRoundRows (6 warm-up rows in x, 8 in y come on top).  256 lanes, fewer where
+// the columns leave a tenth of them idle.  Fixed numbers of waves (about 10500
+// in x, 4096 in y) ended with a nearly empty round at some sizes: 1700x1707
+// FP64 exact 212 us a step, in one round 197, FORCE in the fast numerics 156 and
+// 124, FP32 124 and 91; 2600^2 421 and 434, FP32 200 and 169; 4096^2 fast 714 and
+// 699, FP32 417 and 395.  Short wide grids need the wide workgroups for their
+// number too: the atomics of the CFL maximum (10 ns each, one after the other)
+// of 31250 workgroups of 64 lanes outlast the y sweep of 2000000 x 5 cells
+// (FP32, 566 us a step against 313).
+constexpr int64_t kRoundRows = 96;
+SweepShape round_shape(int dim, int64_t nx, int64_t ny, int ngrids, int waves) {
+  SweepShape best{false, 0, 0};
+  double best_cost = 0.0;
+  for (int B : {256, 128, 64}) {
+    const int64_t cap = (int64_t)1024 * waves / (B / 64);
+    const int64_t bands = ngrids * (dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2));
+    const int64_t least = (bands * ((ny + kRoundRows - 1) / kRoundRows) + cap - 1) / cap;
+    for (int64_t r = least; r < least + 4; ++r) {
+      const int64_t tiles = std::min(r * cap / bands, std::min<int64_t>(ny, 65535));
+      const int64_t rows = (ny + tiles - 1) / tiles;
+      const int64_t rounds = (bands * ((ny + rows - 1) / rows) + cap - 1) / cap;
+      const double cost = (double)(rounds * (rows + (dim ? 8 : 6)));
+      if (!best.block || cost < (B < best.block ? 0.9 : 1.0) * best_cost) {
+        best = {false, B, (int)rows};
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
 // Launch shape of the sweep of dimension dim over ngrids grids of nx x ny
-// cells.  By rule: small grids go cell-parallel (a 64^2 FP64 sweep takes 7 us
-// against 16 (x) and 21 us (y) marching; a step of 1024^2 101 against 124,
-// 3861x515 161 against 176, 2048^2 312 against 284; FP32 3861x515 82 against
-// 117, 2048^2 146 against 159, 4096^2 544 against 419: the line is where the
-// two cross).  Larger ones march, x in 128-lane workgroups of
-// about 10500 waves and y in 64-lane ones of about 4096 in all: fewer, taller
-// tiles end unevenly, shorter ones pay more warm-up rows (FP64 x at 2048^2: 8
-// rows 133 us, 32 rows 186 us; y at 4096^2: 64 rows 441 us, 22 rows 455 us).
+// cells.  By rule small grids go cell-parallel (a 64^2 FP64 sweep takes 7 us
+// against 16 (x) and 21 us (y) marching) and larger ones march.
 template <typename T>
 SweepShape pick_shape(const fl_context* ctx, int dim, int64_t nx, int64_t ny, int ngrids) {
   const fl_tuning& tu = ctx->tuning;
-  const bool few = nx * ny * ngrids <= kCellMax<T>;
+  const bool few = nx * ny * ngrids <= (ngrids > 1 ? kCellMaxTwo<T> : kCellMax);
   // kShapeCell holds for one grid up to the size that it was measured at (a
   // 4096^2 sweep in the shapes tuned at 256^2: FP32 629 us cell-parallel, 535
   // marching); past it, and for two grids past the line, the tuning's march is
@@ -240,13 +273,7 @@ SweepShape pick_shape(const fl_context* ctx, int dim, int64_t nx, int64_t ny, in
     return {false, B, fit_rows(dim ? tu.y_rows : tu.x_rows, ngrids * bands, ny, B)};
   }
   if (cell || few) return {true, 0, 0};
-  const int B = dim ? 64 : 128;
-  const int64_t bands = dim ? (nx + B - 1) / B : (nx + B - 3) / (B - 2);
-  const int64_t waves = ngrids * bands * (B / 64) * ny;  // of one-row tiles
-  const int64_t fit = dim ? (waves + 4095) / 4096 : (waves + 10499) / 10500;
-  int64_t rows = std::max<int64_t>(dim ? 8 : 6, std::min<int64_t>(dim ? 64 : 32, fit));
-  rows = std::max(rows, (ny + 65534) / 65535);  // tile rows are the launch's y extent
-  return {false, B, (int)rows};
+  return round_shape(dim, nx, ny, ngrids, sizeof(T) == 4 ? 4 : ngrids > 1 ? 2 : 3);
 }
 
 // Workgroups of a sweep: the marching tiles over (x, y), or the cell-parallel
