@@ -60,7 +60,9 @@ int64_t grid_bytes(const fl_field* f) { return cells_of(f) * (2 + f->ndim) * 8; 
 // Workgroups of the adjoint of the sweep along dimension d.
 int64_t sweep_blocks(const fl_field* f, int d) {
   const int64_t nx = f->n[0], ny = f->ndim > 1 ? f->n[1] : 1;
-  return ceil_div(d ? ny : nx, aj::kAdjCells) * ceil_div(d ? nx : ny, aj::kAdjWaves);
+  const int64_t segs = ceil_div(d ? ny : nx, aj::kAdjCells);
+  if (f->ndim == 1) return ceil_div(segs, aj::kAdjWaves);
+  return segs * ceil_div(d ? nx : ny, aj::kAdjWaves);
 }
 
 // Scratch of the backward pass for segments of K steps.

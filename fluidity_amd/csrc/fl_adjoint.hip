@@ -202,8 +202,11 @@ __device__ void chi_record(const AGrid& g, const double* __restrict__ P,
 // With a thread per face, which evolved both cells beside it forward and back
 // and passed its 16 contributions through memory to a kernel that gathered
 // them, it took 33 us, the gather 9, the sums 5 and the flattening factors'
-// records 4; now 25 us (x) and 29 (y) in all.  In the y sweep a wave's lanes run down a column: its loads touch a
-// line each, which the columns of a workgroup share.
+// records 4; now 25 us (x) and 29 (y) in all.  In the y sweep a wave's lanes run
+// down a column: its loads touch a line each, which the columns of a workgroup
+// share.  The waves of a workgroup take neighbouring lines, on a 1D grid
+// neighbouring segments (four steps back on 200000 cells 426 us with one wave
+// of four at work, 344 now).
 //
 // rec_k, rec_v and any receive the records of the flattening factors
 // (chi_record) at the positions of the grid's lines, partials the workgroup's
@@ -226,11 +229,12 @@ sweep_adj_kernel(AGrid g, const double* __restrict__ lam, double* __restrict__ l
   const int64_t total = gridDim.x, xcd = blockIdx.x % 8;
   const int64_t tile = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
   const int64_t groups = (lines + kAdjWaves - 1) / kAdjWaves;
-  const int64_t seg = tile / groups;
   const int t = (int)(threadIdx.x & 63);
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t line_of = (tile % groups) * kAdjWaves + w;
-  const bool live = line_of < lines;               // uniform over the wave
+  // a workgroup's waves take neighbouring lines, or segments of the only one
+  const int64_t seg = ND == 1 ? tile * kAdjWaves + w : tile / groups;
+  const int64_t line_of = ND == 1 ? 0 : (tile % groups) * kAdjWaves + w;
+  const bool live = ND == 1 ? seg * kAdjCells < n : line_of < lines;  // uniform over the wave
   const int64_t line = live ? line_of : lines - 1;
   const int64_t j = seg * kAdjCells - kAdjHalo + t;  // this lane's position
   // the cell it names, and whether it is one of the grid
