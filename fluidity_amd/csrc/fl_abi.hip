@@ -1140,7 +1140,7 @@ int fl_simulate(fl_context* c, fl_field* state, fl_field* work, const fl_scheme*
   DeviceGuard g(c->device);
   hipStream_t st = (hipStream_t)stream;
 
-  if (c->use_graphs) {
+  if (c->use_graphs && p->max_iters > 0) {  // (no step: its launch alone is 20 us more)
     const PersistShape sh = persist_shape(state, s);
     if (sh.groups > 0) {
       if (state->dtype == FL_F64)
