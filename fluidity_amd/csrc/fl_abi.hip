@@ -901,12 +901,17 @@ int fl_ctx_autotune(fl_context* c, const fl_field* in, const fl_field* work,
   const int64_t saved_cells[2] = {c->cell_cells[0], c->cell_cells[1]};
   fl_tuning best = c->tuning;
   // the sweep with the context's current shape: milliseconds over reps launches
+  // (on a line with the maximum that its steps reduce: 200000 cells are 3226
+  // workgroups of 64 lanes, whose atomics are most of the 58 us of a step, in
+  // 256 lanes 32)
   auto timed = [&](int dim, float* total) -> int {
     int err = FL_OK;
     *total = 0.0f;
     for (int r = 0; r <= reps && !err; ++r) {  // r = 0 warms up
       if (hipEventRecord(e0, st) != hipSuccess) err = fail(FL_ERR_HIP, "hipEventRecord");
-      if (!err) err = launch_sweep(c, in, work, dim, s, 1e-3, nullptr, nullptr, st);
+      if (!err)
+        err = launch_sweep(c, in, work, dim, s, 1e-3, nullptr, in->ndim == 1 ? c->ws_tmp : nullptr,
+                           st);
       if (!err && hipEventRecord(e1, st) != hipSuccess) err = fail(FL_ERR_HIP, "hipEventRecord");
       if (!err && hipEventSynchronize(e1) != hipSuccess) err = fail(FL_ERR_HIP, "hipEventSynchronize");
       float ms = 0.0f;

@@ -205,8 +205,8 @@ __device__ void chi_record(const AGrid& g, const double* __restrict__ P,
 // records 4; now 25 us (x) and 29 (y) in all.  In the y sweep a wave's lanes run
 // down a column: its loads touch a line each, which the columns of a workgroup
 // share.  The waves of a workgroup take neighbouring lines, on a 1D grid
-// neighbouring segments (four steps back on 200000 cells 426 us with one wave
-// of four at work, 344 now).
+// neighbouring segments (four steps on 200000 cells and back, each recomputed
+// in 64 lanes: 522 us with one wave of four at work, 392 with all).
 //
 // rec_k, rec_v and any receive the records of the flattening factors
 // (chi_record) at the positions of the grid's lines, partials the workgroup's
