@@ -179,12 +179,26 @@ const void* phase_kernel_ptr(const fl_batch* b, int phase) {
 // tall.  The two lines cross at 19M cells in FP64, 17M in FP32.
 constexpr int64_t kBatchCellMax = 1 << 24;
 
-// The rule: whether a batch that was not tuned runs cell-parallel tiles.
-bool cell_by_rule(const fl_batch* b) {
-  int64_t cells = 0;
+// FP32 lines of these many cells in all march: their arithmetic is short, and
+// 56 of a wave's 64 lanes hold cells of a register tile, 254 of 256 of a
+// marching one.  A step of lines of 65536 cells, marching against register
+// tiles, FP32 (FP64 exact): 2.1M cells 56 | 53 us (88 | 75), 4.2M 75 | 85 (137 |
+// 127), 8.4M 119 | 161 (252 | 266); of 10^6 cells 8M 105 | 128 (258 | 247), 16M
+// 219 | 266 (459 | 469); four of 8M cells 727 | 470.
+constexpr int64_t kBatchMarchLines[2] = {3 << 20, 20 << 20};
+
+// The rule: whether a phase of a batch that was not tuned runs cell-parallel tiles.
+bool cell_by_rule(const fl_batch* b, int phase) {
+  int64_t planes = 0, lines = 0;
   for (const fl_batch_problem& q : b->problems)
-    if (q.state.ndim > 1) cells += q.state.n[0] * q.state.n[1];
-  return cells <= kBatchCellMax;
+    if (q.state.ndim > 1) planes += q.state.n[0] * q.state.n[1];
+    else lines += q.state.n[0];
+  // lines and planes share a phase: its kind is that of the lines where they
+  // are nearly all of it
+  if (phase == 0 && b->dtype == FL_F32 && lines > kBatchMarchLines[0] &&
+      lines <= kBatchMarchLines[1] && 8 * planes <= lines)
+    return false;
+  return planes <= kBatchCellMax;
 }
 
 // What the batch runs, as a caller's tuning.
@@ -463,7 +477,7 @@ int fl_batch_create(fl_context* c, const fl_batch_problem* problems, int nprob, 
     hp[p].max_iters = problems[p].params.max_iters;
   }
   const fl_tuning t = {256, 32, 256, 64};
-  const bool cell[2] = {cell_by_rule(b), cell_by_rule(b)};
+  const bool cell[2] = {cell_by_rule(b, 0), cell_by_rule(b, 1)};
   int rc = FL_OK;
   e = hipMemcpy(b->params, hp.data(), sizeof(bt::Params) * nprob, hipMemcpyHostToDevice);
   if (e != hipSuccess) rc = fail(FL_ERR_HIP, "hipMemcpy failed: %s", hipGetErrorString(e));
@@ -497,7 +511,7 @@ int fl_batch_set_tuning(fl_batch* b, const fl_tuning* t) {
   FL_HIP(hipDeviceSynchronize());  // tables in use by queued steps
   bool cell[2];
   for (int ph = 0; ph < 2; ++ph)
-    cell[ph] = shape[ph] == kShapeCell || (shape[ph] == kShapeRule && cell_by_rule(b));
+    cell[ph] = shape[ph] == kShapeCell || (shape[ph] == kShapeRule && cell_by_rule(b, ph));
   return apply_tuning(b, n, cell);
 }
 

@@ -171,3 +171,25 @@ def test_batch_survives_a_failed_autotune():
         for i in range(3):
             assert torch.equal(b.state(i), ref.state(i))
             assert (got[i].iters, got[i].run_time) == (want[i].iters, want[i].run_time) == (7, want[i].run_time)
+
+
+def test_batch_of_many_fp32_cells_on_lines_marches():
+    """The rule of the lines, and its marching tiles against the register tiles
+    of a caller's tuning, bit for bit."""
+    from fluidity_amd import batch as B
+    from fluidity_amd import euler as E
+    shapes = [(65536 - 13 * i,) for i in range(56)] + [(40, 60)]
+    assert 3 << 20 < sum(s[0] for s in shapes[:-1])
+
+    def batch(dtype):
+        r = np.random.default_rng(3)
+        return B.Batch([{"U": (_grid(s, 4) * (1.0 + 0.01 * r.random())).to(dtype),
+                         "scheme": E.Scheme(), "cfl": 0.8, "dh": 1.0 / s[-1]} for s in shapes], layout=1)
+    b, c = batch(torch.float32), batch(torch.float32)
+    assert b.get_tuning().x_rows > 0 and b.get_tuning().y_rows < 0
+    c.set_tuning(x_rows=-32)
+    for x in (b, c):
+        x.step(3)
+        x.finish()
+    assert all(torch.equal(b.state(i), c.state(i)) for i in range(len(shapes)))
+    assert batch(torch.float64).get_tuning().x_rows < 0
