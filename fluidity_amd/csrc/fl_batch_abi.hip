@@ -177,7 +177,16 @@ const void* phase_kernel_ptr(const fl_batch* b, int phase) {
 // The marching tiles of a few large planes are too few to fill the device,
 // and short ones pay their warm-up rows; past the limit they are many and
 // tall.  The two lines cross at 19M cells in FP64, 17M in FP32.
+// Beyond them, planes that make fewer than kBatchFewTiles marching tiles leave
+// CUs without one and go cell-parallel too: 4 planes of 2200^2, 324 tiles, fast
+// FP64 1650 against 1040 us, FP32 1080 against 650; 8 of 2200^2, 648 tiles, 2170
+// against 2010 and 1370 against 1216; 6 of 1900^2, 720 tiles, 1059 against 1130
+// and 745 against 711.
 constexpr int64_t kBatchCellMax = 1 << 24;
+constexpr int64_t kBatchFewTiles = 700;
+
+// Marching tiles of a batch that was not tuned.
+constexpr fl_tuning kMarch = {256, 32, 256, 64};
 
 // FP32 lines of these many cells in all march: their arithmetic is short, and
 // 56 of a wave's 64 lanes hold cells of a register tile, 254 of 256 of a
@@ -189,16 +198,22 @@ constexpr int64_t kBatchMarchLines[2] = {3 << 20, 20 << 20};
 
 // The rule: whether a phase of a batch that was not tuned runs cell-parallel tiles.
 bool cell_by_rule(const fl_batch* b, int phase) {
-  int64_t planes = 0, lines = 0;
-  for (const fl_batch_problem& q : b->problems)
-    if (q.state.ndim > 1) planes += q.state.n[0] * q.state.n[1];
-    else lines += q.state.n[0];
+  int64_t planes = 0, lines = 0, tiles = 0;
+  for (const fl_batch_problem& q : b->problems) {
+    if (q.state.ndim == 1) {
+      lines += q.state.n[0];
+      continue;
+    }
+    const int64_t nx = q.state.n[0], ny = q.state.n[1];
+    planes += nx * ny;
+    tiles += ceil_div(nx, kMarch.x_block - 2) * ceil_div(ny, tile_rows(ny, kMarch.x_rows));
+  }
   // lines and planes share a phase: its kind is that of the lines where they
   // are nearly all of it
   if (phase == 0 && b->dtype == FL_F32 && lines > kBatchMarchLines[0] &&
       lines <= kBatchMarchLines[1] && 8 * planes <= lines)
     return false;
-  return planes <= kBatchCellMax;
+  return planes <= kBatchCellMax || tiles < kBatchFewTiles;
 }
 
 // What the batch runs, as a caller's tuning.
@@ -476,7 +491,7 @@ int fl_batch_create(fl_context* c, const fl_batch_problem* problems, int nprob, 
     hp[p].sim_time = problems[p].params.sim_time;
     hp[p].max_iters = problems[p].params.max_iters;
   }
-  const fl_tuning t = {256, 32, 256, 64};
+  const fl_tuning t = kMarch;
   const bool cell[2] = {cell_by_rule(b, 0), cell_by_rule(b, 1)};
   int rc = FL_OK;
   e = hipMemcpy(b->params, hp.data(), sizeof(bt::Params) * nprob, hipMemcpyHostToDevice);

@@ -314,8 +314,9 @@ int fl_batch_create(fl_context* ctx, const fl_batch_problem* problems, int nprob
 int fl_batch_destroy(fl_batch* batch);
 /* Tiles of the two sweep phases: marching tiles of the given shapes
  * (x_block/x_rows: x tiles of 2D problems, x_block also the width of 1D tiles;
- * y_block/y_rows: y tiles), or with negative rows cell-parallel tiles, which a
- * batch of up to 2^24 2D cells has from the start (FL_ROWS_RULE). */
+ * y_block/y_rows: y tiles), or with negative rows cell-parallel tiles.
+ * FL_ROWS_RULE, as from the start: cell-parallel tiles for batches of up to
+ * 2^24 2D cells or of a few large planes. */
 int fl_batch_set_tuning(fl_batch* batch, const fl_tuning* tuning);
 /* What is set, as fl_batch_set_tuning takes it (negative rows: cell-parallel
  * tiles). */
