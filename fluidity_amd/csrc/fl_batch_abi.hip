@@ -582,7 +582,8 @@ int fl_batch_autotune(fl_batch* b, int reps, fl_tuning* chosen, void* stream) {
         if (b->ntiles[ph] == 0) break;
         float total = 0.0f;
         for (int r = 0; r <= reps && !rc; ++r) {  // r = 0 warms up
-          hipLaunchKernelGGL(bt::reset_counters_kernel, dim3(1), dim3(1), 0, st, b->cnt);
+          hipLaunchKernelGGL(bt::reset_counters_kernel, dim3((unsigned)ceil_div(b->nprob, 256)),
+                             dim3(256), 0, st, b->ctls, b->nprob, b->cnt);
           if (hipEventRecord(e0, st) != hipSuccess) rc = fail(FL_ERR_HIP, "hipEventRecord");
           launch_phases(b, st, 1, dtdh, ph);
           if (hipEventRecord(e1, st) != hipSuccess) rc = fail(FL_ERR_HIP, "hipEventRecord");
