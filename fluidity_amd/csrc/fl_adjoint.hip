@@ -195,14 +195,15 @@ __device__ void chi_record(const AGrid& g, const double* __restrict__ P,
 // PRIM: primitive-form limiting (a template parameter, so that the
 // conservative-form kernel carries none of its code).
 //
-// FP64 arithmetic and its latency at two waves a SIMD bound it (182 registers
-// and more; a 512^2 sweep at three a SIMD 26 us in x and 32 in y, at four, with
-// spills, 38 and 44; workgroups of 8 waves 30 and 36, whose last round is a
-// quarter full).
+// FP64 arithmetic and its latency at two waves a SIMD bound it (2D: HLLC 182
+// registers, FORCE 242, with primitive-form limiting 220 and 256, the latter
+// with 28 to 30 spilled; HLLC at 512^2 at three a SIMD 26 us in x and 32 in y, at
+// four, with spills, 38 and 44; workgroups of 8 waves 30 and 36, whose last round
+// is a quarter full).
 // With a thread per face, which evolved both cells beside it forward and back
 // and passed its 16 contributions through memory to a kernel that gathered
 // them, it took 33 us, the gather 9, the sums 5 and the flattening factors'
-// records 4; now 25 us (x) and 29 (y) in all.  In the y sweep a wave's lanes run
+// records 4; now 24 us (x) and 28 (y) in all.  In the y sweep a wave's lanes run
 // down a column: its loads touch a line each, which the columns of a workgroup
 // share.  The waves of a workgroup take neighbouring lines, on a 1D grid
 // neighbouring segments (four steps on 200000 cells and back, each recomputed

@@ -16,8 +16,8 @@
 // all and the neighbours' cells then start the step.  A word is its own flag,
 // so a step costs one store and one load through device memory; a barrier
 // (atomic counter between release and acquire fences, then the loads of the
-// state) cost three to four.  A step in FP64 HLLC: 100 cells 6.1 -> 2.5 us,
-// 4096 cells 7.3 -> 4.8, 14000 cells 13.3 -> 5.4, 65536 cells 83 -> 8 (the
+// state) cost three to four.  A step in FP64 HLLC: 100 cells 6.1 -> 2.3 us,
+// 4096 cells 7.3 -> 4.6, 14000 cells 13.3 -> 5.1, 65536 cells 83 -> 6.6 (the
 // barrier's counter took one atomic of 1058 workgroups).  Words go to
 // the slots k % 3 in turn.  In step k, after its polls, a workgroup empties
 // its words of slot (k + 2) % 3, which holds the publication of step k - 1:
